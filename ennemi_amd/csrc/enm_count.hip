@@ -15,20 +15,14 @@
 // mode (including ENM_F_BRUTE, which only removes window pruning) 1-D counts
 // use this search.
 //
-// Multi-D spaces: on a grid order (the space's first two columns are the
-// order's columns 0 and 1) a wave takes 64 queries of one strip and scans its
-// own strip and the strips outward, each within the y window of the tile
-// widened by the wave's largest radius, in FP64 (count_grid); with two
-// columns, a strip whose whole key range lies within a lane's radius is
-// counted for that lane by binary searches of its y column.  Otherwise the
-// wave bounds the union of its 64 balls on the key axis and scans that window
-// of the key-sorted order with wave-uniform candidate loads; in FP32-filter
-// mode each lane counts candidates whose FP32 distance is <= the radius
-// rounded down minus the guard (certainly inside) and <= the radius rounded
-// up plus the guard (possibly inside), and if any lane saw a candidate in
-// between the wave rescans its window and settles those in FP64.  (On this
-// ISA FP32 and FP64 compares issue at the same rate, so the grid path counts
-// in FP64 directly: the band bookkeeping would cost more than it saves.)
+// Multi-D spaces are counted on box trees (enm_tree.hip).  The kernel here
+// serves brute force and tunings without strips: a wave bounds the union of
+// its 64 balls on the key axis and scans that window of the key-sorted order
+// with wave-uniform candidate loads; in FP32-filter mode each lane counts
+// candidates whose FP32 distance is <= the radius rounded down minus the guard
+// (certainly inside) and <= the radius rounded up plus the guard (possibly
+// inside), and if any lane saw a candidate in between the wave rescans its
+// window and settles those in FP64.
 //
 // psi(n_i) comes from a table filled once per launch (psi_tab[c], +inf for
 // c = 0: psi(0) = +inf in the reference, :338-339).  Multi-D spaces write it
@@ -254,7 +248,7 @@ void count1d_kernel(CountArgs A, const double* __restrict__ col64, const double*
         queries += (unsigned long long)(it.t1 - it.t0);
         __syncthreads();  // the window is reloaded by the next item
     });
-    if (tid == 0) atomicAdd(stats + ST_CNT_1D, queries);
+    if (tid == 0) add_stat(stats, ST_CNT_1D, queries);
 }
 
 // Deferred 1-D queries: one per thread over all segments at once (entry e
@@ -358,181 +352,11 @@ __global__ void psi_table_kernel(double* __restrict__ tab, int64_t n) {
     if (c <= n) tab[c] = c == 0 ? INFINITY : enm_psi((double)c);
 }
 
-// Count of candidates j in [a, b) with max_d fl64(|c_d[j] - q_d|) <= r, for
-// one lane (wave-uniform candidate range).
-template <int D>
-__device__ __forceinline__ int count_range64(const double* const (&c64)[D], const double (&q64)[D],
-                                             double r, int a, int b) {
-    int cnt = 0;
-    int j = a;
-    for (; j + CH <= b; j += CH) {
-#pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            double m = fabs(c64[0][j + c] - q64[0]);
-#pragma unroll
-            for (int d = 1; d < D; ++d) m = fmax(m, fabs(c64[d][j + c] - q64[d]));
-            cnt += (m <= r);
-        }
-    }
-    for (; j < b; ++j) {
-        double m = fabs(c64[0][j] - q64[0]);
-#pragma unroll
-        for (int d = 1; d < D; ++d) m = fmax(m, fabs(c64[d][j] - q64[d]));
-        cnt += (m <= r);
-    }
-    return cnt;
-}
-
-// count_range64 for three or more columns, candidates through LDS: the wave
-// loads 64 candidates at a time, one per lane (coalesced per column, the
-// next 64 in flight meanwhile), into `stage` (D x 64 doubles), and every
-// lane reads them back with broadcast LDS reads.  [a, b) is wave-uniform.
-template <int D>
-__device__ __forceinline__ int count_range_staged(const double* const (&c64)[D], const double (&q64)[D],
-                                                  double r, int a, int b, double* __restrict__ stage) {
-    const int lane = (int)(threadIdx.x & (ENM_WAVE - 1));
-    int cnt = 0;
-    double nx[D];
-    auto fetch = [&](int j0) {
-        const int p = j0 + lane;
-        const bool ok = p < b;
-#pragma unroll
-        for (int d = 0; d < D; ++d) nx[d] = ok ? c64[d][p] : 0.0;
-    };
-    if (a < b) fetch(a);
-    for (int j = a; j < b; j += ENM_WAVE) {
-        __syncthreads();   // every lane has read the previous block
-#pragma unroll
-        for (int d = 0; d < D; ++d) stage[d * ENM_WAVE + lane] = nx[d];
-        __syncthreads();
-        const int m = min(ENM_WAVE, b - j);
-        if (j + ENM_WAVE < b) fetch(j + ENM_WAVE);
-        int c = 0;
-        for (; c + CH <= m; c += CH) {
-#pragma unroll
-            for (int u = 0; u < CH; ++u) {
-                double e = fabs(stage[c + u] - q64[0]);
-#pragma unroll
-                for (int d = 1; d < D; ++d) e = fmax(e, fabs(stage[d * ENM_WAVE + c + u] - q64[d]));
-                cnt += (e <= r);
-            }
-        }
-        for (; c < m; ++c) {
-            double e = fabs(stage[c] - q64[0]);
-#pragma unroll
-            for (int d = 1; d < D; ++d) e = fmax(e, fabs(stage[d * ENM_WAVE + c] - q64[d]));
-            cnt += (e <= r);
-        }
-    }
-    return cnt;
-}
-
-// Number of positions j in [a, b) of an ascending column with
-// fl64(|y_j - q|) <= r (r >= 0), for one lane: fl64(y - q) is monotone in y,
-// so they are the run from the first j with fl64(y_j - q) >= -r to the first
-// with fl64(y_j - q) > r, found by two binary searches run together (their
-// loads are independent).  [a, b) must hold every such j.
-__device__ __forceinline__ int count_sorted(const double* __restrict__ y, int a, int b, double q, double r) {
-    int l0 = a, n0 = b - a;   // first j with fl(y_j - q) >= -r
-    int l1 = a, n1 = b - a;   // first j with fl(y_j - q) > r
-    while (n0 > 0 || n1 > 0) {
-        const int h0 = n0 >> 1, h1 = n1 >> 1;
-        // Both reads every round (a finished search rereads a position of
-        // the range), issued together ahead of the branches that use them.
-        double v0 = y[min(l0 + h0, b - 1)], v1 = y[min(l1 + h1, b - 1)];
-        pin(v0);
-        pin(v1);
-        if (n0 > 0) {
-            if (v0 - q >= -r) n0 = h0;
-            else { l0 += h0 + 1; n0 -= h0 + 1; }
-        }
-        if (n1 > 0) {
-            if (v1 - q > r) n1 = h1;
-            else { l1 += h1 + 1; n1 -= h1 + 1; }
-        }
-    }
-    return l1 - l0;
-}
-
-// Grid count: the tile's own strip and then strips outward, each within the
-// union of the y intervals [y_i - r_i, y_i + r_i] of the lanes that can
-// reach it (strip_window).  A side stops at the first strip whose column-0
-// bound is more than every live lane's radius away (strictly: a count
-// includes distance == r), and all strips beyond it are further still.
-// With two columns, a lane whose ball covers a strip's whole column-0 range
-// (both end keys within r: fl64(x_j - x_i) is monotone in x_j) counts that
-// strip as a run of its y column, by two binary searches inside the window
-// of such lanes, instead of scanning; the other lanes scan theirs.
-// Returns candidates scanned.
-template <int D>
-__device__ int count_grid(const CountDev& cd, const double* __restrict__ col64,
-                          const double* const (&c64)[D], const double (&q64)[D], double r, bool live,
-                          int lo, int hi, int t0, int t1, int& cnt, double* stage) {
-    const int S = cd.strip;
-    const double* xk = col64 + cd.base_key;
-    const double* yc = c64[1];
-    const int s = (t0 - lo) / S;
-    const int nstrip = (hi - lo + S - 1) / S;
-    if (!wave_any(live)) return 0;
-    int visited = 0;
-    // Strip [ks, ke) for the lanes in `need`.
-    auto visit = [&](int ks, int ke, bool need) {
-        int a, b;
-        if constexpr (D == 2) {
-            const bool inner = need && fabs(xk[ks] - q64[0]) <= r && fabs(xk[ke - 1] - q64[0]) <= r;
-            const bool edge = need && !inner;
-            if (wave_any(inner)) {
-                strip_window(yc, ks, ke, q64[1], r, inner, a, b);
-                if (inner) cnt += count_sorted(yc, a, b, q64[1], r);
-            }
-            if (wave_any(edge)) {
-                strip_window(yc, ks, ke, q64[1], r, edge, a, b);
-                const int c = count_range64<D>(c64, q64, r, a, b);
-                if (!inner) cnt += c;   // lanes outside `need` find no candidate here
-                visited += b - a;
-            }
-        } else {
-            strip_window(yc, ks, ke, q64[1], r, need, a, b);
-            cnt += count_range_staged<D>(c64, q64, r, a, b, stage);
-            visited += b - a;
-        }
-    };
-    visit(lo + s * S, min(hi, lo + s * S + S), live);
-    bool ldone = s == 0, rdone = s == nstrip - 1;
-    for (int d = 1; !(ldone && rdone); ++d) {
-        if (!ldone) {
-            const int sl = s - d;
-            if (sl < 0) {
-                ldone = true;
-            } else {
-                const int le = lo + (sl + 1) * S;
-                const double xb = xk[le - 1];
-                const bool need = live && !(q64[0] - xb > r);
-                ldone = !wave_any(need);
-                if (!ldone) visit(le - S, le, need);
-            }
-        }
-        if (!rdone) {
-            const int sr = s + d;
-            if (sr >= nstrip) {
-                rdone = true;
-            } else {
-                const int rs = lo + sr * S;
-                const double xb = xk[rs];
-                const bool need = live && !(xb - q64[0] > r);
-                rdone = !wave_any(need);
-                if (!rdone) visit(rs, min(hi, rs + S), need);
-            }
-        }
-    }
-    return visited;
-}
-
 template <int D, bool F32>
 __device__ void countnd_item(const CountArgs& A, const Item& it, const CountDev& cd,
                              const double* __restrict__ col64, const float* __restrict__ col32,
                              double* __restrict__ res64, int* __restrict__ res32,
-                             unsigned long long& pairs, unsigned long long& rechecks, double* stage) {
+                             unsigned long long& pairs, unsigned long long& rechecks) {
     const OrderDev od = A.orders[cd.order];
     const int64_t n = od.n;
     const int i = it.t0 + (int)threadIdx.x;
@@ -555,16 +379,6 @@ __device__ void countnd_item(const CountArgs& A, const Item& it, const CountDev&
     double r = active ? query_radius(cd, A, res64, i) : -1.0;
     const bool live = active && !(r < 0.0);
     if (!live) r = -INFINITY;
-
-    if constexpr (D >= 2) {
-        if (cd.strip > 0) {
-            int cnt = 0;
-            const int visited = count_grid<D>(cd, col64, c64, q64, r, live, it.lo, it.hi, it.t0, it.t1, cnt, stage);
-            finish_item(cd, it, active, cnt, res32, res64, i, A.perm, A.psi_tab);
-            pairs += (unsigned long long)(it.t1 - it.t0) * (unsigned long long)visited;
-            return;
-        }
-    }
 
     // Window on the key axis (a superset of every live lane's ball).
     int w0 = it.lo, w1 = it.hi;
@@ -650,7 +464,6 @@ void countnd_kernel(CountArgs A, const double* __restrict__ col64, const float* 
                     unsigned long long* __restrict__ stats) {
     // Counters accumulate per wave and go out once (see knn_kernel).
     unsigned long long pairs = 0, rechecks = 0;
-    __shared__ double stage[D >= 3 ? D * ENM_WAVE : 1];   // grid candidates of three or more columns
     for_each_wave_item(A.qoff, A.counter, A.chunk, [&](int idx) {
         Item it = A.items[idx];
         it.desc = uni(it.desc); it.tile = uni(it.tile);
@@ -659,15 +472,15 @@ void countnd_kernel(CountArgs A, const double* __restrict__ col64, const float* 
         if (F32) {
             bool ok = true;
             (void)enm_guard(A.maxabs[A.orders[cd.order].inst], &ok);
-            if (ok) countnd_item<D, true>(A, it, cd, col64, col32, res64, res32, pairs, rechecks, stage);
-            else    countnd_item<D, false>(A, it, cd, col64, col32, res64, res32, pairs, rechecks, stage);
+            if (ok) countnd_item<D, true>(A, it, cd, col64, col32, res64, res32, pairs, rechecks);
+            else    countnd_item<D, false>(A, it, cd, col64, col32, res64, res32, pairs, rechecks);
         } else {
-            countnd_item<D, false>(A, it, cd, col64, col32, res64, res32, pairs, rechecks, stage);
+            countnd_item<D, false>(A, it, cd, col64, col32, res64, res32, pairs, rechecks);
         }
     });
     if (threadIdx.x == 0) {
-        atomicAdd(stats + ST_CNT_PAIRS, pairs);
-        if (F32) atomicAdd(stats + ST_CNT_RECHECK, rechecks);
+        add_stat(stats, ST_CNT_PAIRS, pairs);
+        if (F32) add_stat(stats, ST_CNT_RECHECK, rechecks);
     }
 }
 

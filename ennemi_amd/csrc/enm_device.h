@@ -127,6 +127,11 @@ __device__ __forceinline__ void list_insert(double (&L)[P], double v) {
     L[0] = vmin(L[0], v);
 }
 
+// Adds to work counter s, in the copy of this workgroup.
+__device__ __forceinline__ void add_stat(unsigned long long* stats, int s, unsigned long long v) {
+    atomicAdd(stats + (s * ENM_ST_COPIES + (int)(blockIdx.x % ENM_ST_COPIES)) * ENM_ST_STRIDE, v);
+}
+
 __device__ __forceinline__ double uni_f64(double v) {
     const long long b = __double_as_longlong(v);
     const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffff));

@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <list>
@@ -80,32 +81,66 @@ struct Group {
                     // deferred 1-D query counts)
     int qoff;       // first of its ENM_NQ + 1 queue offsets in the offset table
     int inst;       // instance (per-instance mode) or -1
-    int walk;       // kNN items on grid orders (per-lane walk kernel)
+    int walk;       // kNN items: ENM_WALK_*; counts: ENM_WALK_TREE on trees
     int k1max;      // largest k+1 of its kNN items (sizes heap lists)
     int waves;      // persistent grid: waves per CU
-    int ticket;     // items per queue ticket (0: automatic)
+    int ticket;     // items per queue ticket (0: automatic); trees: waves per leaf
     int smax;       // strip items: the largest strip (LDS slots)
+    int phase;      // tree counts: the build phase of their trees; else 0
+    int qmax;       // items of the longest queue
 };
 
 struct ExportSpace {
     int64_t counts;   // res32 offset
-    int64_t perm;     // perm offset of the order
+    int64_t perm;     // perm offset of the order (-1: counts are in point order)
 };
 
 struct ExportInst {
     int64_t point_off;
     int64_t n;
-    int64_t eps;      // res64 offset (order A positions)
-    int64_t permA;    // perm offset of order A
+    int64_t eps;      // res64 offset (kNN order positions)
+    int64_t permA;    // perm offset of the kNN order (-1: radii are in point order)
     int nspace;
     ExportSpace sp[ENM_MAX_SPACES];
+};
+
+// A second sort stage: runs of a base order sorted by its column 1, laid out
+// into the orders over it (grid strips, and the slabs that box trees are cut
+// from).
+struct SecondStage {
+    std::vector<SortSeg> segs;
+    std::vector<GatherItem> gitems;
+    int ntiles = 0;
+    int tile = ENM_SORT_TILE;   // block-sort tile
+    int64_t elems = 0, maxlen = 0;
+    size_t off_segs = 0, off_gitems = 0;
+};
+
+// Box-tree phases: the trees of the joint spaces, then those of each count
+// space in turn, in the same memory (the joint trees and the grid orders are
+// not read again after the kNN, nor a count space's trees after its counts).
+constexpr int kPhases = 1 + ENM_MAX_SPACES;
+constexpr int64_t kTreesApart = 64ll << 20;   // bytes of trees that need not share memory
+
+struct TreePhase {
+    std::vector<CellItem> cells, groups;             // in instance order
+    std::vector<std::pair<int, int>> inst_cells, inst_groups;   // per instance: first, count
+    int tile = 0;                                    // largest cell
+    int64_t n64 = 0, nperm = 0;                      // memory used so far
+    size_t off_cells = 0, off_groups = 0;
 };
 
 struct Plan {
     std::string key;
     // host tables
-    std::vector<SortSeg> segs, segs2;        // stage 1 (arena keys), stage 2 (grid strips)
-    std::vector<GatherItem> gitems, gitems2;
+    std::vector<SortSeg> segs;               // stage 1 (arena keys)
+    std::vector<GatherItem> gitems;
+    SecondStage strips, slabs;
+    std::vector<TreeDev> trees;
+    std::vector<int> tree_phase;
+    TreePhase phase[kPhases];
+    int64_t grid64 = 0;                      // col64 of the grid orders (read by the kNN only)
+    std::vector<int> grid_orders;
     std::vector<OrderDev> orders;
     std::vector<KnnDev> kdescs;
     std::vector<CountDev> cdescs;
@@ -120,8 +155,7 @@ struct Plan {
     std::vector<int> qoffs;                          // queue offsets of every group
     std::vector<Group> groups;
     std::vector<ExportInst> exports;
-    int ntiles = 0, ntiles2 = 0;
-    int tile2 = ENM_SORT_TILE;   // block-sort tile of the second stage
+    int ntiles = 0;
     // Sample sort of the first stage (segments longer than one block-sort
     // tile, none longer than ENM_SS_MAXLEN); otherwise merge passes.
     bool sample_sort = false;
@@ -131,8 +165,8 @@ struct Plan {
     std::vector<int> qbase;          // run queue offsets (ENM_NQ + 1)
     int samp_tiles = 0;
     int64_t samp_maxlen = 0, n_samp = 0, n_counts = 0, n_buckets = 0;
-    int64_t maxlen = 0, maxlen2 = 0;
-    int64_t sort_elems = 0, sort_elems2 = 0;
+    int64_t maxlen = 0;
+    int64_t sort_elems = 0;
     int64_t n_col64 = 0, n_col32 = 0, n_perm = 0, n_res64 = 0, n_res32 = 0;
     int64_t psi_tab = 0, psi_n = 0;   // res64 offset of psi(0..psi_n)
     int64_t max_c1_queries = 0;       // 1-D count queries of the largest group
@@ -140,6 +174,7 @@ struct Plan {
     int n_inst = 0;
     bool f32 = true, brute = false, per_instance = false;
     bool want_eps = false;   // the call exports radii (in point order)
+    bool compact = false;    // trees always share memory (the static workspace)
     bool hinted = false;     // the call passes sort hints (first-stage segments of whole columns)
     // Kernels that read the FP32 column copies: the brute-force kNN and
     // multi-D counts off the grid (band filter).  Only then are they made.
@@ -152,7 +187,7 @@ struct Plan {
         deferred, heap, samp_k0, samp_k1, samp_i0, samp_i1, samp_split, bid, ss_counts, ss_tiles, ss_long, ss_ctl,
         hint_bad;
     size_t off_segs = 0, off_gitems = 0, off_orders = 0, off_kdescs = 0, off_cdescs = 0, off_insts = 0,
-           off_cls = 0, off_kitems = 0, off_citems = 0, off_segs2 = 0, off_gitems2 = 0, off_rdescs = 0,
+           off_cls = 0, off_kitems = 0, off_citems = 0, off_trees = 0, off_rdescs = 0,
            off_ritems = 0, off_sitems = 0, off_qoffs = 0, off_ssegs = 0, off_samp_segs = 0, off_cons = 0,
            off_qbase = 0, table_bytes = 0;
     void* pinned = nullptr;
@@ -266,11 +301,16 @@ struct Planner {
 
     explicit Planner(Plan& p, const enm_instance* in, const int64_t* sl) : P(p), inst(in), seg_len(sl) {}
 
+    // Class segments make the key for distinct class layouts differ.
+    std::tuple<int64_t, int64_t, int> sort_key(int ii, int64_t key_src, bool segmented) const {
+        const enm_instance& I = inst[ii];
+        return std::make_tuple(key_src, (int64_t)I.n, segmented ? (int)(I.seg_index * 64 + I.n_segs) : -1);
+    }
+
     int sort_group(int ii, int64_t key_src, bool segmented) {
         const enm_instance& I = inst[ii];
         const int nseg = segmented ? I.n_segs : 1;
-        // Class segments make the key for distinct class layouts differ.
-        auto key = std::make_tuple(key_src, (int64_t)I.n, segmented ? (int)(I.seg_index * 64 + nseg) : -1);
+        const auto key = sort_key(ii, key_src, segmented);
         auto it = sort_groups.find(key);
         if (it != sort_groups.end()) return it->second;
         const int g = (int)group_segs.size();
@@ -345,28 +385,34 @@ struct Planner {
         return id;
     }
 
-    // A grid order over base order `base`: each scope range cut into strips of
-    // S consecutive base positions, each strip sorted by the base order's
-    // column 1 (second-stage sort), all columns gathered in that order.
-    int grid_order(int base, int S) {
-        std::string key = "grid";
+    // An order over base order `base`: each scope range cut into runs of S
+    // consecutive base positions, each run sorted by the base order's column
+    // 1 (second-stage sort).  A grid order (for the kNN) has all columns laid
+    // out in that order; of a slab order only the permutation is wanted.
+    int second_order(int base, int S, bool slab) {
+        std::string key = slab ? "slab" : "grid";
         key += std::string((const char*)&base, sizeof base) + std::string((const char*)&S, sizeof S);
         auto it = order_ids.find(key);
         if (it != order_ids.end()) return it->second;
+        SecondStage& G = slab ? P.slabs : P.strips;
         const OrderDev bo = P.orders[base];
         OrderDev od = bo;
         od.xy = -1;
-        od.xy_only = 0;
-        od.c64 = P.n_col64;
-        od.c32 = P.n_col32;
+        od.xy_only = slab ? 1 : 0;
         od.perm = P.n_perm;
         od.base_perm = bo.perm;
         od.base_c64 = bo.c64;
         od.base_c32 = bo.c32;
-        P.n_col64 += od.ncol * od.n;
-        P.n_col32 += od.ncol * od.n;
-        P.n_perm += od.n;
         const int id = (int)P.orders.size();
+        if (!slab) {
+            // Placed with the trees' memory at the end of planning.
+            od.c64 = P.grid64;
+            od.c32 = P.n_col32;
+            P.grid64 += od.ncol * od.n;
+            P.n_col32 += od.ncol * od.n;
+            P.grid_orders.push_back(id);
+        }
+        P.n_perm += od.n;
         P.orders.push_back(od);
         order_ids[key] = id;
         order_group.push_back(order_group[base]);
@@ -375,21 +421,136 @@ struct Planner {
                 const int len = std::min(S, rg.second - st);
                 SortSeg sg;
                 sg.src = bo.c64 + 1 * bo.n + st;  // column 1 of the base order, in col64
-                sg.sbase = P.sort_elems2;
+                sg.sbase = G.elems;
                 sg.len = len;
-                sg.first_tile = P.ntiles2;
+                sg.first_tile = G.ntiles;
                 sg.p0 = st;
                 sg.hint = 0;
-                P.ntiles2 += (len + P.tile2 - 1) / P.tile2;
-                P.sort_elems2 += len;
-                P.maxlen2 = std::max<int64_t>(P.maxlen2, len);
-                const int sid = (int)P.segs2.size();
-                P.segs2.push_back(sg);
+                G.ntiles += (len + G.tile - 1) / G.tile;
+                G.elems += len;
+                G.maxlen = std::max<int64_t>(G.maxlen, len);
+                const int sid = (int)G.segs.size();
+                G.segs.push_back(sg);
                 for (int off = 0; off < len; off += ENM_SORT_TILE)
-                    P.gitems2.push_back(GatherItem{id, sid, off, st});
+                    G.gitems.push_back(GatherItem{id, sid, off, st});
             }
         }
         return id;
+    }
+
+    // An order of this instance keyed by column c0 (and with column c1 after
+    // it, unless c1 < 0): one that it has already, or a new one of only those
+    // columns.
+    std::vector<int> inst_orders;   // the current instance's first-stage orders
+    int keyed_order(int ii, int64_t c0, int64_t c1, bool segmented) {
+        const int g = sort_group(ii, c0, segmented);
+        for (int o : inst_orders)
+            if (order_group[o] == g && P.orders[o].src[0] == c0 &&
+                (c1 < 0 || (P.orders[o].ncol > 1 && P.orders[o].src[1] == c1)))
+                return o;
+        const int o = order(ii, c1 < 0 ? std::vector<int64_t>{c0} : std::vector<int64_t>{c0, c1}, segmented);
+        inst_orders.push_back(o);
+        return o;
+    }
+
+    // The box trees (one per scope range) of an instance's columns `cols`, in
+    // phase `ph`; returns the first one.  Scopes of one cell are cut from the
+    // point order; longer ones from slabs (runs of the order by column 0, each
+    // sorted by column 1: about as many slabs as cells in a slab), or, up to
+    // ENM_TREE_BASE_CELLS cells, from the order by column 0 itself.
+    int add_trees(int ii, const std::vector<int64_t>& cols, bool segmented, int ph) {
+        const enm_instance& I = inst[ii];
+        const int D = (int)cols.size();
+        std::vector<std::pair<int, int>> scopes;   // first point, points
+        int64_t p0 = 0, longest = 0;
+        for (int sg = 0; sg < (segmented ? I.n_segs : 1); ++sg) {
+            const int64_t len = segmented ? seg_len[I.seg_index + sg] : I.n;
+            if (len > 0) scopes.emplace_back((int)p0, (int)len);
+            p0 += len;
+            longest = std::max(longest, len);
+        }
+        int64_t slab = -1;
+        const int most = (int)((longest + ENM_CELL - 1) / ENM_CELL);   // cells of the longest scope
+        const bool two = most > ENM_TREE_BASE_CELLS;
+        int per_slab = 1;   // cells per slab
+        int sorted = -1;   // the column that the slab order has sorted within a cell
+        if (most == 1) {
+            // A sorted order that is there anyway saves the cell's first sort.
+            const auto g = sort_groups.find(sort_key(ii, cols[0], segmented));
+            for (int o : inst_orders)
+                if (g != sort_groups.end() && order_group[o] == g->second) {
+                    slab = P.orders[o].perm;
+                    sorted = 0;
+                }
+        } else {
+            sorted = two ? 1 : 0;
+            const int base = keyed_order(ii, cols[0], two ? cols[1] : -1, segmented);
+            slab = P.orders[base].perm;
+            if (two) {
+                int ns = 1;
+                while ((ns + 1) * (ns + 1) <= most) ++ns;
+                per_slab = (most + ns - 1) / ns;
+                slab = P.orders[second_order(base, per_slab * ENM_CELL, true)].perm;
+            }
+        }
+        TreePhase& F = P.phase[ph];
+        const int first = (int)P.trees.size();
+        for (auto sc : scopes) {
+            TreeDev t;
+            std::memset(&t, 0, sizeof t);
+            t.n = sc.second;
+            t.p0 = sc.first;
+            t.ncol = D;
+            t.cell = ENM_LEAF;
+            while (t.cell < ENM_CELL && t.cell < t.n) t.cell *= 2;
+            t.ncell = (t.n + t.cell - 1) / t.cell;
+            for (int c = 0; c < D; ++c) t.src[c] = cols[c];
+            t.slab = slab;
+            const int W = t.cell / ENM_LEAF, ngroup = (t.ncell + 63) / 64;
+            t.col = F.n64;
+            F.n64 += (int64_t)((t.n + ENM_LEAF - 1) / ENM_LEAF) * D * ENM_LEAF;
+            t.box = F.n64;
+            if (t.n > ENM_LEAF) F.n64 += (int64_t)t.ncell * 2 * D * 64;
+            t.cbox = F.n64;
+            if (t.ncell > 1) F.n64 += (int64_t)ngroup * 2 * D * 64;
+            t.gbox = F.n64;
+            if (ngroup > 1) F.n64 += (int64_t)((ngroup + 63) / 64) * 2 * D * 64;
+            t.perm = F.nperm;
+            F.nperm += t.n;
+            // The cell's leaves are halved log2(W) times; every halving goes
+            // to the column cut least so far, counting the cuts that made the
+            // cell.  A column the slab order has sorted comes first.
+            std::vector<double> cuts(D, 0.0);
+            if (t.ncell > 1) {
+                cuts[0] = std::log2(two ? std::max(1.0, (double)t.ncell / per_slab) : (double)t.ncell);
+                if (two) cuts[1] = std::log2((double)std::min(t.ncell, per_slab));
+            }
+            std::vector<int> bits(D, 0);
+            int log_cell = 6;
+            for (int w = 1; w < W; w *= 2) {
+                const int c = (int)(std::min_element(cuts.begin(), cuts.end()) - cuts.begin());
+                cuts[c] += 1.0;
+                ++bits[c];
+                ++log_cell;
+            }
+            int run = log_cell;
+            auto step = [&](int c) {
+                t.dim[t.nstep] = (int8_t)c;
+                t.run[t.nstep++] = (int8_t)run;
+                run -= bits[c];
+            };
+            if (sorted >= 0 && bits[sorted] > 0) { step(sorted); t.presorted = 1; }
+            for (int c = 0; c < D; ++c)
+                if (c != sorted && bits[c] > 0) step(c);
+            const int id = (int)P.trees.size();
+            for (int c = 0; c < t.ncell; ++c) F.cells.push_back(CellItem{id, c});
+            if (ngroup > 1)
+                for (int g = 0; g < ngroup; ++g) F.groups.push_back(CellItem{id, g});
+            F.tile = std::max(F.tile, t.cell);
+            P.trees.push_back(t);
+            P.tree_phase.push_back(ph);
+        }
+        return first;
     }
 
     // Scope ranges [lo, hi) of an order (class segments or all points).
@@ -427,7 +588,8 @@ struct PendingItem {
     int64_t cost;
     int inst;
     int dclass, pclass;
-    int walk = 0;   // kNN on a grid order: the per-lane walk kernel
+    int walk = ENM_WALK_NONE;
+    int phase = 0;
     int k1 = 0;     // k+1 of its instance (kNN items)
     int waves = 32, ticket = 0;   // its instance's tile shape
     int strip = 0;  // strip items: the strip size
@@ -462,13 +624,33 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
     // largest strip.
     std::vector<enm_tuning> tunes(n_inst);
     std::set<int> cols_read;   // orders whose column-major columns a kernel reads
+    // How the kNN of an instance of `cols` joint columns runs: strips staged
+    // in LDS (two columns, register lists, strips that three LDS slots hold:
+    // 20 x 100,000 points, k = 3 in 0.29 ms where trees take 0.91, k = 31 in
+    // 1.24 against 1.90), box trees (other spaces of two or more columns, up to
+    // ENM_TREE_K1_MAX neighbours: 4 x 50,000 points in two columns, k = 126 in
+    // 0.57 ms where per-lane walks with heaps take 3.3, in four columns in 1.5
+    // where grid sweeps take 41), grid sweeps (longer lists: heaps in global
+    // memory), or the plain key order (one column, brute force, strips tuned
+    // off).
+    auto route = [&](int cols, int k, const enm_tuning& T) {
+        if (P.brute || T.strip_points <= 0 || cols < 2) return ENM_WALK_NONE;
+        if (cols == 2 && k + 1 <= 32 && T.strip_points <= ENM_STRIP_LDS_MAX) return ENM_WALK_STRIP;
+        if (k < ENM_TREE_K1_MAX) return ENM_WALK_TREE;
+        return cols == 2 ? ENM_WALK_LANES : ENM_WALK_SWEEP;
+    };
     int max_strip = 0;
     for (int ii = 0; ii < n_inst; ++ii) {
         const int cols = std::max(0, inst[ii].dx) + std::max(0, inst[ii].dy) + std::max(0, inst[ii].dz);
         tunes[ii] = tuning_for(ctx, cols, inst[ii].k, inst[ii].n);
-        if (cols >= 2) max_strip = std::max(max_strip, (int)tunes[ii].strip_points);
+        const int r = route(cols, inst[ii].k, tunes[ii]);
+        if (r == ENM_WALK_STRIP || r == ENM_WALK_LANES || r == ENM_WALK_SWEEP)
+            max_strip = std::max(max_strip, (int)tunes[ii].strip_points);
     }
-    P.tile2 = max_strip <= 512 ? 512 : max_strip <= 1024 ? 1024 : ENM_SORT_TILE;
+    P.strips.tile = max_strip <= 512 ? 512 : max_strip <= 1024 ? 1024 : ENM_SORT_TILE;
+    // Queries on trees, made into items once their number is known.
+    struct TreeQueries { PendingItem pi; int first, count; int64_t n; };
+    std::vector<TreeQueries> ktree, ctree;
     int64_t point_off = 0;
     for (int ii = 0; ii < n_inst; ++ii) {
         const enm_instance& I = inst[ii];
@@ -515,13 +697,10 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         ex.n = I.n;
         point_off += I.n;
 
-        // Orders and spaces of this kind.  The kNN order's columns put the
-        // condition's first two columns first (CMI, conditional Ross), so the
-        // key and the grid's second axis are shared by every count space;
-        // each space lists its columns in ascending order (the max-norm does
-        // not depend on column order), so it starts with columns 0 and 1
-        // whenever it contains both.
-        int A = -1;
+        // The joint space's columns: the condition's first two columns come
+        // first (CMI, conditional Ross), so the orders that the trees are cut
+        // from are shared by every count space; each space lists its columns
+        // in ascending order (the max-norm does not depend on it).
         std::vector<int64_t> acols;
         std::vector<int> posX, posY, posZ;
         const bool segA = classes;
@@ -536,21 +715,32 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             for (int64_t c : X) put(posX, c);
             for (int64_t c : Y) put(posY, c);
         }
-        A = pl.order(ii, acols, segA);
-        // The kNN runs on a grid order (strips of the key-sorted order, each
-        // sorted by the second column) when there are two or more columns.
         const enm_tuning& T = tunes[ii];
         const int S = T.strip_points;
-        const bool grid = !P.brute && S > 0 && acols.size() >= 2;
-        const int K = grid ? pl.grid_order(A, S) : A;
-        if (grid && acols.size() == 2 && P.orders[K].xy < 0) {
-            // The per-lane walk reads (column 0, column 1) pairs.
-            P.n_col64 += P.n_col64 & 1;
-            P.orders[K].xy = P.n_col64;
-            P.n_col64 += 2 * I.n;
+        const int walk = route(ncols, I.k, T);
+        const bool grid = walk == ENM_WALK_STRIP || walk == ENM_WALK_LANES || walk == ENM_WALK_SWEEP;
+        // Multi-column count spaces use trees unless strips are tuned off.
+        const bool trees = !P.brute && S > 0;
+        pl.inst_orders.clear();
+        // A: the key-sorted order of all columns (not for trees); K: what the
+        // kNN runs on, A or a grid order over it.
+        int A = -1, K = -1, ktree_first = -1;
+        if (walk != ENM_WALK_TREE) {
+            A = pl.order(ii, acols, segA);
+            pl.inst_orders.push_back(A);
+            K = grid ? pl.second_order(A, S, false) : A;
+            if (grid && ncols == 2 && P.orders[K].xy < 0) {
+                // The strip and per-lane walks read (column 0, column 1) pairs.
+                P.grid64 += P.grid64 & 1;
+                P.orders[K].xy = P.grid64;
+                P.grid64 += 2 * I.n;
+            }
         }
 
-        struct SpaceSpec { int order; std::vector<int> cols; bool segmented; };
+        // The count spaces: columns (indices into acols), and whether balls
+        // are counted within the query's class only.  order, ocols: the order
+        // it is counted on and its columns there; tree: its first tree.
+        struct SpaceSpec { std::vector<int> cols; bool segmented; int order; std::vector<int> ocols; int tree; };
         std::vector<SpaceSpec> spaces;
         auto iota = [](int a, int b) { std::vector<int> v; for (int t = a; t < b; ++t) v.push_back(t); return v; };
         auto join = [](std::vector<int> a, const std::vector<int>& b) {
@@ -558,41 +748,66 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             std::sort(a.begin(), a.end());
             return a;
         };
-        bool need_orig = false;
         if (I.kind == ENM_KIND_KSG) {
-            spaces.push_back({A, posX, false});
-            const int Yo = pl.order(ii, Y, false);
-            spaces.push_back({Yo, iota(0, dy), false});
+            spaces.push_back({posX, false, -1, {}, -1});
+            spaces.push_back({posY, false, -1, {}, -1});
         } else if (I.kind == ENM_KIND_CMI) {
-            spaces.push_back({A, join(posX, posZ), false});
-            spaces.push_back({A, join(posY, posZ), false});
-            spaces.push_back({A, posZ, false});
+            spaces.push_back({join(posX, posZ), false, -1, {}, -1});
+            spaces.push_back({join(posY, posZ), false, -1, {}, -1});
+            spaces.push_back({posZ, false, -1, {}, -1});
         } else if (I.kind == ENM_KIND_ROSS) {
-            const int B = I.n_segs > 1 ? pl.order(ii, X, false) : A;
-            spaces.push_back({B, iota(0, dx), false});
+            spaces.push_back({posX, false, -1, {}, -1});
         } else if (I.kind == ENM_KIND_CROSS) {
-            const int B = I.n_segs > 1 ? pl.order(ii, acols, false) : A;
-            spaces.push_back({B, iota(0, (int)acols.size()), false});
-            spaces.push_back({A, posZ, true});
-            spaces.push_back({B, posZ, false});
+            spaces.push_back({iota(0, ncols), false, -1, {}, -1});
+            spaces.push_back({posZ, true, -1, {}, -1});
+            spaces.push_back({posZ, false, -1, {}, -1});
         }
-        // A multi-dimensional space whose first two columns are the order's
-        // columns 0 and 1 counts on the grid order over that order.
-        std::vector<int> space_strip(spaces.size(), 0);
-        std::vector<int64_t> space_base_key(spaces.size(), -1);
-        for (size_t t = 0; t < spaces.size(); ++t) {
-            SpaceSpec& sp = spaces[t];
-            if (grid && sp.cols.size() >= 2 && sp.cols[0] == 0 && sp.cols[1] == 1) {
-                space_base_key[t] = P.orders[sp.order].c64;
-                sp.order = pl.grid_order(sp.order, S);
-                space_strip[t] = S;
+        // (With one class, its order is the order of all points.)
+        auto scoped = [&](const SpaceSpec& sp) { return sp.segmented || (segA && I.n_segs == 1); };
+        // One-column spaces are counted on an order keyed by the column.
+        // Short instances make theirs first, so that the trees can be cut
+        // from it; longer ones cut them from an order of two columns, which
+        // serves the one-column space too.
+        auto one_column = [&]() {
+            for (SpaceSpec& sp : spaces)
+                if (sp.cols.size() == 1 && sp.order < 0) {
+                    sp.order = pl.keyed_order(ii, acols[sp.cols[0]], -1, scoped(sp));
+                    sp.ocols = {0};
+                }
+        };
+        if (I.n <= ENM_CELL * ENM_TREE_BASE_CELLS) one_column();
+        if (walk == ENM_WALK_TREE) ktree_first = pl.add_trees(ii, acols, segA, 0);
+        int ph = 0;
+        for (SpaceSpec& sp : spaces) {
+            if (!trees || sp.cols.size() < 2) continue;
+            std::vector<int64_t> c;
+            for (int t : sp.cols) c.push_back(acols[t]);
+            sp.tree = pl.add_trees(ii, c, scoped(sp), ++ph);
+        }
+        one_column();
+        for (SpaceSpec& sp : spaces) {
+            if (sp.tree >= 0 || sp.order >= 0) continue;
+            // A scan of the key order: an order whose key is the space's first
+            // column (of the whole joint space where it begins with that
+            // column, as A's scopes allow).
+            const bool seg = scoped(sp);
+            if (sp.cols[0] == 0 && seg == segA) {
+                sp.order = A;
+                sp.ocols = sp.cols;
+            } else {
+                std::vector<int64_t> c;
+                if (sp.cols[0] == 0) c = acols;
+                else for (int t : sp.cols) c.push_back(acols[t]);
+                sp.order = pl.order(ii, c, seg);
+                sp.ocols = sp.cols[0] == 0 ? sp.cols : iota(0, (int)sp.cols.size());
             }
         }
         // The radius in kNN order is kept for spaces on that order and for
         // the export; other spaces read it through the point numbering.
-        bool need_k = P.want_eps;
+        bool need_k = P.want_eps && walk != ENM_WALK_TREE;
+        bool need_orig = walk == ENM_WALK_TREE;
         for (auto& s : spaces) {
-            if (s.order != K) need_orig = true;
+            if (s.order < 0 || s.order != K) need_orig = true;
             else need_k = true;
         }
         // Entropy sums log radii in point order, whatever the kNN order.
@@ -604,17 +819,17 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         kd.order = K;
         kd.inst = ii;
         kd.strip = grid ? S : 0;
-        kd.base_key = P.orders[A].c64;
+        kd.base_key = A >= 0 ? P.orders[A].c64 : -1;
         kd.k = I.k;
         kd.kl = I.kind == ENM_KIND_KL;
+        kd.tree = ktree_first;
         kd.eps = -1;
         if (need_k) { kd.eps = P.n_res64; P.n_res64 += I.n; }
         kd.eps_orig = -1;
         if (need_orig) { kd.eps_orig = P.n_res64; P.n_res64 += I.n; }
         kd.part = -1;
         const int kdi = (int)P.kdescs.size();
-        const int D = (int)acols.size();
-        const int dcl = enm_knn_dim_class(D);
+        const int dcl = enm_knn_dim_class(ncols);
         // A register list may be given more slots than k+1 needs (the
         // extra ones stay pinned at -inf).
         const int pcl = I.k + 1 <= 32 && T.list_slots > 0 ? enm_knn_list_class(std::max(I.k + 1, (int)T.list_slots))
@@ -622,38 +837,35 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         if (dcl < 0) return bad("joint dimension above 16");
         if (I.k > 0x3fffffff) return bad("k out of range");
         int ktiles = 0;
-        std::vector<PendingItem> mine;
-        // Two-column grid orders with register lists and strips that three
-        // LDS slots hold: a strip per workgroup.
-        const bool strip_items = grid && D == 2 && pcl > 0 && S <= ENM_STRIP_LDS_MAX;
-        for (auto rg : pl.ranges(K)) {
-            if (strip_items) {
-                for (int t0 = rg.first; t0 < rg.second; t0 += S) {
-                    PendingItem pi;
-                    pi.it = Item{kdi, ktiles++, rg.first, rg.second, t0, std::min(t0 + S, rg.second)};
-                    pi.cost = (std::min(t0 + S, rg.second) - t0 + ENM_TILE - 1) / ENM_TILE;
-                    pi.inst = ii; pi.dclass = dcl; pi.pclass = pcl; pi.walk = 2;
-                    pi.k1 = I.k + 1;
-                    pi.waves = T.waves_per_cu; pi.ticket = T.items_per_ticket;
-                    pi.strip = S;
-                    mine.push_back(pi);
+        PendingItem kp;
+        kp.cost = 1;
+        kp.inst = ii; kp.dclass = dcl; kp.pclass = pcl; kp.walk = walk;
+        kp.k1 = I.k + 1;
+        kp.waves = T.waves_per_cu; kp.ticket = T.items_per_ticket;
+        kp.strip = walk == ENM_WALK_STRIP ? S : 0;
+        if (walk == ENM_WALK_TREE) {
+            // Lists across the lanes, one register of ranks or two.
+            kp.pclass = I.k + 1 <= 64 ? 1 : 2;
+            kp.it = Item{kdi, 0, 0, 0, 0, 0};
+            ktree.push_back({kp, ktree_first, (int)P.trees.size(), I.n});
+            int c = ktree_first;
+            while (c < (int)P.trees.size() && P.tree_phase[c] == 0) ++c;
+            ktree.back().count = c - ktree_first;
+        } else {
+            // Strips are items of their own; tiles never straddle a strip
+            // (strips start at lo + s*strip and the strip size is a multiple
+            // of the tile size).  Work per tile: the scope range in brute
+            // force, about constant with window pruning.
+            const int step = walk == ENM_WALK_STRIP ? S : ENM_TILE;
+            for (auto rg : pl.ranges(K)) {
+                for (int t0 = rg.first; t0 < rg.second; t0 += step) {
+                    PendingItem pi = kp;
+                    pi.it = Item{kdi, ktiles++, rg.first, rg.second, t0, std::min(t0 + step, rg.second)};
+                    pi.cost = walk == ENM_WALK_STRIP ? (pi.it.t1 - t0 + ENM_TILE - 1) / ENM_TILE
+                              : P.brute              ? (int64_t)(rg.second - rg.first)
+                                                     : 1;
+                    kpend.push_back(pi);
                 }
-                continue;
-            }
-            // Tiles never straddle a strip: strips start at lo + s*strip and
-            // the strip size is a multiple of the tile size.
-            for (int t0 = rg.first; t0 < rg.second; t0 += ENM_TILE) {
-                PendingItem pi;
-                pi.it = Item{kdi, ktiles++, rg.first, rg.second, t0, std::min(t0 + ENM_TILE, rg.second)};
-                // Work per tile: the scope range in brute force, about
-                // constant with window pruning.
-                pi.cost = P.brute ? (int64_t)(rg.second - rg.first) : 1;
-                // Per-lane walks on two-column grids; with more columns the
-                // gridded two prune less and tiles share candidates.
-                pi.inst = ii; pi.dclass = dcl; pi.pclass = pcl; pi.walk = grid && D == 2 ? 1 : 0;
-                pi.k1 = I.k + 1;
-                pi.waves = T.waves_per_cu; pi.ticket = T.items_per_ticket;
-                mine.push_back(pi);
             }
         }
         const int red_first = (int)P.ritems.size();
@@ -667,10 +879,9 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             id.ntile[0] = chunks;
         }
         P.kdescs.push_back(kd);
-        if (!strip_items) cols_read.insert(K);
-        kpend.insert(kpend.end(), mine.begin(), mine.end());
-        ex.eps = kd.eps;
-        ex.permA = P.orders[K].perm;
+        if (K >= 0 && walk != ENM_WALK_STRIP) cols_read.insert(K);
+        ex.eps = K >= 0 ? kd.eps : kd.eps_orig;
+        ex.permA = K >= 0 ? P.orders[K].perm : -1;
 
         // Count descriptors and items.
         if (!kd.kl) id.nspace = (int)spaces.size();
@@ -678,25 +889,37 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             const SpaceSpec& sp = spaces[s];
             CountDev cd;
             std::memset(&cd, 0, sizeof(cd));
-            cd.strip = space_strip[s];
-            cd.base_key = space_base_key[s];
+            cd.tree = sp.tree;
             cd.order = sp.order;
             cd.inst = ii;
             cd.ncol = (int)sp.cols.size();
-            for (int c = 0; c < cd.ncol; ++c) cd.cols[c] = sp.cols[c];
-            cd.same_order = sp.order == K;
+            for (int c = 0; c < cd.ncol; ++c) cd.cols[c] = sp.tree >= 0 ? c : sp.ocols[c];
+            cd.same_order = sp.order >= 0 && sp.order == K;
             cd.eps = cd.same_order ? kd.eps : kd.eps_orig;
-            cd.eps_perm = P.orders[sp.order].perm;
+            cd.eps_perm = sp.order >= 0 ? P.orders[sp.order].perm : -1;
             cd.counts = P.n_res32;
             P.n_res32 += I.n;
-            if (cd.ncol >= 2 && cd.strip == 0) P.need32 = true;
+            if (cd.ncol >= 2 && sp.tree < 0) P.need32 = true;
             const int cdi = (int)P.cdescs.size();
             const int ccl = enm_count_dim_class(cd.ncol);
             cd.psi_pt = -1;
             int ctiles = 0;
             std::vector<std::pair<int, int>> rgs;
-            if (sp.segmented) rgs = pl.ranges(sp.order);
-            else rgs.emplace_back(0, (int)I.n);
+            if (sp.tree >= 0) {
+                PendingItem pi;
+                pi.it = Item{cdi, 0, 0, 0, 0, 0};
+                pi.cost = 0;
+                pi.inst = ii; pi.dclass = ccl; pi.pclass = 0; pi.walk = ENM_WALK_TREE;
+                pi.waves = T.waves_per_cu; pi.ticket = T.items_per_ticket;
+                pi.phase = P.tree_phase[sp.tree];
+                int c = sp.tree;
+                while (c < (int)P.trees.size() && P.tree_phase[c] == pi.phase) ++c;
+                ctree.push_back({pi, sp.tree, c - sp.tree, I.n});
+            } else if (sp.segmented) {
+                rgs = pl.ranges(sp.order);
+            } else {
+                rgs.emplace_back(0, (int)I.n);
+            }
             // 1-D counts take ENM_C1_ITEM positions per item (and psi tiles
             // of ENM_PSI_TILE), multi-D ENM_TILE.
             const int step = ccl == 1 ? ENM_C1_ITEM : ENM_TILE;
@@ -740,6 +963,12 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             P.cdescs.push_back(cd);
         }
         ex.nspace = (int)spaces.size();
+        for (TreePhase& F : P.phase) {
+            const int c0 = F.inst_cells.empty() ? 0 : F.inst_cells.back().first + F.inst_cells.back().second;
+            const int g0 = F.inst_groups.empty() ? 0 : F.inst_groups.back().first + F.inst_groups.back().second;
+            F.inst_cells.emplace_back(c0, (int)F.cells.size() - c0);
+            F.inst_groups.emplace_back(g0, (int)F.groups.size() - g0);
+        }
         P.inst_ritems.emplace_back(red_first, (int)P.ritems.size() - red_first);
         P.inst_sitems.emplace_back(sit_first, (int)P.sitems.size() - sit_first);
         P.psi_n = std::max<int64_t>(P.psi_n, I.n);
@@ -753,7 +982,76 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
 
     // Grid orders read through their interleaved copy only (by the strip
     // kNN) skip the column-major layout.
-    for (const CountDev& cd : P.cdescs) cols_read.insert(cd.order);
+    for (const CountDev& cd : P.cdescs) cols_read.insert(cd.order);   // (-1: a tree)
+
+    // The grid orders and the trees follow the orders.  Small batches keep
+    // every tree, so one launch builds them and one counts the spaces of a
+    // dimension class; larger ones share the memory: the grid orders and the
+    // joint trees are read by the kNN, each phase's trees by its counts.  (One
+    // instance at a time, the grid orders of the later instances still have to
+    // be there.)
+    P.n_col64 += P.n_col64 & 1;
+    {
+        const int64_t base = P.n_col64;
+        int64_t all = P.grid64;
+        for (const TreePhase& F : P.phase) all += F.n64;
+        const bool apart = !P.per_instance && !P.compact && all * 8 <= kTreesApart;
+        int64_t at64[kPhases], atp[kPhases], end64 = P.grid64, endp = 0;
+        for (int f = 0; f < kPhases; ++f) {
+            at64[f] = apart ? end64 : f == 0 || P.per_instance ? P.grid64 : 0;
+            atp[f] = apart ? endp : 0;
+            end64 = std::max(end64, at64[f] + P.phase[f].n64);
+            endp = std::max(endp, atp[f] + P.phase[f].nperm);
+        }
+        for (int o : P.grid_orders) {
+            P.orders[o].c64 += base;
+            if (P.orders[o].xy >= 0) P.orders[o].xy += base;
+        }
+        for (size_t t = 0; t < P.trees.size(); ++t) {
+            TreeDev& tr = P.trees[t];
+            const int f = P.tree_phase[t];
+            tr.col += base + at64[f]; tr.box += base + at64[f];
+            tr.cbox += base + at64[f]; tr.gbox += base + at64[f];
+            tr.perm += P.n_perm + atp[f];
+        }
+        P.n_col64 += end64;
+        P.n_perm += endp;
+        if (apart) {
+            TreePhase& F = P.phase[0];
+            for (int f = 1; f < kPhases; ++f) {
+                TreePhase& G = P.phase[f];
+                F.cells.insert(F.cells.end(), G.cells.begin(), G.cells.end());
+                F.groups.insert(F.groups.end(), G.groups.begin(), G.groups.end());
+                F.tile = std::max(F.tile, G.tile);
+                G.cells.clear();
+                G.groups.clear();
+            }
+            for (TreeQueries& q : ctree) q.pi.phase = 0;
+        }
+    }
+
+    // Tree queries: an item is a leaf, shared by as many waves (of as few
+    // queries each) as make four for every wave slot of the GPU.
+    auto tree_items = [&](const std::vector<TreeQueries>& all, std::vector<PendingItem>& pend) {
+        int64_t total = 0;
+        for (const TreeQueries& q : all) total = P.per_instance ? std::max(total, q.n) : total + q.n;
+        int share = 1;
+        while (share < ENM_LEAF && total * share / ENM_LEAF < (int64_t)4 * 32 * ctx->num_cus) share *= 2;
+        for (const TreeQueries& q : all)
+            for (int t = q.first; t < q.first + q.count; ++t)
+                for (int t0 = 0; t0 < P.trees[t].n; t0 += ENM_LEAF) {
+                    PendingItem pi = q.pi;
+                    pi.it.tile = t;
+                    pi.it.t0 = t0;
+                    pi.it.t1 = std::min(t0 + ENM_LEAF, (int)P.trees[t].n);
+                    pi.cost = 1;
+                    pi.ticket = share;
+                    pend.push_back(pi);
+                }
+    };
+    tree_items(ktree, kpend);
+    tree_items(ctree, cpend);
+
     for (size_t o = 0; o < P.orders.size(); ++o)
         if (P.orders[o].xy >= 0 && !cols_read.count((int)o)) P.orders[o].xy_only = 1;
 
@@ -768,6 +1066,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             if (a.dclass != b.dclass) return a.dclass < b.dclass;
             if (a.pclass != b.pclass) return a.pclass < b.pclass;
             if (a.walk != b.walk) return a.walk < b.walk;
+            if (a.phase != b.phase) return a.phase < b.phase;
             return a.cost > b.cost;
         });
         // A deferred 1-D query code holds the item index in its upper bits.
@@ -776,7 +1075,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         while (i < pend.size()) {
             size_t j = i;
             while (j < pend.size() && pend[j].dclass == pend[i].dclass && pend[j].pclass == pend[i].pclass &&
-                   pend[j].walk == pend[i].walk && (!P.per_instance || pend[j].inst == pend[i].inst) &&
+                   pend[j].walk == pend[i].walk && pend[j].phase == pend[i].phase && (!P.per_instance || pend[j].inst == pend[i].inst) &&
                    j - i < max_group)
                 ++j;
             Group g;
@@ -788,6 +1087,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             g.counter = (int)P.groups.size() * (ENM_NQ + ENM_NDEF) * ENM_CSTRIDE;
             g.inst = P.per_instance ? pend[i].inst : -1;
             g.walk = pend[i].walk;
+            g.phase = pend[i].phase;
             g.k1max = 1;
             g.smax = 0;
             for (size_t t = i; t < j; ++t) {
@@ -797,11 +1097,11 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             // The group runs with the shape of its costliest item's instance.
             g.waves = pend[i].waves;
             g.ticket = pend[i].ticket;
-            if (!is_count && g.pclass == ENM_LIST_HEAP_GLOBAL) {
+            if (!is_count && g.walk != ENM_WALK_TREE && g.pclass == ENM_LIST_HEAP_GLOBAL) {
                 const int hg = enm_knn_heap_grid(grid_for(ctx, g.waves, g.n_items), g.k1max);
                 P.heap_bytes = std::max<int64_t>(P.heap_bytes, (int64_t)hg * ENM_TILE * g.k1max * 8);
             }
-            if (!is_count && g.walk == 2) {
+            if (!is_count && g.walk == ENM_WALK_STRIP) {
                 // Room for one query in 16 of the group (about 1 % reach past
                 // their neighbours on the lag scans), at most 64 MiB; the
                 // groups run one after the other and share it.
@@ -838,6 +1138,8 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
                 }
             }
             P.qoffs.push_back((int)(out.size() - g.first));
+            g.qmax = 0;
+            for (const auto& q : queue) g.qmax = std::max(g.qmax, (int)q.size());
             if (is_count && g.dclass == 1) P.max_c1_queries = std::max(P.max_c1_queries, queries);
             P.groups.push_back(g);
             i = j;
@@ -942,8 +1244,15 @@ std::vector<char> pack_tables(Plan& P) {
     P.off_cls = append(blob, P.cls);
     P.off_kitems = append(blob, P.kitems);
     P.off_citems = append(blob, P.citems);
-    P.off_segs2 = append(blob, P.segs2);
-    P.off_gitems2 = append(blob, P.gitems2);
+    for (SecondStage* g : {&P.strips, &P.slabs}) {
+        g->off_segs = append(blob, g->segs);
+        g->off_gitems = append(blob, g->gitems);
+    }
+    P.off_trees = append(blob, P.trees);
+    for (TreePhase& f : P.phase) {
+        f.off_cells = append(blob, f.cells);
+        f.off_groups = append(blob, f.groups);
+    }
     P.off_rdescs = append(blob, P.rdescs);
     P.off_ritems = append(blob, P.ritems);
     P.off_sitems = append(blob, P.sitems);
@@ -965,7 +1274,7 @@ struct BufSpec {
 // Every device buffer of a plan and its size in bytes.
 std::vector<BufSpec> workspace_layout(Plan& P) {
     std::vector<BufSpec> v;
-    const int64_t se = std::max(P.sort_elems, P.sort_elems2);
+    const int64_t se = std::max(P.sort_elems, std::max(P.strips.elems, P.slabs.elems));
     // FP32 column copies exist only when a kernel reads them.
     const bool with32 = P.f32 && P.need32;
     v.push_back({&P.tables, P.table_bytes, "tables"});
@@ -973,7 +1282,7 @@ std::vector<BufSpec> workspace_layout(Plan& P) {
     v.push_back({&P.sk1, (size_t)se * 8, "sort keys"});
     v.push_back({&P.si0, (size_t)se * 4, "sort index"});
     v.push_back({&P.si1, (size_t)se * 4, "sort index"});
-    v.push_back({&P.split, (size_t)std::max(P.ntiles, P.ntiles2) * 4 + 4, "merge splits"});
+    v.push_back({&P.split, (size_t)std::max(P.ntiles, std::max(P.strips.ntiles, P.slabs.ntiles)) * 4 + 4, "merge splits"});
     v.push_back({&P.col64, (size_t)P.n_col64 * 8, "columns"});
     v.push_back({&P.col32, with32 ? (size_t)P.n_col32 * 4 : 256, "FP32 columns"});
     v.push_back({&P.perm, (size_t)P.n_perm * 4, "permutations"});
@@ -982,7 +1291,7 @@ std::vector<BufSpec> workspace_layout(Plan& P) {
     v.push_back({&P.maxabs, (size_t)P.n_inst * 8, "maxima"});
     v.push_back({&P.counters, P.groups.size() * (ENM_NQ + ENM_NDEF) * ENM_CSTRIDE * 4 + 4, "counters"});
     v.push_back({&P.deferred, (size_t)P.deferred_seg * ENM_NDEF * 4, "deferred queries"});
-    v.push_back({&P.stats, ST_N * 8, "stats"});
+    v.push_back({&P.stats, ENM_ST_SLOTS * 8, "stats"});
     if (P.heap_bytes > 0) v.push_back({&P.heap, (size_t)P.heap_bytes, "heap lists"});
     if (P.far_bytes > 0) v.push_back({&P.far, (size_t)P.far_bytes, "strip kNN far list"});
     if (P.sample_sort) {
@@ -1056,7 +1365,7 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
     };
     if ((rc = mark(0))) return rc;
     unsigned long long* stats = P.stats.as<unsigned long long>();
-    if ((rc = chk(enm_launch_fill_u64(stats, ST_N, 0ull, st), "fill"))) return rc;
+    if ((rc = chk(enm_launch_fill_u64(stats, ENM_ST_SLOTS, 0ull, st), "fill"))) return rc;
     if ((rc = chk(enm_launch_fill_u64(P.maxabs.as<unsigned long long>(), P.n_inst, 0ull, st), "fill"))) return rc;
     if ((rc = chk(enm_launch_fill_i32(P.counters.as<int>(),
                                       (int64_t)P.groups.size() * (ENM_NQ + ENM_NDEF) * ENM_CSTRIDE, 0, st),
@@ -1109,7 +1418,8 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
         if ((rc = chk(enm_launch_sample_sort(a, arena, P.sk0.as<double>(), P.si0.as<int>(), P.sk1.as<double>(),
                                              P.si1.as<int>(), &nl, st), "sort")))
             return rc;
-    } else if ((rc = chk(enm_launch_sort(tab<SortSeg>(P, P.off_segs), (int)P.segs.size(), P.ntiles, P.maxlen,
+    } else if (!P.segs.empty() &&
+               (rc = chk(enm_launch_sort(tab<SortSeg>(P, P.off_segs), (int)P.segs.size(), P.ntiles, P.maxlen,
                                          ENM_SORT_TILE, arena, nullptr,
                                          P.sk0.as<double>(), P.si0.as<int>(), P.sk1.as<double>(), P.si1.as<int>(),
                                          P.split.as<int>(), &fb, &nl, st), "sort"))) {
@@ -1119,40 +1429,51 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
     const double* skey = fb ? P.sk1.as<double>() : P.sk0.as<double>();
     const int* sidx = fb ? P.si1.as<int>() : P.si0.as<int>();
     // (The sample sort lays its segments out into the orders itself.)
-    if (!P.sample_sort && (rc = chk(enm_launch_gather(tab<GatherItem>(P, P.off_gitems), (int)P.gitems.size(),
+    if (!P.sample_sort && !P.gitems.empty() && (rc = chk(enm_launch_gather(tab<GatherItem>(P, P.off_gitems), (int)P.gitems.size(),
                                     tab<SortSeg>(P, P.off_segs), tab<OrderDev>(P, P.off_orders), arena, skey,
                                     sidx, P.col64.as<double>(), P.col32.as<float>(), P.perm.as<int>(),
                                     P.maxabs.as<unsigned long long>(), P.f32 && P.need32 ? 1 : 0, &nl, st),
                       "gather")))
         return rc;
-    if (!P.segs2.empty()) {
-        // Second stage: sort each grid strip by the base order's column 1
-        // (keys read from col64) and lay out the grid orders; strips that
-        // fit one block do both in one kernel.
-        if (P.maxlen2 <= ENM_SORT_TILE) {
-            if ((rc = chk(enm_launch_strip_sort(tab<GatherItem>(P, P.off_gitems2), (int)P.gitems2.size(),
-                                                tab<SortSeg>(P, P.off_segs2), tab<OrderDev>(P, P.off_orders),
-                                                P.tile2, P.col64.as<double>(), P.col32.as<float>(),
-                                                P.perm.as<int>(), P.f32 && P.need32 ? 1 : 0, &nl, st),
+    // Second stages: sort each grid strip or slab by the base order's column 1
+    // (keys read from col64) and lay out the orders; strips that fit one
+    // block do both in one kernel.
+    for (const SecondStage* g : {&P.strips, &P.slabs}) {
+        if (g->segs.empty()) continue;
+        const SortSeg* gsegs = tab<SortSeg>(P, g->off_segs);
+        const GatherItem* gits = tab<GatherItem>(P, g->off_gitems);
+        const int with32 = P.f32 && P.need32 ? 1 : 0;
+        if (g->maxlen <= ENM_SORT_TILE) {
+            if ((rc = chk(enm_launch_strip_sort(gits, (int)g->gitems.size(), gsegs, tab<OrderDev>(P, P.off_orders),
+                                                g->tile, P.col64.as<double>(), P.col32.as<float>(), P.perm.as<int>(),
+                                                with32, &nl, st), "sort")))
+                return rc;
+        } else {
+            if ((rc = chk(enm_launch_sort(gsegs, (int)g->segs.size(), g->ntiles, g->maxlen, g->tile,
+                                          P.col64.as<double>(), nullptr, P.sk0.as<double>(), P.si0.as<int>(),
+                                          P.sk1.as<double>(), P.si1.as<int>(), P.split.as<int>(), &fb, &nl, st),
                           "sort")))
                 return rc;
-        } else if ((rc = chk(enm_launch_sort(tab<SortSeg>(P, P.off_segs2), (int)P.segs2.size(), P.ntiles2, P.maxlen2,
-                                      P.tile2, P.col64.as<double>(), nullptr, P.sk0.as<double>(), P.si0.as<int>(),
-                                      P.sk1.as<double>(), P.si1.as<int>(), P.split.as<int>(), &fb, &nl, st),
-                      "sort"))) {
-            return rc;
-        } else {
-            const double* skey2 = fb ? P.sk1.as<double>() : P.sk0.as<double>();
-            const int* sidx2 = fb ? P.si1.as<int>() : P.si0.as<int>();
-            if ((rc = chk(enm_launch_gather(tab<GatherItem>(P, P.off_gitems2), (int)P.gitems2.size(),
-                                            tab<SortSeg>(P, P.off_segs2), tab<OrderDev>(P, P.off_orders), arena,
-                                            skey2, sidx2, P.col64.as<double>(), P.col32.as<float>(),
-                                            P.perm.as<int>(), P.maxabs.as<unsigned long long>(),
-                                            P.f32 && P.need32 ? 1 : 0, &nl, st),
+            if ((rc = chk(enm_launch_gather(gits, (int)g->gitems.size(), gsegs, tab<OrderDev>(P, P.off_orders), arena,
+                                            fb ? P.sk1.as<double>() : P.sk0.as<double>(),
+                                            fb ? P.si1.as<int>() : P.si0.as<int>(), P.col64.as<double>(),
+                                            P.col32.as<float>(), P.perm.as<int>(),
+                                            P.maxabs.as<unsigned long long>(), with32, &nl, st),
                           "gather")))
                 return rc;
         }
     }
+    // The box trees of one phase, of all instances or of one.
+    const TreeDev* trees = tab<TreeDev>(P, P.off_trees);
+    auto build_trees = [&](int f, int ii) -> int {
+        const TreePhase& F = P.phase[f];
+        const auto cells = ii < 0 ? std::make_pair(0, (int)F.cells.size()) : F.inst_cells[ii];
+        const auto groups = ii < 0 ? std::make_pair(0, (int)F.groups.size()) : F.inst_groups[ii];
+        return chk(enm_launch_tree_build(tab<CellItem>(P, F.off_cells) + cells.first, cells.second,
+                                         tab<CellItem>(P, F.off_groups) + groups.first, groups.second, F.tile, trees,
+                                         arena, P.col64.as<double>(), P.perm.as<int>(), &nl, st), "trees");
+    };
+    if (!P.per_instance && (rc = build_trees(0, -1))) return rc;
     if ((rc = mark(3))) return rc;
     const OrderDev* orders = tab<OrderDev>(P, P.off_orders);
     const unsigned long long* maxabs = P.maxabs.as<unsigned long long>();
@@ -1161,10 +1482,22 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
     const int* qoffs = tab<int>(P, P.off_qoffs);
     const double* psi_tab = P.res64.as<double>() + P.psi_tab;
     auto run_group = [&](const Group& g) -> int {
+        if (g.walk == ENM_WALK_TREE) {
+            ++nl;
+            if (!g.is_count)
+                return chk(enm_launch_tree_knn(tab<Item>(P, P.off_kitems) + g.first, qoffs + g.qoff, g.n_items,
+                                               g.qmax, g.ticket, tab<KnnDev>(P, P.off_kdescs), trees, P.perm.as<int>(),
+                                               P.col64.as<double>(), P.res64.as<double>(), stats, g.dclass, g.k1max,
+                                               st), "knn");
+            return chk(enm_launch_tree_count(tab<Item>(P, P.off_citems) + g.first, qoffs + g.qoff, g.n_items, g.qmax,
+                                             g.ticket, tab<CountDev>(P, P.off_cdescs), trees, P.perm.as<int>(), psi_tab,
+                                             P.col64.as<double>(), P.res64.as<double>(), P.res32.as<int>(), stats,
+                                             g.dclass, st), "count");
+        }
         if (!g.is_count) {
             int grid = g.pclass == ENM_LIST_HEAP_GLOBAL ? enm_knn_heap_grid(grid_for(ctx, g.waves, g.n_items), g.k1max)
                                                         : grid_for(ctx, g.waves, g.n_items);
-            if (g.walk == 2) {
+            if (g.walk == ENM_WALK_STRIP) {
                 // Strip workgroups: as many per CU as the waves per CU and
                 // the LDS (three slots of the largest strip) allow.
                 const int nt = std::min(512, ((g.smax + 63) / 64) * 64);
@@ -1178,9 +1511,9 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
                                P.col64.as<double>(), P.col32.as<float>(), P.res64.as<double>(), stats,
                                g.dclass, g.pclass, P.f32 && P.brute, P.brute, g.walk, grid,
                                g.k1max, P.heap.as<double>(), g.ticket, g.smax,
-                               g.walk == 2 && P.far_bytes > 0 ? P.far.as<char>() : nullptr,
+                               g.walk == ENM_WALK_STRIP && P.far_bytes > 0 ? P.far.as<char>() : nullptr,
                                counters + g.counter + ENM_NQ * ENM_CSTRIDE, P.far_bytes, st);
-            nl += g.walk == 2 && P.far_bytes > 0 ? 2 : 1;
+            nl += g.walk == ENM_WALK_STRIP && P.far_bytes > 0 ? 2 : 1;
             return chk(e, "knn");
         }
         e = enm_launch_count(tab<Item>(P, P.off_citems) + g.first, qoffs + g.qoff, g.n_items,
@@ -1202,10 +1535,14 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
     };
     if (P.per_instance) {
         for (int ii = 0; ii < P.n_inst; ++ii) {
+            for (int f = 0; f < kPhases; ++f) {
+                if ((rc = build_trees(f, ii))) return rc;
+                for (const Group& g : P.groups)
+                    if (g.inst == ii && (f == 0) == !g.is_count && (f == 0 || g.phase == f) && (rc = run_group(g)))
+                        return rc;
+            }
             for (const Group& g : P.groups)
-                if (g.inst == ii && !g.is_count && (rc = run_group(g))) return rc;
-            for (const Group& g : P.groups)
-                if (g.inst == ii && g.is_count && (rc = run_group(g))) return rc;
+                if (g.inst == ii && g.is_count && g.phase == 0 && (rc = run_group(g))) return rc;
             if ((rc = psi_tiles(P.inst_sitems[ii].first, P.inst_sitems[ii].second))) return rc;
             const auto ri = P.inst_ritems[ii];
             if ((rc = chk(enm_launch_reduce_pt(tab<RedItem>(P, P.off_ritems) + ri.first, ri.second,
@@ -1224,8 +1561,13 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
         for (const Group& g : P.groups)
             if (!g.is_count && (rc = run_group(g))) return rc;
         if ((rc = mark(4))) return rc;
+        for (int f = 1; f < kPhases; ++f) {
+            if ((rc = build_trees(f, -1))) return rc;
+            for (const Group& g : P.groups)
+                if (g.is_count && g.phase == f && (rc = run_group(g))) return rc;
+        }
         for (const Group& g : P.groups)
-            if (g.is_count && (rc = run_group(g))) return rc;
+            if (g.is_count && g.phase == 0 && (rc = run_group(g))) return rc;
         if ((rc = psi_tiles(0, (int)P.sitems.size()))) return rc;
         if ((rc = chk(enm_launch_reduce_pt(tab<RedItem>(P, P.off_ritems), (int)P.ritems.size(),
                                            tab<RedDev>(P, P.off_rdescs), P.res64.as<double>(), st),
@@ -1241,7 +1583,8 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
     if (d_eps || d_counts) {
         for (const ExportInst& ex : P.exports) {
             if (d_eps) {
-                if ((rc = chk(enm_launch_export_eps(P.res64.as<double>() + ex.eps, P.perm.as<int>() + ex.permA,
+                if ((rc = chk(enm_launch_export_eps(P.res64.as<double>() + ex.eps,
+                                                    ex.permA >= 0 ? P.perm.as<int>() + ex.permA : nullptr,
                                                     ex.n, d_eps + ex.point_off, st), "export")))
                     return rc;
                 ++nl;
@@ -1252,7 +1595,7 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
                 ++nl;
                 for (int s = 0; s < ex.nspace; ++s) {
                     if ((rc = chk(enm_launch_export_cnt(P.res32.as<int>() + ex.sp[s].counts,
-                                                        P.perm.as<int>() + ex.sp[s].perm, ex.n,
+                                                        ex.sp[s].perm >= 0 ? P.perm.as<int>() + ex.sp[s].perm : nullptr, ex.n,
                                                         base + s * ex.n, st), "export")))
                         return rc;
                     ++nl;
@@ -1477,6 +1820,7 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     P.need32 = P.brute;
     P.per_instance = (flags & ENM_F_PER_INSTANCE) != 0;
     P.want_eps = d_eps != nullptr;
+    P.compact = true;
     int rc = plan_batch(ctx, P, inst, n_inst, seg_len);
     if (rc) return rc;
     const std::vector<char> blob = pack_tables(P);
@@ -1998,15 +2342,18 @@ int enm_get_stats(enm_ctx* ctx, enm_stats* out) {
     if (!ctx->last) return fail(ctx, ENM_E_ARG, "no batch has run");
     hipError_t e = hipStreamSynchronize(ctx->last_stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
-    unsigned long long h[ST_N];
-    e = hipMemcpy(h, ctx->last->stats.p, sizeof h, hipMemcpyDeviceToHost);
+    std::vector<unsigned long long> parts(ENM_ST_SLOTS);
+    e = hipMemcpy(parts.data(), ctx->last->stats.p, ENM_ST_SLOTS * 8, hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipMemcpy(stats)");
+    unsigned long long h[ST_N] = {};
+    for (int s = 0; s < ST_N; ++s)
+        for (int c = 0; c < ENM_ST_COPIES; ++c) h[s] += parts[(s * ENM_ST_COPIES + c) * ENM_ST_STRIDE];
     out->knn_pairs = h[ST_KNN_PAIRS];
     out->knn_rechecks = h[ST_KNN_RECHECK];
     out->count_pairs = h[ST_CNT_PAIRS];
     out->count_rechecks = h[ST_CNT_RECHECK];
     out->count_queries_1d = h[ST_CNT_1D];
-    out->sort_keys = (uint64_t)(ctx->last->sort_elems + ctx->last->sort_elems2);
+    out->sort_keys = (uint64_t)(ctx->last->sort_elems + ctx->last->strips.elems + ctx->last->slabs.elems);
     out->n_launches = (uint32_t)ctx->last->n_launch;
     out->graph_replayed = ctx->last->graph != nullptr && ctx->last->n_launch == 0;
     if (ctx->last->timing) {

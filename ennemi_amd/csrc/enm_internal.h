@@ -45,8 +45,22 @@
 // Two-column kNN: strips up to this size are walked a strip per workgroup
 // with the strip and its two neighbours staged in LDS (3 x 1024 x 16 B).
 #define ENM_STRIP_LDS_MAX 1024
-// Default strip of instances of three or more joint columns.
+// Default strip of instances of three or more joint columns.  Their kNN and
+// counts run on box trees; strips of this size serve only the grid sweeps
+// of k+1 > ENM_TREE_K1_MAX.
 #define ENM_STRIP_WIDE 4096
+// Box trees (enm_tree.hip).
+#define ENM_LEAF 64            // points per leaf (one per lane)
+#define ENM_CELL 4096          // points per cell: ENM_LEAF leaves of ENM_LEAF points
+#define ENM_TREE_STEPS 6       // most sorted columns of a cell (one halving of its leaves each at least)
+#define ENM_TREE_K1_MAX 128    // longest neighbour list held across a wave's lanes
+// How a kNN group runs (and, on trees, a count group).
+#define ENM_WALK_NONE 0        // key order: plain or brute force
+#define ENM_WALK_LANES 1       // two-column grid order, per-lane walks (global heaps)
+#define ENM_WALK_STRIP 2       // two-column grid order, a strip per workgroup
+#define ENM_WALK_SWEEP 3       // wider grid order, tile-shared sweeps (global heaps)
+#define ENM_WALK_TREE 4        // box tree
+#define ENM_TREE_BASE_CELLS 4  // scopes of more cells are cut by two columns, not one
 
 // One contiguous key range to sort: keys at arena[src + t], t in [0, len),
 // carried with their instance point index p0 + t.
@@ -130,6 +144,44 @@ struct OrderDev {
     int32_t pad2;
 };
 
+// A box tree over one scope of an instance (all points or one class) in the
+// columns of the joint space or of one count space.  Positions [0, n) are the
+// scope's points in tree order: cells of `cell` consecutive positions (a power
+// of two of at least ENM_LEAF, ENM_CELL where there are several cells), each
+// cut into leaves of ENM_LEAF positions.  The last leaf and the last cell may
+// be partly filled.  A leaf is a block of ENM_LEAF values of each column, one
+// column after the other (NaN past the last point), a cell's leaf boxes are
+// 2 * ncol rows (lo and hi of each column) of 64 values, so every load of a
+// leaf, or of 64 boxes, is a fixed offset from one address.  Groups of 64
+// cells have the boxes of their cells in the same form, blocks of 64 groups
+// those of the groups.
+struct TreeDev {
+    int64_t col;      // col64 offset of the leaves: leaf l at col + l * ncol * ENM_LEAF
+    int64_t box;      // col64 offset of the leaf boxes: cell k at box + k * 2 * ncol * 64
+    int64_t cbox;     // col64 offset of the cell boxes: group g at cbox + g * 2 * ncol * 64
+    int64_t gbox;     // col64 offset of the group boxes: block b at gbox + b * 2 * ncol * 64
+    int64_t perm;     // perm offset: tree position -> instance point
+    int64_t slab;     // perm offset of the order the cells are cut from (-1: the point order)
+    int64_t src[16];  // arena offset of each column
+    int32_t n;
+    int32_t ncol;
+    int32_t cell;
+    int32_t ncell;
+    int32_t p0;       // first instance point of the scope (its first position in the slab order, too)
+    // A cell's sorts: step s sorts runs of 1 << run[s] positions by column
+    // dim[s] (the first is skipped when the slab order has it sorted already).
+    int32_t nstep;
+    int32_t presorted;
+    int8_t dim[ENM_TREE_STEPS];
+    int8_t run[ENM_TREE_STEPS];
+};
+
+// Tree build work: one cell.
+struct CellItem {
+    int32_t tree;
+    int32_t cell;
+};
+
 // kNN over one order (its scope ranges are the class segments, or all points).
 // With strip > 0 the order is a grid order: positions [lo + s*strip,
 // lo + (s+1)*strip) of each scope range [lo, hi) form strip s, whose points
@@ -145,7 +197,7 @@ struct KnnDev {
     int64_t part;       // unused (-1)
     int64_t base_key;   // col64 offset of the base order's sorted column 0
     int32_t strip;      // points per strip (0: plain key-sorted order)
-    int32_t pad;
+    int32_t tree;       // >= 0: its first box tree (one per scope range); the order is unused
 };
 
 // Ball count in one space (a subset of an order's columns, key first).
@@ -157,13 +209,12 @@ struct CountDev {
     int32_t cols[16];    // indices into the order's columns; cols[0] == 0
     int64_t eps;         // res64 offset of the radius source
     int64_t eps_perm;    // perm offset of the order's permutation (radius via eps_orig)
-    int64_t counts;      // res32 offset: count per order position
+    int64_t counts;      // res32 offset: count per order position (trees: per point)
     int64_t part;        // res64 offset: per-tile sum of psi(count)
     int64_t zero;        // res32 offset: per-tile "some count is 0" flag
-    // With strip > 0 the order is a grid order (as for KnnDev) and the space
-    // starts with the order's columns 0 and 1.
-    int64_t base_key;
-    int32_t strip;
+    // >= 0: its first box tree (one per scope range), which holds the
+    // space's columns; radii and counts are in point order then.
+    int32_t tree;
     int32_t pad;
     // >= 0: res64 offset of a point-order array receiving psi(count) (+inf
     // for a count of 0) instead of per-tile partial sums; a reduction in
@@ -188,7 +239,8 @@ struct RedItem {
 // One work item: a tile of consecutive order positions [t0, t1) inside the
 // scope range [lo, hi) (64 for kNN and multi-D counts, ENM_C1_ITEM for 1-D
 // counts, ENM_PSI_TILE for 1-D psi sums).  A persistent launch takes its
-// items from ENM_NQ queues, queue q being items [qoff[q], qoff[q+1]).
+// items from ENM_NQ queues, queue q being items [qoff[q], qoff[q+1]).  A tree
+// item is a range of tree positions inside one leaf; `tile` is its tree.
 struct Item {
     int32_t desc;
     int32_t tile;   // tile index within its descriptor (partials slot)
@@ -214,6 +266,12 @@ struct InstDev {
 
 // Device counters (enm_stats order).
 enum { ST_KNN_PAIRS = 0, ST_KNN_RECHECK, ST_CNT_PAIRS, ST_CNT_RECHECK, ST_CNT_1D, ST_SORT_KEYS, ST_N };
+// Each is kept in ENM_ST_COPIES parts, a cache line apart (copy c of counter
+// s at (s * ENM_ST_COPIES + c) * ENM_ST_STRIDE), and summed by the host: every
+// wave of a launch adds to one at its end, and additions to one address queue.
+#define ENM_ST_COPIES 64
+#define ENM_ST_STRIDE 16
+#define ENM_ST_SLOTS (ST_N * ENM_ST_COPIES * ENM_ST_STRIDE)
 
 // Device-side preparation of estimate_mi tasks (enm_prep_count / enm_prep_write).
 #define ENM_PREP_BLOCK 2048     // window rows per compaction block

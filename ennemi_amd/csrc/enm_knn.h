@@ -6,28 +6,28 @@
 // all j of the query's scope range, i itself included (distance 0); fewer
 // than k+1 points leave it +inf, as cKDTree does.
 //
-// Grid orders: the key-sorted points cut into strips, each strip sorted by
-// the second column.  A work item is one wave and 64 consecutive positions
-// of one strip (one query per lane).  With two columns each lane walks the
-// strips around its own point by itself (knn_walk): its own strip from its
-// own position, then the strips outward that its current radius still
-// reaches on the key axis, each from the lane's y position in both
-// directions until the y distance reaches the radius.  Candidates arrive in
-// about increasing distance, so each lane evaluates about ten candidates.
-// Each lane keeps an ascending FP64 list of its K1 = k+1 smallest distances
-// in registers (P slots, the lowest P-K1 pinned at -inf).
+// Box trees (enm_tree_knn.hip) serve spaces of two or more columns, except:
 //
-// Grid orders of three or more columns, where the two gridded columns prune
-// less and a lane's walk would be long, share candidates instead: a wave
-// takes a tile of 64 consecutive positions of a strip and walks candidates
-// in wave-uniform order (grid_sweep: its own strip, then the strips outward,
-// each within the union of the lanes' y intervals).  Other orders (one
-// column, or ENM_F_BRUTE) do the same over the key-sorted order, 8
+// Two columns and register lists: grid orders (the key-sorted points cut into
+// strips, each strip sorted by the second column), a strip per workgroup with
+// its neighbours staged in LDS (knn_strip_kernel below).
+//
+// Lists of more than ENM_TREE_K1_MAX distances: heaps in global memory, on grid
+// orders.  With two columns each lane walks the strips around its own point by
+// itself (knn_walk): its own strip from its own position, then the strips
+// outward that its current radius still reaches on the key axis, each from the
+// lane's y position in both directions until the y distance reaches the
+// radius.  With more columns a wave takes a tile of 64 consecutive positions
+// of a strip and walks candidates in wave-uniform order (grid_sweep: its own
+// strip, then the strips outward, each within the union of the lanes' y
+// intervals).
+//
+// One column, ENM_F_BRUTE and tunings without strips: the key-sorted order, 8
 // candidates at a time through the scalar cache (candidate coordinates are
-// SGPR operands); with one column, from the tile outward in key order, alternating
-// left and right in steps of 64, a side stopping once every lane's key
-// distance to the last visited candidate is >= its current K1-th distance T.
-// With ENM_F_BRUTE the whole scope range is scanned.
+// SGPR operands), from the tile outward in key order, alternating left and
+// right in steps of 64, a side stopping once every lane's key distance to the
+// last visited candidate is >= its current K1-th distance T.  With ENM_F_BRUTE
+// the whole scope range is scanned.
 //
 // Precision.  Every distance that enters a list is exact FP64.  The FP32
 // filter (brute force in FP32-filter mode) computes the bulk distance from
@@ -651,7 +651,7 @@ __device__ void knn_item(const KnnArgs& A, const Item& it, const double* __restr
     int visited = t1 - t0;
     w.range(t0, t1);
     bool swept = false;
-    if constexpr (D >= 2) {
+    if constexpr (D >= 2 && P == ENM_LIST_HEAP_GLOBAL) {
         if (kd.strip > 0 && !A.brute) {
             visited += grid_sweep(w, kd, col64, lo, hi, t0, t1, active);
             swept = true;
@@ -732,7 +732,7 @@ void knn_walk_kernel(KnnArgs A, const double* __restrict__ col64, double* __rest
         it.lo = uni(it.lo); it.hi = uni(it.hi); it.t0 = uni(it.t0); it.t1 = uni(it.t1);
         walk_item<P>(A, it, col64, res64, pairs);
     });
-    if (threadIdx.x == 0) atomicAdd(stats + ST_KNN_PAIRS, pairs);
+    if (threadIdx.x == 0) add_stat(stats, ST_KNN_PAIRS, pairs);
 }
 
 // ---------------------------------------------------------------------------
@@ -1082,7 +1082,7 @@ void knn_strip_kernel(KnnArgs A, const double* __restrict__ col64, double* __res
         __syncthreads();   // the slots are restaged by the next item
     });
     const unsigned long long total = wave_sum_u64((unsigned long long)pairs);
-    if ((threadIdx.x & (ENM_WAVE - 1)) == 0) atomicAdd(stats + ST_KNN_PAIRS, total);
+    if ((threadIdx.x & (ENM_WAVE - 1)) == 0) add_stat(stats, ST_KNN_PAIRS, total);
 }
 
 // The far list of a knn_strip_kernel launch, one query per thread: its
@@ -1121,7 +1121,7 @@ void knn_far_kernel(KnnArgs A, const double* __restrict__ col64, double* __restr
         pairs += visited;
     }
     pairs = wave_sum_u64(pairs);
-    if ((threadIdx.x & (ENM_WAVE - 1)) == 0 && pairs) atomicAdd(stats + ST_KNN_PAIRS, pairs);
+    if ((threadIdx.x & (ENM_WAVE - 1)) == 0 && pairs) add_stat(stats, ST_KNN_PAIRS, pairs);
 }
 
 template <int D, int P, bool F32>
@@ -1148,8 +1148,8 @@ void knn_kernel(KnnArgs A, const double* __restrict__ col64, const float* __rest
         }
     });
     if (threadIdx.x == 0) {
-        atomicAdd(stats + ST_KNN_PAIRS, pairs);
-        if (F32) atomicAdd(stats + ST_KNN_RECHECK, rechecks);
+        add_stat(stats, ST_KNN_PAIRS, pairs);
+        if (F32) add_stat(stats, ST_KNN_RECHECK, rechecks);
     }
 }
 
@@ -1158,28 +1158,26 @@ hipError_t launch_dp(const KnnArgs& a, bool f32, int walk, int grid, const doubl
                      double* res64, unsigned long long* stats, hipStream_t st) {
     // LDS heaps: 64 lanes x the group's largest K1 doubles per workgroup.
     const unsigned shmem = P == ENM_LIST_HEAP_LDS ? (unsigned)(a.heap_stride * sizeof(double)) : 0u;
-    // Per-lane walks and strip workgroups exist for two-column grid orders
-    // only; strip workgroups for register lists (their LDS holds strips).
-    if (walk) {
-        if constexpr (D == 2) {
-            if constexpr (P > 0) {
-                if (walk == 2) {
-                    const int nt = a.smax >= SK_THREADS_MAX ? SK_THREADS_MAX : ((a.smax + 63) / 64) * 64;
-                    const unsigned lds = (unsigned)(3 * a.smax * sizeof(double2));
-                    hipLaunchKernelGGL((knn_strip_kernel<P>), dim3(grid), dim3(nt), lds, st, a, col64, res64, stats);
-                    // The far list: eight 4-wave blocks per CU of the strip grid's
-                    // three (latency-bound walks need every wave slot).
-                    if (a.far != nullptr)
-                        hipLaunchKernelGGL((knn_far_kernel<P>), dim3(std::max(1, grid) * 8 / 3 + 1), dim3(256), 0, st,
-                                           a, col64, res64, stats);
-                    return hipGetLastError();
-                }
-            }
-            if (walk == 1) {
-                hipLaunchKernelGGL((knn_walk_kernel<P>), dim3(grid), dim3(ENM_WAVE), shmem, st, a, col64, res64,
-                                   stats);
-                return hipGetLastError();
-            }
+    // Strip workgroups: two-column grid orders, register lists (their LDS
+    // holds strips); per-lane walks: the same orders, global heaps.
+    if (walk == ENM_WALK_STRIP) {
+        if constexpr (D == 2 && P > 0) {
+            const int nt = a.smax >= SK_THREADS_MAX ? SK_THREADS_MAX : ((a.smax + 63) / 64) * 64;
+            const unsigned lds = (unsigned)(3 * a.smax * sizeof(double2));
+            hipLaunchKernelGGL((knn_strip_kernel<P>), dim3(grid), dim3(nt), lds, st, a, col64, res64, stats);
+            // The far list: eight 4-wave blocks per CU of the strip grid's
+            // three (latency-bound walks need every wave slot).
+            if (a.far != nullptr)
+                hipLaunchKernelGGL((knn_far_kernel<P>), dim3(std::max(1, grid) * 8 / 3 + 1), dim3(256), 0, st,
+                                   a, col64, res64, stats);
+            return hipGetLastError();
+        }
+        return hipErrorInvalidValue;
+    }
+    if (walk == ENM_WALK_LANES) {
+        if constexpr (D == 2 && P == ENM_LIST_HEAP_GLOBAL) {
+            hipLaunchKernelGGL((knn_walk_kernel<P>), dim3(grid), dim3(ENM_WAVE), 0, st, a, col64, res64, stats);
+            return hipGetLastError();
         }
         return hipErrorInvalidValue;
     }

@@ -71,6 +71,20 @@ hipError_t enm_launch_knn(const Item* items, const int* qoff, int n_items, unsig
 // ENM_HEAP_GLOBAL_BYTES: at most `grid` blocks of 64 x k1max doubles.
 int enm_knn_heap_grid(int grid, int k1max);
 
+// Box trees (enm_tree.hip, enm_tree_knn.hip): the build of a phase's cells
+// (and of its trees' cell groups), and the queries on them.
+hipError_t enm_launch_tree_build(const CellItem* items, int n_items, const CellItem* groups, int n_groups, int tile,
+                                 const TreeDev* trees, const double* arena, double* col64, int* perm, int* n_launch,
+                                 hipStream_t st);
+hipError_t enm_launch_tree_knn(const Item* items, const int* qoff, int n_items, int qmax, int share,
+                               const KnnDev* descs,
+                               const TreeDev* trees, const int* perm, const double* col64, double* res64,
+                               unsigned long long* stats, int dclass, int k1max, hipStream_t st);
+hipError_t enm_launch_tree_count(const Item* items, const int* qoff, int n_items, int qmax, int share,
+                                 const CountDev* descs,
+                                 const TreeDev* trees, const int* perm, const double* psi_tab, const double* col64,
+                                 double* res64, int* res32, unsigned long long* stats, int dclass, hipStream_t st);
+
 int enm_count_dim_class(int d);
 hipError_t enm_launch_count(const Item* items, const int* qoff, int n_items, unsigned* counter,
                             const CountDev* descs, const OrderDev* orders,

@@ -106,17 +106,18 @@ void reduce_pt_kernel(const RedItem* __restrict__ items, const RedDev* __restric
     if (threadIdx.x == 0) res64[rd.part + it.chunk] = acc;
 }
 
-// Export one order-positioned array into instance numbering.
+// Export one order-positioned array into instance numbering (perm NULL: it
+// is in instance numbering already).
 __global__ void export_eps_kernel(const double* __restrict__ src, const int* __restrict__ perm,
                                   int64_t n, double* __restrict__ dst) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < n) dst[perm[p]] = src[p];
+    if (p < n) dst[perm ? perm[p] : p] = src[p];
 }
 
 __global__ void export_cnt_kernel(const int* __restrict__ src, const int* __restrict__ perm,
                                   int64_t n, int* __restrict__ dst) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < n) dst[perm[p]] = src[p];
+    if (p < n) dst[perm ? perm[p] : p] = src[p];
 }
 
 __global__ void fill_i32_kernel(int* __restrict__ p, int64_t n, int v) {

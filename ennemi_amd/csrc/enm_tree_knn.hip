@@ -1,0 +1,170 @@
+// k-th-neighbour radii on box trees: eps_i is the (k+1)-th smallest distance
+// over the scope, the query itself included (+inf with fewer points).
+//
+// A wave takes the queries of one leaf one after the other.  The leaf's own 64
+// points, held one per lane for all of its queries, are sorted across the
+// lanes and give the first k+1 neighbours and radius T; then the leaves of the
+// own cell and of the other cells whose boxes come nearer than T are visited,
+// the nearest first, so T is close to its final value after a leaf or two.  A
+// leaf's few distances below T go into the list one at a time (a shift by one
+// lane, a minimum and a maximum for up to 64 neighbours); where there are
+// many, as with long lists, they are sorted and merged.
+#include "enm_tree.h"
+
+namespace {
+
+// Distances below T at which sorting and merging all 64 beats inserting one by
+// one: about 140 (one register of ranks) or 200 instructions against 11 or 15
+// each.
+constexpr int MERGE_FROM = 13;
+
+template <int D, int NR>
+struct TreeQuery {
+    const TreeDev& T;
+    const double* col64;
+    int ncol;
+    double q[D];
+    LaneList<NR> list;
+    int K1;
+    double t;            // the current radius
+    unsigned visited;    // leaves
+
+    __device__ __forceinline__ void visit_leaf(const double* leaf) {
+        double a[D];
+        load_leaf<D>(a, leaf, ncol);
+        const double e = point_dist<D>(a, q);
+        unsigned long long m = __builtin_amdgcn_ballot_w64(e < t);
+        ++visited;
+        if (__popcll(m) >= MERGE_FROM) {
+            list.merge(e < t ? e : INFINITY);
+            t = list.rank(K1 - 1);
+        } else {
+            while (m) {
+                list.insert(lane_f64(e, __builtin_ctzll(m)));
+                t = list.rank(K1 - 1);
+                m &= (m - 1) & __builtin_amdgcn_ballot_w64(e < t);
+            }
+        }
+    }
+
+    // The nearest of the lanes in m by their gaps.
+    __device__ __forceinline__ int nearest(unsigned long long m, double gap) {
+        const int lane = (int)(threadIdx.x & (ENM_WAVE - 1));
+        const float g = (m >> lane) & 1 ? (float)gap : INFINITY;
+        const unsigned long long s = __builtin_amdgcn_ballot_w64(g == wave_min_f32(g)) & m;
+        return __builtin_ctzll(s ? s : m);
+    }
+
+    // The leaves of a cell but leaf `own` (-1: all).
+    __device__ __forceinline__ void visit_cell(int cell, int own) {
+        const int nleaf = (min(T.cell, T.n - cell * T.cell) + ENM_LEAF - 1) / ENM_LEAF;
+        double far;
+        const double g = box_gap<D, false>(col64 + T.box + (int64_t)cell * 2 * ncol * 64, ncol, q, far);
+        unsigned long long open = low_mask(nleaf);
+        if (own >= 0) open &= ~(1ull << own);
+        const double* leaves = col64 + T.col + (int64_t)cell * T.cell * ncol;
+        for (;;) {
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(g < t) & open;
+            if (!m) break;
+            const int l = nearest(m, g);
+            open &= ~(1ull << l);
+            visit_leaf(leaves + l * ENM_LEAF * ncol);
+        }
+    }
+
+    __device__ __forceinline__ void visit_others(int own_cell) {
+        const int ncell = T.ncell, ngroup = (ncell + 63) / 64;
+        double far;
+        for (int gb = 0; gb < ngroup; gb += 64) {
+            double gg = 0.0;
+            unsigned long long gopen = low_mask(ngroup - gb);
+            if (ngroup > 1) gg = box_gap<D, false>(col64 + T.gbox + (int64_t)(gb / 64) * 2 * ncol * 64, ncol, q, far);
+            for (;;) {
+                const unsigned long long gm = ngroup > 1 ? __builtin_amdgcn_ballot_w64(gg < t) & gopen : gopen;
+                if (!gm) break;
+                const int gl = ngroup > 1 ? nearest(gm, gg) : 0;
+                gopen &= ~(1ull << gl);
+                const int gr = gb + gl;
+                const double g = box_gap<D, false>(col64 + T.cbox + (int64_t)gr * 2 * ncol * 64, ncol, q, far);
+                unsigned long long open = low_mask(ncell - gr * 64);
+                if (own_cell / 64 == gr) open &= ~(1ull << (own_cell % 64));
+                for (;;) {
+                    const unsigned long long m = __builtin_amdgcn_ballot_w64(g < t) & open;
+                    if (!m) break;
+                    const int c = nearest(m, g);
+                    open &= ~(1ull << c);
+                    visit_cell(gr * 64 + c, -1);
+                }
+            }
+        }
+    }
+};
+
+template <int D, int NR>
+__global__ __launch_bounds__(TREE_WG* ENM_WAVE, tree_waves(D))
+void tree_knn_kernel(TreeArgs A, const KnnDev* __restrict__ descs, const double* __restrict__ col64,
+                     double* __restrict__ res64, unsigned long long* __restrict__ stats) {
+    const TreeWork it = tree_work(A);
+    if (it.nq <= 0) return;
+    const int lane = (int)(threadIdx.x & (ENM_WAVE - 1));
+    const KnnDev& kd = descs[it.desc];
+    const TreeDev& T = A.trees[it.tile];
+    const int t0 = it.t0, nq = it.nq;
+    const int ncol = T.ncol;
+    // The queries' leaf, one point per lane.
+    const int leaf = t0 / ENM_LEAF, j0 = t0 % ENM_LEAF;
+    const int cell = leaf * ENM_LEAF / T.cell;
+    double own[D];
+    load_leaf<D>(own, col64 + T.col + (int64_t)leaf * ncol * ENM_LEAF, ncol);
+    double mine = 0.0;
+    unsigned visited = 0;
+    for (int j = 0; j < nq; ++j) {
+        TreeQuery<D, NR> w{T, col64, ncol};
+#pragma unroll
+        for (int d = 0; d < D; ++d) w.q[d] = lane_f64(own[d], j0 + j);
+        w.K1 = kd.k + 1;
+        w.visited = visited + 1;
+        w.list.seed(vmin(point_dist<D>(own, w.q), INFINITY));   // (NaN: +inf)
+        w.t = w.list.rank(w.K1 - 1);
+        if (T.n > ENM_LEAF) w.visit_cell(cell, leaf - cell * (T.cell / ENM_LEAF));
+        if (T.ncell > 1) w.visit_others(cell);
+        if (lane == j) mine = w.t;
+        visited = w.visited;
+    }
+    if (lane < nq) res64[kd.eps_orig + A.perm[T.perm + t0 + lane]] = mine;
+    if (lane == 0) add_stat(stats, ST_KNN_PAIRS, (unsigned long long)visited * ENM_LEAF);
+}
+
+template <int D>
+hipError_t launch(const TreeArgs& a, int qmax, int k1max, const KnnDev* descs, const double* col64, double* res64,
+                  unsigned long long* stats, hipStream_t st) {
+    const dim3 grid(tree_grid(qmax, a.share)), block(TREE_WG * ENM_WAVE);
+    if (k1max <= 64)
+        hipLaunchKernelGGL((tree_knn_kernel<D, 1>), grid, block, 0, st, a, descs, col64, res64, stats);
+    else if (k1max <= ENM_TREE_K1_MAX)
+        hipLaunchKernelGGL((tree_knn_kernel<D, 2>), grid, block, 0, st, a, descs, col64, res64, stats);
+    else
+        return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t enm_launch_tree_knn(const Item* items, const int* qoff, int n_items, int qmax, int share,
+                               const KnnDev* descs,
+                               const TreeDev* trees, const int* perm, const double* col64, double* res64,
+                               unsigned long long* stats, int dclass, int k1max, hipStream_t st) {
+    if (n_items <= 0) return hipSuccess;
+    const TreeArgs a{items, qoff, share, trees, perm, nullptr};
+    switch (dclass) {
+        case 2: return launch<2>(a, qmax, k1max, descs, col64, res64, stats, st);
+        case 3: return launch<3>(a, qmax, k1max, descs, col64, res64, stats, st);
+        case 4: return launch<4>(a, qmax, k1max, descs, col64, res64, stats, st);
+        case 5: return launch<5>(a, qmax, k1max, descs, col64, res64, stats, st);
+        case 6: return launch<6>(a, qmax, k1max, descs, col64, res64, stats, st);
+        case 8: return launch<8>(a, qmax, k1max, descs, col64, res64, stats, st);
+        case 12: return launch<12>(a, qmax, k1max, descs, col64, res64, stats, st);
+        case 16: return launch<16>(a, qmax, k1max, descs, col64, res64, stats, st);
+        default: return hipErrorInvalidValue;
+    }
+}
