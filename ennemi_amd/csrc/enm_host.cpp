@@ -631,10 +631,12 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
     // ENM_TREE_K1_MAX neighbours: 4 x 50,000 points in two columns, k = 126 in
     // 0.57 ms where per-lane walks with heaps take 3.3, in four columns in 1.5
     // where grid sweeps take 41), grid sweeps (longer lists: heaps in global
-    // memory), or the plain key order (one column, brute force, strips tuned
-    // off).
+    // memory), or the plain key order (brute force, strips tuned off); one
+    // column by windows of its sorted keys.
     auto route = [&](int cols, int k, const enm_tuning& T) {
-        if (P.brute || T.strip_points <= 0 || cols < 2) return ENM_WALK_NONE;
+        if (P.brute) return ENM_WALK_NONE;
+        if (cols < 2) return ENM_WALK_LINE;
+        if (T.strip_points <= 0) return ENM_WALK_NONE;
         if (cols == 2 && k + 1 <= 32 && T.strip_points <= ENM_STRIP_LDS_MAX) return ENM_WALK_STRIP;
         if (k < ENM_TREE_K1_MAX) return ENM_WALK_TREE;
         return cols == 2 ? ENM_WALK_LANES : ENM_WALK_SWEEP;
@@ -856,7 +858,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             // (strips start at lo + s*strip and the strip size is a multiple
             // of the tile size).  Work per tile: the scope range in brute
             // force, about constant with window pruning.
-            const int step = walk == ENM_WALK_STRIP ? S : ENM_TILE;
+            const int step = walk == ENM_WALK_STRIP ? S : walk == ENM_WALK_LINE ? ENM_LINE_ITEM : ENM_TILE;
             for (auto rg : pl.ranges(K)) {
                 for (int t0 = rg.first; t0 < rg.second; t0 += step) {
                     PendingItem pi = kp;
@@ -1097,7 +1099,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             // The group runs with the shape of its costliest item's instance.
             g.waves = pend[i].waves;
             g.ticket = pend[i].ticket;
-            if (!is_count && g.walk != ENM_WALK_TREE && g.pclass == ENM_LIST_HEAP_GLOBAL) {
+            if (!is_count && g.walk != ENM_WALK_TREE && g.walk != ENM_WALK_LINE && g.pclass == ENM_LIST_HEAP_GLOBAL) {
                 const int hg = enm_knn_heap_grid(grid_for(ctx, g.waves, g.n_items), g.k1max);
                 P.heap_bytes = std::max<int64_t>(P.heap_bytes, (int64_t)hg * ENM_TILE * g.k1max * 8);
             }
@@ -1493,6 +1495,12 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
                                              g.ticket, tab<CountDev>(P, P.off_cdescs), trees, P.perm.as<int>(), psi_tab,
                                              P.col64.as<double>(), P.res64.as<double>(), P.res32.as<int>(), stats,
                                              g.dclass, st), "count");
+        }
+        if (g.walk == ENM_WALK_LINE) {
+            ++nl;
+            return chk(enm_launch_knn_line(tab<Item>(P, P.off_kitems) + g.first, g.n_items,
+                                           tab<KnnDev>(P, P.off_kdescs), orders, P.perm.as<int>(),
+                                           P.col64.as<double>(), P.res64.as<double>(), stats, st), "knn");
         }
         if (!g.is_count) {
             int grid = g.pclass == ENM_LIST_HEAP_GLOBAL ? enm_knn_heap_grid(grid_for(ctx, g.waves, g.n_items), g.k1max)

@@ -60,6 +60,9 @@
 #define ENM_WALK_STRIP 2       // two-column grid order, a strip per workgroup
 #define ENM_WALK_SWEEP 3       // wider grid order, tile-shared sweeps (global heaps)
 #define ENM_WALK_TREE 4        // box tree
+#define ENM_WALK_LINE 5        // one column: windows of the sorted keys
+#define ENM_LINE_THREADS 256
+#define ENM_LINE_ITEM 2048     // positions per one-column item
 #define ENM_TREE_BASE_CELLS 4  // scopes of more cells are cut by two columns, not one
 
 // One contiguous key range to sort: keys at arena[src + t], t in [0, len),
