@@ -223,22 +223,6 @@ __device__ __forceinline__ void wave_bounds(const double* __restrict__ v, int lo
     b = __builtin_amdgcn_readlane(L, 32);
 }
 
-// Positions [a, b) of the strip [s0, s1) of a y-sorted column that can
-// hold a candidate j with fl(|y_j - y_i|) <= T_i for some live lane i: the
-// union of the lanes' intervals [y_i - T_i, y_i + T_i], each widened by a
-// relative 2^-50 so that the rounding of the bounds (far below the
-// widening) cannot exclude such a candidate.  Wave-uniform result.
-__device__ __forceinline__ void strip_window(const double* __restrict__ yc, int s0, int s1, double yq, double T,
-                                         bool live, int& a, int& b) {
-    const double slack = 0x1p-50 * (fabs(yq) + T);
-    const double lq = live ? (yq - T * (1.0 + 0x1p-50)) - slack : INFINITY;
-    const double uq = live ? (yq + T * (1.0 + 0x1p-50)) + slack : -INFINITY;
-    const double lb = uni_f64(wave_min(lq));
-    const double ub = uni_f64(wave_max(uq));
-    if (!(lb <= ub)) { a = b = s0; return; }
-    wave_bounds(yc, s0, s1, lb, ub, a, b);
-}
-
 // The block number that block b of an nb-block launch works on when
 // consecutive numbers should share an XCD's L2: the hardware deals
 // workgroups to the ENM_NQ XCDs round-robin, so this gives XCD x the x-th of

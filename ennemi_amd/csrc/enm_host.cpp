@@ -175,6 +175,7 @@ struct Plan {
     bool f32 = true, brute = false, per_instance = false;
     bool want_eps = false;   // the call exports radii (in point order)
     bool compact = false;    // trees always share memory (the static workspace)
+    bool plain = false;      // no trees: the key orders alone (a static batch whose trees do not fit)
     bool hinted = false;     // the call passes sort hints (first-stage segments of whole columns)
     // Kernels that read the FP32 column copies: the brute-force kNN and
     // multi-D counts off the grid (band filter).  Only then are they made.
@@ -627,26 +628,21 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
     // How the kNN of an instance of `cols` joint columns runs: strips staged
     // in LDS (two columns, register lists, strips that three LDS slots hold:
     // 20 x 100,000 points, k = 3 in 0.29 ms where trees take 0.91, k = 31 in
-    // 1.24 against 1.90), box trees (other spaces of two or more columns, up to
-    // ENM_TREE_K1_MAX neighbours: 4 x 50,000 points in two columns, k = 126 in
-    // 0.57 ms where per-lane walks with heaps take 3.3, in four columns in 1.5
-    // where grid sweeps take 41), grid sweeps (longer lists: heaps in global
-    // memory), or the plain key order (brute force, strips tuned off); one
-    // column by windows of its sorted keys.
+    // 1.24 against 1.90), box trees (other spaces of two or more columns),
+    // or the plain key order (brute force, strips tuned off); one column by
+    // windows of its sorted keys.
     auto route = [&](int cols, int k, const enm_tuning& T) {
         if (P.brute) return ENM_WALK_NONE;
         if (cols < 2) return ENM_WALK_LINE;
-        if (T.strip_points <= 0) return ENM_WALK_NONE;
+        if (T.strip_points <= 0 || (P.plain && (cols > 2 || k + 1 > 32))) return ENM_WALK_NONE;
         if (cols == 2 && k + 1 <= 32 && T.strip_points <= ENM_STRIP_LDS_MAX) return ENM_WALK_STRIP;
-        if (k < ENM_TREE_K1_MAX) return ENM_WALK_TREE;
-        return cols == 2 ? ENM_WALK_LANES : ENM_WALK_SWEEP;
+        return ENM_WALK_TREE;
     };
     int max_strip = 0;
     for (int ii = 0; ii < n_inst; ++ii) {
         const int cols = std::max(0, inst[ii].dx) + std::max(0, inst[ii].dy) + std::max(0, inst[ii].dz);
         tunes[ii] = tuning_for(ctx, cols, inst[ii].k, inst[ii].n);
-        const int r = route(cols, inst[ii].k, tunes[ii]);
-        if (r == ENM_WALK_STRIP || r == ENM_WALK_LANES || r == ENM_WALK_SWEEP)
+        if (route(cols, inst[ii].k, tunes[ii]) == ENM_WALK_STRIP)
             max_strip = std::max(max_strip, (int)tunes[ii].strip_points);
     }
     P.strips.tile = max_strip <= 512 ? 512 : max_strip <= 1024 ? 1024 : ENM_SORT_TILE;
@@ -720,9 +716,8 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         const enm_tuning& T = tunes[ii];
         const int S = T.strip_points;
         const int walk = route(ncols, I.k, T);
-        const bool grid = walk == ENM_WALK_STRIP || walk == ENM_WALK_LANES || walk == ENM_WALK_SWEEP;
         // Multi-column count spaces use trees unless strips are tuned off.
-        const bool trees = !P.brute && S > 0;
+        const bool trees = !P.brute && !P.plain && S > 0;
         pl.inst_orders.clear();
         // A: the key-sorted order of all columns (not for trees); K: what the
         // kNN runs on, A or a grid order over it.
@@ -730,9 +725,9 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         if (walk != ENM_WALK_TREE) {
             A = pl.order(ii, acols, segA);
             pl.inst_orders.push_back(A);
-            K = grid ? pl.second_order(A, S, false) : A;
-            if (grid && ncols == 2 && P.orders[K].xy < 0) {
-                // The strip and per-lane walks read (column 0, column 1) pairs.
+            K = walk == ENM_WALK_STRIP ? pl.second_order(A, S, false) : A;
+            if (walk == ENM_WALK_STRIP && P.orders[K].xy < 0) {
+                // The strip walks read (column 0, column 1) pairs.
                 P.grid64 += P.grid64 & 1;
                 P.orders[K].xy = P.grid64;
                 P.grid64 += 2 * I.n;
@@ -820,7 +815,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         std::memset(&kd, 0, sizeof(kd));
         kd.order = K;
         kd.inst = ii;
-        kd.strip = grid ? S : 0;
+        kd.strip = walk == ENM_WALK_STRIP ? S : 0;
         kd.base_key = A >= 0 ? P.orders[A].c64 : -1;
         kd.k = I.k;
         kd.kl = I.kind == ENM_KIND_KL;
@@ -845,9 +840,9 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         kp.k1 = I.k + 1;
         kp.waves = T.waves_per_cu; kp.ticket = T.items_per_ticket;
         kp.strip = walk == ENM_WALK_STRIP ? S : 0;
+        if (walk == ENM_WALK_LINE) kp.pclass = 0;   // one kernel for any k
         if (walk == ENM_WALK_TREE) {
-            // Lists across the lanes, one register of ranks or two.
-            kp.pclass = I.k + 1 <= 64 ? 1 : 2;
+            kp.pclass = enm_tree_list_class(I.k + 1);
             kp.it = Item{kdi, 0, 0, 0, 0, 0};
             ktree.push_back({kp, ktree_first, (int)P.trees.size(), I.n});
             int c = ktree_first;
@@ -1489,7 +1484,7 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
             if (!g.is_count)
                 return chk(enm_launch_tree_knn(tab<Item>(P, P.off_kitems) + g.first, qoffs + g.qoff, g.n_items,
                                                g.qmax, g.ticket, tab<KnnDev>(P, P.off_kdescs), trees, P.perm.as<int>(),
-                                               P.col64.as<double>(), P.res64.as<double>(), stats, g.dclass, g.k1max,
+                                               P.col64.as<double>(), P.res64.as<double>(), stats, g.dclass, g.pclass,
                                                st), "knn");
             return chk(enm_launch_tree_count(tab<Item>(P, P.off_citems) + g.first, qoffs + g.qoff, g.n_items, g.qmax,
                                              g.ticket, tab<CountDev>(P, P.off_cdescs), trees, P.perm.as<int>(), psi_tab,
@@ -1821,21 +1816,31 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
         if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
     }
     ctx->last_stream = st;
-    std::unique_ptr<Plan> up(new Plan());
-    Plan& P = *up;
-    P.f32 = (flags & ENM_F_FP64) == 0;
-    P.brute = (flags & ENM_F_BRUTE) != 0;
-    P.need32 = P.brute;
-    P.per_instance = (flags & ENM_F_PER_INSTANCE) != 0;
-    P.want_eps = d_eps != nullptr;
-    P.compact = true;
-    int rc = plan_batch(ctx, P, inst, n_inst, seg_len);
-    if (rc) return rc;
-    const std::vector<char> blob = pack_tables(P);
-    const std::vector<BufSpec> layout = workspace_layout(P);
     auto rounded = [](size_t b) { return (std::max<size_t>(b, 256) + 255) & ~(size_t)255; };
+    std::unique_ptr<Plan> up;
+    std::vector<char> blob;
+    std::vector<BufSpec> layout;
     size_t total = 0;
-    for (const BufSpec& b : layout) total += rounded(b.bytes);
+    // A batch whose box trees do not fit may fit without them (slower).
+    for (int plain = 0; plain < 2; ++plain) {
+        up.reset(new Plan());
+        Plan& P = *up;
+        P.f32 = (flags & ENM_F_FP64) == 0;
+        P.brute = (flags & ENM_F_BRUTE) != 0;
+        P.need32 = P.brute;
+        P.per_instance = (flags & ENM_F_PER_INSTANCE) != 0;
+        P.want_eps = d_eps != nullptr;
+        P.compact = true;
+        P.plain = plain != 0;
+        int rc = plan_batch(ctx, P, inst, n_inst, seg_len);
+        if (rc) return rc;
+        blob = pack_tables(P);
+        layout = workspace_layout(P);
+        total = 0;
+        for (const BufSpec& b : layout) total += rounded(b.bytes);
+        if (total <= (size_t)ENM_STATIC_WORKSPACE_BYTES || P.trees.empty()) break;
+    }
+    Plan& P = *up;
     if (total > (size_t)ENM_STATIC_WORKSPACE_BYTES) {
         char msg[200];
         std::snprintf(msg, sizeof msg,
@@ -1855,7 +1860,7 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     if (e != hipSuccess) return hip_fail(ctx, e, "hipMemcpyAsync(tables)");
     e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
-    rc = enqueue(ctx, P, d_arena, nullptr, d_out, d_eps, d_counts, st, false);
+    const int rc = enqueue(ctx, P, d_arena, nullptr, d_out, d_eps, d_counts, st, false);
     if (rc) return rc;
     ctx->static_plan = std::move(up);
     ctx->last = ctx->static_plan.get();

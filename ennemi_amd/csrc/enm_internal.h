@@ -45,22 +45,19 @@
 // Two-column kNN: strips up to this size are walked a strip per workgroup
 // with the strip and its two neighbours staged in LDS (3 x 1024 x 16 B).
 #define ENM_STRIP_LDS_MAX 1024
-// Default strip of instances of three or more joint columns.  Their kNN and
-// counts run on box trees; strips of this size serve only the grid sweeps
-// of k+1 > ENM_TREE_K1_MAX.
+// Default strip of instances of three or more joint columns.  (Any size but
+// 0 puts them on box trees, which are cut without it.)
 #define ENM_STRIP_WIDE 4096
 // Box trees (enm_tree.hip).
 #define ENM_LEAF 64            // points per leaf (one per lane)
 #define ENM_CELL 4096          // points per cell: ENM_LEAF leaves of ENM_LEAF points
 #define ENM_TREE_STEPS 6       // most sorted columns of a cell (one halving of its leaves each at least)
-#define ENM_TREE_K1_MAX 128    // longest neighbour list held across a wave's lanes
+#define ENM_TREE_LISTS 8       // most registers of a neighbour list held across a wave's lanes (64 each)
 // How a kNN group runs (and, on trees, a count group).
 #define ENM_WALK_NONE 0        // key order: plain or brute force
-#define ENM_WALK_LANES 1       // two-column grid order, per-lane walks (global heaps)
-#define ENM_WALK_STRIP 2       // two-column grid order, a strip per workgroup
-#define ENM_WALK_SWEEP 3       // wider grid order, tile-shared sweeps (global heaps)
-#define ENM_WALK_TREE 4        // box tree
-#define ENM_WALK_LINE 5        // one column: windows of the sorted keys
+#define ENM_WALK_STRIP 1       // two-column grid order, a strip per workgroup
+#define ENM_WALK_TREE 2        // box tree
+#define ENM_WALK_LINE 3        // one column: windows of the sorted keys
 #define ENM_LINE_THREADS 256
 #define ENM_LINE_ITEM 2048     // positions per one-column item
 #define ENM_TREE_BASE_CELLS 4  // scopes of more cells are cut by two columns, not one

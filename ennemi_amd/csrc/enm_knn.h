@@ -6,28 +6,19 @@
 // all j of the query's scope range, i itself included (distance 0); fewer
 // than k+1 points leave it +inf, as cKDTree does.
 //
-// Box trees (enm_tree_knn.hip) serve spaces of two or more columns, except:
+// Box trees (enm_tree_knn.hip) serve spaces of two or more columns and sorted
+// windows (enm_knn.hip) one column, except:
 //
 // Two columns and register lists: grid orders (the key-sorted points cut into
 // strips, each strip sorted by the second column), a strip per workgroup with
 // its neighbours staged in LDS (knn_strip_kernel below).
 //
-// Lists of more than ENM_TREE_K1_MAX distances: heaps in global memory, on grid
-// orders.  With two columns each lane walks the strips around its own point by
-// itself (knn_walk): its own strip from its own position, then the strips
-// outward that its current radius still reaches on the key axis, each from the
-// lane's y position in both directions until the y distance reaches the
-// radius.  With more columns a wave takes a tile of 64 consecutive positions
-// of a strip and walks candidates in wave-uniform order (grid_sweep: its own
-// strip, then the strips outward, each within the union of the lanes' y
-// intervals).
-//
-// One column, ENM_F_BRUTE and tunings without strips: the key-sorted order, 8
-// candidates at a time through the scalar cache (candidate coordinates are
-// SGPR operands), from the tile outward in key order, alternating left and
-// right in steps of 64, a side stopping once every lane's key distance to the
-// last visited candidate is >= its current K1-th distance T.  With ENM_F_BRUTE
-// the whole scope range is scanned.
+// ENM_F_BRUTE and tunings without strips: the key-sorted order, 8 candidates
+// at a time through the scalar cache (candidate coordinates are SGPR
+// operands), from the tile outward in key order, alternating left and right in
+// steps of 64, a side stopping once every lane's key distance to the last
+// visited candidate is >= its current K1-th distance T.  With ENM_F_BRUTE the
+// whole scope range is scanned.
 //
 // Precision.  Every distance that enters a list is exact FP64.  The FP32
 // filter (brute force in FP32-filter mode) computes the bulk distance from
@@ -392,228 +383,6 @@ struct KnnTile {
     }
 };
 
-// First position in [ks, ke) whose key is >= y, one search per lane (the
-// trip count depends only on ke - ks, up to one step).
-__device__ __forceinline__ int lane_lower_bound(const double* __restrict__ v, int ks, int ke, double y) {
-    int first = ks, len = ke - ks;
-    while (len > 0) {
-        const int half = len >> 1;
-        const bool go = v[first + half] < y;
-        first = go ? first + half + 1 : first;
-        len = go ? len - half - 1 : half;
-    }
-    return first;
-}
-
-// Every live lane's lower bound lane_lower_bound(v, ks, ke, y), found by
-// the whole wave: the bounds [a, b) of the live lanes' y range in the strip
-// (wave_bounds, two rounds of independent probes for a 1024-point strip),
-// then, when that window holds at most 64 keys (the usual case: a wave's
-// 64 queries are consecutive in y, and so are their entry points), each
-// lane counts the window keys below its y by a binary search over the
-// window held one key per lane (shuffles, no memory round trips).  Wider
-// windows fall back to a per-lane search inside the window.  The result is
-// the exact lower bound of every live lane; other lanes get ks.
-__device__ __forceinline__ int wave_lower_bounds(const double* __restrict__ v, int ks, int ke, double y, bool live) {
-    const double lo = uni_f64(wave_min(live ? y : INFINITY));
-    const double hi = uni_f64(wave_max(live ? y : -INFINITY));
-    if (!(lo <= hi)) return ks;
-    int a, b;
-    wave_bounds(v, ks, ke, lo, hi, a, b);
-    const int L = b - a;
-    const int lane = (int)(threadIdx.x & (ENM_WAVE - 1));
-    if (L <= ENM_WAVE) {
-        const double key = lane < L ? v[a + lane] : INFINITY;
-        int pos = 0;
-#pragma unroll
-        for (int step = ENM_WAVE; step > 0; step >>= 1) {
-            const int idx = pos + step - 1;
-            const double kv = __shfl(key, idx < ENM_WAVE ? idx : ENM_WAVE - 1, ENM_WAVE);
-            if (idx < L && kv < y) pos += step;
-        }
-        return live ? a + pos : ks;
-    }
-    return live ? lane_lower_bound(v, a, b, y) : ks;
-}
-
-// Walk of one strip [ks, ke) (sorted by column 1) for every live lane, from
-// its own start: upward from u and downward from dn, one candidate per
-// direction and iteration, so candidates come in about increasing y
-// distance.  A direction stops at the first candidate whose y distance is
-// >= the lane's current radius T (the strip is sorted, so every later one
-// is further still, and T only decreases); the others are evaluated and
-// offered to the list (an insertion at or above T leaves it unchanged).
-// Candidates are (x, y) pairs of the interleaved copy, one 16-byte load
-// each (the lanes of a wave walk different positions, so every load
-// instruction touches up to 64 cache lines: one per candidate, not two);
-// the next candidate is loaded before the current one is evaluated.  Adds
-// the lane's evaluated candidates to `visited`.
-template <int P, bool F32>
-__device__ __forceinline__ void walk_strip(KnnTile<2, P, F32>& w, const double2* __restrict__ xy, int ks, int ke,
-                                           int u, int dn, bool live, unsigned& visited) {
-    const double qx = w.q64[0], qy = w.q64[1];
-    bool up = live && u < ke;
-    bool down = live && dn >= ks;
-    double2 cu = xy[up ? u : ks], cd = xy[down ? dn : ks];
-    while (wave_any(up || down)) {
-        const double2 nu = xy[up && u + 1 < ke ? u + 1 : ks];
-        const double2 nd = xy[down && dn - 1 >= ks ? dn - 1 : ks];
-        {
-            const double dy = cu.y - qy;
-            up = up && dy < w.T;
-            const double m = fmax(dy, fabs(cu.x - qx));
-            w.L.insert(up ? m : INFINITY);
-            w.T = w.L.top();
-            visited += up;
-        }
-        {
-            const double dy = qy - cd.y;
-            down = down && dy < w.T;
-            const double m = fmax(dy, fabs(cd.x - qx));
-            w.L.insert(down ? m : INFINITY);
-            w.T = w.L.top();
-            visited += down;
-        }
-        ++u;
-        --dn;
-        up = up && u < ke;
-        down = down && dn >= ks;
-        cu = nu;
-        cd = nd;
-    }
-}
-
-// kNN on a grid order by per-lane walks: each lane walks its own strip
-// from its own position, then the strips outward on each side that its
-// radius still reaches on the key axis (x gap to the strip < T), entering
-// each at its own y position (per-lane binary search).  A side stops for
-// the wave once no lane reaches the next strip (strips further out are
-// further in x).  Every candidate that could enter a lane's list is
-// evaluated, in about increasing distance, so lists settle early; a lane
-// evaluates a few dozen candidates instead of the whole tile's window.
-// Returns the lane's number of evaluated candidates (the query itself
-// included).
-template <int P, bool F32>
-__device__ unsigned knn_walk(KnnTile<2, P, F32>& w, const double2* __restrict__ xy, const KnnDev& kd,
-                             const double* __restrict__ col64, int lo, int hi, int t0, int i, bool active) {
-    const int S = kd.strip;
-    const double* xk = col64 + kd.base_key;  // base order: column 0 sorted over [lo, hi)
-    const int s = (t0 - lo) / S;
-    const int nstrip = (hi - lo + S - 1) / S;
-    unsigned visited = active ? 1u : 0u;
-    if (active) {
-        w.L.insert(0.0);  // the query itself
-        w.T = w.L.top();
-    }
-    {
-        const int ss = lo + s * S, se = min(hi, ss + S);
-        walk_strip(w, xy, ss, se, i + 1, i - 1, active, visited);
-    }
-    bool ldone = s == 0, rdone = s == nstrip - 1;
-    for (int d = 1; !(ldone && rdone); ++d) {
-        if (!ldone) {
-            const int sl = s - d;
-            if (sl < 0) {
-                ldone = true;
-            } else {
-                const int ks = lo + sl * S, ke = ks + S;  // a full strip (left of s)
-                const bool need = active && w.q64[0] - xk[ke - 1] < w.T;
-                ldone = !wave_any(need);
-                if (!ldone) {
-                    const int p = wave_lower_bounds(w.c64[1], ks, ke, w.q64[1], need);
-                    walk_strip(w, xy, ks, ke, p, p - 1, need, visited);
-                }
-            }
-        }
-        if (!rdone) {
-            const int sr = s + d;
-            if (sr >= nstrip) {
-                rdone = true;
-            } else {
-                const int ks = lo + sr * S, ke = min(hi, ks + S);
-                const bool need = active && xk[ks] - w.q64[0] < w.T;
-                rdone = !wave_any(need);
-                if (!rdone) {
-                    const int p = wave_lower_bounds(w.c64[1], ks, ke, w.q64[1], need);
-                    walk_strip(w, xy, ks, ke, p, p - 1, need, visited);
-                }
-            }
-        }
-    }
-    return visited;
-}
-
-// Grid sweep of one tile (already seeded with its own 64 points): the rest
-// of the tile's strip near the tile in y order, then whole strips outward on
-// both sides.  A strip is visited only within the y window of the lanes'
-// current radii; a side stops at the first strip whose x bound is at least
-// every lane's radius away (all strips beyond it are further in x).  Each
-// candidate is visited at most once, and every candidate that could still
-// enter a lane's list is visited.  Returns the number of candidates visited.
-template <int D, int P, bool F32>
-__device__ int grid_sweep(KnnTile<D, P, F32>& w, const KnnDev& kd, const double* __restrict__ col64,
-                          int lo, int hi, int t0, int t1, bool active) {
-    constexpr int SEED = 64;
-    const int S = kd.strip;
-    const double* xk = col64 + kd.base_key;  // base order: column 0 sorted over [lo, hi)
-    const double* yc = w.c64[1];             // column 1, sorted inside each strip
-    const int s = (t0 - lo) / S;
-    const int nstrip = (hi - lo + S - 1) / S;
-    const int ss = lo + s * S, se = min(hi, ss + S);
-    const double yq = w.q64[1];
-    int visited = 0;
-    // Seed: up to SEED neighbours in y on each side of the tile.
-    const int a0 = max(ss, t0 - SEED), b0 = min(se, t1 + SEED);
-    w.range(a0, t0);
-    w.range(t1, b0);
-    visited += (t0 - a0) + (b0 - t1);
-    {
-        int a, b;
-        strip_window(yc, ss, se, yq, w.T, active, a, b);
-        if (a < a0) { w.range(a, a0); visited += a0 - a; }
-        if (b > b0) { w.range(b0, b); visited += b - b0; }
-    }
-    bool ldone = s == 0, rdone = s == nstrip - 1;
-    for (int d = 1; !(ldone && rdone); ++d) {
-        if (!ldone) {
-            const int sl = s - d;
-            if (sl < 0) {
-                ldone = true;
-            } else {
-                const int le = lo + (sl + 1) * S;  // strip sl is [le - S, le)
-                const double xb = xk[le - 1];      // largest x of strip sl
-                // Lanes whose radius reaches this strip on the key axis.
-                const bool need = w.q64[0] - xb < w.T;
-                ldone = !wave_any(need);
-                if (!ldone) {
-                    int a, b;
-                    strip_window(yc, le - S, le, yq, w.T, need, a, b);
-                    w.range(a, b);
-                    visited += b - a;
-                }
-            }
-        }
-        if (!rdone) {
-            const int sr = s + d;
-            if (sr >= nstrip) {
-                rdone = true;
-            } else {
-                const int rs = lo + sr * S;
-                const double xb = xk[rs];          // smallest x of strip sr
-                const bool need = xb - w.q64[0] < w.T;
-                rdone = !wave_any(need);
-                if (!rdone) {
-                    int a, b;
-                    strip_window(yc, rs, min(hi, rs + S), yq, w.T, need, a, b);
-                    w.range(a, b);
-                    visited += b - a;
-                }
-            }
-        }
-    }
-    return visited;
-}
-
 template <int D, int P, bool F32>
 __device__ void knn_item(const KnnArgs& A, const Item& it, const double* __restrict__ col64,
                          const float* __restrict__ col32, double* __restrict__ res64,
@@ -650,15 +419,7 @@ __device__ void knn_item(const KnnArgs& A, const Item& it, const double* __restr
     const int lo = it.lo, hi = it.hi, t0 = it.t0, t1 = it.t1;
     int visited = t1 - t0;
     w.range(t0, t1);
-    bool swept = false;
-    if constexpr (D >= 2 && P == ENM_LIST_HEAP_GLOBAL) {
-        if (kd.strip > 0 && !A.brute) {
-            visited += grid_sweep(w, kd, col64, lo, hi, t0, t1, active);
-            swept = true;
-        }
-    }
-    if (swept) {
-    } else if (A.brute) {
+    if (A.brute) {
         w.range(lo, t0);
         w.range(t1, hi);
         visited = hi - lo;
@@ -691,48 +452,6 @@ __device__ void knn_item(const KnnArgs& A, const Item& it, const double* __restr
     }
     pairs += (unsigned long long)(t1 - t0) * (unsigned long long)visited;
     if (F32) rechecks += wave_sum_u64(w.rechecks);
-}
-
-// One grid-order item of a two-column order by per-lane walks (knn_walk).
-template <int P>
-__device__ void walk_item(const KnnArgs& A, const Item& it, const double* __restrict__ col64,
-                          double* __restrict__ res64, unsigned long long& pairs) {
-    const KnnDev kd = A.descs[it.desc];
-    const OrderDev od = A.orders[kd.order];
-    const int64_t n = od.n;
-    const int i = it.t0 + (int)threadIdx.x;
-    const bool active = i < it.t1;
-    KnnTile<2, P, false> w;
-#pragma unroll
-    for (int d = 0; d < 2; ++d) {
-        w.c64[d] = col64 + od.c64 + d * n;
-        w.q64[d] = active ? w.c64[d][i] : 0.0;
-    }
-    const double2* xy = reinterpret_cast<const double2*>(col64 + od.xy);
-    const int K1 = kd.k + 1;
-    w.L.init(K1, heap_base<P>(A));
-    w.T = active ? INFINITY : -INFINITY;
-    const unsigned v = knn_walk(w, xy, kd, col64, it.lo, it.hi, it.t0, i, active);
-    const double eps = w.L.top();
-    if (active) {
-        if (kd.eps >= 0) res64[kd.eps + i] = eps;
-        if (kd.eps_orig >= 0) res64[kd.eps_orig + A.perm[od.perm + i]] = eps;
-    }
-    pairs += wave_sum_u64(v);
-}
-
-template <int P>
-__global__ __launch_bounds__(ENM_WAVE)
-void knn_walk_kernel(KnnArgs A, const double* __restrict__ col64, double* __restrict__ res64,
-                     unsigned long long* __restrict__ stats) {
-    unsigned long long pairs = 0;
-    for_each_wave_item(A.qoff, A.counter, A.chunk, [&](int idx) {
-        Item it = A.items[idx];
-        it.desc = uni(it.desc); it.tile = uni(it.tile);
-        it.lo = uni(it.lo); it.hi = uni(it.hi); it.t0 = uni(it.t0); it.t1 = uni(it.t1);
-        walk_item<P>(A, it, col64, res64, pairs);
-    });
-    if (threadIdx.x == 0) add_stat(stats, ST_KNN_PAIRS, pairs);
 }
 
 // ---------------------------------------------------------------------------
@@ -1159,7 +878,7 @@ hipError_t launch_dp(const KnnArgs& a, bool f32, int walk, int grid, const doubl
     // LDS heaps: 64 lanes x the group's largest K1 doubles per workgroup.
     const unsigned shmem = P == ENM_LIST_HEAP_LDS ? (unsigned)(a.heap_stride * sizeof(double)) : 0u;
     // Strip workgroups: two-column grid orders, register lists (their LDS
-    // holds strips); per-lane walks: the same orders, global heaps.
+    // holds strips).
     if (walk == ENM_WALK_STRIP) {
         if constexpr (D == 2 && P > 0) {
             const int nt = a.smax >= SK_THREADS_MAX ? SK_THREADS_MAX : ((a.smax + 63) / 64) * 64;
@@ -1170,13 +889,6 @@ hipError_t launch_dp(const KnnArgs& a, bool f32, int walk, int grid, const doubl
             if (a.far != nullptr)
                 hipLaunchKernelGGL((knn_far_kernel<P>), dim3(std::max(1, grid) * 8 / 3 + 1), dim3(256), 0, st,
                                    a, col64, res64, stats);
-            return hipGetLastError();
-        }
-        return hipErrorInvalidValue;
-    }
-    if (walk == ENM_WALK_LANES) {
-        if constexpr (D == 2 && P == ENM_LIST_HEAP_GLOBAL) {
-            hipLaunchKernelGGL((knn_walk_kernel<P>), dim3(grid), dim3(ENM_WAVE), 0, st, a, col64, res64, stats);
             return hipGetLastError();
         }
         return hipErrorInvalidValue;

@@ -82,7 +82,8 @@ hipError_t enm_launch_tree_build(const CellItem* items, int n_items, const CellI
 hipError_t enm_launch_tree_knn(const Item* items, const int* qoff, int n_items, int qmax, int share,
                                const KnnDev* descs,
                                const TreeDev* trees, const int* perm, const double* col64, double* res64,
-                               unsigned long long* stats, int dclass, int k1max, hipStream_t st);
+                               unsigned long long* stats, int dclass, int lists, hipStream_t st);
+int enm_tree_list_class(int k1);   // registers of the neighbour list for k1 = k + 1
 hipError_t enm_launch_tree_count(const Item* items, const int* qoff, int n_items, int qmax, int share,
                                  const CountDev* descs,
                                  const TreeDev* trees, const int* perm, const double* psi_tab, const double* col64,

@@ -146,8 +146,11 @@ struct LaneList {
     }
 
     __device__ __forceinline__ double rank(int t) const {
-        if constexpr (NR == 1) return lane_f64(L[0], t);
-        else return t < 64 ? lane_f64(L[0], t) : lane_f64(L[1], t - 64);
+        double v = lane_f64(L[0], t & 63);
+#pragma unroll
+        for (int r = 1; r < NR; ++r)
+            if (t >= 64 * r) v = lane_f64(L[r], t & 63);
+        return v;
     }
 
     // One value (the same in every lane): every rank takes
@@ -236,6 +239,80 @@ __device__ __forceinline__ double box_gap(const double* __restrict__ b, int ncol
 
 __device__ __forceinline__ unsigned long long low_mask(int n) {
     return n >= 64 ? ~0ull : ((1ull << n) - 1ull);
+}
+
+// Points within r of q, max_d fl64(|a_d - q_d|) <= r: a node whose box lies
+// within the radius in every column adds its points unopened, one out of reach
+// adds none; the others are opened, leaves by their points.
+template <int D>
+__device__ __forceinline__ int count_cell(const TreeDev& T, const double* __restrict__ col64, int cell,
+                                          const double (&q)[D], double r, unsigned& opened) {
+    const int ncol = T.ncol;
+    const int cnt = min(T.cell, T.n - cell * T.cell);
+    const int nleaf = (cnt + ENM_LEAF - 1) / ENM_LEAF;
+    unsigned long long part = 1;
+    int c = 0;
+    if (T.n > ENM_LEAF) {
+        double far;
+        const double g = box_gap<D, true>(col64 + T.box + (int64_t)cell * 2 * ncol * 64, ncol, q, far);
+        const unsigned long long inside = __builtin_amdgcn_ballot_w64(far <= r) & low_mask(nleaf);
+        part = __builtin_amdgcn_ballot_w64(g <= r) & low_mask(nleaf) & ~inside;
+        c = (int)__popcll(inside) * ENM_LEAF;
+        if ((inside >> (nleaf - 1)) & 1) c -= nleaf * ENM_LEAF - cnt;
+    }
+    opened += (unsigned)__popcll(part);
+    const double* leaves = col64 + T.col + (int64_t)cell * T.cell * ncol;
+    // Two leaves at a time, so that their loads overlap (an odd last one is
+    // loaded twice and counted once).
+    while (part) {
+        const int l0 = __builtin_ctzll(part);
+        part &= part - 1;
+        const int l1 = part ? __builtin_ctzll(part) : l0;
+        const bool two = part != 0;
+        part &= part - 1;
+        double a[D], b[D];
+        load_leaf<D>(a, leaves + l0 * ENM_LEAF * ncol, ncol);
+        load_leaf<D>(b, leaves + l1 * ENM_LEAF * ncol, ncol);
+        const int ca = (int)__popcll(__builtin_amdgcn_ballot_w64(point_dist<D>(a, q) <= r));
+        const int cb = (int)__popcll(__builtin_amdgcn_ballot_w64(point_dist<D>(b, q) <= r));
+        c += ca + (two ? cb : 0);
+    }
+    return c;
+}
+
+template <int D>
+__device__ __forceinline__ int count_query(const TreeDev& T, const double* __restrict__ col64, const double (&q)[D],
+                                           double r, unsigned& opened) {
+    const int ncell = T.ncell, ncol = T.ncol;
+    if (ncell == 1) return count_cell<D>(T, col64, 0, q, r, opened);
+    const int ngroup = (ncell + 63) / 64;
+    int c = 0;
+    double far;
+    // Groups that the ball meets, 64 at a time; then their cells.
+    for (int gb = 0; gb < ngroup; gb += 64) {
+        unsigned long long gm = 1;
+        if (ngroup > 1) {
+            const double g = box_gap<D, false>(col64 + T.gbox + (int64_t)(gb / 64) * 2 * ncol * 64, ncol, q, far);
+            gm = __builtin_amdgcn_ballot_w64(g <= r) & low_mask(ngroup - gb);
+        }
+        while (gm) {
+            const int gr = gb + __builtin_ctzll(gm);
+            gm &= gm - 1;
+            const double g = box_gap<D, true>(col64 + T.cbox + (int64_t)gr * 2 * ncol * 64, ncol, q, far);
+            const unsigned long long valid = low_mask(ncell - gr * 64);
+            const unsigned long long inside = __builtin_amdgcn_ballot_w64(far <= r) & valid;
+            unsigned long long part = __builtin_amdgcn_ballot_w64(g <= r) & valid & ~inside;
+            c += (int)__popcll(inside) * T.cell;
+            const int last = ncell - 1 - gr * 64;   // the scope's last cell, if it is here
+            if (last < 64 && ((inside >> last) & 1)) c -= ncell * T.cell - T.n;
+            while (part) {
+                const int k = gr * 64 + __builtin_ctzll(part);
+                part &= part - 1;
+                c += count_cell<D>(T, col64, k, q, r, opened);
+            }
+        }
+    }
+    return c;
 }
 
 // Waves per SIMD that the kernels of dimension class D are held to registers

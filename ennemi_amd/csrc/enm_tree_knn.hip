@@ -8,15 +8,20 @@
 // the nearest first, so T is close to its final value after a leaf or two.  A
 // leaf's few distances below T go into the list one at a time (a shift by one
 // lane, a minimum and a maximum for up to 64 neighbours); where there are
-// many, as with long lists, they are sorted and merged.
+// many, as with long lists, they are sorted and merged.  Lists longer than
+// 64 * ENM_TREE_LISTS are taken in passes: each finds the next ranks above the
+// last pass's highest distance B, after counting the points within B.  4 x
+// 50,000 points in two columns: k = 126 in 0.59 ms, 200 in 1.13, 600 in 8.5,
+// where walks with a heap per lane took 3.1, 6.4 and 28; in four columns 1.6,
+// 3.3 and 23 ms, where sweeps shared by 64 queries took 49, 77 and 267.
 #include "enm_tree.h"
 
 namespace {
 
 // Distances below T at which sorting and merging all 64 beats inserting one by
-// one: about 140 (one register of ranks) or 200 instructions against 11 or 15
-// each.
-constexpr int MERGE_FROM = 13;
+// one: about 140, 210, 350 or 630 instructions (1, 2, 4 or 8 registers of
+// ranks) against 11, 15, 23 or 39 each.
+constexpr int MERGE_FROM = 14;
 
 template <int D, int NR>
 struct TreeQuery {
@@ -27,12 +32,16 @@ struct TreeQuery {
     LaneList<NR> list;
     int K1;
     double t;            // the current radius
+    double above;        // only distances above this are ranked (last registers only)
     unsigned visited;    // leaves
+
+    static constexpr bool PASSES = NR == ENM_TREE_LISTS;
 
     __device__ __forceinline__ void visit_leaf(const double* leaf) {
         double a[D];
         load_leaf<D>(a, leaf, ncol);
-        const double e = point_dist<D>(a, q);
+        double e = point_dist<D>(a, q);
+        if (PASSES) e = e > above ? e : INFINITY;
         unsigned long long m = __builtin_amdgcn_ballot_w64(e < t);
         ++visited;
         if (__popcll(m) >= MERGE_FROM) {
@@ -101,7 +110,7 @@ struct TreeQuery {
 };
 
 template <int D, int NR>
-__global__ __launch_bounds__(TREE_WG* ENM_WAVE, tree_waves(D))
+__global__ __launch_bounds__(TREE_WG* ENM_WAVE, std::min(tree_waves(D), NR <= 2 ? 8 : NR <= 4 ? 6 : 4))
 void tree_knn_kernel(TreeArgs A, const KnnDev* __restrict__ descs, const double* __restrict__ col64,
                      double* __restrict__ res64, unsigned long long* __restrict__ stats) {
     const TreeWork it = tree_work(A);
@@ -116,18 +125,30 @@ void tree_knn_kernel(TreeArgs A, const KnnDev* __restrict__ descs, const double*
     const int cell = leaf * ENM_LEAF / T.cell;
     double own[D];
     load_leaf<D>(own, col64 + T.col + (int64_t)leaf * ncol * ENM_LEAF, ncol);
+    constexpr bool PASSES = TreeQuery<D, NR>::PASSES;
     double mine = 0.0;
     unsigned visited = 0;
     for (int j = 0; j < nq; ++j) {
         TreeQuery<D, NR> w{T, col64, ncol};
 #pragma unroll
         for (int d = 0; d < D; ++d) w.q[d] = lane_f64(own[d], j0 + j);
-        w.K1 = kd.k + 1;
-        w.visited = visited + 1;
-        w.list.seed(vmin(point_dist<D>(own, w.q), INFINITY));   // (NaN: +inf)
-        w.t = w.list.rank(w.K1 - 1);
-        if (T.n > ENM_LEAF) w.visit_cell(cell, leaf - cell * (T.cell / ENM_LEAF));
-        if (T.ncell > 1) w.visit_others(cell);
+        const int k1 = kd.k + 1;
+        const double e0 = vmin(point_dist<D>(own, w.q), INFINITY);   // (NaN: +inf)
+        w.visited = visited;
+        w.above = -INFINITY;
+        int found = 0;   // points ranked by the passes before
+        for (;;) {
+            w.K1 = PASSES ? min(k1 - found, 64 * NR) : k1;
+            w.list.seed(PASSES ? (e0 > w.above ? e0 : INFINITY) : e0);
+            w.t = w.list.rank(w.K1 - 1);
+            ++w.visited;
+            if (T.n > ENM_LEAF) w.visit_cell(cell, leaf - cell * (T.cell / ENM_LEAF));
+            if (T.ncell > 1) w.visit_others(cell);
+            if (!PASSES || found + w.K1 == k1 || !(w.t < INFINITY)) break;
+            found = count_query<D>(T, col64, w.q, w.t, w.visited);
+            if (found >= k1) break;   // ties at the last rank
+            w.above = w.t;
+        }
         if (lane == j) mine = w.t;
         visited = w.visited;
     }
@@ -136,35 +157,41 @@ void tree_knn_kernel(TreeArgs A, const KnnDev* __restrict__ descs, const double*
 }
 
 template <int D>
-hipError_t launch(const TreeArgs& a, int qmax, int k1max, const KnnDev* descs, const double* col64, double* res64,
+hipError_t launch(const TreeArgs& a, int qmax, int lists, const KnnDev* descs, const double* col64, double* res64,
                   unsigned long long* stats, hipStream_t st) {
     const dim3 grid(tree_grid(qmax, a.share)), block(TREE_WG * ENM_WAVE);
-    if (k1max <= 64)
-        hipLaunchKernelGGL((tree_knn_kernel<D, 1>), grid, block, 0, st, a, descs, col64, res64, stats);
-    else if (k1max <= ENM_TREE_K1_MAX)
-        hipLaunchKernelGGL((tree_knn_kernel<D, 2>), grid, block, 0, st, a, descs, col64, res64, stats);
-    else
-        return hipErrorInvalidValue;
+#define ENM_TREE_KNN(NR) \
+    case NR: hipLaunchKernelGGL((tree_knn_kernel<D, NR>), grid, block, 0, st, a, descs, col64, res64, stats); break;
+    switch (lists) {
+        ENM_TREE_KNN(1)
+        ENM_TREE_KNN(2)
+        ENM_TREE_KNN(4)
+        ENM_TREE_KNN(ENM_TREE_LISTS)
+        default: return hipErrorInvalidValue;
+    }
+#undef ENM_TREE_KNN
     return hipGetLastError();
 }
 
 }  // namespace
 
+int enm_tree_list_class(int k1) { return k1 <= 64 ? 1 : k1 <= 128 ? 2 : k1 <= 256 ? 4 : ENM_TREE_LISTS; }
+
 hipError_t enm_launch_tree_knn(const Item* items, const int* qoff, int n_items, int qmax, int share,
                                const KnnDev* descs,
                                const TreeDev* trees, const int* perm, const double* col64, double* res64,
-                               unsigned long long* stats, int dclass, int k1max, hipStream_t st) {
+                               unsigned long long* stats, int dclass, int lists, hipStream_t st) {
     if (n_items <= 0) return hipSuccess;
     const TreeArgs a{items, qoff, share, trees, perm, nullptr};
     switch (dclass) {
-        case 2: return launch<2>(a, qmax, k1max, descs, col64, res64, stats, st);
-        case 3: return launch<3>(a, qmax, k1max, descs, col64, res64, stats, st);
-        case 4: return launch<4>(a, qmax, k1max, descs, col64, res64, stats, st);
-        case 5: return launch<5>(a, qmax, k1max, descs, col64, res64, stats, st);
-        case 6: return launch<6>(a, qmax, k1max, descs, col64, res64, stats, st);
-        case 8: return launch<8>(a, qmax, k1max, descs, col64, res64, stats, st);
-        case 12: return launch<12>(a, qmax, k1max, descs, col64, res64, stats, st);
-        case 16: return launch<16>(a, qmax, k1max, descs, col64, res64, stats, st);
+        case 2: return launch<2>(a, qmax, lists, descs, col64, res64, stats, st);
+        case 3: return launch<3>(a, qmax, lists, descs, col64, res64, stats, st);
+        case 4: return launch<4>(a, qmax, lists, descs, col64, res64, stats, st);
+        case 5: return launch<5>(a, qmax, lists, descs, col64, res64, stats, st);
+        case 6: return launch<6>(a, qmax, lists, descs, col64, res64, stats, st);
+        case 8: return launch<8>(a, qmax, lists, descs, col64, res64, stats, st);
+        case 12: return launch<12>(a, qmax, lists, descs, col64, res64, stats, st);
+        case 16: return launch<16>(a, qmax, lists, descs, col64, res64, stats, st);
         default: return hipErrorInvalidValue;
     }
 }

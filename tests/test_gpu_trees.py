@@ -89,11 +89,24 @@ def test_sizes_and_forms(n, form):
         assert vals[i] == w or abs(vals[i] - w) <= 1e-12 or (np.isnan(w) and np.isnan(vals[i]))
 
 
+@pytest.mark.parametrize("form", ["plain", "ties"])
+@pytest.mark.parametrize("k", [255, 256, 511, 512, 1100, 1999, 2000])
+@pytest.mark.parametrize("d", [2, 3, 16])
+def test_long_lists(d, k, form):
+    """The longest lists, and those that take several passes (ties at the
+    rank where one ends), up to more neighbours than points."""
+    nat = _nat()
+    a = _data(2000, d, 7 * d + k, form)
+    _, eps, _ = _both(lambda b: b.add(nat.KIND_KL, k, _cols(a)))
+    _, ref = orc.estimate_single_entropy(a, k, detail=True)
+    np.testing.assert_array_equal(eps[0], ref["eps"])
+
+
 @pytest.mark.parametrize("k", [3, 63, 64, 127, 128])
 @pytest.mark.parametrize("d", [2, 3, 4, 5, 6, 7, 9, 13, 16])
 def test_columns_and_list_lengths(d, k):
-    """Every column class and the ends of both list lengths (two columns with
-    short lists run on strips, k = 128 on the grid sweeps)."""
+    """Every column class and the ends of the shorter list lengths (two
+    columns with short lists run on strips)."""
     nat = _nat()
     a = _data(5000, d, 31 * d + k)
     _, eps, _ = _both(lambda b: b.add(nat.KIND_KL, k, _cols(a)))
