@@ -99,7 +99,7 @@ def _instance_table(inst: List[tuple], col_offsets: Optional[np.ndarray]):
     inst_arr = (nat.EnmInstance * n_inst)()
     if n_inst == 0:
         return inst_arr
-    tab = np.ctypeslib.as_array(inst_arr)   # the same memory, field by field
+    tab = nat.struct_array(inst_arr)
     head = np.array([t[:8] for t in inst], dtype=np.int64).reshape(n_inst, 8)
     for f, name in enumerate(("kind", "k", "n", "dx", "dy", "dz", "n_segs", "seg_index")):
         tab[name] = head[:, f]
@@ -177,29 +177,48 @@ class DeviceBatch:
 
 class ArenaBatch:
     """A batch whose float64 arena was written on the device (the columns
-    of device-prepared estimate_mi tasks, enm_prep_write), with the sort
-    hints of its columns when they were made (enm_prep_hints); instances
-    name their columns by arena offset.  Same interface as Batch."""
+    of device-prepared tasks, enm_prep_write), with the sort hints of its
+    columns when they were made (enm_prep_hints); instances name their
+    columns by arena offset.  Same interface as Batch."""
 
     def __init__(self, device_arena, device_hint=None) -> None:
         self.device_arena = device_arena
         self.device_hint = device_hint
-        self._inst: List[tuple] = []
+        self._runs: List[tuple] = []   # (kind, k, n per instance, dx, dy, dz, offsets per instance)
 
     def __len__(self) -> int:
-        return len(self._inst)
+        return sum(len(r[2]) for r in self._runs)
 
     def add(self, kind: int, k: int, n: int, offsets: Sequence[int], dx: int, dy: int, dz: int) -> int:
-        self._inst.append((kind, int(k), int(n), dx, dy, dz, 1, 0, [int(o) for o in offsets]))
-        return len(self._inst) - 1
+        self.add_many(kind, k, [n], [offsets], dx, dy, dz)
+        return len(self) - 1
+
+    def add_many(self, kind: int, k: int, n, offsets, dx: int, dy: int, dz: int) -> None:
+        """Instances of one kind: their points n (per instance) and column
+        offsets (per instance and column)."""
+        self._runs.append((kind, int(k), np.asarray(n, dtype=np.int64), dx, dy, dz,
+                           np.asarray(offsets, dtype=np.int64)))
+
+    @property
+    def _inst(self) -> List[tuple]:
+        return [(kind, k, int(n), dx, dy, dz, 1, 0, [int(o) for o in offs])
+                for kind, k, ns, dx, dy, dz, cols in self._runs for n, offs in zip(ns, cols)]
 
     def pack(self):
-        inst_arr = _instance_table(self._inst, None)
+        inst_arr = (nat.EnmInstance * len(self))()
+        tab = nat.struct_array(inst_arr)
+        at = 0
+        for kind, k, n, dx, dy, dz, cols in self._runs:
+            t = tab[at:at + len(n)]
+            at += len(n)
+            for name, v in (("kind", kind), ("k", k), ("n", n), ("dx", dx), ("dy", dy), ("dz", dz), ("n_segs", 1)):
+                t[name] = v
+            t["col"][:, :cols.shape[1]] = cols
         seg_arr = (ctypes.c_int64 * 1)(0)
         return None, inst_arr, seg_arr
 
     def point_offsets(self) -> np.ndarray:
-        n = np.array([t[2] for t in self._inst], dtype=np.int64)
+        n = np.concatenate([np.zeros(0, dtype=np.int64)] + [r[2] for r in self._runs])
         return np.concatenate([[0], np.cumsum(n)])
 
     def device(self, flags: int = 0, export: bool = False, hints: bool = True):

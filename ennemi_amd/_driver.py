@@ -427,7 +427,11 @@ def _device_prep_eligible(x, y, cond, discrete_x: bool, discrete_y: bool) -> boo
     boolean, which NumPy computes with in float64) x, y and condition."""
     if discrete_x or discrete_y:
         return False
-    for a in (x, y) if cond is None else (x, y, cond):
+    return _device_prep_arrays((x, y) if cond is None else (x, y, cond), cond)
+
+
+def _device_prep_arrays(arrays, cond) -> bool:
+    for a in arrays:
         if a.dtype.kind not in "fiub" or (a.dtype.kind == "f" and a.dtype != np.float64):
             return False
     if cond is not None and cond.shape[1] > nat.PREP_MAXZ:
@@ -466,50 +470,61 @@ class DevicePrep:
 
     def __init__(self, y, x, lag, cond, cond_lag, mask, preprocess, drop_nan, min_lag, max_lag, indices,
                  hints: bool = True):
+        n_rows = len(y)
+        nvar = 1 if x.ndim == 1 else x.shape[1]
+        dz = 0 if cond is None else cond.shape[1]
+        n_tasks = len(indices)
+        self._begin([y, x] + ([] if cond is None else [cond]), mask, dz, n_tasks, preprocess, drop_nan, hints)
+        min_lag = min(min_lag, 0)
+        max_lag = max(max_lag, 0)
+        # Device order: by x column, then lag, so a kernel's consecutive
+        # blocks (one XCD's share) read one x series.
+        idx = np.asarray(indices, dtype=np.int64).reshape(n_tasks, 2)
+        order = np.lexsort((idx[:, 0], idx[:, 1]))
+        self.place[order] = np.arange(n_tasks)
+        li, v = idx[order, 0], idx[order, 1]
+        tab = nat.struct_array(self.tasks)
+        tab["x_col"] = (1 + v) * n_rows
+        tab["y_col"] = 0
+        tab["x0"] = max_lag - np.asarray(lag, dtype=np.int64)[li]
+        tab["y0"] = max_lag
+        tab["w"] = n_rows - max_lag + min_lag
+        if dz:
+            cl = np.asarray(cond_lag, dtype=np.int64).reshape(len(lag), -1)
+            tab["z_col"][:, :dz] = (1 + nvar + np.arange(dz)) * n_rows
+            tab["z0"][:, :dz] = max_lag - cl[li, :dz]
+
+    @classmethod
+    def of_columns(cls, data, cond, mask, preprocess, drop_nan, pairs) -> "DevicePrep":
+        """The preparation of column pairs (i, j) of a table, x = column i and
+        y = column j, all rows; tasks stay in the given order."""
+        self = cls.__new__(cls)
+        n_rows, nvar = data.shape
+        dz = 0 if cond is None else cond.shape[1]
+        self._begin([data] + ([] if cond is None else [cond]), mask, dz, len(pairs), preprocess, drop_nan, True)
+        tab = nat.struct_array(self.tasks)
+        tab["x_col"] = pairs[:, 0] * n_rows
+        tab["y_col"] = pairs[:, 1] * n_rows
+        tab["w"] = n_rows
+        if dz:
+            tab["z_col"][:, :dz] = (nvar + np.arange(dz)) * n_rows
+        return self
+
+    def _begin(self, arrays, mask, dz: int, n_tasks: int, preprocess, drop_nan, hints: bool) -> None:
         import torch
         from ._batch import _stream
         self.ctx = nat.context()
         self.dev = torch.device("cuda", self.ctx.device)
         self.st = _stream()
-        n_rows = len(y)
-        nvar = 1 if x.ndim == 1 else x.shape[1]
-        self.dz = dz = 0 if cond is None else cond.shape[1]
-        series = [y] + ([x] if x.ndim == 1 else [x[:, v] for v in range(nvar)]) + \
-            ([] if cond is None else [cond[:, c] for c in range(dz)])
-        # The series go up from pinned host memory, asynchronously on the
-        # preparation stream (ahead of the kernels that read them), while
-        # the host builds the task table.
-        self.raw_host = torch.empty(n_rows * len(series), dtype=torch.float64, pin_memory=True)
-        raw = self.raw_host.numpy()
-        for i, col in enumerate(series):
-            raw[i * n_rows:(i + 1) * n_rows] = col
+        self.dz = dz
+        self.n_tasks = n_tasks
+        self._upload(arrays)
         with torch.cuda.stream(self.st):
-            self.d_raw = self.raw_host.to(self.dev, non_blocking=True)
             self.d_mask = torch.from_numpy(np.ascontiguousarray(mask, dtype=np.uint8)).to(self.dev) \
                 if mask is not None else None
-        min_lag = min(min_lag, 0)
-        max_lag = max(max_lag, 0)
-        w = n_rows - max_lag + min_lag
-        self.n_tasks = n_tasks = len(indices)
-        # Device order: by x column, then lag, so a kernel's consecutive
-        # blocks (one XCD's share) read one x series.
-        idx = np.asarray(indices, dtype=np.int64).reshape(n_tasks, 2)
-        order = np.lexsort((idx[:, 0], idx[:, 1]))
-        self.place = np.empty(n_tasks, dtype=np.int64)   # task -> its device slot
-        self.place[order] = np.arange(n_tasks)
+        self.place = np.arange(n_tasks, dtype=np.int64)   # task -> its device slot
         self.tasks = (nat.EnmPrepTask * n_tasks)()
-        li, v = idx[order, 0], idx[order, 1]
-        tab = np.ctypeslib.as_array(self.tasks)   # the same memory, field by field
-        tab["x_col"] = (1 + v) * n_rows
-        tab["y_col"] = 0
-        tab["x0"] = max_lag - np.asarray(lag, dtype=np.int64)[li]
-        tab["y0"] = max_lag
-        tab["w"] = w
-        tab["dz"] = dz
-        if dz:
-            cl = np.asarray(cond_lag, dtype=np.int64).reshape(len(lag), -1)
-            tab["z_col"][:, :dz] = (1 + nvar + np.arange(dz)) * n_rows
-            tab["z0"][:, :dz] = max_lag - cl[li, :dz]
+        nat.struct_array(self.tasks)["dz"] = dz
         self.preprocess = preprocess
         self.hints = hints
         self.flags = (nat.P_DROP_NAN if drop_nan else 0) | (nat.P_RESCALE if preprocess else 0) | \
@@ -519,22 +534,65 @@ class DevicePrep:
         self.arena = self.hint = self.d_const = self.d_noise = None
         self.noise_len = 0
 
+    def _upload(self, arrays) -> None:
+        """The arrays' columns in d_raw, one after the other.  They go up from
+        pinned host memory, asynchronously on the preparation stream (ahead
+        of the kernels that read them), while the host builds the task table;
+        a table held row by row is turned into columns on the device."""
+        import torch
+        n = len(arrays[0])
+        blocks = []   # values as they lie in memory (rows of `m`, or a column each), m
+        for a in arrays:
+            m = 1 if a.ndim == 1 else a.shape[1]
+            by_column = m == 1 or a.flags.f_contiguous
+            blocks.append((a.reshape(n) if m == 1 else a.T if by_column else a, 1 if by_column else m, n * m))
+        total = sum(size for _, _, size in blocks)
+        self.raw_host = torch.empty(total, dtype=torch.float64, pin_memory=True)
+        host = self.raw_host.numpy()
+        with torch.cuda.stream(self.st):
+            self.d_raw = torch.empty(total, dtype=torch.float64, device=self.dev)
+            at = 0
+            for a, m, size in blocks:
+                part = self.raw_host[at:at + size]
+                if a.dtype == np.float64 and a.flags.c_contiguous and a.flags.writeable and size >= 1 << 18:
+                    part.copy_(torch.from_numpy(a).reshape(-1))   # on several threads
+                else:
+                    host[at:at + size].reshape(a.shape)[...] = a
+                dst = self.d_raw[at:at + size]
+                if m == 1:
+                    dst.copy_(part, non_blocking=True)
+                else:
+                    rows = torch.empty(size, dtype=torch.float64, device=self.dev)
+                    rows.copy_(part, non_blocking=True)
+                    with self.ctx.lock:
+                        self.ctx.prep_columns(rows.data_ptr(), n, m, dst.data_ptr(), self.st.cuda_stream)
+                at += size
+
     def _ptrs(self):
         return self.d_raw.data_ptr(), self.d_mask.data_ptr() if self.d_mask is not None else 0
 
-    def count(self, k: int) -> None:
-        """Kept rows of every task; validation in task order with the
-        reference's messages."""
+    def _count(self, k: int):
+        """Kept rows of every task; per task, whether they are too few for k,
+        and whether a NaN is left among them."""
         raw, mask = self._ptrs()
         with self.ctx.lock:
             self.ctx.prep_count(self.tasks, self.n_tasks, raw, mask, self.flags & ~nat.P_HINTS,
                                 self.h_n, self.h_nan, self.st.cuda_stream)
-        small = self.h_n[self.place] <= k
-        nan = self.h_nan[self.place] != 0
+        return self.h_n[self.place] <= k, self.h_nan[self.place] != 0
+
+    def count(self, k: int) -> None:
+        """Kept rows of every task; validation in task order with the
+        reference's messages."""
+        small, nan = self._count(k)
         failing = np.flatnonzero(small | nan)
         if len(failing):
             # The first failing task in task order, its first failed check.
             raise ValueError(K_TOO_LARGE_MSG if small[failing[0]] else NANS_LEFT_MSG)
+
+    def valid(self, k: int) -> bool:
+        """count(), but only whether every task passes."""
+        small, nan = self._count(k)
+        return not (small.any() or nan.any())
 
     def write(self) -> None:
         """The arena (and hints) from the counts of the last count(); the
@@ -562,6 +620,10 @@ class DevicePrep:
                 self.ctx.prep_hints(self.tasks, self.n_tasks, raw, mask, noise, nlen, self.flags, self.arena_off,
                                     self.arena.data_ptr(), self.hint.data_ptr(), self.st.cuda_stream)
 
+    def columns(self) -> np.ndarray:
+        """Arena offset of every column of every device slot."""
+        return self.arena_off[:, None] + self.h_n[:, None] * np.arange(2 + self.dz)
+
     def constant_flags(self) -> np.ndarray:
         """Per task (task order): bit 0/1/2 when x/y/the condition was
         constant (left unscaled).  Synchronises the preparation stream."""
@@ -580,30 +642,29 @@ def _plan_mi_device(y, x, lag, k, cond, cond_lag, mask, preprocess, drop_nan, mi
     arena, with the sort hints of every column."""
     from ._batch import ArenaBatch
     prep = DevicePrep(y, x, lag, cond, cond_lag, mask, preprocess, drop_nan, min_lag, max_lag, indices)
-    prep.count(k)
-    prep.write()
+    with prep.ctx.prep_lock:
+        prep.count(k)
+        prep.write()
     dz = prep.dz
 
-    def constant_warnings():
-        # Read after the batch is launched (the flags are ready by then):
-        # reading them first would wait for the preparation before the
-        # batch could be planned and launched.
-        const = prep.constant_flags()
-        for t in range(prep.n_tasks):
-            for bit in (1, 2, 4):
-                if const[t] & bit and (bit != 4 or dz > 0):
-                    warn(PREPROCESS_CONSTANT_DATA_WARNING)
-
     tasks_out = _Tasks()
-    tasks_out.deferred.append(constant_warnings)
+    tasks_out.deferred.append(lambda: _constant_warnings(prep))
     tasks_out.batch = ArenaBatch(prep.arena, prep.hint)
     tasks_out.batch.prep = prep
-    kind = nat.KIND_KSG if dz == 0 else nat.KIND_CMI
-    offs = (prep.arena_off[:, None] + prep.h_n[:, None] * np.arange(2 + dz)).tolist()
-    for n, o in zip(prep.h_n.tolist(), offs):
-        tasks_out.batch.add(kind, k, n, o, 1, 1, dz)
+    tasks_out.batch.add_many(nat.KIND_KSG if dz == 0 else nat.KIND_CMI, k, prep.h_n, prep.columns(), 1, 1, dz)
     tasks_out.slots = [("gpu", p) for p in prep.place.tolist()]
     return tasks_out
+
+
+def _constant_warnings(prep) -> None:
+    """The warnings of constant variables, task by task.  Read after the batch
+    is launched (the flags are ready by then): reading them first would wait
+    for the preparation before the batch could be planned and launched."""
+    const = prep.constant_flags()
+    for t in np.flatnonzero(const):
+        for bit in (1, 2, 4):
+            if const[t] & bit and (bit != 4 or prep.dz > 0):
+                warn(PREPROCESS_CONSTANT_DATA_WARNING)
 
 
 # ---------------------------------------------------------------------------
@@ -658,9 +719,10 @@ def _pairwise_mi(data, k, cond, preprocess, drop_nan, mask, discrete, callback):
     tasks, indices, nvar = _plan_pairwise(data, k, cond, preprocess, drop_nan, mask, discrete)
     values = tasks.run()
     result = np.full((nvar, nvar), np.nan)
-    for (i, j), res in zip(indices, values):
-        result[i, j] = res
-        result[j, i] = res
+    if indices:
+        i, j = np.asarray(indices).T
+        result[i, j] = values
+        result[j, i] = values
     if callback is not None:
         for (i, j) in indices:
             callback(i, j)
@@ -677,6 +739,7 @@ def plan_pairwise_mi(data, *, k: int = 3, cond=None, mask=None, discrete=False,
     discrete_arr = np.broadcast_to(discrete, data_arr.shape[1])
     tasks, indices, _ = _plan_pairwise(data_arr, k, cond_arr, preprocess, drop_nan, mask_arr,
                                        discrete_arr)
+    tasks.finish()
     if tasks.host_values:
         raise ValueError("plan_pairwise_mi covers the GPU estimators only")
     return tasks.batch, indices
@@ -692,6 +755,10 @@ def _plan_pairwise(data, k, cond, preprocess, drop_nan, mask, discrete):
     cond_lag = np.full(cond.shape[1], 0) if cond is not None else np.asarray(0)
 
     indices = [(i, j) for i in range(nvar) for j in range(i + 1, nvar)]
+    if len(data) and not np.any(discrete) and _device_prep_arrays((data,) if cond is None else (data, cond), cond):
+        tasks = _plan_pairwise_device(data, k, cond, preprocess, drop_nan, mask, indices)
+        if tasks is not None:
+            return tasks, indices, nvar
     tasks = _Tasks()
     noise = _Noise()
     # Without a mask, a NaN drop or a condition, a column's rescaled x-role
@@ -734,6 +801,44 @@ def _plan_pairwise(data, k, cond, preprocess, drop_nan, mask, discrete):
             continue
         _add_mi_task(tasks, xs, ys, None, k, dx, dy)
     return tasks, indices, nvar
+
+
+def _plan_pairwise_device(data, k, cond, preprocess, drop_nan, mask, indices):
+    """_plan_pairwise with the columns prepared on the device.  None where a
+    pair fails validation (or a shared column is constant): the host path
+    then warns and raises in the reference's order.
+
+    Without a mask, a NaN drop or a condition, a column's x-role and y-role
+    are the same in every pair: they are prepared once per column, as the pair
+    (i, i), whose x draws the noise's first n values and whose y the next n.
+    Otherwise every pair is prepared by itself."""
+    from ._batch import ArenaBatch
+    pairs = np.asarray(indices, dtype=np.int64).reshape(-1, 2)
+    shared = mask is None and cond is None and not drop_nan
+    cols = np.arange(data.shape[1])
+    prep = DevicePrep.of_columns(data, cond, mask, preprocess, drop_nan,
+                                 np.column_stack((cols, cols)) if shared else pairs)
+    with prep.ctx.prep_lock:
+        if not prep.valid(k):
+            return None
+        prep.write()
+    tasks = _Tasks()
+    tasks.batch = ArenaBatch(prep.arena, prep.hint)
+    tasks.batch.prep = prep
+    if shared:
+        # (A constant x draws no noise, so the pair's y would take other values.)
+        if prep.constant_flags().any():
+            return None
+        role = prep.columns()
+        # Unscaled, both roles are the column itself.
+        offs = np.column_stack((role[pairs[:, 0], 0], role[pairs[:, 1], 1 if preprocess else 0]))
+        tasks.batch.add_many(nat.KIND_KSG, k, prep.h_n[pairs[:, 0]], offs, 1, 1, 0)
+    else:
+        tasks.deferred.append(lambda: _constant_warnings(prep))
+        tasks.batch.add_many(nat.KIND_KSG if cond is None else nat.KIND_CMI, k, prep.h_n, prep.columns(), 1, 1,
+                             prep.dz)
+    tasks.slots = [("gpu", p) for p in range(len(pairs))]
+    return tasks
 
 
 # ---------------------------------------------------------------------------

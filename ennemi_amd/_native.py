@@ -29,7 +29,7 @@ F_TIMING = 0x10
 STAGES = ("fill", "sort", "gather", "knn", "count", "combine")
 
 EXPORTED_SYMBOLS = ("enm_init", "enm_shutdown", "enm_last_error", "enm_run_batch", "enm_run_batch_hinted",
-                    "enm_run_batch_static", "enm_prep_count", "enm_prep_write", "enm_prep_hints",
+                    "enm_run_batch_static", "enm_prep_columns", "enm_prep_count", "enm_prep_write", "enm_prep_hints",
                     "enm_unique_rows", "enm_get_stats",
                     "enm_autotune", "enm_set_tuning", "enm_set_tuning_ex", "enm_get_tuning",
                     "enm_get_tuning_for")
@@ -59,6 +59,18 @@ class EnmPrepTask(ctypes.Structure):
                 ("x0", ctypes.c_int64), ("y0", ctypes.c_int64), ("w", ctypes.c_int64),
                 ("dz", ctypes.c_int32), ("pad", ctypes.c_int32),
                 ("z_col", ctypes.c_int64 * PREP_MAXZ), ("z0", ctypes.c_int64 * PREP_MAXZ)]
+
+
+_dtypes = {}
+
+
+def struct_array(arr) -> np.ndarray:
+    """A ctypes array of structures as a NumPy array over the same memory,
+    field by field."""
+    t = arr._type_
+    if t not in _dtypes:
+        _dtypes[t] = np.dtype(t)
+    return np.frombuffer(arr, dtype=_dtypes[t]) if len(arr) else np.empty(0, dtype=_dtypes[t])
 
 
 class EnmRowset(ctypes.Structure):
@@ -115,6 +127,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.enm_run_batch_hinted.restype = ctypes.c_int
     lib.enm_run_batch_static.argtypes = lib.enm_run_batch.argtypes
     lib.enm_run_batch_static.restype = ctypes.c_int
+    lib.enm_prep_columns.argtypes = [vp, vp, ctypes.c_int64, ctypes.c_int32, vp, vp]
+    lib.enm_prep_columns.restype = ctypes.c_int
     lib.enm_prep_count.argtypes = [vp, ctypes.POINTER(EnmPrepTask), ctypes.c_int32, vp, vp,
                                    ctypes.c_uint32, vp, vp, vp]
     lib.enm_prep_count.restype = ctypes.c_int
@@ -160,6 +174,9 @@ class Context:
                 raise NativeUnavailable("enm_init failed: " + self.lib.enm_last_error(None).decode())
         self.ctx = ptr
         self.lock = threading.Lock()
+        # Held from a preparation's count to its last write: the context keeps
+        # the count's state for the calls that follow it.
+        self.prep_lock = threading.Lock()
 
     def error(self) -> str:
         return self.lib.enm_last_error(self.ctx).decode()
@@ -188,6 +205,10 @@ class Context:
         rc = self.lib.enm_run_batch_static(self.ctx, inst_arr, n_inst, seg_arr, arena_ptr, out_ptr,
                                            eps_ptr or None, cnt_ptr or None, flags, stream_ptr or None)
         self.check(rc, "enm_run_batch_static")
+
+    def prep_columns(self, rows_ptr: int, n: int, m: int, cols_ptr: int, stream_ptr: int = 0) -> None:
+        rc = self.lib.enm_prep_columns(self.ctx, rows_ptr, n, m, cols_ptr, stream_ptr or None)
+        self.check(rc, "enm_prep_columns")
 
     def prep_count(self, tasks, n_tasks: int, raw_ptr: int, mask_ptr: int, flags: int,
                    h_n: np.ndarray, h_nan: np.ndarray, stream_ptr: int = 0) -> None:

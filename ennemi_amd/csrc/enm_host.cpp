@@ -1867,6 +1867,18 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     return ENM_OK;
 }
 
+int enm_prep_columns(enm_ctx* ctx, const double* d_rows, int64_t n, int32_t m, double* d_cols, void* stream) {
+    if (!ctx) { g_init_error = "ctx is NULL"; return ENM_E_ARG; }
+    ctx->err.clear();
+    if (!d_rows || !d_cols || n < 1 || m < 1 || m > 65535 * 64 || n > ((int64_t)0x7fffffff - 1) * 64)
+        return fail(ctx, ENM_E_ARG, "a table of at least one row and one column is required");
+    hipError_t e = hipSetDevice(ctx->device);
+    if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
+    e = enm_launch_prep_columns(d_rows, n, m, d_cols, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(ctx, e, "prep columns");
+    return ENM_OK;
+}
+
 int enm_prep_count(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks, const double* d_raw,
                    const uint8_t* d_mask, uint32_t flags, int64_t* h_n, uint32_t* h_nan, void* stream) {
     if (!ctx) { g_init_error = "ctx is NULL"; return ENM_E_ARG; }

@@ -108,6 +108,7 @@ hipError_t enm_launch_reduce_pt(const RedItem* items, int n_items, const RedDev*
 hipError_t enm_launch_export_eps(const double* src, const int* perm, int64_t n, double* dst, hipStream_t st);
 hipError_t enm_launch_export_cnt(const int* src, const int* perm, int64_t n, int* dst, hipStream_t st);
 
+hipError_t enm_launch_prep_columns(const double* rows, int64_t n, int m, double* cols, hipStream_t st);
 hipError_t enm_launch_prep_count(const PrepTaskDev* tasks, int64_t stride, int n_tasks,
                                  const double* raw, const unsigned char* mask, int drop_nan, int* blk_count,
                                  int64_t* blk_off, unsigned* nan_flag, int64_t* n_out, hipStream_t st);

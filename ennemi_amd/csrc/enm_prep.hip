@@ -70,6 +70,28 @@ __device__ __forceinline__ bool row_keep(const PrepTaskDev& t, const double* __r
     return pass && !(drop_nan && nan);
 }
 
+// Rows of m columns (row-major, as NumPy holds a table) to columns of n rows:
+// 64 x 64 tiles through LDS, both sides in whole lines.
+constexpr int PC_TILE = 64;
+constexpr int PC_THREADS = 256;
+__global__ __launch_bounds__(PC_THREADS)
+void prep_columns_kernel(const double* __restrict__ rows, int64_t n, int m, double* __restrict__ cols) {
+    __shared__ double tile[PC_TILE][PC_TILE + 1];
+    const int64_t r0 = (int64_t)blockIdx.x * PC_TILE;
+    const int c0 = (int)blockIdx.y * PC_TILE;
+    // Narrow tables: consecutive threads read consecutive values of the rows.
+    const int w = min(PC_TILE, m - c0), h = (int)min((int64_t)PC_TILE, n - r0);
+    for (int t = (int)threadIdx.x; t < h * w; t += PC_THREADS) {
+        const int r = t / w, c = t - r * w;
+        tile[r][c] = rows[(r0 + r) * m + c0 + c];
+    }
+    __syncthreads();
+    for (int t = (int)threadIdx.x; t < w * PC_TILE; t += PC_THREADS) {
+        const int c = t / PC_TILE, r = t % PC_TILE;
+        if (r < h) cols[(int64_t)(c0 + c) * n + r0 + r] = tile[r][c];
+    }
+}
+
 // Blocks are laid out `stride` per task (the most any task needs; the
 // rest of a shorter task's blocks find no rows), so a block's task is a
 // division, not a search.
@@ -510,6 +532,12 @@ void prep_scale_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, co
 }
 
 }  // namespace
+
+hipError_t enm_launch_prep_columns(const double* rows, int64_t n, int m, double* cols, hipStream_t st) {
+    const dim3 grid((unsigned)((n + PC_TILE - 1) / PC_TILE), (unsigned)((m + PC_TILE - 1) / PC_TILE));
+    hipLaunchKernelGGL(prep_columns_kernel, grid, dim3(PC_THREADS), 0, st, rows, n, m, cols);
+    return hipGetLastError();
+}
 
 hipError_t enm_launch_prep_count(const PrepTaskDev* tasks, int64_t stride, int n_tasks,
                                  const double* raw, const unsigned char* mask, int drop_nan, int* blk_count,

@@ -257,6 +257,12 @@ typedef struct enm_prep_task {
 #define ENM_P_RESCALE  0x2u
 #define ENM_P_HINTS    0x4u  /* enm_prep_write keeps what enm_prep_hints needs */
 
+/*
+ * enm_prep_columns: a row-major table (n rows of m float64 values, as NumPy
+ * holds one) as m columns of n values, d_cols[c * n + r] = d_rows[r * m + c],
+ * for callers whose series are the columns of a table.  Asynchronous.
+ */
+int enm_prep_columns(enm_ctx* ctx, const double* d_rows, int64_t n, int32_t m, double* d_cols, void* stream);
 int enm_prep_count(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks,
                    const double* d_raw, const uint8_t* d_mask, uint32_t flags,
                    int64_t* h_n, uint32_t* h_nan, void* stream);
