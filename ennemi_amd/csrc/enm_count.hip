@@ -301,19 +301,24 @@ void count1d_deferred_kernel(CountArgs A, const double* __restrict__ col64, cons
     }
 }
 
-// psi sums of 1-D spaces: one wave per ENM_PSI_TILE positions of a space's
-// key-sorted order, 8 per lane in lane-major order, then a butterfly sum;
+// psi sums of 1-D spaces: one workgroup per count item, one wave per
+// ENM_PSI_TILE positions of it, 8 per lane in lane-major order, then a butterfly sum;
 // psi values come from the table psi_tab[c] = psi(c).  A zero count sets the
 // tile's flag (psi(0) poisons the reference's mean).
-__global__ __launch_bounds__(ENM_WAVE)
+constexpr int PSI_WAVES = ENM_C1_ITEM / ENM_PSI_TILE;
+__global__ __launch_bounds__(PSI_WAVES* ENM_WAVE)
 void psi_tile_kernel(const Item* __restrict__ items, int n_items, const CountDev* __restrict__ descs,
                      const double* __restrict__ psi_tab, const int* __restrict__ counts_in,
                      double* __restrict__ res64, int* __restrict__ res32) {
-    const int item = blockIdx.x;
-    if (item >= n_items) return;
-    const Item it = items[item];
+    if ((int)blockIdx.x >= n_items) return;
+    Item it = items[blockIdx.x];
+    const int wave = uni((int)threadIdx.x / ENM_WAVE);
+    it.t0 += wave * ENM_PSI_TILE;
+    if (it.t0 >= it.t1) return;
+    it.t1 = min(it.t1, it.t0 + ENM_PSI_TILE);
+    it.tile += wave;   // the item's first partials slot
     const CountDev& cd = descs[it.desc];
-    const int lane = threadIdx.x;
+    const int lane = (int)(threadIdx.x & (ENM_WAVE - 1));
     constexpr int Q = ENM_PSI_TILE / ENM_WAVE;
     // Every count is read (positions past the tile reread its last one),
     // then every table entry, each batch issued together; the sum then takes
@@ -553,7 +558,7 @@ hipError_t enm_launch_psi_table(double* tab, int64_t n, hipStream_t st) {
 hipError_t enm_launch_psi_tiles(const Item* items, int n_items, const CountDev* descs, const double* psi_tab,
                                 const int* counts, double* res64, int* res32, hipStream_t st) {
     if (n_items <= 0) return hipSuccess;
-    hipLaunchKernelGGL(psi_tile_kernel, dim3(n_items), dim3(ENM_WAVE), 0, st, items, n_items, descs, psi_tab,
-                       counts, res64, res32);
+    hipLaunchKernelGGL(psi_tile_kernel, dim3(n_items), dim3(PSI_WAVES * ENM_WAVE), 0, st, items, n_items, descs,
+                       psi_tab, counts, res64, res32);
     return hipGetLastError();
 }

@@ -45,6 +45,16 @@ struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
     bool borrowed = false;
+    DevBuf() = default;
+    DevBuf(const DevBuf&) = delete;
+    DevBuf& operator=(const DevBuf&) = delete;
+    DevBuf(DevBuf&& o) noexcept { *this = std::move(o); }
+    DevBuf& operator=(DevBuf&& o) noexcept {
+        std::swap(p, o.p);
+        std::swap(bytes, o.bytes);
+        std::swap(borrowed, o.borrowed);
+        return *this;
+    }
     ~DevBuf() { release(); }
     void release() {
         if (p && !borrowed) (void)hipFree(p);
@@ -56,7 +66,17 @@ struct DevBuf {
         if (b <= bytes && p && !borrowed) return hipSuccess;
         release();
         if (b == 0) b = 256;
-        hipError_t e = hipMalloc(&p, b);
+        // An eighth more than asked for, where there is room: the next call's
+        // kept rows are rarely the same number, and a larger buffer costs a
+        // free and an allocation (10 ms for the masked lag scan's).
+        const size_t more = b + b / 8;
+        hipError_t e = hipMalloc(&p, more);
+        if (e == hipSuccess) {
+            bytes = more;
+            return e;
+        }
+        (void)hipGetLastError();
+        e = hipMalloc(&p, b);
         if (e == hipSuccess) bytes = b;
         else p = nullptr;
         return e;
@@ -108,12 +128,30 @@ struct ExportInst {
 // into the orders over it (grid strips, and the slabs that box trees are cut
 // from).
 struct SecondStage {
-    std::vector<SortSeg> segs;
+    std::vector<StripItem> strips;
+    int strip_tile = ENM_SORT_TILE;   // block-sort tile that holds the longest strip
+    int64_t strip_points = 0;
+    std::vector<SortSeg> segs;        // slabs
     std::vector<GatherItem> gitems;
     int ntiles = 0;
-    int tile = ENM_SORT_TILE;   // block-sort tile
     int64_t elems = 0, maxlen = 0;
-    size_t off_segs = 0, off_gitems = 0;
+    size_t off_strips = 0, off_segs = 0, off_gitems = 0;
+};
+
+// First-stage sort segment sseg laid out into an order from position pos0 on.
+struct Consumer {
+    int order, sseg;
+    int32_t pos0;
+};
+
+// Device memory that a run needs besides its plan's tables: one set per
+// context, shared by its plans (runs of a context follow one another), or the
+// static workspace.  `moved` counts reallocations: a graph captured before one
+// holds stale addresses.
+struct Work {
+    DevBuf far, sk0, si0, sk1, si1, split, col64, col32, perm, res64, res32, maxabs, counters, stats, deferred, heap,
+        samp_k0, samp_k1, samp_i0, samp_i1, samp_split, bid, ss_counts, ss_tiles, ss_long, ss_ctl, hint_bad;
+    uint64_t moved = 0;
 };
 
 // Box-tree phases: the trees of the joint spaces, then those of each count
@@ -135,7 +173,8 @@ struct Plan {
     // host tables
     std::vector<SortSeg> segs;               // stage 1 (arena keys)
     std::vector<GatherItem> gitems;
-    SecondStage strips, slabs;
+    std::vector<Consumer> consumers;         // order by order
+    SecondStage second;
     std::vector<TreeDev> trees;
     std::vector<int> tree_phase;
     TreePhase phase[kPhases];
@@ -150,8 +189,6 @@ struct Plan {
     std::vector<std::pair<int, int>> inst_ritems;   // per instance: first item, count
     std::vector<double> cls;
     std::vector<Item> kitems, citems;
-    std::vector<Item> sitems;                        // psi tiles of 1-D spaces
-    std::vector<std::pair<int, int>> inst_sitems;    // per instance: first item, count
     std::vector<int> qoffs;                          // queue offsets of every group
     std::vector<Group> groups;
     std::vector<ExportInst> exports;
@@ -183,17 +220,16 @@ struct Plan {
     // device
     int64_t heap_bytes = 0;   // global heap lists of kNN groups with k+1 > ENM_LIST_LDS_MAX
     int64_t far_bytes = 0;    // far list of the strip kNN (queries reaching past the staged strips)
-    DevBuf far,
-        tables, sk0, si0, sk1, si1, split, col64, col32, perm, res64, res32, maxabs, counters, stats,
-        deferred, heap, samp_k0, samp_k1, samp_i0, samp_i1, samp_split, bid, ss_counts, ss_tiles, ss_long, ss_ctl,
-        hint_bad;
+    DevBuf tables;
+    Work* work = nullptr;
+    std::unique_ptr<Work> own_work;   // the static workspace's
+    std::vector<size_t> need;         // bytes of each workspace buffer
     size_t off_segs = 0, off_gitems = 0, off_orders = 0, off_kdescs = 0, off_cdescs = 0, off_insts = 0,
            off_cls = 0, off_kitems = 0, off_citems = 0, off_trees = 0, off_rdescs = 0,
-           off_ritems = 0, off_sitems = 0, off_qoffs = 0, off_ssegs = 0, off_samp_segs = 0, off_cons = 0,
+           off_ritems = 0, off_qoffs = 0, off_ssegs = 0, off_samp_segs = 0, off_cons = 0,
            off_qbase = 0, table_bytes = 0;
-    void* pinned = nullptr;
-    hipEvent_t upload_done = nullptr;
     hipGraphExec_t graph = nullptr;
+    uint64_t graph_moved = 0;         // the workspace it was captured with
     const void* graph_ptrs[5] = {};   // arena, out, eps, counts, hints the graph was captured with
     int n_launch = 0;
     bool timing = false;       // events recorded by the last enqueue
@@ -201,8 +237,6 @@ struct Plan {
     ~Plan() {
         for (hipEvent_t e : ev) if (e) (void)hipEventDestroy(e);
         if (graph) (void)hipGraphExecDestroy(graph);
-        if (upload_done) (void)hipEventDestroy(upload_done);
-        if (pinned) (void)hipHostFree(pinned);
     }
 };
 
@@ -235,6 +269,15 @@ struct enm_ctx {
     std::map<std::tuple<int, int, int>, enm_tuning> tuned;
     uint64_t tuning_gen = 0;
     std::list<std::unique_ptr<Plan>> cache;   // most recent first
+    Work work;                                // of every plan in the cache
+    DevBuf spare_tables;                      // of a plan that has left the cache
+    void* stage = nullptr;                    // pinned: tables on their way up
+    size_t stage_bytes = 0;
+    hipEvent_t stage_done = nullptr;          // the last upload from it
+    ~enm_ctx() {
+        if (stage_done) (void)hipEventDestroy(stage_done);
+        if (stage) (void)hipHostFree(stage);
+    }
     Plan* last = nullptr;
     hipStream_t last_stream = nullptr;
     // Device-side task preparation: the state enm_prep_count leaves for
@@ -372,17 +415,8 @@ struct Planner {
         P.orders.push_back(od);
         order_ids[key] = id;
         order_group.push_back(g);
-        for (size_t t = 0; t < group_segs[g].size(); ++t) {
-            const int s = group_segs[g][t];
-            for (int off = 0; off < P.segs[s].len; off += ENM_SORT_TILE) {
-                GatherItem gi;
-                gi.order = id;
-                gi.sseg = s;
-                gi.off = off;
-                gi.pos0 = (int32_t)group_pos0[g][t];
-                P.gitems.push_back(gi);
-            }
-        }
+        for (size_t t = 0; t < group_segs[g].size(); ++t)
+            P.consumers.push_back(Consumer{id, group_segs[g][t], (int32_t)group_pos0[g][t]});
         return id;
     }
 
@@ -395,7 +429,7 @@ struct Planner {
         key += std::string((const char*)&base, sizeof base) + std::string((const char*)&S, sizeof S);
         auto it = order_ids.find(key);
         if (it != order_ids.end()) return it->second;
-        SecondStage& G = slab ? P.slabs : P.strips;
+        SecondStage& G = P.second;
         const OrderDev bo = P.orders[base];
         OrderDev od = bo;
         od.xy = -1;
@@ -420,6 +454,11 @@ struct Planner {
         for (auto rg : ranges(base)) {
             for (int st = rg.first; st < rg.second; st += S) {
                 const int len = std::min(S, rg.second - st);
+                if (!slab) {
+                    G.strips.push_back(StripItem{id, st, len});
+                    G.strip_points += len;
+                    continue;
+                }
                 SortSeg sg;
                 sg.src = bo.c64 + 1 * bo.n + st;  // column 1 of the base order, in col64
                 sg.sbase = G.elems;
@@ -427,7 +466,7 @@ struct Planner {
                 sg.first_tile = G.ntiles;
                 sg.p0 = st;
                 sg.hint = 0;
-                G.ntiles += (len + G.tile - 1) / G.tile;
+                G.ntiles += (len + ENM_SORT_TILE - 1) / ENM_SORT_TILE;
                 G.elems += len;
                 G.maxlen = std::max<int64_t>(G.maxlen, len);
                 const int sid = (int)G.segs.size();
@@ -584,16 +623,27 @@ int64_t add_reduction(Plan& P, int64_t src, int64_t n, int log_values, int* nchu
     return rd.part;
 }
 
-struct PendingItem {
+// Work items to be: positions [it.t0, it.t1) of `it`, `step` at a time, each
+// item's tile tile_step after the one before.
+struct PendingRun {
     Item it;
-    int64_t cost;
-    int inst;
-    int dclass, pclass;
+    int step = 1, tile_step = 0;
+    int64_t cost = 1;   // of an item
+    int inst = 0;
+    int dclass = 0, pclass = 0;
     int walk = ENM_WALK_NONE;
     int phase = 0;
     int k1 = 0;     // k+1 of its instance (kNN items)
     int waves = 32, ticket = 0;   // its instance's tile shape
     int strip = 0;  // strip items: the strip size
+    int count() const { return (it.t1 - it.t0 + step - 1) / step; }
+    Item item(int i) const {
+        Item r = it;
+        r.tile += i * tile_step;
+        r.t0 += i * step;
+        r.t1 = std::min(r.t0 + step, it.t1);
+        return r;
+    }
 };
 
 int grid_for(const enm_ctx* ctx, int waves_per_cu, int n_items) {
@@ -618,7 +668,7 @@ enm_tuning tuning_for(const enm_ctx* ctx, int dims, int k, int64_t n) {
 
 int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, const int64_t* seg_len) {
     Planner pl(P, inst, seg_len);
-    std::vector<PendingItem> kpend, cpend;
+    std::vector<PendingRun> kpend, cpend;
     P.n_inst = n_inst;
     // Every instance's tile shape; grid strips up to 2048 points are sorted
     // by one block each, with the smallest block tile that holds the
@@ -645,9 +695,9 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         if (route(cols, inst[ii].k, tunes[ii]) == ENM_WALK_STRIP)
             max_strip = std::max(max_strip, (int)tunes[ii].strip_points);
     }
-    P.strips.tile = max_strip <= 512 ? 512 : max_strip <= 1024 ? 1024 : ENM_SORT_TILE;
+    P.second.strip_tile = max_strip <= 512 ? 512 : max_strip <= 1024 ? 1024 : ENM_SORT_TILE;
     // Queries on trees, made into items once their number is known.
-    struct TreeQueries { PendingItem pi; int first, count; int64_t n; };
+    struct TreeQueries { PendingRun pi; int first, count; int64_t n; };
     std::vector<TreeQueries> ktree, ctree;
     int64_t point_off = 0;
     for (int ii = 0; ii < n_inst; ++ii) {
@@ -833,9 +883,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
                                                           : enm_knn_list_class(I.k + 1);
         if (dcl < 0) return bad("joint dimension above 16");
         if (I.k > 0x3fffffff) return bad("k out of range");
-        int ktiles = 0;
-        PendingItem kp;
-        kp.cost = 1;
+        PendingRun kp;
         kp.inst = ii; kp.dclass = dcl; kp.pclass = pcl; kp.walk = walk;
         kp.k1 = I.k + 1;
         kp.waves = T.waves_per_cu; kp.ticket = T.items_per_ticket;
@@ -853,20 +901,14 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             // (strips start at lo + s*strip and the strip size is a multiple
             // of the tile size).  Work per tile: the scope range in brute
             // force, about constant with window pruning.
-            const int step = walk == ENM_WALK_STRIP ? S : walk == ENM_WALK_LINE ? ENM_LINE_ITEM : ENM_TILE;
+            kp.step = walk == ENM_WALK_STRIP ? S : walk == ENM_WALK_LINE ? ENM_LINE_ITEM : ENM_TILE;
             for (auto rg : pl.ranges(K)) {
-                for (int t0 = rg.first; t0 < rg.second; t0 += step) {
-                    PendingItem pi = kp;
-                    pi.it = Item{kdi, ktiles++, rg.first, rg.second, t0, std::min(t0 + step, rg.second)};
-                    pi.cost = walk == ENM_WALK_STRIP ? (pi.it.t1 - t0 + ENM_TILE - 1) / ENM_TILE
-                              : P.brute              ? (int64_t)(rg.second - rg.first)
-                                                     : 1;
-                    kpend.push_back(pi);
-                }
+                kp.it = Item{kdi, 0, rg.first, rg.second, rg.first, rg.second};
+                kp.cost = walk == ENM_WALK_STRIP ? S / ENM_TILE : P.brute ? (int64_t)(rg.second - rg.first) : 1;
+                kpend.push_back(kp);
             }
         }
         const int red_first = (int)P.ritems.size();
-        const int sit_first = (int)P.sitems.size();
         if (kd.kl) {
             // Entropy: log radii summed in point order.
             int chunks = 0;
@@ -902,38 +944,30 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             cd.psi_pt = -1;
             int ctiles = 0;
             std::vector<std::pair<int, int>> rgs;
+            PendingRun cp;
+            cp.it = Item{cdi, 0, 0, 0, 0, 0};
+            cp.inst = ii; cp.dclass = ccl;
+            cp.waves = T.waves_per_cu; cp.ticket = T.items_per_ticket;
             if (sp.tree >= 0) {
-                PendingItem pi;
-                pi.it = Item{cdi, 0, 0, 0, 0, 0};
-                pi.cost = 0;
-                pi.inst = ii; pi.dclass = ccl; pi.pclass = 0; pi.walk = ENM_WALK_TREE;
-                pi.waves = T.waves_per_cu; pi.ticket = T.items_per_ticket;
-                pi.phase = P.tree_phase[sp.tree];
+                cp.walk = ENM_WALK_TREE;
+                cp.phase = P.tree_phase[sp.tree];
                 int c = sp.tree;
-                while (c < (int)P.trees.size() && P.tree_phase[c] == pi.phase) ++c;
-                ctree.push_back({pi, sp.tree, c - sp.tree, I.n});
+                while (c < (int)P.trees.size() && P.tree_phase[c] == cp.phase) ++c;
+                ctree.push_back({cp, sp.tree, c - sp.tree, I.n});
             } else if (sp.segmented) {
                 rgs = pl.ranges(sp.order);
             } else {
                 rgs.emplace_back(0, (int)I.n);
             }
-            // 1-D counts take ENM_C1_ITEM positions per item (and psi tiles
-            // of ENM_PSI_TILE), multi-D ENM_TILE.
-            const int step = ccl == 1 ? ENM_C1_ITEM : ENM_TILE;
+            // 1-D counts take ENM_C1_ITEM positions per item, each of whole
+            // psi tiles; multi-D ENM_TILE.
+            cp.step = ccl == 1 ? ENM_C1_ITEM : ENM_TILE;
+            cp.tile_step = ccl == 1 ? ENM_C1_ITEM / ENM_PSI_TILE : 0;
             for (auto rg : rgs) {
-                for (int t0 = rg.first; t0 < rg.second; t0 += step) {
-                    PendingItem pi;
-                    pi.it = Item{cdi, ccl == 1 ? 0 : ctiles++, rg.first, rg.second, t0,
-                                 std::min(t0 + step, rg.second)};
-                    pi.cost = P.brute && ccl != 1 ? (int64_t)(rg.second - rg.first) : (int64_t)step;
-                    pi.inst = ii; pi.dclass = ccl; pi.pclass = 0;
-                    pi.waves = T.waves_per_cu; pi.ticket = T.items_per_ticket;
-                    cpend.push_back(pi);
-                }
-                if (ccl == 1)
-                    for (int t0 = rg.first; t0 < rg.second; t0 += ENM_PSI_TILE)
-                        P.sitems.push_back(Item{cdi, ctiles++, rg.first, rg.second, t0,
-                                                std::min(t0 + ENM_PSI_TILE, rg.second)});
+                cp.it = Item{cdi, ctiles, rg.first, rg.second, rg.first, rg.second};
+                cp.cost = P.brute && ccl != 1 ? (int64_t)(rg.second - rg.first) : (int64_t)cp.step;
+                cpend.push_back(cp);
+                if (ccl == 1) ctiles += (rg.second - rg.first + ENM_PSI_TILE - 1) / ENM_PSI_TILE;
             }
             if (ccl == 1) {
                 // 1-D spaces sum per tile of their key-sorted order.
@@ -967,7 +1001,6 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             F.inst_groups.emplace_back(g0, (int)F.groups.size() - g0);
         }
         P.inst_ritems.emplace_back(red_first, (int)P.ritems.size() - red_first);
-        P.inst_sitems.emplace_back(sit_first, (int)P.sitems.size() - sit_first);
         P.psi_n = std::max<int64_t>(P.psi_n, I.n);
         if (I.kind == ENM_KIND_ROSS) {
             id.seg_len = (int64_t)P.cls.size();
@@ -1029,22 +1062,21 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
 
     // Tree queries: an item is a leaf, shared by as many waves (of as few
     // queries each) as make four for every wave slot of the GPU.
-    auto tree_items = [&](const std::vector<TreeQueries>& all, std::vector<PendingItem>& pend) {
+    auto tree_items = [&](const std::vector<TreeQueries>& all, std::vector<PendingRun>& pend) {
         int64_t total = 0;
         for (const TreeQueries& q : all) total = P.per_instance ? std::max(total, q.n) : total + q.n;
         int share = 1;
         while (share < ENM_LEAF && total * share / ENM_LEAF < (int64_t)4 * 32 * ctx->num_cus) share *= 2;
         for (const TreeQueries& q : all)
-            for (int t = q.first; t < q.first + q.count; ++t)
-                for (int t0 = 0; t0 < P.trees[t].n; t0 += ENM_LEAF) {
-                    PendingItem pi = q.pi;
-                    pi.it.tile = t;
-                    pi.it.t0 = t0;
-                    pi.it.t1 = std::min(t0 + ENM_LEAF, (int)P.trees[t].n);
-                    pi.cost = 1;
-                    pi.ticket = share;
-                    pend.push_back(pi);
-                }
+            for (int t = q.first; t < q.first + q.count; ++t) {
+                PendingRun pi = q.pi;
+                pi.it.tile = t;
+                pi.it.t0 = 0;
+                pi.it.t1 = P.trees[t].n;
+                pi.step = ENM_LEAF;
+                pi.ticket = share;
+                pend.push_back(pi);
+            }
     };
     tree_items(ktree, kpend);
     tree_items(ctree, cpend);
@@ -1057,8 +1089,12 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
     // instance's items in blocks of consecutive tiles (one block unless the
     // instance is a large share of the group), blocks placed largest first
     // on the least-loaded queue.
-    auto build = [&](std::vector<PendingItem>& pend, std::vector<Item>& out, int is_count) {
-        std::stable_sort(pend.begin(), pend.end(), [&](const PendingItem& a, const PendingItem& b) {
+    auto build = [&](std::vector<PendingRun>& pend, std::vector<Item>& out, int is_count) {
+        auto same = [&](const PendingRun& a, const PendingRun& b) {
+            return a.dclass == b.dclass && a.pclass == b.pclass && a.walk == b.walk && a.phase == b.phase &&
+                   (!P.per_instance || a.inst == b.inst);
+        };
+        std::stable_sort(pend.begin(), pend.end(), [&](const PendingRun& a, const PendingRun& b) {
             if (P.per_instance && a.inst != b.inst) return a.inst < b.inst;
             if (a.dclass != b.dclass) return a.dclass < b.dclass;
             if (a.pclass != b.pclass) return a.pclass < b.pclass;
@@ -1067,20 +1103,22 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             return a.cost > b.cost;
         });
         // A deferred 1-D query code holds the item index in its upper bits.
-        const size_t max_group = (size_t)1 << (32 - ENM_C1_OFF_BITS);
+        const int64_t max_group = (int64_t)1 << (32 - ENM_C1_OFF_BITS);
         size_t i = 0;
+        int done = 0;   // items of run i that earlier groups have
         while (i < pend.size()) {
+            // The group's runs, and the last one's items left for the next.
+            int64_t items = 0;
             size_t j = i;
-            while (j < pend.size() && pend[j].dclass == pend[i].dclass && pend[j].pclass == pend[i].pclass &&
-                   pend[j].walk == pend[i].walk && pend[j].phase == pend[i].phase && (!P.per_instance || pend[j].inst == pend[i].inst) &&
-                   j - i < max_group)
-                ++j;
+            while (j < pend.size() && same(pend[j], pend[i]) && items < max_group)
+                items += pend[j++].count() - (items == 0 ? done : 0);
+            const int left = (int)std::max<int64_t>(0, items - max_group);
             Group g;
             g.is_count = is_count;
             g.dclass = pend[i].dclass;
             g.pclass = pend[i].pclass;
             g.first = (int)out.size();
-            g.n_items = (int)(j - i);
+            g.n_items = (int)(items - left);
             g.counter = (int)P.groups.size() * (ENM_NQ + ENM_NDEF) * ENM_CSTRIDE;
             g.inst = P.per_instance ? pend[i].inst : -1;
             g.walk = pend[i].walk;
@@ -1094,7 +1132,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
             // The group runs with the shape of its costliest item's instance.
             g.waves = pend[i].waves;
             g.ticket = pend[i].ticket;
-            if (!is_count && g.walk != ENM_WALK_TREE && g.walk != ENM_WALK_LINE && g.pclass == ENM_LIST_HEAP_GLOBAL) {
+            if (!is_count && g.walk == ENM_WALK_NONE && g.pclass == ENM_LIST_HEAP_GLOBAL) {
                 const int hg = enm_knn_heap_grid(grid_for(ctx, g.waves, g.n_items), g.k1max);
                 P.heap_bytes = std::max<int64_t>(P.heap_bytes, (int64_t)hg * ENM_TILE * g.k1max * 8);
             }
@@ -1106,82 +1144,62 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
                 const int64_t want = (int64_t)g.n_items * g.smax / 16 * rec;
                 P.far_bytes = std::max<int64_t>(P.far_bytes, std::min<int64_t>(want, (int64_t)64 << 20));
             }
-            const size_t blk = std::max<size_t>(64, (j - i + 4 * ENM_NQ - 1) / (4 * ENM_NQ));
-            struct Block { int64_t cost; size_t a, b; };
+            const int blk = (int)std::max<int64_t>(64, (g.n_items + 4 * ENM_NQ - 1) / (4 * ENM_NQ));
+            struct Block { int64_t cost; size_t run; int a, b; };   // items [a, b) of a run
             std::vector<Block> blocks;
-            for (size_t t = i; t < j;) {
-                size_t u = t;
-                int64_t c = 0;
-                while (u < j && pend[u].inst == pend[t].inst && u - t < blk) c += pend[u++].cost;
-                blocks.push_back(Block{c, t, u});
-                t = u;
+            for (size_t t = i; t < j; ++t) {
+                const int a0 = t == i ? done : 0, n = pend[t].count() - (t + 1 == j ? left : 0);
+                for (int a = a0; a < n; a += blk) {
+                    const int b = std::min(n, a + blk);
+                    blocks.push_back(Block{pend[t].cost * (b - a), t, a, b});
+                }
             }
             std::stable_sort(blocks.begin(), blocks.end(),
                              [](const Block& a, const Block& b) { return a.cost > b.cost; });
             std::vector<std::vector<size_t>> queue(ENM_NQ);
             std::vector<int64_t> load(ENM_NQ, 0);
-            for (const Block& b : blocks) {
+            for (size_t t = 0; t < blocks.size(); ++t) {
                 const int q = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-                load[q] += b.cost;
-                for (size_t t = b.a; t < b.b; ++t) queue[q].push_back(t);
+                load[q] += blocks[t].cost;
+                queue[q].push_back(t);
             }
             g.qoff = (int)P.qoffs.size();
+            g.qmax = 0;
+            out.reserve(out.size() + g.n_items);
             int64_t queries = 0;
             for (int q = 0; q < ENM_NQ; ++q) {
-                P.qoffs.push_back((int)(out.size() - g.first));
+                const int q0 = (int)(out.size() - g.first);
+                P.qoffs.push_back(q0);
                 for (size_t t : queue[q]) {
-                    out.push_back(pend[t].it);
-                    queries += pend[t].it.t1 - pend[t].it.t0;
+                    const Block& bl = blocks[t];
+                    const PendingRun& run = pend[bl.run];
+                    for (int a = bl.a; a < bl.b; ++a) out.push_back(run.item(a));
+                    queries += std::min(run.it.t1, run.it.t0 + bl.b * run.step) - (run.it.t0 + bl.a * run.step);
                 }
+                g.qmax = std::max(g.qmax, (int)(out.size() - g.first) - q0);
             }
             P.qoffs.push_back((int)(out.size() - g.first));
-            g.qmax = 0;
-            for (const auto& q : queue) g.qmax = std::max(g.qmax, (int)q.size());
             if (is_count && g.dclass == 1) P.max_c1_queries = std::max(P.max_c1_queries, queries);
             P.groups.push_back(g);
-            i = j;
+            done = left > 0 ? pend[j - 1].count() - left : 0;
+            i = left > 0 ? j - 1 : j;
         }
     };
     build(kpend, P.kitems, 0);
     build(cpend, P.citems, 1);
-    // Stage-1 gathers read their columns at random positions of one
-    // instance: interleave the items so that block b (dispatched to XCD
-    // b % ENM_NQ) only serves the instances of queue b % ENM_NQ, and each
-    // instance's columns are cached in one XCD's L2.
-    {
-        std::vector<std::vector<GatherItem>> lists(ENM_NQ);
-        for (const GatherItem& gi : P.gitems) lists[P.orders[gi.order].inst % ENM_NQ].push_back(gi);
-        std::vector<GatherItem> mixed;
-        mixed.reserve(P.gitems.size());
-        for (size_t k = 0; mixed.size() < P.gitems.size(); ++k)
-            for (int q = 0; q < ENM_NQ; ++q)
-                if (k < lists[q].size()) mixed.push_back(lists[q][k]);
-        P.gitems.swap(mixed);
-    }
     // First stage: sample sort when segments need more than one block-sort
     // tile and none is longer than ENM_SS_MAXLEN.
     P.sample_sort = P.maxlen > ENM_SORT_TILE && P.maxlen <= ENM_SS_MAXLEN;
     if (P.sample_sort) {
-        // The orders each segment is laid out into (the first-stage gather
-        // items, one per order and segment), and the run queue of the
-        // segment: by instance, as the gather items are interleaved.
+        // The orders each segment is laid out into, and its run queue, by
+        // instance.
         std::vector<std::vector<SsCons>> seg_cons(P.segs.size());
-        std::set<std::pair<int, int>> seen;
-        for (const GatherItem& gi : P.gitems) {
-            if (!seen.insert({gi.sseg, gi.order}).second) continue;
-            SsCons c;
-            c.pos0 = gi.pos0;
-            c.order = gi.order;
-            c.pad = 0;
-            seg_cons[gi.sseg].push_back(c);
-        }
+        for (const Consumer& c : P.consumers) seg_cons[c.sseg].push_back(SsCons{c.pos0, c.order, 0});
         std::vector<int64_t> qload(ENM_NQ, 0);
         for (size_t si = 0; si < P.segs.size(); ++si) {
             const SortSeg& sg = P.segs[si];
             SampleSeg q;
             std::memset(&q, 0, sizeof(q));
-            std::sort(seg_cons[si].begin(), seg_cons[si].end(),
-                      [](const SsCons& a, const SsCons& b) { return a.order < b.order; });
             q.cons0 = (int32_t)P.cons.size();
             q.ncons = (int32_t)seg_cons[si].size();
             P.cons.insert(P.cons.end(), seg_cons[si].begin(), seg_cons[si].end());
@@ -1210,6 +1228,20 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         }
         P.qbase.assign(ENM_NQ + 1, 0);
         for (int q = 0; q < ENM_NQ; ++q) P.qbase[q + 1] = P.qbase[q] + (int)qload[q];
+    } else {
+        // Gathers read their columns at random positions of one instance:
+        // interleave the items so that block b (dispatched to XCD b % ENM_NQ)
+        // only serves the instances of queue b % ENM_NQ, and each instance's
+        // columns are cached in one XCD's L2.
+        std::vector<std::vector<GatherItem>> lists(ENM_NQ);
+        size_t total = 0;
+        for (const Consumer& c : P.consumers)
+            for (int off = 0; off < P.segs[c.sseg].len; off += ENM_SORT_TILE, ++total)
+                lists[P.orders[c.order].inst % ENM_NQ].push_back(GatherItem{c.order, c.sseg, off, c.pos0});
+        P.gitems.reserve(total);
+        for (size_t k = 0; P.gitems.size() < total; ++k)
+            for (int q = 0; q < ENM_NQ; ++q)
+                if (k < lists[q].size()) P.gitems.push_back(lists[q][k]);
     }
     // psi(0..max n) for the count kernels.
     P.psi_tab = P.n_res64;
@@ -1229,37 +1261,52 @@ size_t append(std::vector<char>& blob, const std::vector<T>& v) {
     return off;
 }
 
-// The plan's device tables, packed into one host blob (256-byte aligned).
-std::vector<char> pack_tables(Plan& P) {
-    std::vector<char> blob;
-    P.off_segs = append(blob, P.segs);
-    P.off_gitems = append(blob, P.gitems);
-    P.off_orders = append(blob, P.orders);
-    P.off_kdescs = append(blob, P.kdescs);
-    P.off_cdescs = append(blob, P.cdescs);
-    P.off_insts = append(blob, P.insts);
-    P.off_cls = append(blob, P.cls);
-    P.off_kitems = append(blob, P.kitems);
-    P.off_citems = append(blob, P.citems);
-    for (SecondStage* g : {&P.strips, &P.slabs}) {
-        g->off_segs = append(blob, g->segs);
-        g->off_gitems = append(blob, g->gitems);
-    }
-    P.off_trees = append(blob, P.trees);
+// The plan's device tables, one after the other (256-byte aligned): their
+// offsets and total size, and the pieces to copy there.
+struct TablePiece {
+    size_t off;
+    const void* p;
+    size_t bytes;
+};
+std::vector<TablePiece> layout_tables(Plan& P) {
+    std::vector<TablePiece> v;
+    size_t end = 0;
+    auto put = [&](const auto& t) {
+        const size_t off = (end + 255) & ~(size_t)255, bytes = t.size() * sizeof(t[0]);
+        if (bytes) v.push_back(TablePiece{off, t.data(), bytes});
+        end = off + bytes;
+        return off;
+    };
+    P.off_segs = put(P.segs);
+    P.off_gitems = put(P.gitems);
+    P.off_orders = put(P.orders);
+    P.off_kdescs = put(P.kdescs);
+    P.off_cdescs = put(P.cdescs);
+    P.off_insts = put(P.insts);
+    P.off_cls = put(P.cls);
+    P.off_kitems = put(P.kitems);
+    P.off_citems = put(P.citems);
+    P.second.off_strips = put(P.second.strips);
+    P.second.off_segs = put(P.second.segs);
+    P.second.off_gitems = put(P.second.gitems);
+    P.off_trees = put(P.trees);
     for (TreePhase& f : P.phase) {
-        f.off_cells = append(blob, f.cells);
-        f.off_groups = append(blob, f.groups);
+        f.off_cells = put(f.cells);
+        f.off_groups = put(f.groups);
     }
-    P.off_rdescs = append(blob, P.rdescs);
-    P.off_ritems = append(blob, P.ritems);
-    P.off_sitems = append(blob, P.sitems);
-    P.off_qoffs = append(blob, P.qoffs);
-    P.off_ssegs = append(blob, P.ssegs);
-    P.off_samp_segs = append(blob, P.samp_segs);
-    P.off_cons = append(blob, P.cons);
-    P.off_qbase = append(blob, P.qbase);
-    P.table_bytes = blob.size();
-    return blob;
+    P.off_rdescs = put(P.rdescs);
+    P.off_ritems = put(P.ritems);
+    P.off_qoffs = put(P.qoffs);
+    P.off_ssegs = put(P.ssegs);
+    P.off_samp_segs = put(P.samp_segs);
+    P.off_cons = put(P.cons);
+    P.off_qbase = put(P.qbase);
+    P.table_bytes = end;
+    return v;
+}
+
+void copy_tables(const std::vector<TablePiece>& pieces, char* to) {
+    for (const TablePiece& t : pieces) std::memcpy(to + t.off, t.p, t.bytes);
 }
 
 struct BufSpec {
@@ -1268,69 +1315,104 @@ struct BufSpec {
     const char* what;
 };
 
-// Every device buffer of a plan and its size in bytes.
-std::vector<BufSpec> workspace_layout(Plan& P) {
+// Every workspace buffer of a plan and its size in bytes (0: not needed).
+std::vector<BufSpec> workspace_layout(const Plan& P, Work& W) {
     std::vector<BufSpec> v;
-    const int64_t se = std::max(P.sort_elems, std::max(P.strips.elems, P.slabs.elems));
+    const int64_t se = std::max(P.sort_elems, P.second.elems);
     // FP32 column copies exist only when a kernel reads them.
     const bool with32 = P.f32 && P.need32;
-    v.push_back({&P.tables, P.table_bytes, "tables"});
-    v.push_back({&P.sk0, (size_t)se * 8, "sort keys"});
-    v.push_back({&P.sk1, (size_t)se * 8, "sort keys"});
-    v.push_back({&P.si0, (size_t)se * 4, "sort index"});
-    v.push_back({&P.si1, (size_t)se * 4, "sort index"});
-    v.push_back({&P.split, (size_t)std::max(P.ntiles, std::max(P.strips.ntiles, P.slabs.ntiles)) * 4 + 4, "merge splits"});
-    v.push_back({&P.col64, (size_t)P.n_col64 * 8, "columns"});
-    v.push_back({&P.col32, with32 ? (size_t)P.n_col32 * 4 : 256, "FP32 columns"});
-    v.push_back({&P.perm, (size_t)P.n_perm * 4, "permutations"});
-    v.push_back({&P.res64, (size_t)P.n_res64 * 8, "radii"});
-    v.push_back({&P.res32, (size_t)P.n_res32 * 4, "counts"});
-    v.push_back({&P.maxabs, (size_t)P.n_inst * 8, "maxima"});
-    v.push_back({&P.counters, P.groups.size() * (ENM_NQ + ENM_NDEF) * ENM_CSTRIDE * 4 + 4, "counters"});
-    v.push_back({&P.deferred, (size_t)P.deferred_seg * ENM_NDEF * 4, "deferred queries"});
-    v.push_back({&P.stats, ENM_ST_SLOTS * 8, "stats"});
-    if (P.heap_bytes > 0) v.push_back({&P.heap, (size_t)P.heap_bytes, "heap lists"});
-    if (P.far_bytes > 0) v.push_back({&P.far, (size_t)P.far_bytes, "strip kNN far list"});
-    if (P.sample_sort) {
-        v.push_back({&P.samp_k0, (size_t)P.n_samp * 8 + 8, "samples"});
-        v.push_back({&P.samp_k1, (size_t)P.n_samp * 8 + 8, "samples"});
-        v.push_back({&P.samp_i0, (size_t)P.n_samp * 4 + 4, "samples"});
-        v.push_back({&P.samp_i1, (size_t)P.n_samp * 4 + 4, "samples"});
-        v.push_back({&P.samp_split, (size_t)P.samp_tiles * 4 + 4, "sample splits"});
-        v.push_back({&P.bid, (size_t)P.sort_elems * 2 + 2, "buckets"});
-        v.push_back({&P.ss_counts, (size_t)P.n_counts * 4 + 4, "bucket counts"});
-        v.push_back({&P.ss_tiles, (size_t)P.n_buckets * sizeof(SsTile), "bucket runs"});
-        v.push_back({&P.ss_long, (size_t)P.n_buckets * sizeof(SsTile), "long bucket runs"});
-        v.push_back({&P.ss_ctl, (2 * ENM_NQ + 1) * ENM_CSTRIDE * 4, "run queue counters"});
-        if (P.hinted) v.push_back({&P.hint_bad, P.segs.size() * 4 + 4, "hint checks"});
-    }
+    v.push_back({&W.sk0, (size_t)se * 8, "sort keys"});
+    v.push_back({&W.sk1, (size_t)se * 8, "sort keys"});
+    v.push_back({&W.si0, (size_t)se * 4, "sort index"});
+    v.push_back({&W.si1, (size_t)se * 4, "sort index"});
+    v.push_back({&W.split, (size_t)std::max(P.ntiles, P.second.ntiles) * 4 + 4, "merge splits"});
+    v.push_back({&W.col64, (size_t)P.n_col64 * 8, "columns"});
+    v.push_back({&W.col32, with32 ? (size_t)P.n_col32 * 4 : 256, "FP32 columns"});
+    v.push_back({&W.perm, (size_t)P.n_perm * 4, "permutations"});
+    v.push_back({&W.res64, (size_t)P.n_res64 * 8, "radii"});
+    v.push_back({&W.res32, (size_t)P.n_res32 * 4, "counts"});
+    v.push_back({&W.maxabs, (size_t)P.n_inst * 8, "maxima"});
+    v.push_back({&W.counters, P.groups.size() * (ENM_NQ + ENM_NDEF) * ENM_CSTRIDE * 4 + 4, "counters"});
+    v.push_back({&W.deferred, (size_t)P.deferred_seg * ENM_NDEF * 4, "deferred queries"});
+    v.push_back({&W.stats, ENM_ST_SLOTS * 8, "stats"});
+    // (Buffers a plan does without have size 0, so every plan lists the same ones.)
+    v.push_back({&W.heap, (size_t)P.heap_bytes, "heap lists"});
+    v.push_back({&W.far, (size_t)P.far_bytes, "strip kNN far list"});
+    const bool ss = P.sample_sort;
+    v.push_back({&W.samp_k0, ss ? (size_t)P.n_samp * 8 + 8 : 0, "samples"});
+    v.push_back({&W.samp_k1, ss ? (size_t)P.n_samp * 8 + 8 : 0, "samples"});
+    v.push_back({&W.samp_i0, ss ? (size_t)P.n_samp * 4 + 4 : 0, "samples"});
+    v.push_back({&W.samp_i1, ss ? (size_t)P.n_samp * 4 + 4 : 0, "samples"});
+    v.push_back({&W.samp_split, ss ? (size_t)P.samp_tiles * 4 + 4 : 0, "sample splits"});
+    v.push_back({&W.bid, ss ? (size_t)P.sort_elems * 2 + 2 : 0, "buckets"});
+    v.push_back({&W.ss_counts, ss ? (size_t)P.n_counts * 4 + 4 : 0, "bucket counts"});
+    v.push_back({&W.ss_tiles, ss ? (size_t)P.n_buckets * sizeof(SsTile) : 0, "bucket runs"});
+    v.push_back({&W.ss_long, ss ? (size_t)P.n_buckets * sizeof(SsTile) : 0, "long bucket runs"});
+    v.push_back({&W.ss_ctl, ss ? (size_t)(2 * ENM_NQ + 1) * ENM_CSTRIDE * 4 : 0, "run queue counters"});
+    v.push_back({&W.hint_bad, ss && P.hinted ? P.segs.size() * 4 + 4 : 0, "hint checks"});
     return v;
 }
 
-int allocate_and_upload(enm_ctx* ctx, Plan& P, hipStream_t st) {
-    std::vector<char> blob = pack_tables(P);
-    hipError_t e;
-    if (P.upload_done) {
-        e = hipEventSynchronize(P.upload_done);
-        if (e != hipSuccess) return hip_fail(ctx, e, "hipEventSynchronize");
-    } else {
-        e = hipEventCreateWithFlags(&P.upload_done, hipEventDisableTiming);
-        if (e != hipSuccess) return hip_fail(ctx, e, "hipEventCreate");
-    }
-    if (P.pinned) { (void)hipHostFree(P.pinned); P.pinned = nullptr; }
-    e = hipHostMalloc(&P.pinned, std::max<size_t>(P.table_bytes, 256), hipHostMallocDefault);
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipHostMalloc");
-    std::memcpy(P.pinned, blob.data(), P.table_bytes);
-
-    for (const BufSpec& b : workspace_layout(P)) {
-        if (b.buf->ensure(b.bytes) != hipSuccess) {
+// The plan's share of the context's workspace, in place before every run of
+// it (another plan's run may have moved or released a buffer).
+int ensure_workspace(enm_ctx* ctx, Plan& P) {
+    const std::vector<BufSpec> v = workspace_layout(P, *P.work);
+    P.need.resize(v.size());
+    for (size_t i = 0; i < v.size(); ++i) {
+        P.need[i] = v[i].bytes;
+        if (v[i].bytes == 0 || (v[i].buf->p && v[i].buf->bytes >= v[i].bytes)) continue;
+        ++P.work->moved;
+        if (v[i].buf->ensure(v[i].bytes) != hipSuccess) {
             (void)hipGetLastError();
-            return fail(ctx, ENM_E_NOMEM, std::string("hipMalloc failed for ") + b.what);
+            return fail(ctx, ENM_E_NOMEM, std::string("hipMalloc failed for ") + v[i].what);
         }
     }
-    e = hipMemcpyAsync(P.tables.p, P.pinned, P.table_bytes, hipMemcpyHostToDevice, st);
+    return ENM_OK;
+}
+
+// Releases workspace buffers of more than twice what any cached plan (or
+// `next`) needs.
+void trim_workspace(enm_ctx* ctx, const Plan& next) {
+    const std::vector<BufSpec> v = workspace_layout(next, ctx->work);
+    for (size_t i = 0; i < v.size(); ++i) {
+        size_t need = v[i].bytes;
+        for (const auto& p : ctx->cache)
+            if (i < p->need.size()) need = std::max(need, p->need[i]);
+        if (v[i].buf->p && v[i].buf->bytes > 2 * std::max<size_t>(need, 1 << 20)) {
+            v[i].buf->release();
+            ++ctx->work.moved;
+        }
+    }
+}
+
+// The plan's tables through the context's pinned buffer.
+int upload_tables(enm_ctx* ctx, Plan& P, hipStream_t st) {
+    const std::vector<TablePiece> pieces = layout_tables(P);
+    const size_t bytes = std::max<size_t>(P.table_bytes, 256);
+    hipError_t e;
+    if (!ctx->stage_done) {
+        e = hipEventCreateWithFlags(&ctx->stage_done, hipEventDisableTiming);
+        if (e != hipSuccess) { ctx->stage_done = nullptr; return hip_fail(ctx, e, "hipEventCreate"); }
+    } else if ((e = hipEventSynchronize(ctx->stage_done)) != hipSuccess) {
+        return hip_fail(ctx, e, "hipEventSynchronize");
+    }
+    if (ctx->stage_bytes < bytes) {
+        if (ctx->stage) (void)hipHostFree(ctx->stage);
+        ctx->stage = nullptr;
+        ctx->stage_bytes = 0;
+        e = hipHostMalloc(&ctx->stage, bytes + bytes / 4, hipHostMallocDefault);
+        if (e != hipSuccess) { ctx->stage = nullptr; return hip_fail(ctx, e, "hipHostMalloc"); }
+        ctx->stage_bytes = bytes + bytes / 4;
+    }
+    copy_tables(pieces, static_cast<char*>(ctx->stage));
+    if (ctx->spare_tables.p && ctx->spare_tables.bytes >= bytes) std::swap(P.tables, ctx->spare_tables);
+    if (P.tables.ensure(bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(ctx, ENM_E_NOMEM, "hipMalloc failed for tables");
+    }
+    e = hipMemcpyAsync(P.tables.p, ctx->stage, bytes, hipMemcpyHostToDevice, st);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipMemcpyAsync(tables)");
-    e = hipEventRecord(P.upload_done, st);
+    e = hipEventRecord(ctx->stage_done, st);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipEventRecord");
     return ENM_OK;
 }
@@ -1344,6 +1426,7 @@ const T* tab(const Plan& P, size_t off) {
 // event is recorded on `st` before the first and after every stage.
 int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double* out, double* d_eps, int* d_counts,
             hipStream_t st, bool timing) {
+    Work& W = *P.work;
     hipError_t e;
     int nl = 0;
     auto chk = [&](hipError_t er, const char* what) -> int {
@@ -1361,18 +1444,18 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
         return chk(hipEventRecord(P.ev[stage], st), "hipEventRecord");
     };
     if ((rc = mark(0))) return rc;
-    unsigned long long* stats = P.stats.as<unsigned long long>();
+    unsigned long long* stats = W.stats.as<unsigned long long>();
     if ((rc = chk(enm_launch_fill_u64(stats, ENM_ST_SLOTS, 0ull, st), "fill"))) return rc;
-    if ((rc = chk(enm_launch_fill_u64(P.maxabs.as<unsigned long long>(), P.n_inst, 0ull, st), "fill"))) return rc;
-    if ((rc = chk(enm_launch_fill_i32(P.counters.as<int>(),
+    if ((rc = chk(enm_launch_fill_u64(W.maxabs.as<unsigned long long>(), P.n_inst, 0ull, st), "fill"))) return rc;
+    if ((rc = chk(enm_launch_fill_i32(W.counters.as<int>(),
                                       (int64_t)P.groups.size() * (ENM_NQ + ENM_NDEF) * ENM_CSTRIDE, 0, st),
                   "fill")))
         return rc;
-    if ((rc = chk(enm_launch_psi_table(P.res64.as<double>() + P.psi_tab, P.psi_n, st), "fill"))) return rc;
+    if ((rc = chk(enm_launch_psi_table(W.res64.as<double>() + P.psi_tab, P.psi_n, st), "fill"))) return rc;
     nl += 4;
     const bool hints = P.hinted && P.sample_sort && hint != nullptr;
     if (hints) {
-        if ((rc = chk(enm_launch_fill_i32(P.hint_bad.as<int>(), (int64_t)P.segs.size() + 1, 0, st), "fill")))
+        if ((rc = chk(enm_launch_fill_i32(W.hint_bad.as<int>(), (int64_t)P.segs.size() + 1, 0, st), "fill")))
             return rc;
         ++nl;
     }
@@ -1388,77 +1471,72 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
         a.n_samp_segs = (int)P.samp_segs.size();
         a.samp_tiles = P.samp_tiles;
         a.samp_maxlen = P.samp_maxlen;
-        a.samp_k0 = P.samp_k0.as<double>();
-        a.samp_k1 = P.samp_k1.as<double>();
-        a.samp_i0 = P.samp_i0.as<int>();
-        a.samp_i1 = P.samp_i1.as<int>();
-        a.samp_split = P.samp_split.as<int>();
-        a.bid = P.bid.as<unsigned short>();
-        a.counts = P.ss_counts.as<int>();
-        a.tiles = P.ss_tiles.as<SsTile>();
+        a.samp_k0 = W.samp_k0.as<double>();
+        a.samp_k1 = W.samp_k1.as<double>();
+        a.samp_i0 = W.samp_i0.as<int>();
+        a.samp_i1 = W.samp_i1.as<int>();
+        a.samp_split = W.samp_split.as<int>();
+        a.bid = W.bid.as<unsigned short>();
+        a.counts = W.ss_counts.as<int>();
+        a.tiles = W.ss_tiles.as<SsTile>();
         a.qbase = tab<int>(P, P.off_qbase);
-        a.qctl = P.ss_ctl.as<unsigned>();
-        a.long_runs = P.ss_long.as<SsTile>();
+        a.qctl = W.ss_ctl.as<unsigned>();
+        a.long_runs = W.ss_long.as<SsTile>();
         a.long_grid = std::max(1, ctx->num_cus);
         // ss_tile_kernel holds 50 KB of LDS: three blocks per CU.
         a.tile_grid = std::max(1, ctx->num_cus * 3);
         a.cons = tab<SsCons>(P, P.off_cons);
         a.orders = tab<OrderDev>(P, P.off_orders);
-        a.col64 = P.col64.as<double>();
-        a.col32 = P.col32.as<float>();
-        a.perm = P.perm.as<int>();
-        a.maxabs = P.maxabs.as<unsigned long long>();
+        a.col64 = W.col64.as<double>();
+        a.col32 = W.col32.as<float>();
+        a.perm = W.perm.as<int>();
+        a.maxabs = W.maxabs.as<unsigned long long>();
         a.with32 = P.f32 && P.need32 ? 1 : 0;
         a.hint = hints ? hint : nullptr;
-        a.hint_bad = hints ? P.hint_bad.as<int>() : nullptr;
+        a.hint_bad = hints ? W.hint_bad.as<int>() : nullptr;
         a.all_hinted = hints && std::all_of(P.segs.begin(), P.segs.end(), [](const SortSeg& g) { return g.hint != 0; });
-        if ((rc = chk(enm_launch_sample_sort(a, arena, P.sk0.as<double>(), P.si0.as<int>(), P.sk1.as<double>(),
-                                             P.si1.as<int>(), &nl, st), "sort")))
+        if ((rc = chk(enm_launch_sample_sort(a, arena, W.sk0.as<double>(), W.si0.as<int>(), W.sk1.as<double>(),
+                                             W.si1.as<int>(), &nl, st), "sort")))
             return rc;
     } else if (!P.segs.empty() &&
                (rc = chk(enm_launch_sort(tab<SortSeg>(P, P.off_segs), (int)P.segs.size(), P.ntiles, P.maxlen,
                                          ENM_SORT_TILE, arena, nullptr,
-                                         P.sk0.as<double>(), P.si0.as<int>(), P.sk1.as<double>(), P.si1.as<int>(),
-                                         P.split.as<int>(), &fb, &nl, st), "sort"))) {
+                                         W.sk0.as<double>(), W.si0.as<int>(), W.sk1.as<double>(), W.si1.as<int>(),
+                                         W.split.as<int>(), &fb, &nl, st), "sort"))) {
         return rc;
     }
     if ((rc = mark(2))) return rc;
-    const double* skey = fb ? P.sk1.as<double>() : P.sk0.as<double>();
-    const int* sidx = fb ? P.si1.as<int>() : P.si0.as<int>();
+    const double* skey = fb ? W.sk1.as<double>() : W.sk0.as<double>();
+    const int* sidx = fb ? W.si1.as<int>() : W.si0.as<int>();
     // (The sample sort lays its segments out into the orders itself.)
     if (!P.sample_sort && !P.gitems.empty() && (rc = chk(enm_launch_gather(tab<GatherItem>(P, P.off_gitems), (int)P.gitems.size(),
                                     tab<SortSeg>(P, P.off_segs), tab<OrderDev>(P, P.off_orders), arena, skey,
-                                    sidx, P.col64.as<double>(), P.col32.as<float>(), P.perm.as<int>(),
-                                    P.maxabs.as<unsigned long long>(), P.f32 && P.need32 ? 1 : 0, &nl, st),
+                                    sidx, W.col64.as<double>(), W.col32.as<float>(), W.perm.as<int>(),
+                                    W.maxabs.as<unsigned long long>(), P.f32 && P.need32 ? 1 : 0, &nl, st),
                       "gather")))
         return rc;
-    // Second stages: sort each grid strip or slab by the base order's column 1
-    // (keys read from col64) and lay out the orders; strips that fit one
-    // block do both in one kernel.
-    for (const SecondStage* g : {&P.strips, &P.slabs}) {
-        if (g->segs.empty()) continue;
-        const SortSeg* gsegs = tab<SortSeg>(P, g->off_segs);
-        const GatherItem* gits = tab<GatherItem>(P, g->off_gitems);
-        const int with32 = P.f32 && P.need32 ? 1 : 0;
-        if (g->maxlen <= ENM_SORT_TILE) {
-            if ((rc = chk(enm_launch_strip_sort(gits, (int)g->gitems.size(), gsegs, tab<OrderDev>(P, P.off_orders),
-                                                g->tile, P.col64.as<double>(), P.col32.as<float>(), P.perm.as<int>(),
-                                                with32, &nl, st), "sort")))
-                return rc;
-        } else {
-            if ((rc = chk(enm_launch_sort(gsegs, (int)g->segs.size(), g->ntiles, g->maxlen, g->tile,
-                                          P.col64.as<double>(), nullptr, P.sk0.as<double>(), P.si0.as<int>(),
-                                          P.sk1.as<double>(), P.si1.as<int>(), P.split.as<int>(), &fb, &nl, st),
-                          "sort")))
-                return rc;
-            if ((rc = chk(enm_launch_gather(gits, (int)g->gitems.size(), gsegs, tab<OrderDev>(P, P.off_orders), arena,
-                                            fb ? P.sk1.as<double>() : P.sk0.as<double>(),
-                                            fb ? P.si1.as<int>() : P.si0.as<int>(), P.col64.as<double>(),
-                                            P.col32.as<float>(), P.perm.as<int>(),
-                                            P.maxabs.as<unsigned long long>(), with32, &nl, st),
-                          "gather")))
-                return rc;
-        }
+    // Second stage: sort each grid strip (one block each) or slab by the base
+    // order's column 1 and lay out the orders.
+    const int with32 = P.f32 && P.need32 ? 1 : 0;
+    if ((rc = chk(enm_launch_strip_sort(tab<StripItem>(P, P.second.off_strips), (int)P.second.strips.size(),
+                                        tab<OrderDev>(P, P.off_orders), P.second.strip_tile, W.col64.as<double>(),
+                                        W.col32.as<float>(), W.perm.as<int>(), with32, &nl, st), "sort")))
+        return rc;
+    if (!P.second.segs.empty()) {
+        const SortSeg* gsegs = tab<SortSeg>(P, P.second.off_segs);
+        if ((rc = chk(enm_launch_sort(gsegs, (int)P.second.segs.size(), P.second.ntiles, P.second.maxlen,
+                                      ENM_SORT_TILE, W.col64.as<double>(), nullptr, W.sk0.as<double>(),
+                                      W.si0.as<int>(), W.sk1.as<double>(), W.si1.as<int>(), W.split.as<int>(), &fb,
+                                      &nl, st), "sort")))
+            return rc;
+        if ((rc = chk(enm_launch_gather(tab<GatherItem>(P, P.second.off_gitems), (int)P.second.gitems.size(), gsegs,
+                                        tab<OrderDev>(P, P.off_orders), arena,
+                                        fb ? W.sk1.as<double>() : W.sk0.as<double>(),
+                                        fb ? W.si1.as<int>() : W.si0.as<int>(), W.col64.as<double>(),
+                                        W.col32.as<float>(), W.perm.as<int>(), W.maxabs.as<unsigned long long>(),
+                                        with32, &nl, st),
+                      "gather")))
+            return rc;
     }
     // The box trees of one phase, of all instances or of one.
     const TreeDev* trees = tab<TreeDev>(P, P.off_trees);
@@ -1468,34 +1546,34 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
         const auto groups = ii < 0 ? std::make_pair(0, (int)F.groups.size()) : F.inst_groups[ii];
         return chk(enm_launch_tree_build(tab<CellItem>(P, F.off_cells) + cells.first, cells.second,
                                          tab<CellItem>(P, F.off_groups) + groups.first, groups.second, F.tile, trees,
-                                         arena, P.col64.as<double>(), P.perm.as<int>(), &nl, st), "trees");
+                                         arena, W.col64.as<double>(), W.perm.as<int>(), &nl, st), "trees");
     };
     if (!P.per_instance && (rc = build_trees(0, -1))) return rc;
     if ((rc = mark(3))) return rc;
     const OrderDev* orders = tab<OrderDev>(P, P.off_orders);
-    const unsigned long long* maxabs = P.maxabs.as<unsigned long long>();
-    unsigned* counters = P.counters.as<unsigned>();
+    const unsigned long long* maxabs = W.maxabs.as<unsigned long long>();
+    unsigned* counters = W.counters.as<unsigned>();
     // Per-instance mode interleaves each instance's kNN, counts and combine.
     const int* qoffs = tab<int>(P, P.off_qoffs);
-    const double* psi_tab = P.res64.as<double>() + P.psi_tab;
+    const double* psi_tab = W.res64.as<double>() + P.psi_tab;
     auto run_group = [&](const Group& g) -> int {
         if (g.walk == ENM_WALK_TREE) {
             ++nl;
             if (!g.is_count)
                 return chk(enm_launch_tree_knn(tab<Item>(P, P.off_kitems) + g.first, qoffs + g.qoff, g.n_items,
-                                               g.qmax, g.ticket, tab<KnnDev>(P, P.off_kdescs), trees, P.perm.as<int>(),
-                                               P.col64.as<double>(), P.res64.as<double>(), stats, g.dclass, g.pclass,
+                                               g.qmax, g.ticket, tab<KnnDev>(P, P.off_kdescs), trees, W.perm.as<int>(),
+                                               W.col64.as<double>(), W.res64.as<double>(), stats, g.dclass, g.pclass,
                                                st), "knn");
             return chk(enm_launch_tree_count(tab<Item>(P, P.off_citems) + g.first, qoffs + g.qoff, g.n_items, g.qmax,
-                                             g.ticket, tab<CountDev>(P, P.off_cdescs), trees, P.perm.as<int>(), psi_tab,
-                                             P.col64.as<double>(), P.res64.as<double>(), P.res32.as<int>(), stats,
+                                             g.ticket, tab<CountDev>(P, P.off_cdescs), trees, W.perm.as<int>(), psi_tab,
+                                             W.col64.as<double>(), W.res64.as<double>(), W.res32.as<int>(), stats,
                                              g.dclass, st), "count");
         }
         if (g.walk == ENM_WALK_LINE) {
             ++nl;
             return chk(enm_launch_knn_line(tab<Item>(P, P.off_kitems) + g.first, g.n_items,
-                                           tab<KnnDev>(P, P.off_kdescs), orders, P.perm.as<int>(),
-                                           P.col64.as<double>(), P.res64.as<double>(), stats, st), "knn");
+                                           tab<KnnDev>(P, P.off_kdescs), orders, W.perm.as<int>(),
+                                           W.col64.as<double>(), W.res64.as<double>(), stats, st), "knn");
         }
         if (!g.is_count) {
             int grid = g.pclass == ENM_LIST_HEAP_GLOBAL ? enm_knn_heap_grid(grid_for(ctx, g.waves, g.n_items), g.k1max)
@@ -1510,31 +1588,27 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
             }
             e = enm_launch_knn(tab<Item>(P, P.off_kitems) + g.first, qoffs + g.qoff, g.n_items,
                                counters + g.counter,
-                               tab<KnnDev>(P, P.off_kdescs), orders, maxabs, P.perm.as<int>(),
-                               P.col64.as<double>(), P.col32.as<float>(), P.res64.as<double>(), stats,
+                               tab<KnnDev>(P, P.off_kdescs), orders, maxabs, W.perm.as<int>(),
+                               W.col64.as<double>(), W.col32.as<float>(), W.res64.as<double>(), stats,
                                g.dclass, g.pclass, P.f32 && P.brute, P.brute, g.walk, grid,
-                               g.k1max, P.heap.as<double>(), g.ticket, g.smax,
-                               g.walk == ENM_WALK_STRIP && P.far_bytes > 0 ? P.far.as<char>() : nullptr,
+                               g.k1max, W.heap.as<double>(), g.ticket, g.smax,
+                               g.walk == ENM_WALK_STRIP && P.far_bytes > 0 ? W.far.as<char>() : nullptr,
                                counters + g.counter + ENM_NQ * ENM_CSTRIDE, P.far_bytes, st);
             nl += g.walk == ENM_WALK_STRIP && P.far_bytes > 0 ? 2 : 1;
             return chk(e, "knn");
         }
         e = enm_launch_count(tab<Item>(P, P.off_citems) + g.first, qoffs + g.qoff, g.n_items,
                              counters + g.counter, tab<CountDev>(P, P.off_cdescs), orders, maxabs,
-                             P.perm.as<int>(), psi_tab, P.col64.as<double>(), P.col32.as<float>(),
-                             P.res64.as<double>(), P.res32.as<int>(), stats, g.dclass, P.f32, P.brute,
+                             W.perm.as<int>(), psi_tab, W.col64.as<double>(), W.col32.as<float>(),
+                             W.res64.as<double>(), W.res32.as<int>(), stats, g.dclass, P.f32, P.brute,
                              grid_for(ctx, g.waves, g.n_items * (g.dclass == 1 ? ENM_C1_THREADS / 64 : 1)),
-                             P.deferred.as<unsigned>(), counters + g.counter + ENM_NQ * ENM_CSTRIDE,
+                             W.deferred.as<unsigned>(), counters + g.counter + ENM_NQ * ENM_CSTRIDE,
                              P.deferred_seg, g.ticket, st);
-        nl += g.dclass == 1 ? 2 : 1;
+        nl += g.dclass == 1 ? 3 : 1;
+        if (e == hipSuccess && g.dclass == 1)
+            e = enm_launch_psi_tiles(tab<Item>(P, P.off_citems) + g.first, g.n_items, tab<CountDev>(P, P.off_cdescs),
+                                     psi_tab, W.res32.as<int>(), W.res64.as<double>(), W.res32.as<int>(), st);
         return chk(e, "count");
-    };
-    auto psi_tiles = [&](int first, int count) -> int {
-        if (count <= 0) return ENM_OK;
-        ++nl;
-        return chk(enm_launch_psi_tiles(tab<Item>(P, P.off_sitems) + first, count, tab<CountDev>(P, P.off_cdescs),
-                                        psi_tab, P.res32.as<int>(), P.res64.as<double>(), P.res32.as<int>(), st),
-                   "psi");
     };
     if (P.per_instance) {
         for (int ii = 0; ii < P.n_inst; ++ii) {
@@ -1546,15 +1620,14 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
             }
             for (const Group& g : P.groups)
                 if (g.inst == ii && g.is_count && g.phase == 0 && (rc = run_group(g))) return rc;
-            if ((rc = psi_tiles(P.inst_sitems[ii].first, P.inst_sitems[ii].second))) return rc;
             const auto ri = P.inst_ritems[ii];
             if ((rc = chk(enm_launch_reduce_pt(tab<RedItem>(P, P.off_ritems) + ri.first, ri.second,
-                                               tab<RedDev>(P, P.off_rdescs), P.res64.as<double>(), st),
+                                               tab<RedDev>(P, P.off_rdescs), W.res64.as<double>(), st),
                           "reduce")))
                 return rc;
             if (ri.second > 0) ++nl;
             if ((rc = chk(enm_launch_combine(tab<InstDev>(P, P.off_insts), tab<double>(P, P.off_cls), ii, 1,
-                                             P.res64.as<double>(), P.res32.as<int>(), out, st), "combine")))
+                                             W.res64.as<double>(), W.res32.as<int>(), out, st), "combine")))
                 return rc;
             ++nl;
         }
@@ -1571,23 +1644,22 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
         }
         for (const Group& g : P.groups)
             if (g.is_count && g.phase == 0 && (rc = run_group(g))) return rc;
-        if ((rc = psi_tiles(0, (int)P.sitems.size()))) return rc;
         if ((rc = chk(enm_launch_reduce_pt(tab<RedItem>(P, P.off_ritems), (int)P.ritems.size(),
-                                           tab<RedDev>(P, P.off_rdescs), P.res64.as<double>(), st),
+                                           tab<RedDev>(P, P.off_rdescs), W.res64.as<double>(), st),
                       "reduce")))
             return rc;
         if (!P.ritems.empty()) ++nl;
         if ((rc = mark(5))) return rc;
         if ((rc = chk(enm_launch_combine(tab<InstDev>(P, P.off_insts), tab<double>(P, P.off_cls), 0, P.n_inst,
-                                         P.res64.as<double>(), P.res32.as<int>(), out, st), "combine")))
+                                         W.res64.as<double>(), W.res32.as<int>(), out, st), "combine")))
             return rc;
         ++nl;
     }
     if (d_eps || d_counts) {
         for (const ExportInst& ex : P.exports) {
             if (d_eps) {
-                if ((rc = chk(enm_launch_export_eps(P.res64.as<double>() + ex.eps,
-                                                    ex.permA >= 0 ? P.perm.as<int>() + ex.permA : nullptr,
+                if ((rc = chk(enm_launch_export_eps(W.res64.as<double>() + ex.eps,
+                                                    ex.permA >= 0 ? W.perm.as<int>() + ex.permA : nullptr,
                                                     ex.n, d_eps + ex.point_off, st), "export")))
                     return rc;
                 ++nl;
@@ -1597,8 +1669,8 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
                 if ((rc = chk(enm_launch_fill_i32(base, 3 * ex.n, 0, st), "export"))) return rc;
                 ++nl;
                 for (int s = 0; s < ex.nspace; ++s) {
-                    if ((rc = chk(enm_launch_export_cnt(P.res32.as<int>() + ex.sp[s].counts,
-                                                        ex.sp[s].perm >= 0 ? P.perm.as<int>() + ex.sp[s].perm : nullptr, ex.n,
+                    if ((rc = chk(enm_launch_export_cnt(W.res32.as<int>() + ex.sp[s].counts,
+                                                        ex.sp[s].perm >= 0 ? W.perm.as<int>() + ex.sp[s].perm : nullptr, ex.n,
                                                         base + s * ex.n, st), "export")))
                         return rc;
                     ++nl;
@@ -1735,6 +1807,7 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
         (void)hipGraphDestroy(graph);
         if (er != hipSuccess) { P.graph = nullptr; return hip_fail(ctx, er, "hipGraphInstantiate"); }
         std::memcpy(P.graph_ptrs, ptrs, sizeof ptrs);
+        P.graph_moved = P.work->moved;
         er = hipGraphLaunch(P.graph, st);
         if (er != hipSuccess) return hip_fail(ctx, er, "hipGraphLaunch");
         return ENM_OK;
@@ -1746,8 +1819,10 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
             if (it != ctx->cache.begin()) ctx->cache.splice(ctx->cache.begin(), ctx->cache, it);
             ctx->last = P;
             P->timing = false;
+            const int r = ensure_workspace(ctx, *P);
+            if (r) return r;
             if (use_graph) {
-                if (P->graph && std::memcmp(P->graph_ptrs, ptrs, sizeof ptrs) == 0) {
+                if (P->graph && P->graph_moved == P->work->moved && std::memcmp(P->graph_ptrs, ptrs, sizeof ptrs) == 0) {
                     e = hipGraphLaunch(P->graph, st);
                     if (e != hipSuccess) return hip_fail(ctx, e, "hipGraphLaunch");
                     P->n_launch = 0;
@@ -1767,23 +1842,35 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     P.per_instance = (flags & ENM_F_PER_INSTANCE) != 0;
     P.want_eps = d_eps != nullptr;
     P.hinted = d_hint != nullptr;
+    P.work = &ctx->work;
     int rc = plan_batch(ctx, P, inst, n_inst, seg_len);
     if (rc) return rc;
-    // Evict before allocating so a cache full of large plans frees memory first.
+    // Plans past the newest few leave (their runs may still be queued, and one
+    // set of tables is kept for the next plan).
     auto evict = [&](size_t keep) {
         while (ctx->cache.size() > keep) {
             if (ctx->cache.back().get() == ctx->last) ctx->last = nullptr;
             (void)hipStreamSynchronize(st);
+            DevBuf& t = ctx->cache.back()->tables;
+            if (t.bytes > ctx->spare_tables.bytes) std::swap(t, ctx->spare_tables);
             ctx->cache.pop_back();
         }
     };
     evict(kMaxCachedPlans - 1);
-    rc = allocate_and_upload(ctx, P, st);
-    if (rc == ENM_E_NOMEM && !ctx->cache.empty()) {
-        // Out of device memory with other plans resident: drop them all and
+    rc = upload_tables(ctx, P, st);
+    if (!rc) {
+        trim_workspace(ctx, P);
+        rc = ensure_workspace(ctx, P);
+    }
+    if (rc == ENM_E_NOMEM) {
+        // Out of device memory: drop the other plans and every buffer, and
         // try once more.
         evict(0);
-        rc = allocate_and_upload(ctx, P, st);
+        ctx->spare_tables.release();
+        for (const BufSpec& b : workspace_layout(P, ctx->work)) b.buf->release();
+        ++ctx->work.moved;
+        rc = P.tables.p ? ENM_OK : upload_tables(ctx, P, st);
+        if (!rc) rc = ensure_workspace(ctx, P);
     }
     if (rc) return rc;
     if (use_graph) {
@@ -1818,7 +1905,7 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     ctx->last_stream = st;
     auto rounded = [](size_t b) { return (std::max<size_t>(b, 256) + 255) & ~(size_t)255; };
     std::unique_ptr<Plan> up;
-    std::vector<char> blob;
+    std::vector<TablePiece> pieces;
     std::vector<BufSpec> layout;
     size_t total = 0;
     // A batch whose box trees do not fit may fit without them (slower).
@@ -1834,9 +1921,11 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
         P.plain = plain != 0;
         int rc = plan_batch(ctx, P, inst, n_inst, seg_len);
         if (rc) return rc;
-        blob = pack_tables(P);
-        layout = workspace_layout(P);
-        total = 0;
+        P.own_work.reset(new Work());
+        P.work = P.own_work.get();
+        pieces = layout_tables(P);
+        layout = workspace_layout(P, *P.work);
+        total = rounded(P.table_bytes);
         for (const BufSpec& b : layout) total += rounded(b.bytes);
         if (total <= (size_t)ENM_STATIC_WORKSPACE_BYTES || P.trees.empty()) break;
     }
@@ -1849,11 +1938,14 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
         return fail(ctx, ENM_E_NOMEM, msg);
     }
     char* base = static_cast<char*>(ctx->scratch);
-    size_t off = 0;
+    P.tables.borrow(base, P.table_bytes);
+    size_t off = rounded(P.table_bytes);
     for (const BufSpec& b : layout) {
         b.buf->borrow(base + off, b.bytes);
         off += rounded(b.bytes);
     }
+    std::vector<char> blob(P.table_bytes);
+    copy_tables(pieces, blob.data());
     // The tables go up from pageable host memory; the copy is complete
     // before the blob is released.
     e = hipMemcpyAsync(P.tables.p, blob.data(), P.table_bytes, hipMemcpyHostToDevice, st);
@@ -2368,7 +2460,7 @@ int enm_get_stats(enm_ctx* ctx, enm_stats* out) {
     hipError_t e = hipStreamSynchronize(ctx->last_stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
     std::vector<unsigned long long> parts(ENM_ST_SLOTS);
-    e = hipMemcpy(parts.data(), ctx->last->stats.p, ENM_ST_SLOTS * 8, hipMemcpyDeviceToHost);
+    e = hipMemcpy(parts.data(), ctx->last->work->stats.p, ENM_ST_SLOTS * 8, hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipMemcpy(stats)");
     unsigned long long h[ST_N] = {};
     for (int s = 0; s < ST_N; ++s)
@@ -2378,7 +2470,7 @@ int enm_get_stats(enm_ctx* ctx, enm_stats* out) {
     out->count_pairs = h[ST_CNT_PAIRS];
     out->count_rechecks = h[ST_CNT_RECHECK];
     out->count_queries_1d = h[ST_CNT_1D];
-    out->sort_keys = (uint64_t)(ctx->last->sort_elems + ctx->last->strips.elems + ctx->last->slabs.elems);
+    out->sort_keys = (uint64_t)(ctx->last->sort_elems + ctx->last->second.elems + ctx->last->second.strip_points);
     out->n_launches = (uint32_t)ctx->last->n_launch;
     out->graph_replayed = ctx->last->graph != nullptr && ctx->last->n_launch == 0;
     if (ctx->last->timing) {

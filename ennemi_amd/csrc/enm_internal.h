@@ -111,6 +111,14 @@ struct SsTile {
     int32_t seg;
 };
 
+// A strip of a grid order: positions [st, st + len) of its base order, sorted
+// by the base order's column 1.
+struct StripItem {
+    int32_t order;
+    int32_t st;
+    int32_t len;
+};
+
 // Gather work: one ENM_SORT_TILE chunk of one sort segment into one order.
 struct GatherItem {
     int32_t order;
@@ -238,7 +246,7 @@ struct RedItem {
 
 // One work item: a tile of consecutive order positions [t0, t1) inside the
 // scope range [lo, hi) (64 for kNN and multi-D counts, ENM_C1_ITEM for 1-D
-// counts, ENM_PSI_TILE for 1-D psi sums).  A persistent launch takes its
+// counts, whose psi sums follow tile by tile).  A persistent launch takes its
 // items from ENM_NQ queues, queue q being items [qoff[q], qoff[q+1]).  A tree
 // item is a range of tree positions inside one leaf; `tile` is its tree.
 struct Item {

@@ -49,8 +49,8 @@ struct SampleSortArgs {
 };
 hipError_t enm_launch_sample_sort(const SampleSortArgs& a, const double* arena, double* k0, int* i0,
                                   double* k1, int* i1, int* n_launch, hipStream_t st);
-hipError_t enm_launch_strip_sort(const GatherItem* d_items, int nitems, const SortSeg* d_segs,
-                                 const OrderDev* d_orders, int tile, double* col64, float* col32, int* perm,
+hipError_t enm_launch_strip_sort(const StripItem* d_items, int nitems, const OrderDev* d_orders, int tile,
+                                 double* col64, float* col32, int* perm,
                                  int with32, int* n_launch, hipStream_t st);
 hipError_t enm_launch_gather(const GatherItem* d_items, int nitems, const SortSeg* d_segs,
                              const OrderDev* d_orders, const double* arena,
@@ -98,6 +98,7 @@ hipError_t enm_launch_count(const Item* items, const int* qoff, int n_items, uns
                             int grid, unsigned* deferred, unsigned* n_deferred, unsigned seg_cap,
                             int ticket, hipStream_t st);
 hipError_t enm_launch_psi_table(double* tab, int64_t n, hipStream_t st);
+// items: the items of a 1-D count group.
 hipError_t enm_launch_psi_tiles(const Item* items, int n_items, const CountDev* descs, const double* psi_tab,
                                 const int* counts, double* res64, int* res32, hipStream_t st);
 

@@ -130,20 +130,17 @@ void block_sort_kernel(const SortSeg* __restrict__ segs, int nsegs,
 // points) sorts the strip's points by the base order's column 1 in LDS and
 // copies each point's columns and instance index from the base order into
 // the grid order directly (strip-local reads, coalesced writes), with no
-// pass through the sort buffers.  Item: the strip's sort segment (src =
-// column 1 of the base order at the strip, p0 = the strip's first position,
-// which is the same in both orders).
+// pass through the sort buffers.
 template <int TILE>
 __global__ __launch_bounds__(ENM_SORT_THREADS)
-void strip_sort_kernel(const GatherItem* __restrict__ items, const SortSeg* __restrict__ segs,
-                       const OrderDev* __restrict__ orders, double* col64, float* col32, int* perm,
+void strip_sort_kernel(const StripItem* __restrict__ items, const OrderDev* __restrict__ orders, double* col64, float* col32, int* perm,
                        int with32) {
     __shared__ double sk[ENM_LDS_PAD(TILE)];
     __shared__ int si[ENM_LDS_PAD(TILE)];
-    const GatherItem it = items[blockIdx.x];
-    const SortSeg sg = segs[it.sseg];
+    const StripItem it = items[blockIdx.x];
     const OrderDev& od = orders[it.order];
-    const int len = sg.len;
+    const int len = it.len;
+    const double* key = col64 + od.base_c64 + od.n + it.st;   // column 1 of the base order
     // A thread's PER elements: every load of a column goes out before any
     // store (a store between two loads would hold the second one back).
     constexpr int PER = TILE / ENM_SORT_THREADS;
@@ -152,13 +149,13 @@ void strip_sort_kernel(const GatherItem* __restrict__ items, const SortSeg* __re
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
             const int t = k * ENM_SORT_THREADS + (int)threadIdx.x;
-            kv[k] = t < len ? col64[sg.src + t] : INFINITY;
+            kv[k] = t < len ? key[t] : INFINITY;
         }
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
             const int t = k * ENM_SORT_THREADS + (int)threadIdx.x;
             sk[lp(t)] = kv[k];
-            si[lp(t)] = t < len ? sg.p0 + t : 0x7fffffff;
+            si[lp(t)] = t < len ? it.st + t : 0x7fffffff;
         }
     }
     block_sort_lds<TILE>(sk, si);
@@ -166,7 +163,7 @@ void strip_sort_kernel(const GatherItem* __restrict__ items, const SortSeg* __re
     const int ncol = od.ncol;
     int idx[PER];
     auto in = [&](int k) { return k * ENM_SORT_THREADS + (int)threadIdx.x < len; };
-    auto pos = [&](int k) { return it.pos0 + k * ENM_SORT_THREADS + (int)threadIdx.x; };
+    auto pos = [&](int k) { return it.st + k * ENM_SORT_THREADS + (int)threadIdx.x; };
 #pragma unroll
     for (int k = 0; k < PER; ++k) idx[k] = in(k) ? si[lp(k * ENM_SORT_THREADS + (int)threadIdx.x)] : 0;
     {
@@ -1128,19 +1125,19 @@ hipError_t enm_launch_sample_sort(const SampleSortArgs& a, const double* arena, 
     return hipGetLastError();
 }
 
-hipError_t enm_launch_strip_sort(const GatherItem* d_items, int nitems, const SortSeg* d_segs,
-                                 const OrderDev* d_orders, int tile, double* col64, float* col32, int* perm,
+hipError_t enm_launch_strip_sort(const StripItem* d_items, int nitems, const OrderDev* d_orders, int tile,
+                                 double* col64, float* col32, int* perm,
                                  int with32, int* n_launch, hipStream_t st) {
     if (nitems <= 0) return hipSuccess;
     if (tile == 512)
         hipLaunchKernelGGL(strip_sort_kernel<512>, dim3(nitems), dim3(ENM_SORT_THREADS), 0, st,
-                           d_items, d_segs, d_orders, col64, col32, perm, with32);
+                           d_items, d_orders, col64, col32, perm, with32);
     else if (tile == 1024)
         hipLaunchKernelGGL(strip_sort_kernel<1024>, dim3(nitems), dim3(ENM_SORT_THREADS), 0, st,
-                           d_items, d_segs, d_orders, col64, col32, perm, with32);
+                           d_items, d_orders, col64, col32, perm, with32);
     else if (tile == ENM_SORT_TILE)
         hipLaunchKernelGGL(strip_sort_kernel<ENM_SORT_TILE>, dim3(nitems), dim3(ENM_SORT_THREADS), 0, st,
-                           d_items, d_segs, d_orders, col64, col32, perm, with32);
+                           d_items, d_orders, col64, col32, perm, with32);
     else
         return hipErrorInvalidValue;
     ++*n_launch;
