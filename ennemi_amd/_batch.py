@@ -230,6 +230,45 @@ class ArenaBatch:
         return db.results()
 
 
+def upload_columns(arrays, device, stream):
+    """The values of arrays (equally long: columns, or tables of columns) as
+    float64 columns in HBM, one after the other; returns (device columns,
+    pinned host copy).  They go up from pinned host memory, asynchronously on
+    `stream`, while the host goes on; a table held row by row is turned into
+    columns on the device."""
+    import torch
+    n = len(arrays[0])
+    blocks = []   # values as they lie in memory (rows of `m`, or column by column), m
+    for a in arrays:
+        m = 1 if a.ndim == 1 else a.shape[1]
+        by_column = m == 1 or a.flags.f_contiguous
+        blocks.append((a.reshape(n) if m == 1 else a.T if by_column else a, 1 if by_column else m, n * m))
+    total = sum(size for _, _, size in blocks)
+    pinned = torch.empty(total, dtype=torch.float64, pin_memory=True)
+    host = pinned.numpy()
+    ctx = nat.context()
+    with torch.cuda.stream(stream):
+        d_cols = torch.empty(total, dtype=torch.float64, device=device)
+        at = 0
+        for a, m, size in blocks:
+            part = pinned[at:at + size]
+            if size >= 1 << 18 and a.flags.c_contiguous and a.flags.writeable and \
+                    a.dtype in (np.float64, np.int64, np.int32):
+                part.copy_(torch.from_numpy(a).reshape(-1))   # on several threads
+            else:
+                host[at:at + size].reshape(a.shape)[...] = a
+            dst = d_cols[at:at + size]
+            if m == 1:
+                dst.copy_(part, non_blocking=True)
+            else:
+                rows = torch.empty(size, dtype=torch.float64, device=device)
+                rows.copy_(part, non_blocking=True)
+                with ctx.lock:
+                    ctx.prep_columns(rows.data_ptr(), n, m, dst.data_ptr(), stream.cuda_stream)
+            at += size
+    return d_cols, pinned
+
+
 _side_stream = None
 
 

@@ -53,7 +53,7 @@ def _numeric(a: np.ndarray) -> bool:
     if a.dtype.kind == "b":
         return True
     if a.dtype.kind in "iu":
-        return a.size == 0 or float(np.max(np.abs(a.astype(np.float64)))) < _EXACT_INT
+        return a.dtype.itemsize <= 4 or a.size == 0 or (float(a.max()) < _EXACT_INT and float(a.min()) > -_EXACT_INT)
     return a.dtype.kind == "f" and a.dtype.itemsize <= 8
 
 
@@ -118,6 +118,45 @@ def _device_unique(row_sets: Sequence[Sequence[np.ndarray]]) -> List[Tuple[np.nd
              counts[out_off[s]:out_off[s] + int(h_distinct[s])].copy()) for s in range(n_sets)]
 
 
+def _count_rows(cols: Sequence[np.ndarray]):
+    """The distinct rows of numeric columns of whole numbers in small ranges:
+    (code of each column in every distinct row, points per distinct row,
+    values a column's codes range over), rows in lexicographic order, codes in
+    value order; None for other columns.  From enm_count_rows."""
+    import torch
+    from ._batch import _stream, upload_columns
+    if len(cols) > nat.MAX_COLS or len(cols[0]) == 0:
+        return None
+    ctx = nat.context()
+    st = _stream()
+    rowset = nat.EnmRowset()
+    rowset.n = n = len(cols[0])
+    rowset.ncol = len(cols)
+    for c in range(len(cols)):
+        rowset.col[c] = c * n
+    values, pinned = upload_columns(cols, torch.device("cuda", ctx.device), st)
+    least = np.zeros(len(cols))
+    radix = np.zeros(len(cols), dtype=np.int64)
+    counts = np.zeros(nat.COUNT_ROWS_MAX, dtype=np.uint32)
+    with ctx.lock:
+        rc = ctx.count_rows(rowset, values.data_ptr(), least, radix, counts, st.cuda_stream)
+    if rc == nat.E_UNSUPPORTED:
+        return None
+    keys = np.flatnonzero(counts[:int(np.prod(radix))])
+    rest = keys
+    codes = [None] * len(cols)
+    for c in range(len(cols) - 1, -1, -1):
+        rest, codes[c] = np.divmod(rest, radix[c])
+    return codes, counts[keys].astype(np.int64), radix
+
+
+def _sums(codes: np.ndarray, counts: np.ndarray, size: int) -> np.ndarray:
+    """Points per code."""
+    out = np.zeros(size, dtype=np.int64)
+    np.add.at(out, codes, counts)
+    return out
+
+
 def _host_unique(cols: Sequence[np.ndarray]) -> Tuple[np.ndarray, np.ndarray]:
     rows = cols[0] if len(cols) == 1 else np.column_stack(cols)
     _, inverse, counts = np.unique(rows, axis=0, return_inverse=True, return_counts=True)
@@ -143,18 +182,36 @@ def _mi_terms(n: int, cj: np.ndarray, nj: np.ndarray, cx: np.ndarray, nx: np.nda
 def estimate_discrete_entropy(x) -> float:
     """-sum p log p over the distinct rows of x."""
     reject_object(x)
-    _, counts = _unique([_columns(x)])[0]
+    cols = _columns(x)
+    direct = _count_rows(cols) if all(_numeric(c) for c in cols) else None
+    counts = direct[1] if direct is not None else _unique([cols])[0][1]
     p = counts / x.shape[0]
     return -float(np.dot(p, np.log(p)))
 
 
-def estimate_discrete_mi(x, y) -> float:
-    """Plug-in MI of two discrete variables (both converted to their common
-    type first, as np.column_stack does in the reference)."""
-    n = len(x)
+def _pair(x, y):
+    """x and y with the values that their common type gives them, as
+    np.column_stack converts them in the reference (numbers that float64
+    holds exactly keep theirs)."""
+    x, y = np.asarray(x), np.asarray(y)
+    if x.ndim == 1 and y.ndim == 1 and len(x) == len(y) and _numeric(x) and _numeric(y):
+        return x, y
     pair = np.column_stack((x, y))
     reject_object(pair)
-    xs, ys = pair[:, 0], pair[:, 1]
+    return pair[:, 0], pair[:, 1]
+
+
+def estimate_discrete_mi(x, y) -> float:
+    """Plug-in MI of two discrete variables."""
+    n = len(x)
+    xs, ys = _pair(x, y)
+    direct = _count_rows([xs, ys]) if _numeric(xs) and _numeric(ys) else None
+    if direct is not None:
+        (xj, yj), nj, radix = direct
+        nx, ny = _sums(xj, nj, radix[0]), _sums(yj, nj, radix[1])
+        verify_not_continuous(np.flatnonzero(nx), n)
+        verify_not_continuous(np.flatnonzero(ny), n)
+        return float(np.sum(nj * np.log(n * nj / (nx[xj] * ny[yj])))) / n
     (cx, nx), (cy, ny), (cj, nj) = _unique([[xs], [ys], [xs, ys]])
     verify_not_continuous(nx, n)
     verify_not_continuous(ny, n)
@@ -169,9 +226,11 @@ def estimate_conditional_discrete_mi(x, y, cond) -> float:
     n = len(x)
     reject_object(cond)
     zc = _columns(cond)
-    pair = np.column_stack((x, y))
-    reject_object(pair)
-    xs, ys = pair[:, 0], pair[:, 1]
+    xs, ys = _pair(x, y)
+    cols = zc + [xs, ys]
+    direct = _count_rows(cols) if all(_numeric(c) for c in cols) else None
+    if direct is not None:
+        return _conditional_mi_of_rows(n, *direct)
     (cz, nz), (czx, nzx), (czy, nzy), (czxy, nzxy) = _unique([zc, zc + [xs], zc + [ys], zc + [xs, ys]])
     # Condition row of every (z, x), (z, y) and (z, x, y) row.
     g_zx = np.empty(len(nzx), dtype=np.int64)
@@ -189,8 +248,31 @@ def estimate_conditional_discrete_mi(x, y, cond) -> float:
     zx_of[czxy] = czx
     zy_of = np.empty(len(nzxy), dtype=np.int64)
     zy_of[czxy] = czy
-    n_sub = nz[g_zxy]
-    terms = nzxy * np.log(n_sub * nzxy / (nzx[zx_of] * nzy[zy_of]))
+    return _sum_over_conditions(n, nz, g_zxy, nzxy, nzx[zx_of], nzy[zy_of])
+
+
+def _conditional_mi_of_rows(n: int, codes, nzxy: np.ndarray, radix: np.ndarray) -> float:
+    """The same from the distinct (condition, x, y) rows alone: the condition
+    rows, (z, x) and (z, y) cells and their points are sums over them."""
+    zkey = np.zeros(len(nzxy), dtype=np.int64)
+    for c in range(len(radix) - 2):
+        zkey = zkey * radix[c] + codes[c]
+    _, g = np.unique(zkey, return_inverse=True)   # condition row of every distinct row, lexicographic
+    nz = _sums(g, nzxy, int(g[-1]) + 1)
+    cells = []
+    for c, r in ((codes[-2], radix[-2]), (codes[-1], radix[-1])):
+        key, inv = np.unique(g * r + c, return_inverse=True)
+        if np.any(np.bincount(key // r, minlength=len(nz)) > nz / 4):
+            warn(MANY_VALUES_MESSAGE, UserWarning)
+        cells.append(_sums(inv, nzxy, len(key))[inv])
+    return _sum_over_conditions(n, nz, g, nzxy, cells[0], cells[1])
+
+
+def _sum_over_conditions(n: int, nz, g_zxy, nzxy, nzx, nzy) -> float:
+    """sum over condition rows of n_z MI(x; y | z), over n, from the distinct
+    (z, x, y) rows: their condition row and points, and the points of their
+    (z, x) and (z, y) rows."""
+    terms = nzxy * np.log(nz[g_zxy] * nzxy / (nzx * nzy))
     ends = np.cumsum(np.bincount(g_zxy, minlength=len(nz)))
     weighted = np.zeros(len(nz))
     for g in range(len(nz)):

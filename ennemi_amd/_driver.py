@@ -512,13 +512,13 @@ class DevicePrep:
 
     def _begin(self, arrays, mask, dz: int, n_tasks: int, preprocess, drop_nan, hints: bool) -> None:
         import torch
-        from ._batch import _stream
+        from ._batch import _stream, upload_columns
         self.ctx = nat.context()
         self.dev = torch.device("cuda", self.ctx.device)
         self.st = _stream()
         self.dz = dz
         self.n_tasks = n_tasks
-        self._upload(arrays)
+        self.d_raw, self.raw_host = upload_columns(arrays, self.dev, self.st)
         with torch.cuda.stream(self.st):
             self.d_mask = torch.from_numpy(np.ascontiguousarray(mask, dtype=np.uint8)).to(self.dev) \
                 if mask is not None else None
@@ -533,40 +533,6 @@ class DevicePrep:
         self.h_nan = np.zeros(n_tasks, dtype=np.uint32)
         self.arena = self.hint = self.d_const = self.d_noise = None
         self.noise_len = 0
-
-    def _upload(self, arrays) -> None:
-        """The arrays' columns in d_raw, one after the other.  They go up from
-        pinned host memory, asynchronously on the preparation stream (ahead
-        of the kernels that read them), while the host builds the task table;
-        a table held row by row is turned into columns on the device."""
-        import torch
-        n = len(arrays[0])
-        blocks = []   # values as they lie in memory (rows of `m`, or a column each), m
-        for a in arrays:
-            m = 1 if a.ndim == 1 else a.shape[1]
-            by_column = m == 1 or a.flags.f_contiguous
-            blocks.append((a.reshape(n) if m == 1 else a.T if by_column else a, 1 if by_column else m, n * m))
-        total = sum(size for _, _, size in blocks)
-        self.raw_host = torch.empty(total, dtype=torch.float64, pin_memory=True)
-        host = self.raw_host.numpy()
-        with torch.cuda.stream(self.st):
-            self.d_raw = torch.empty(total, dtype=torch.float64, device=self.dev)
-            at = 0
-            for a, m, size in blocks:
-                part = self.raw_host[at:at + size]
-                if a.dtype == np.float64 and a.flags.c_contiguous and a.flags.writeable and size >= 1 << 18:
-                    part.copy_(torch.from_numpy(a).reshape(-1))   # on several threads
-                else:
-                    host[at:at + size].reshape(a.shape)[...] = a
-                dst = self.d_raw[at:at + size]
-                if m == 1:
-                    dst.copy_(part, non_blocking=True)
-                else:
-                    rows = torch.empty(size, dtype=torch.float64, device=self.dev)
-                    rows.copy_(part, non_blocking=True)
-                    with self.ctx.lock:
-                        self.ctx.prep_columns(rows.data_ptr(), n, m, dst.data_ptr(), self.st.cuda_stream)
-                at += size
 
     def _ptrs(self):
         return self.d_raw.data_ptr(), self.d_mask.data_ptr() if self.d_mask is not None else 0

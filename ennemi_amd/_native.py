@@ -30,7 +30,7 @@ STAGES = ("fill", "sort", "gather", "knn", "count", "combine")
 
 EXPORTED_SYMBOLS = ("enm_init", "enm_shutdown", "enm_last_error", "enm_run_batch", "enm_run_batch_hinted",
                     "enm_run_batch_static", "enm_prep_columns", "enm_prep_count", "enm_prep_write", "enm_prep_hints",
-                    "enm_unique_rows", "enm_get_stats",
+                    "enm_unique_rows", "enm_count_rows", "enm_get_stats",
                     "enm_autotune", "enm_set_tuning", "enm_set_tuning_ex", "enm_get_tuning",
                     "enm_get_tuning_for")
 # Workspace of enm_run_batch_static, bytes (ENM_STATIC_WORKSPACE_BYTES).
@@ -79,6 +79,8 @@ class EnmRowset(ctypes.Structure):
 
 
 E_UNSUPPORTED = -4
+# Counters of enm_count_rows (ENM_COUNT_ROWS_MAX).
+COUNT_ROWS_MAX = 65536
 
 
 class EnmTuning(ctypes.Structure):
@@ -140,6 +142,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.enm_prep_hints.restype = ctypes.c_int
     lib.enm_unique_rows.argtypes = [vp, ctypes.POINTER(EnmRowset), ctypes.c_int32, vp, vp, vp, vp, vp]
     lib.enm_unique_rows.restype = ctypes.c_int
+    lib.enm_count_rows.argtypes = [vp, ctypes.POINTER(EnmRowset), vp, vp, vp, vp, ctypes.c_int64, vp]
+    lib.enm_count_rows.restype = ctypes.c_int
     lib.enm_get_stats.argtypes = [vp, ctypes.POINTER(EnmStats)]
     lib.enm_get_stats.restype = ctypes.c_int
     lib.enm_autotune.argtypes = [vp, ctypes.POINTER(EnmInstance), ctypes.c_int32,
@@ -240,6 +244,16 @@ class Context:
                                       h_distinct.ctypes.data, stream_ptr or None)
         if rc != E_UNSUPPORTED:
             self.check(rc, "enm_unique_rows")
+        return rc
+
+    def count_rows(self, rowset, values_ptr: int, h_least: np.ndarray, h_radix: np.ndarray, h_counts: np.ndarray,
+                   stream_ptr: int = 0) -> int:
+        """enm_count_rows; returns its status (0, or E_UNSUPPORTED when the
+        rows are not whole numbers in small ranges)."""
+        rc = self.lib.enm_count_rows(self.ctx, ctypes.byref(rowset), values_ptr, h_least.ctypes.data,
+                                     h_radix.ctypes.data, h_counts.ctypes.data, len(h_counts), stream_ptr or None)
+        if rc != E_UNSUPPORTED:
+            self.check(rc, "enm_count_rows")
         return rc
 
     def stats(self) -> dict:

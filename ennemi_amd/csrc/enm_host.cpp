@@ -308,7 +308,7 @@ struct enm_ctx {
     } prep;
     // Workspace of enm_unique_rows.
     struct Unique {
-        DevBuf tables, k0, k1, i0, i1, split, ccodes, cstarts, ccounts, cdist, rkeys, rstarts, rdist;
+        DevBuf tables, k0, k1, i0, i1, split, heads, ccodes, cstarts, ccounts, cdist, rkeys, rstarts, rdist, hist;
         std::vector<char> blob1, blob2;
     } uq;
     void* scratch = nullptr;          // this device's static workspace
@@ -2324,6 +2324,7 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
             u.start_off = tot1 + id;   // n + 1 slots each
             u.count_off = tot1;
             u.slot = id;
+            u.first_tile = sg.first_tile;
             segs1.push_back(sg);
             useg1.push_back(u);
             tot1 += R.n;
@@ -2337,6 +2338,7 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
         return U.k0.ensure(sort_n * 8) == hipSuccess && U.k1.ensure(sort_n * 8) == hipSuccess &&
                U.i0.ensure(sort_n * 4) == hipSuccess && U.i1.ensure(sort_n * 4) == hipSuccess &&
                U.split.ensure((size_t)tiles_max * 4 + 4) == hipSuccess &&
+               U.heads.ensure((size_t)tiles_max * 4 + 4) == hipSuccess &&
                U.ccodes.ensure(tot1 * 4) == hipSuccess && U.cstarts.ensure((tot1 + ncols) * 8) == hipSuccess &&
                U.ccounts.ensure(tot1 * 8) == hipSuccess && U.cdist.ensure((size_t)ncols * 8) == hipSuccess &&
                U.rkeys.ensure(tot2 * 8 + 8) == hipSuccess && U.rstarts.ensure((tot2 + n_sets) * 8 + 8) == hipSuccess &&
@@ -2356,9 +2358,9 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
                         ENM_SORT_TILE, d_values, nullptr, U.k0.as<double>(), U.i0.as<int>(), U.k1.as<double>(),
                         U.i1.as<int>(), U.split.as<int>(), &fb, &nl, st);
     if (e == hipSuccess)
-        e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(U.tables.as<char>() + o_u1), ncols,
+        e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(U.tables.as<char>() + o_u1), ncols, tiles1,
                                 fb ? U.k1.as<double>() : U.k0.as<double>(), fb ? U.i1.as<int>() : U.i0.as<int>(),
-                                U.ccodes.as<int>(), U.cstarts.as<int64_t>(), U.ccounts.as<int64_t>(),
+                                U.heads.as<int>(), U.ccodes.as<int>(), U.cstarts.as<int64_t>(), U.ccounts.as<int64_t>(),
                                 U.cdist.as<int64_t>(), st);
     std::vector<int64_t> cdist(ncols);
     if (e == hipSuccess) e = hipMemcpyAsync(cdist.data(), U.cdist.p, (size_t)ncols * 8, hipMemcpyDeviceToHost, st);
@@ -2404,6 +2406,7 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
         u.start_off = koff + (int64_t)useg2.size();
         u.count_off = set_off[s];
         u.slot = (int32_t)useg2.size();
+        u.first_tile = sg.first_tile;
         rks.push_back(rk);
         segs2.push_back(sg);
         useg2.push_back(u);
@@ -2427,9 +2430,9 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
                                 ENM_SORT_TILE, U.rkeys.as<double>(), nullptr, U.k0.as<double>(), U.i0.as<int>(),
                                 U.k1.as<double>(), U.i1.as<int>(), U.split.as<int>(), &fb, &nl, st);
         if (e == hipSuccess)
-            e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(tb + o_u2), (int)useg2.size(),
+            e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(tb + o_u2), (int)useg2.size(), tiles2,
                                     fb ? U.k1.as<double>() : U.k0.as<double>(), fb ? U.i1.as<int>() : U.i0.as<int>(),
-                                    d_codes, U.rstarts.as<int64_t>(), d_counts, U.rdist.as<int64_t>(), st);
+                                    U.heads.as<int>(), d_codes, U.rstarts.as<int64_t>(), d_counts, U.rdist.as<int64_t>(), st);
         if (e == hipSuccess)
             e = hipMemcpyAsync(rdist.data(), U.rdist.p, rdist.size() * 8, hipMemcpyDeviceToHost, st);
         if (e != hipSuccess) return hip_fail(ctx, e, "distinct rows");
@@ -2450,6 +2453,65 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
     e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
     for (size_t t = 0; t < multi_set.size(); ++t) h_distinct[multi_set[t]] = rdist[t];
+    return ENM_OK;
+}
+
+int enm_count_rows(enm_ctx* ctx, const enm_rowset* set, const double* d_values, double* h_least, int64_t* h_radix,
+                   uint32_t* h_counts, int64_t cap, void* stream) {
+    if (!ctx) { g_init_error = "ctx is NULL"; return ENM_E_ARG; }
+    ctx->err.clear();
+    if (!set || !d_values || !h_least || !h_radix || !h_counts || cap < 1)
+        return fail(ctx, ENM_E_ARG, "missing argument");
+    if (set->n < 1 || set->n > 0x7fffffffLL || set->ncol < 1 || set->ncol > ENM_MAX_COLS)
+        return fail(ctx, ENM_E_ARG, "bad row set");
+    hipError_t e = hipSetDevice(ctx->device);
+    if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
+    hipStream_t st = (hipStream_t)stream;
+    auto& U = ctx->uq;
+    cap = std::min<int64_t>(cap, ENM_COUNT_ROWS_MAX);
+    EnmRowsDev rows;
+    std::memset(&rows, 0, sizeof rows);
+    rows.n = set->n;
+    rows.ncol = set->ncol;
+    for (int c = 0; c < set->ncol; ++c) rows.col[c] = set->col[c];
+    const int next = 3 * ENM_MAX_COLS;
+    if (U.hist.ensure((size_t)next * 8 + (size_t)cap * 4) != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(ctx, ENM_E_NOMEM, "hipMalloc failed for the row counts");
+    }
+    // ext: least, greatest and oddity of every column, then the counts.
+    unsigned long long* ext = U.hist.as<unsigned long long>();
+    unsigned* counts = reinterpret_cast<unsigned*>(ext + next);
+    unsigned long long init[3 * ENM_MAX_COLS], got[3 * ENM_MAX_COLS];
+    for (int c = 0; c < ENM_MAX_COLS; ++c) { init[3 * c] = ~0ull; init[3 * c + 1] = init[3 * c + 2] = 0; }
+    e = hipMemcpyAsync(ext, init, sizeof init, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = enm_launch_uq_range(rows, d_values, ext, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(got, ext, sizeof got, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return hip_fail(ctx, e, "ranges of the columns");
+    auto value = [](unsigned long long m) {
+        const unsigned long long b = m >> 63 ? m & ~(1ull << 63) : ~m;
+        double v;
+        std::memcpy(&v, &b, 8);
+        return v;
+    };
+    double keys = 1.0;
+    for (int c = 0; c < set->ncol; ++c) {
+        if (got[3 * c + 2]) return fail(ctx, ENM_E_UNSUPPORTED, "a column holds values that are not whole numbers");
+        h_least[c] = value(got[3 * c]);
+        const double range = value(got[3 * c + 1]) - h_least[c] + 1.0;
+        keys *= range;
+        if (!(keys <= (double)cap)) return fail(ctx, ENM_E_UNSUPPORTED, "more value combinations than counters");
+        h_radix[c] = (int64_t)range;
+        rows.least[c] = h_least[c];
+        rows.radix[c] = (int32_t)range;
+    }
+    const int nk = (int)keys;
+    e = enm_launch_fill_i32(reinterpret_cast<int*>(counts), nk, 0, st);
+    if (e == hipSuccess) e = enm_launch_uq_hist(rows, d_values, nk, counts, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(h_counts, counts, (size_t)nk * 4, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return hip_fail(ctx, e, "row counts");
     return ENM_OK;
 }
 

@@ -349,7 +349,17 @@ struct UqSeg {
     int64_t start_off;  // run starts (n + 1 slots)
     int64_t count_off;  // points per code
     int32_t slot;       // its distinct-count slot
-    int32_t pad;
+    int32_t first_tile; // index of its first ENM_SORT_TILE positions
+};
+
+// A row set of whole numbers (enm_count_rows): its columns, their least
+// values and ranges.
+struct EnmRowsDev {
+    int64_t n;
+    int64_t col[16];
+    double least[16];
+    int32_t radix[16];
+    int32_t ncol;
 };
 
 // The mixed-radix keys of a multi-column row set.

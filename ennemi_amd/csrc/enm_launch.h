@@ -145,7 +145,11 @@ hipError_t enm_launch_hint_order(const HintCol* cols, int n_cols, int64_t max_w,
                                  int64_t noise_len, double* noise_max, unsigned* cont, int64_t cont_words,
                                  const HintSegs& sg, const double* arena, int* hint, int* bad, hipStream_t st);
 
-hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, const double* skeys, const int* sidx, int* codes,
-                               int64_t* starts, int64_t* counts, int64_t* distinct, hipStream_t st);
+hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, int ntiles, const double* skeys, const int* sidx,
+                               int* tile_heads, int* codes, int64_t* starts, int64_t* counts, int64_t* distinct,
+                               hipStream_t st);
+hipError_t enm_launch_uq_range(const EnmRowsDev& rows, const double* values, unsigned long long* ext, hipStream_t st);
+hipError_t enm_launch_uq_hist(const EnmRowsDev& rows, const double* values, int keys, unsigned* counts,
+                              hipStream_t st);
 hipError_t enm_launch_uq_keys(const UqRowKey* rk, int n_rk, int64_t max_n, const int* ccodes, double* keys,
                               hipStream_t st);

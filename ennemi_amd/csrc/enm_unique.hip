@@ -21,67 +21,197 @@
 namespace {
 
 constexpr int UQ_THREADS = 256;
-constexpr int UQ_PER = 4;                       // elements per thread and tile
-constexpr int UQ_TILE = UQ_THREADS * UQ_PER;
+constexpr int UQ_PER = 8;                       // elements per thread of a tile
+constexpr int UQ_TILE = UQ_THREADS * UQ_PER;    // as the sort's chunks
+constexpr int UQ_LDS_KEYS = 8192;              // counters of a workgroup in LDS
+static_assert(UQ_TILE == ENM_SORT_TILE, "tiles are numbered by the segments' first_tile");
 
-// One block per segment: codes (by point), run starts, counts and the
-// number of distinct values.
-__global__ __launch_bounds__(UQ_THREADS)
-void uq_codes_kernel(const UqSeg* __restrict__ segs, const double* __restrict__ skeys, const int* __restrict__ sidx,
-                     int* __restrict__ codes, int64_t* __restrict__ starts, int64_t* __restrict__ counts,
-                     int64_t* __restrict__ distinct) {
-    __shared__ int s_wave[UQ_THREADS / ENM_WAVE];
-    __shared__ int64_t s_carry;
-    const UqSeg sg = segs[blockIdx.x];
-    const int lane = threadIdx.x & (ENM_WAVE - 1), wv = threadIdx.x / ENM_WAVE;
-    if (threadIdx.x == 0) s_carry = 0;
-    __syncthreads();
-    for (int64_t t0 = 0; t0 < sg.n; t0 += UQ_TILE) {
-        // Thread-local heads of UQ_PER consecutive positions.
-        int heads = 0;
-        bool h[UQ_PER];
+__device__ __forceinline__ int uq_seg(const UqSeg* __restrict__ segs, int nsegs, int tile) {
+    int lo = 0, hi = nsegs - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (segs[mid].first_tile <= tile) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+// Run heads among a thread's UQ_PER consecutive positions.
+__device__ __forceinline__ int uq_heads(const UqSeg& sg, const double* __restrict__ skeys, int64_t i0,
+                                        bool (&h)[UQ_PER]) {
+    int heads = 0;
 #pragma unroll
-        for (int j = 0; j < UQ_PER; ++j) {
-            const int64_t i = t0 + threadIdx.x * UQ_PER + j;
-            h[j] = i < sg.n && (i == 0 || skeys[sg.sbase + i] != skeys[sg.sbase + i - 1]);
-            heads += h[j];
-        }
-        // Block-wide inclusive scan of the per-thread head counts.
-        int inc = heads;
+    for (int j = 0; j < UQ_PER; ++j) {
+        const int64_t i = i0 + j;
+        h[j] = i < sg.n && (i == 0 || skeys[sg.sbase + i] != skeys[sg.sbase + i - 1]);
+        heads += h[j];
+    }
+    return heads;
+}
+
+// Three passes over tiles of 2,048 sorted positions (one workgroup per segment
+// walked its tiles in sequence: 1.9 ms for two columns of 1,000,000): the run
+// heads of every tile, their running sums per segment, then codes (by point)
+// and run starts.
+__global__ __launch_bounds__(UQ_THREADS)
+void uq_heads_kernel(const UqSeg* __restrict__ segs, int nsegs, const double* __restrict__ skeys,
+                     int* __restrict__ tile_heads) {
+    __shared__ int s_wave[UQ_THREADS / ENM_WAVE];
+    const UqSeg& sg = segs[uq_seg(segs, nsegs, (int)blockIdx.x)];
+    const int64_t t0 = ((int64_t)blockIdx.x - sg.first_tile) * UQ_TILE;
+    bool h[UQ_PER];
+    int c = uq_heads(sg, skeys, t0 + threadIdx.x * UQ_PER, h);
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, ENM_WAVE);
+    if ((threadIdx.x & (ENM_WAVE - 1)) == 0) s_wave[threadIdx.x / ENM_WAVE] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int total = 0;
+        for (int w = 0; w < UQ_THREADS / ENM_WAVE; ++w) total += s_wave[w];
+        tile_heads[blockIdx.x] = total;
+    }
+}
+
+__global__ __launch_bounds__(ENM_WAVE)
+void uq_scan_kernel(const UqSeg* __restrict__ segs, int* __restrict__ tile_heads, int64_t* __restrict__ starts,
+                    int64_t* __restrict__ distinct) {
+    const UqSeg sg = segs[blockIdx.x];
+    const int lane = threadIdx.x;
+    const int nt = (int)((sg.n + UQ_TILE - 1) / UQ_TILE);
+    int carry = 0;
+    for (int base = 0; base < nt; base += ENM_WAVE) {
+        const int v = base + lane < nt ? tile_heads[sg.first_tile + base + lane] : 0;
+        int inc = v;
         for (int off = 1; off < ENM_WAVE; off <<= 1) {
             const int o = __shfl_up(inc, off, ENM_WAVE);
             if (lane >= off) inc += o;
         }
-        if (lane == ENM_WAVE - 1) s_wave[wv] = inc;
-        __syncthreads();
-        int before = 0, total = 0;
-        for (int w = 0; w < UQ_THREADS / ENM_WAVE; ++w) {
-            before += w < wv ? s_wave[w] : 0;
-            total += s_wave[w];
-        }
-        const int64_t carry = s_carry;
-        int64_t rank = carry + before + inc - heads - 1;  // code of the position before this thread's first
-#pragma unroll
-        for (int j = 0; j < UQ_PER; ++j) {
-            const int64_t i = t0 + threadIdx.x * UQ_PER + j;
-            if (i < sg.n) {
-                rank += h[j];
-                codes[sg.code_off + sidx[sg.sbase + i]] = (int)rank;
-                if (h[j]) starts[sg.start_off + rank] = i;
-            }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) s_carry = carry + total;
-        __syncthreads();
+        if (base + lane < nt) tile_heads[sg.first_tile + base + lane] = carry + inc - v;
+        carry += __shfl(inc, ENM_WAVE - 1, ENM_WAVE);
     }
-    const int64_t m = s_carry;
-    if (threadIdx.x == 0) {
-        starts[sg.start_off + m] = sg.n;
-        distinct[sg.slot] = m;
+    if (lane == 0) {
+        starts[sg.start_off + carry] = sg.n;
+        distinct[sg.slot] = carry;
+    }
+}
+
+__global__ __launch_bounds__(UQ_THREADS)
+void uq_codes_kernel(const UqSeg* __restrict__ segs, int nsegs, const double* __restrict__ skeys,
+                     const int* __restrict__ sidx, const int* __restrict__ tile_heads, int* __restrict__ codes,
+                     int64_t* __restrict__ starts) {
+    __shared__ int s_wave[UQ_THREADS / ENM_WAVE];
+    const UqSeg& sg = segs[uq_seg(segs, nsegs, (int)blockIdx.x)];
+    const int64_t i0 = ((int64_t)blockIdx.x - sg.first_tile) * UQ_TILE + threadIdx.x * UQ_PER;
+    const int lane = threadIdx.x & (ENM_WAVE - 1), wv = threadIdx.x / ENM_WAVE;
+    bool h[UQ_PER];
+    const int heads = uq_heads(sg, skeys, i0, h);
+    int inc = heads;
+    for (int off = 1; off < ENM_WAVE; off <<= 1) {
+        const int o = __shfl_up(inc, off, ENM_WAVE);
+        if (lane >= off) inc += o;
+    }
+    if (lane == ENM_WAVE - 1) s_wave[wv] = inc;
+    __syncthreads();
+    int64_t rank = tile_heads[blockIdx.x] + inc - heads - 1;   // code of the position before this thread's first
+    for (int w = 0; w < wv; ++w) rank += s_wave[w];
+#pragma unroll
+    for (int j = 0; j < UQ_PER; ++j) {
+        const int64_t i = i0 + j;
+        if (i < sg.n) {
+            rank += h[j];
+            codes[sg.code_off + sidx[sg.sbase + i]] = (int)rank;
+            if (h[j]) starts[sg.start_off + rank] = i;
+        }
+    }
+}
+
+// Points per code: run lengths.
+__global__ __launch_bounds__(UQ_THREADS)
+void uq_counts_kernel(const UqSeg* __restrict__ segs, int nsegs, const int64_t* __restrict__ starts,
+                      const int64_t* __restrict__ distinct, int64_t* __restrict__ counts) {
+    const UqSeg& sg = segs[uq_seg(segs, nsegs, (int)blockIdx.x)];
+    const int64_t m = distinct[sg.slot];
+    const int64_t r0 = ((int64_t)blockIdx.x - sg.first_tile) * UQ_TILE;
+    for (int64_t r = r0 + threadIdx.x; r < min(m, r0 + UQ_TILE); r += UQ_THREADS)
+        counts[sg.count_off + r] = starts[sg.start_off + r + 1] - starts[sg.start_off + r];
+}
+
+// ---------------------------------------------------------------------------
+// Rows of whole numbers in small ranges (class labels, levels): counted
+// directly, without a sort.
+
+// An order-preserving integer image of a double, for atomic extrema.
+__device__ __forceinline__ unsigned long long uq_image(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    return b >> 63 ? ~b : b | (1ull << 63);
+}
+
+// Per column: the images of its least and greatest value, and whether a value
+// is not a whole number below 2^53.  ext[3 c] starts at all ones, the others
+// at 0.
+__global__ __launch_bounds__(UQ_THREADS)
+void uq_range_kernel(EnmRowsDev rows, const double* __restrict__ values, unsigned long long* __restrict__ ext) {
+    __shared__ unsigned long long s_ext[UQ_THREADS / ENM_WAVE][3];
+    const double* v = values + rows.col[blockIdx.y];
+    unsigned long long lo = ~0ull, hi = 0;
+    bool odd = false;
+    for (int64_t i = (int64_t)blockIdx.x * UQ_THREADS + threadIdx.x; i < rows.n; i += (int64_t)gridDim.x * UQ_THREADS) {
+        const double x = v[i] + 0.0;   // (-0.0 is 0.0)
+        odd = odd || !(fabs(x) < 9007199254740992.0 && x == floor(x));
+        const unsigned long long m = uq_image(x);
+        lo = m < lo ? m : lo;
+        hi = m > hi ? m : hi;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long a = __shfl_xor(lo, off, ENM_WAVE), b = __shfl_xor(hi, off, ENM_WAVE);
+        lo = a < lo ? a : lo;
+        hi = b > hi ? b : hi;
+    }
+    const bool any = wave_any(odd);
+    const int wv = threadIdx.x / ENM_WAVE;
+    if ((threadIdx.x & (ENM_WAVE - 1)) == 0) {
+        s_ext[wv][0] = lo;
+        s_ext[wv][1] = hi;
+        s_ext[wv][2] = any ? 1 : 0;
     }
     __syncthreads();
-    for (int64_t r = threadIdx.x; r < m; r += UQ_THREADS)
-        counts[sg.count_off + r] = starts[sg.start_off + r + 1] - starts[sg.start_off + r];
+    if (threadIdx.x == 0) {
+        unsigned long long o = s_ext[0][2];
+        lo = s_ext[0][0];
+        hi = s_ext[0][1];
+        for (int w = 1; w < UQ_THREADS / ENM_WAVE; ++w) {
+            lo = s_ext[w][0] < lo ? s_ext[w][0] : lo;
+            hi = s_ext[w][1] > hi ? s_ext[w][1] : hi;
+            o |= s_ext[w][2];
+        }
+        atomicMin(ext + 3 * blockIdx.y, lo);
+        atomicMax(ext + 3 * blockIdx.y + 1, hi);
+        if (o) atomicOr(ext + 3 * blockIdx.y + 2, 1ull);
+    }
+}
+
+// Points per mixed-radix key of their values' offsets from the columns' least.
+// Bound by the reads of the columns; the counters of a workgroup are in LDS
+// where they fit (a few labels are many additions to few addresses).
+template <bool LDS>
+__global__ __launch_bounds__(UQ_THREADS)
+void uq_hist_kernel(EnmRowsDev rows, const double* __restrict__ values, int keys, unsigned* __restrict__ counts) {
+    extern __shared__ unsigned s_counts[];
+    if (LDS) {
+        for (int k = threadIdx.x; k < keys; k += UQ_THREADS) s_counts[k] = 0;
+        __syncthreads();
+    }
+    for (int64_t i = (int64_t)blockIdx.x * UQ_THREADS + threadIdx.x; i < rows.n; i += (int64_t)gridDim.x * UQ_THREADS) {
+        int key = 0;
+        for (int c = 0; c < rows.ncol; ++c)
+            key = key * rows.radix[c] + (int)(values[rows.col[c] + i] - rows.least[c]);
+        atomicAdd((LDS ? s_counts : counts) + key, 1u);
+    }
+    if (LDS) {
+        __syncthreads();
+        for (int k = threadIdx.x; k < keys; k += UQ_THREADS) {
+            const unsigned c = s_counts[k];
+            if (c) atomicAdd(counts + k, c);
+        }
+    }
 }
 
 // Mixed-radix keys of the rows of multi-column row sets (exact doubles).
@@ -99,11 +229,32 @@ __global__ void uq_key_kernel(const UqRowKey* __restrict__ rk, int n_rk, const i
 
 }  // namespace
 
-hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, const double* skeys, const int* sidx, int* codes,
-                               int64_t* starts, int64_t* counts, int64_t* distinct, hipStream_t st) {
+hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, int ntiles, const double* skeys, const int* sidx,
+                               int* tile_heads, int* codes, int64_t* starts, int64_t* counts, int64_t* distinct,
+                               hipStream_t st) {
     if (nsegs <= 0) return hipSuccess;
-    hipLaunchKernelGGL(uq_codes_kernel, dim3(nsegs), dim3(UQ_THREADS), 0, st, segs, skeys, sidx, codes, starts,
-                       counts, distinct);
+    hipLaunchKernelGGL(uq_heads_kernel, dim3(ntiles), dim3(UQ_THREADS), 0, st, segs, nsegs, skeys, tile_heads);
+    hipLaunchKernelGGL(uq_scan_kernel, dim3(nsegs), dim3(ENM_WAVE), 0, st, segs, tile_heads, starts, distinct);
+    hipLaunchKernelGGL(uq_codes_kernel, dim3(ntiles), dim3(UQ_THREADS), 0, st, segs, nsegs, skeys, sidx, tile_heads,
+                       codes, starts);
+    hipLaunchKernelGGL(uq_counts_kernel, dim3(ntiles), dim3(UQ_THREADS), 0, st, segs, nsegs, starts, distinct, counts);
+    return hipGetLastError();
+}
+
+hipError_t enm_launch_uq_range(const EnmRowsDev& rows, const double* values, unsigned long long* ext, hipStream_t st) {
+    const int blocks = (int)std::min<int64_t>((rows.n + UQ_TILE - 1) / UQ_TILE, 256);
+    hipLaunchKernelGGL(uq_range_kernel, dim3(blocks, rows.ncol), dim3(UQ_THREADS), 0, st, rows, values, ext);
+    return hipGetLastError();
+}
+
+hipError_t enm_launch_uq_hist(const EnmRowsDev& rows, const double* values, int keys, unsigned* counts,
+                              hipStream_t st) {
+    const int blocks = (int)std::min<int64_t>((rows.n + UQ_TILE - 1) / UQ_TILE, 512);
+    if (keys <= UQ_LDS_KEYS)
+        hipLaunchKernelGGL(uq_hist_kernel<true>, dim3(blocks), dim3(UQ_THREADS), (size_t)keys * 4, st, rows, values,
+                           keys, counts);
+    else
+        hipLaunchKernelGGL(uq_hist_kernel<false>, dim3(blocks), dim3(UQ_THREADS), 0, st, rows, values, keys, counts);
     return hipGetLastError();
 }
 

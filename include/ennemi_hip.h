@@ -321,6 +321,21 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets,
                     const double* d_values, int32_t* d_codes, int64_t* d_counts,
                     int64_t* h_distinct, void* stream);
 
+/*
+ * enm_count_rows: the points of every combination of values of one row set
+ * whose columns hold whole numbers in small ranges (class labels, levels),
+ * counted directly.  Column c takes values h_least[c] .. h_least[c] +
+ * h_radix[c] - 1, and a row's key is the mixed-radix number of its offsets
+ * from the least values, column 0 first (so keys ascend with the rows'
+ * lexicographic order): h_counts[key] points have it (0: none), for key <
+ * h_radix[0] * h_radix[1] * ...  ENM_E_UNSUPPORTED when a value is no whole
+ * number or the keys would exceed cap (at most ENM_COUNT_ROWS_MAX are used).
+ * Synchronous.
+ */
+#define ENM_COUNT_ROWS_MAX 65536
+int enm_count_rows(enm_ctx* ctx, const enm_rowset* set, const double* d_values, double* h_least, int64_t* h_radix,
+                   uint32_t* h_counts, int64_t cap, void* stream);
+
 /* Counters of the last enm_run_batch; synchronises the stream it used. */
 int enm_get_stats(enm_ctx* ctx, enm_stats* out);
 
