@@ -185,6 +185,7 @@ class ArenaBatch:
         self.device_arena = device_arena
         self.device_hint = device_hint
         self._runs: List[tuple] = []   # (kind, k, n per instance, dx, dy, dz, offsets per instance)
+        self._classes = None           # class sizes per instance (Ross kinds): n_segs, seg_index, all sizes
 
     def __len__(self) -> int:
         return sum(len(r[2]) for r in self._runs)
@@ -198,6 +199,12 @@ class ArenaBatch:
         offsets (per instance and column)."""
         self._runs.append((kind, int(k), np.asarray(n, dtype=np.int64), dx, dy, dz,
                            np.asarray(offsets, dtype=np.int64)))
+
+    def set_classes(self, sizes: np.ndarray) -> None:
+        """Rows of every class (instances by classes, 0: none) of the Ross
+        instances that are the whole batch."""
+        n_segs = (sizes > 0).sum(axis=1)
+        self._classes = (n_segs, np.cumsum(n_segs) - n_segs, sizes[sizes > 0])
 
     @property
     def _inst(self) -> List[tuple]:
@@ -215,6 +222,9 @@ class ArenaBatch:
                 t[name] = v
             t["col"][:, :cols.shape[1]] = cols
         seg_arr = (ctypes.c_int64 * 1)(0)
+        if self._classes is not None:
+            tab["n_segs"], tab["seg_index"] = self._classes[:2]
+            seg_arr = (ctypes.c_int64 * len(self._classes[2]))(*self._classes[2].tolist())
         return None, inst_arr, seg_arr
 
     def point_offsets(self) -> np.ndarray:

@@ -246,8 +246,7 @@ def _add_mi_task(tasks: _Tasks, xs, ys, zs, k: int, discrete_x: bool, discrete_y
             cont = np.column_stack((cont,))
             values, counts, grouped = _group_by_class(disc, [cont[:, c] for c in range(cont.shape[1])])
             if len(values) > len(disc) / 4:
-                warn("The discrete variable has relatively many unique values." +
-                     " Did you pass y and x in correct order?", UserWarning)
+                _warn_many_values(False)
             tasks.gpu(b.add(nat.KIND_ROSS, k, grouped, class_sizes=counts))
             return
         tasks.gpu(b.add(nat.KIND_KSG, k, _cols(xs), _cols(ys)))
@@ -410,6 +409,11 @@ def _plan_mi(y, x, lag, k, cond, cond_lag, mask, discrete_x, discrete_y, preproc
     if prep != "host" and _device_prep_eligible(x, y, cond, discrete_x, discrete_y):
         return _plan_mi_device(y, x, lag, k, cond, cond_lag, mask, preprocess, drop_nan,
                                min_lag, max_lag, indices), indices, nvar
+    if prep != "host" and bool(discrete_x) != bool(discrete_y) and _classes_eligible(x, y, cond, discrete_x):
+        tasks = _plan_classes_device(y, x, lag, k, cond, cond_lag, mask, bool(discrete_x), preprocess, drop_nan,
+                                     min_lag, max_lag, indices)
+        if tasks is not None:
+            return tasks, indices, nvar
     tasks = _Tasks()
     noise = _Noise()
     for (li, v) in indices:
@@ -469,12 +473,14 @@ class DevicePrep:
     device order (by x column, then lag); place[t] is task t's slot."""
 
     def __init__(self, y, x, lag, cond, cond_lag, mask, preprocess, drop_nan, min_lag, max_lag, indices,
-                 hints: bool = True):
+                 hints: bool = True, labels: int = 0):
+        # labels: P_X_RAW or P_Y_RAW where x or y holds class labels.
         n_rows = len(y)
         nvar = 1 if x.ndim == 1 else x.shape[1]
         dz = 0 if cond is None else cond.shape[1]
         n_tasks = len(indices)
         self._begin([y, x] + ([] if cond is None else [cond]), mask, dz, n_tasks, preprocess, drop_nan, hints)
+        self.flags |= labels
         min_lag = min(min_lag, 0)
         max_lag = max(max_lag, 0)
         # Device order: by x column, then lag, so a kernel's consecutive
@@ -622,15 +628,94 @@ def _plan_mi_device(y, x, lag, k, cond, cond_lag, mask, preprocess, drop_nan, mi
     return tasks_out
 
 
-def _constant_warnings(prep) -> None:
+def _classes_eligible(x, y, cond, discrete_x: bool) -> bool:
+    """Class labels that are numbers, with a continuous variable (and
+    condition) that the device prepares."""
+    cont, labels = (y, x) if discrete_x else (x, y)
+    return labels.dtype.kind in "biuf" and labels.dtype.itemsize <= 8 and \
+        _device_prep_arrays((cont,) if cond is None else (cont, cond), cond)
+
+
+def _plan_classes_device(y, x, lag, k, cond, cond_lag, mask, discrete_x: bool, preprocess, drop_nan, min_lag, max_lag,
+                         indices):
+    """_plan_mi of class labels against continuous variables, prepared and
+    grouped by class on the device.  None where the labels are not whole
+    numbers in a small range or a task fails validation (the host path then
+    takes the call, and raises in the reference's order)."""
+    import torch
+    from ._batch import ArenaBatch
+    prep = DevicePrep(y, x, lag, cond, cond_lag, mask, preprocess, drop_nan, min_lag, max_lag, indices,
+                      hints=False, labels=nat.P_X_RAW if discrete_x else nat.P_Y_RAW)
+    ctx, dz, n_rows = prep.ctx, prep.dz, len(y)
+    tab = nat.struct_array(prep.tasks)
+    label_col = tab["x_col"] if discrete_x else tab["y_col"]
+    least = np.empty(prep.n_tasks)
+    classes = 1
+    rowset = nat.EnmRowset()
+    rowset.n, rowset.ncol = n_rows, 1
+    low, radix = np.zeros(1), np.zeros(1, dtype=np.int64)
+    counts = np.zeros(nat.GROUP_CLASSES_MAX, dtype=np.uint32)
+    with ctx.prep_lock:
+        for col in np.unique(label_col):
+            rowset.col[0] = int(col)
+            with ctx.lock:
+                if ctx.count_rows(rowset, prep.d_raw.data_ptr(), low, radix, counts, prep.st.cuda_stream):
+                    return None
+            least[label_col == col] = low[0]
+            classes = max(classes, int(radix[0]))
+        if not prep.valid(k):
+            return None
+        prep.write()
+    n, cols = prep.h_n, prep.columns()
+    # Grouped columns: the continuous variable, then the condition.
+    src = np.column_stack([cols[:, 1 if discrete_x else 0]] + [cols[:, 2 + c] for c in range(dz)])
+    first = np.cumsum(n * (1 + dz)) - n * (1 + dz)
+    dst = first[:, None] + n[:, None] * np.arange(1 + dz)
+    tasks = (nat.EnmGroupTask * prep.n_tasks)()
+    g = nat.struct_array(tasks)
+    g["n"], g["least"], g["ncol"] = n, least, 1 + dz
+    g["label"] = cols[:, 0 if discrete_x else 1]
+    g["src"][:, :1 + dz] = src
+    g["dst"][:, :1 + dz] = dst
+    sizes = np.zeros((prep.n_tasks, classes), dtype=np.int64)
+    with torch.cuda.stream(prep.st):
+        arena = torch.empty(int((n * (1 + dz)).sum()), dtype=torch.float64, device=prep.dev)
+    with ctx.lock:
+        ctx.group_rows(tasks, prep.n_tasks, classes, prep.arena.data_ptr(), arena.data_ptr(), sizes,
+                       prep.st.cuda_stream)
+    out = _Tasks()
+    out.batch = ArenaBatch(arena)
+    out.batch.prep = prep
+    out.batch.add_many(nat.KIND_ROSS if dz == 0 else nat.KIND_CROSS, k, n, dst, 1, 0, dz)
+    out.batch.set_classes(sizes)
+    out.slots = [("gpu", p) for p in prep.place.tolist()]
+    many = ((sizes > 0).sum(axis=1) > n / 4)[prep.place]
+
+    def warnings():
+        _constant_warnings(prep, lambda t: many[t] and _warn_many_values(dz > 0))
+    out.deferred.append(warnings)
+    return out
+
+
+def _warn_many_values(conditional: bool) -> None:
+    if conditional:
+        warn(_discrete.MANY_VALUES_MESSAGE, UserWarning)
+    else:
+        warn("The discrete variable has relatively many unique values." +
+             " Did you pass y and x in correct order?", UserWarning)
+
+
+def _constant_warnings(prep, and_then=None) -> None:
     """The warnings of constant variables, task by task.  Read after the batch
     is launched (the flags are ready by then): reading them first would wait
     for the preparation before the batch could be planned and launched."""
     const = prep.constant_flags()
-    for t in np.flatnonzero(const):
+    for t in range(prep.n_tasks) if and_then else np.flatnonzero(const):
         for bit in (1, 2, 4):
             if const[t] & bit and (bit != 4 or prep.dz > 0):
                 warn(PREPROCESS_CONSTANT_DATA_WARNING)
+        if and_then:
+            and_then(t)
 
 
 # ---------------------------------------------------------------------------

@@ -30,7 +30,7 @@ STAGES = ("fill", "sort", "gather", "knn", "count", "combine")
 
 EXPORTED_SYMBOLS = ("enm_init", "enm_shutdown", "enm_last_error", "enm_run_batch", "enm_run_batch_hinted",
                     "enm_run_batch_static", "enm_prep_columns", "enm_prep_count", "enm_prep_write", "enm_prep_hints",
-                    "enm_unique_rows", "enm_count_rows", "enm_get_stats",
+                    "enm_group_rows", "enm_unique_rows", "enm_count_rows", "enm_get_stats",
                     "enm_autotune", "enm_set_tuning", "enm_set_tuning_ex", "enm_get_tuning",
                     "enm_get_tuning_for")
 # Workspace of enm_run_batch_static, bytes (ENM_STATIC_WORKSPACE_BYTES).
@@ -52,6 +52,10 @@ PREP_MAXZ = MAX_COLS - 2
 P_DROP_NAN = 0x1
 P_RESCALE = 0x2
 P_HINTS = 0x4
+P_X_RAW = 0x8
+P_Y_RAW = 0x10
+# Classes of enm_group_rows (ENM_GROUP_CLASSES_MAX).
+GROUP_CLASSES_MAX = 1024
 
 
 class EnmPrepTask(ctypes.Structure):
@@ -59,6 +63,12 @@ class EnmPrepTask(ctypes.Structure):
                 ("x0", ctypes.c_int64), ("y0", ctypes.c_int64), ("w", ctypes.c_int64),
                 ("dz", ctypes.c_int32), ("pad", ctypes.c_int32),
                 ("z_col", ctypes.c_int64 * PREP_MAXZ), ("z0", ctypes.c_int64 * PREP_MAXZ)]
+
+
+class EnmGroupTask(ctypes.Structure):
+    _fields_ = [("n", ctypes.c_int64), ("label", ctypes.c_int64), ("least", ctypes.c_double),
+                ("src", ctypes.c_int64 * MAX_COLS), ("dst", ctypes.c_int64 * MAX_COLS),
+                ("ncol", ctypes.c_int32), ("pad", ctypes.c_int32)]
 
 
 _dtypes = {}
@@ -140,6 +150,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.enm_prep_hints.argtypes = [vp, ctypes.POINTER(EnmPrepTask), ctypes.c_int32, vp, vp, vp,
                                    ctypes.c_int64, ctypes.c_uint32, vp, vp, vp, vp]
     lib.enm_prep_hints.restype = ctypes.c_int
+    lib.enm_group_rows.argtypes = [vp, ctypes.POINTER(EnmGroupTask), ctypes.c_int32, ctypes.c_int32, vp, vp, vp, vp]
+    lib.enm_group_rows.restype = ctypes.c_int
     lib.enm_unique_rows.argtypes = [vp, ctypes.POINTER(EnmRowset), ctypes.c_int32, vp, vp, vp, vp, vp]
     lib.enm_unique_rows.restype = ctypes.c_int
     lib.enm_count_rows.argtypes = [vp, ctypes.POINTER(EnmRowset), vp, vp, vp, vp, ctypes.c_int64, vp]
@@ -235,6 +247,12 @@ class Context:
                                      noise_ptr or None, noise_len, flags, arena_off.ctypes.data,
                                      arena_ptr, hint_ptr, stream_ptr or None)
         self.check(rc, "enm_prep_hints")
+
+    def group_rows(self, tasks, n_tasks: int, classes: int, src_ptr: int, dst_ptr: int, h_sizes: np.ndarray,
+                   stream_ptr: int = 0) -> None:
+        rc = self.lib.enm_group_rows(self.ctx, tasks, n_tasks, classes, src_ptr, dst_ptr, h_sizes.ctypes.data,
+                                     stream_ptr or None)
+        self.check(rc, "enm_group_rows")
 
     def unique_rows(self, sets, n_sets: int, values_ptr: int, codes_ptr: int, counts_ptr: int,
                     h_distinct: np.ndarray, stream_ptr: int = 0) -> int:

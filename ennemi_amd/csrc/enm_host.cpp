@@ -306,7 +306,11 @@ struct enm_ctx {
         DevBuf kept, tables3, hkeys, hk0, hk1, hi0, hi1, hsplit, hcont, hbad, hmax, sg_cnt, sg_last, sg_off,
             sg_cin, sg_chas;
     } prep;
-    // Workspace of enm_unique_rows.
+    // Workspace of enm_group_rows.
+    struct Grouping {
+        DevBuf tables, counts, sizes;
+    } group;
+    // Workspace of enm_unique_rows and enm_count_rows.
     struct Unique {
         DevBuf tables, k0, k1, i0, i1, split, heads, ccodes, cstarts, ccounts, cdist, rkeys, rstarts, rdist, hist;
         std::vector<char> blob1, blob2;
@@ -2042,6 +2046,8 @@ int enm_prep_write(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks, co
         return fail(ctx, ENM_E_ARG, "enm_prep_write must follow enm_prep_count of the same tasks and inputs");
     if (!tasks || !arena_off || !d_arena || !d_const) return fail(ctx, ENM_E_ARG, "missing argument");
     const bool rescale = (flags & ENM_P_RESCALE) != 0;
+    const unsigned raw_vars = ((flags & ENM_P_X_RAW) ? 1u : 0u) | ((flags & ENM_P_Y_RAW) ? 2u : 0u);
+    if (raw_vars && (flags & ENM_P_HINTS)) return fail(ctx, ENM_E_ARG, "no sort hints with class labels");
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
     hipStream_t st = (hipStream_t)stream;
@@ -2065,6 +2071,7 @@ int enm_prep_write(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks, co
         // multi-column condition: row-by-row sums.
         const int narr = 2 + D.dz;
         for (int a = 0; a < narr; ++a) {
+            if (a < 2 && ((raw_vars >> a) & 1u)) continue;   // labels: never rescaled
             PrepSumDev sd;
             std::memset(&sd, 0, sizeof sd);
             sd.src = D.arena_off + a * n;
@@ -2125,7 +2132,7 @@ int enm_prep_write(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks, co
                               reinterpret_cast<const int*>(base + o_cs), reinterpret_cast<const int*>(base + o_ci),
                               reinterpret_cast<const int*>(base + o_cl), (int)chunk_sum_of.size(), n_full,
                               S.chunk_val.as<double>(), S.stats.as<double>(), sstride,
-                              d_noise, d_const, d_arena, hints ? S.kept.as<KeptWord>() : nullptr, st);
+                              d_noise, raw_vars, d_const, d_arena, hints ? S.kept.as<KeptWord>() : nullptr, st);
     if (e != hipSuccess) return hip_fail(ctx, e, "prep write");
     if (!rescale) {
         e = enm_launch_fill_i32(reinterpret_cast<int*>(d_const), n_tasks, 0, st);
@@ -2276,6 +2283,47 @@ int enm_prep_hints(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks, co
                               (flags & ENM_P_RESCALE) ? d_noise : nullptr, noise_len, S.hmax.as<double>(),
                               S.hcont.as<unsigned>(), cont_words, hsg, d_arena, d_hint, S.hbad.as<int>(), st);
     if (e != hipSuccess) return hip_fail(ctx, e, "hint order");
+    return ENM_OK;
+}
+
+int enm_group_rows(enm_ctx* ctx, const enm_group_task* tasks, int32_t n_tasks, int32_t classes, const double* d_src,
+                   double* d_dst, int64_t* h_sizes, void* stream) {
+    if (!ctx) { g_init_error = "ctx is NULL"; return ENM_E_ARG; }
+    ctx->err.clear();
+    if (!tasks || n_tasks <= 0 || !d_src || !d_dst || !h_sizes) return fail(ctx, ENM_E_ARG, "missing argument");
+    if (classes < 1 || classes > ENM_GROUP_CLASSES_MAX) return fail(ctx, ENM_E_UNSUPPORTED, "too many classes");
+    hipError_t e = hipSetDevice(ctx->device);
+    if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
+    hipStream_t st = (hipStream_t)stream;
+    auto& G = ctx->group;
+    std::vector<GroupTaskDev> dev(n_tasks);
+    int64_t stride = 1;
+    for (int i = 0; i < n_tasks; ++i) {
+        const enm_group_task& t = tasks[i];
+        if (t.n < 1 || t.n > 0x7fffffffLL || t.ncol < 1 || t.ncol > ENM_MAX_COLS)
+            return fail(ctx, ENM_E_ARG, "bad rows or columns to group");
+        GroupTaskDev& d = dev[i];
+        std::memset(&d, 0, sizeof d);
+        d.n = t.n;
+        d.label = t.label;
+        d.least = t.least;
+        d.ncol = t.ncol;
+        for (int c = 0; c < t.ncol; ++c) { d.src[c] = t.src[c]; d.dst[c] = t.dst[c]; }
+        stride = std::max(stride, (t.n + ENM_PREP_BLOCK - 1) / ENM_PREP_BLOCK);
+    }
+    const size_t sizes = (size_t)n_tasks * classes;
+    if (G.tables.ensure(dev.size() * sizeof(GroupTaskDev)) != hipSuccess ||
+        G.counts.ensure((size_t)stride * sizes * 4) != hipSuccess || G.sizes.ensure(sizes * 8) != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(ctx, ENM_E_NOMEM, "hipMalloc failed for the class counts");
+    }
+    e = hipMemcpyAsync(G.tables.p, dev.data(), dev.size() * sizeof(GroupTaskDev), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess)
+        e = enm_launch_group(G.tables.as<GroupTaskDev>(), n_tasks, stride, classes, d_src, G.counts.as<int>(),
+                             G.sizes.as<int64_t>(), d_dst, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(h_sizes, G.sizes.p, sizes * 8, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return hip_fail(ctx, e, "group rows");
     return ENM_OK;
 }
 

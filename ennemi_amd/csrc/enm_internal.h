@@ -331,6 +331,15 @@ struct HintCol {
 #define ENM_HINT_BLOCK 1024   // sorted series rows per filter chunk (256 threads x 4)
 #define ENM_HINT_RUN 32       // longest run of near-equal values re-sorted (longer: no hint)
 
+// Rows grouped by class (enm_group_rows).
+struct GroupTaskDev {
+    int64_t n;
+    int64_t label;              // source offset of the labels
+    double least;               // the smallest label
+    int64_t src[16], dst[16];   // offsets of each column, before and after
+    int32_t ncol, pad;
+};
+
 // One array whose mean and standard deviation NumPy's way are needed.
 struct PrepSumDev {
     int64_t src;        // arena offset

@@ -118,8 +118,8 @@ hipError_t enm_launch_prep_write(PrepTaskDev* tasks, int64_t stride, int n_tasks
                                  const int64_t* blk_off, const PrepSumDev* sums, int n_sums,
                                  const int* chunk_sum_of, const int* chunk_index, const int* chunk_list,
                                  int n_chunks, int n_full, double* chunk_val, double* stats, int64_t sstride,
-                                 const double* noise, unsigned* const_flag, double* arena, KeptWord* kept,
-                                 hipStream_t st);
+                                 const double* noise, unsigned raw_vars, unsigned* const_flag, double* arena,
+                                 KeptWord* kept, hipStream_t st);
 // Sort hints (enm_hint.hip).
 hipError_t enm_launch_hint_keys(const HintSeries* series, int n_series, int64_t maxlen, const double* raw,
                                 double* keys, hipStream_t st);
@@ -145,6 +145,8 @@ hipError_t enm_launch_hint_order(const HintCol* cols, int n_cols, int64_t max_w,
                                  int64_t noise_len, double* noise_max, unsigned* cont, int64_t cont_words,
                                  const HintSegs& sg, const double* arena, int* hint, int* bad, hipStream_t st);
 
+hipError_t enm_launch_group(const GroupTaskDev* tasks, int n_tasks, int64_t stride, int classes, const double* src,
+                            int* counts, int64_t* sizes, double* dst, hipStream_t st);
 hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, int ntiles, const double* skeys, const int* sidx,
                                int* tile_heads, int* codes, int64_t* starts, int64_t* counts, int64_t* distinct,
                                hipStream_t st);

@@ -483,17 +483,21 @@ void prep_finish_kernel(const PrepSumDev* __restrict__ sums, int n_sums, const d
 }
 
 // Phase 2d: which variables are rescaled, where their noise starts, and
-// their flag bits (bit 0 x, bit 1 y, bit 2 z constant).  One thread per task.
+// their flag bits (bit 0 x, bit 1 y, bit 2 z constant).  Variables of
+// raw_vars (bit 0 x, bit 1 y) are class labels: never rescaled, no noise drawn,
+// not called constant.  One thread per task.
 __global__ void prep_noise_kernel(PrepTaskDev* __restrict__ tasks, int n_tasks, const double* __restrict__ stats,
-                                  unsigned* __restrict__ const_flag) {
+                                  unsigned raw_vars, unsigned* __restrict__ const_flag) {
     const int ti = blockIdx.x * blockDim.x + threadIdx.x;
     if (ti >= n_tasks) return;
     PrepTaskDev& t = tasks[ti];
     unsigned fl = 0;
-    if (fabs(stats[t.stat + 1]) < 1e-20) fl |= 1u;
-    if (fabs(stats[t.stat + 3]) < 1e-20) fl |= 2u;
+    if (!(raw_vars & 1u) && fabs(stats[t.stat + 1]) < 1e-20) fl |= 1u;
+    if (!(raw_vars & 2u) && fabs(stats[t.stat + 3]) < 1e-20) fl |= 2u;
     for (int c = 0; c < t.dz; ++c)
         if (fabs(stats[t.stat + 4 + 2 * c + 1]) < 1e-20) fl |= 4u;
+    const_flag[ti] = fl;
+    fl |= raw_vars;
     int64_t drawn = 0;
     t.noise_x = drawn;
     if (!(fl & 1u)) drawn += t.n;
@@ -501,7 +505,6 @@ __global__ void prep_noise_kernel(PrepTaskDev* __restrict__ tasks, int n_tasks, 
     if (!(fl & 2u)) drawn += t.n;
     t.noise_z = drawn;
     t.flags = fl;
-    const_flag[ti] = fl;
 }
 
 // Phase 2e: (v - mean) / std + noise for every rescaled value, in place.
@@ -559,8 +562,8 @@ hipError_t enm_launch_prep_write(PrepTaskDev* tasks, int64_t stride, int n_tasks
                                  const int64_t* blk_off, const PrepSumDev* sums, int n_sums,
                                  const int* chunk_sum_of, const int* chunk_index, const int* chunk_list,
                                  int n_chunks, int n_full, double* chunk_val, double* stats, int64_t sstride,
-                                 const double* noise, unsigned* const_flag, double* arena, KeptWord* kept,
-                                 hipStream_t st) {
+                                 const double* noise, unsigned raw_vars, unsigned* const_flag, double* arena,
+                                 KeptWord* kept, hipStream_t st) {
     if (n_tasks <= 0) return hipSuccess;
     const int64_t n_blocks = stride * n_tasks, n_sblocks = sstride * n_tasks;
     if (n_blocks > 0)
@@ -583,7 +586,7 @@ hipError_t enm_launch_prep_write(PrepTaskDev* tasks, int64_t stride, int n_tasks
                            chunk_val, pass, stats);
     }
     hipLaunchKernelGGL(prep_noise_kernel, dim3((unsigned)((n_tasks + 63) / 64)), dim3(64), 0, st, tasks, n_tasks,
-                       stats, const_flag);
+                       stats, raw_vars, const_flag);
     if (n_sblocks > 0)
         hipLaunchKernelGGL(prep_scale_kernel, dim3((unsigned)n_sblocks), dim3(PB_THREADS), 0, st, tasks, sstride,
                            stats, noise, arena);

@@ -255,6 +255,8 @@ typedef struct enm_prep_task {
 
 #define ENM_P_DROP_NAN 0x1u
 #define ENM_P_RESCALE  0x2u
+#define ENM_P_X_RAW    0x8u  /* x holds class labels: left as it is, no noise drawn */
+#define ENM_P_Y_RAW   0x10u  /* the same for y                                     */
 #define ENM_P_HINTS    0x4u  /* enm_prep_write keeps what enm_prep_hints needs */
 
 /*
@@ -291,6 +293,32 @@ int enm_prep_hints(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks,
                    const double* d_noise, int64_t noise_len, uint32_t flags,
                    const int64_t* arena_off, const double* d_arena, int32_t* d_hint,
                    void* stream);
+
+/*
+ * enm_group_rows: rows grouped by class, for the discrete-continuous
+ * estimators, whose points go class by class (enm_instance), replacing
+ *
+ *   np.unique(y) and x[y == value]   ennemi/_entropy_estimators.py:177-196
+ *
+ * Task t has n rows, whose labels d_src[label ..] are whole numbers least ..
+ * least + classes - 1; each of its columns d_src[src[c] ..] is written to
+ * d_dst[dst[c] ..] with the rows of a class together, classes in ascending
+ * order, rows in their own order within a class.  h_sizes[t * classes + c]
+ * rows are of class c (0: none).  d_src and d_dst must not overlap.
+ * ENM_E_UNSUPPORTED for more than ENM_GROUP_CLASSES_MAX classes.  Synchronous.
+ */
+#define ENM_GROUP_CLASSES_MAX 1024
+typedef struct enm_group_task {
+    int64_t n;
+    int64_t label;
+    double least;
+    int64_t src[ENM_MAX_COLS], dst[ENM_MAX_COLS];
+    int32_t ncol;
+    int32_t pad;
+} enm_group_task;
+
+int enm_group_rows(enm_ctx* ctx, const enm_group_task* tasks, int32_t n_tasks, int32_t classes, const double* d_src,
+                   double* d_dst, int64_t* h_sizes, void* stream);
 
 /*
  * enm_unique_rows: the distinct rows of row sets and their counts, as
