@@ -240,6 +240,13 @@ class ArenaBatch:
         return db.results()
 
 
+# Values that are copied to pinned memory and sent up at a time, so that one piece
+# goes up while the next is copied.  The calling thread copies them: where the
+# caller's own program keeps all processors busy (NumPy's threads spin on after a
+# matrix product), one that waits for helpers, woken or new, waited 4 ms for them.
+_PIECE = 1 << 18
+
+
 def upload_columns(arrays, device, stream):
     """The values of arrays (equally long: columns, or tables of columns) as
     float64 columns in HBM, one after the other; returns (device columns,
@@ -255,26 +262,32 @@ def upload_columns(arrays, device, stream):
         blocks.append((a.reshape(n) if m == 1 else a.T if by_column else a, 1 if by_column else m, n * m))
     total = sum(size for _, _, size in blocks)
     pinned = torch.empty(total, dtype=torch.float64, pin_memory=True)
-    host = pinned.numpy()
     ctx = nat.context()
     with torch.cuda.stream(stream):
         d_cols = torch.empty(total, dtype=torch.float64, device=device)
         at = 0
         for a, m, size in blocks:
-            part = pinned[at:at + size]
-            if size >= 1 << 18 and a.flags.c_contiguous and a.flags.writeable and \
-                    a.dtype in (np.float64, np.int64, np.int32):
-                part.copy_(torch.from_numpy(a).reshape(-1))   # on several threads
-            else:
-                host[at:at + size].reshape(a.shape)[...] = a
             dst = d_cols[at:at + size]
-            if m == 1:
-                dst.copy_(part, non_blocking=True)
+            whole = a.dtype in (np.int64, np.int32)   # go up as they are, become doubles there
+            dtype = getattr(torch, a.dtype.name) if whole else torch.float64
+            up = torch.empty(size, dtype=dtype, device=device) if whole or m > 1 else dst
+            part = pinned[at:at + size].view(dtype)[:size]
+            host = part.numpy()
+            if a.flags.c_contiguous:
+                a = a.reshape(-1)
+                for i in range(0, size, _PIECE):
+                    piece = slice(i, min(i + _PIECE, size))
+                    host[piece] = a[piece]
+                    up[piece].copy_(part[piece], non_blocking=True)
             else:
-                rows = torch.empty(size, dtype=torch.float64, device=device)
-                rows.copy_(part, non_blocking=True)
+                host.reshape(a.shape)[...] = a
+                up.copy_(part, non_blocking=True)
+            if m > 1:
+                rows = up.to(torch.float64)
                 with ctx.lock:
                     ctx.prep_columns(rows.data_ptr(), n, m, dst.data_ptr(), stream.cuda_stream)
+            elif whole:
+                dst.copy_(up)
             at += size
     return d_cols, pinned
 
