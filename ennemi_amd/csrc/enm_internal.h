@@ -346,8 +346,15 @@ struct PrepSumDev {
     int64_t n;
     int32_t stat;       // stats slot of the mean (the std follows)
     int32_t sequential; // 1: accumulated row by row (a column of a multi-column condition)
-    int32_t chunk0;     // pairwise arrays: first of its 8192-value chunks
-    int32_t n_chunks;
+    int32_t chunk0;     // first of its chunks of 8192 values (pairwise) or of its
+    int32_t n_chunks;   // blocks of ENM_PREP_SEQ_BLOCK rows (row by row; none: short)
+};
+
+// A column summed row by row: 64 rows of it (see enm_prep.hip).
+#define ENM_PREP_SEQ_BLOCK 4096
+struct PrepSeqTile {
+    double add, lo, hi;   // units the sum gains, its least and greatest gain on the way
+    int32_t odd, bits;    // 1 or -1: gains so much more if the sum was odd; flags
 };
 
 // Distinct rows (enm_unique_rows): one sorted segment of keys.
