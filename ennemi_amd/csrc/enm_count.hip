@@ -352,9 +352,13 @@ void psi_tile_kernel(const Item* __restrict__ items, int n_items, const CountDev
 }
 
 // psi_tab[c] = psi(c) for c in [1, n], psi_tab[0] = +inf.
-__global__ void psi_table_kernel(double* __restrict__ tab, int64_t n) {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c <= n) tab[c] = c == 0 ? INFINITY : enm_psi((double)c);
+__global__ void init_kernel(InitArgs a) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i <= a.n) a.tab[i] = i == 0 ? INFINITY : enm_psi((double)i);
+    if (i < ENM_ST_SLOTS) a.stats[i] = 0;
+    if (i < a.n_maxabs) a.maxabs[i] = 0;
+    if (i < a.n_counters) a.counters[i] = 0;
+    if (i < a.n_hint_bad) a.hint_bad[i] = 0;
 }
 
 template <int D, bool F32>
@@ -548,10 +552,9 @@ hipError_t enm_launch_count(const Item* items, const int* qoff, int n_items, uns
     }
 }
 
-hipError_t enm_launch_psi_table(double* tab, int64_t n, hipStream_t st) {
-    const int threads = 256;
-    const int64_t blocks = (n + threads) / threads;
-    hipLaunchKernelGGL(psi_table_kernel, dim3((unsigned)blocks), dim3(threads), 0, st, tab, n);
+hipError_t enm_launch_init(const InitArgs& a, hipStream_t st) {
+    const int64_t n = std::max({a.n + 1, (int64_t)ENM_ST_SLOTS, a.n_maxabs, a.n_counters, a.n_hint_bad});
+    hipLaunchKernelGGL(init_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

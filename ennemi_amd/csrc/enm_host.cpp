@@ -277,6 +277,7 @@ struct enm_ctx {
     ~enm_ctx() {
         if (stage_done) (void)hipEventDestroy(stage_done);
         if (stage) (void)hipHostFree(stage);
+        if (prep.out) (void)hipHostFree(prep.out);
     }
     Plan* last = nullptr;
     hipStream_t last_stream = nullptr;
@@ -290,8 +291,10 @@ struct enm_ctx {
         const void* mask = nullptr;
         uint32_t drop_nan = 0;
         bool counted = false;
+        PrepCounted* out = nullptr;       // host memory that the kernels write (n_counted tasks)
+        int n_counted = 0;
         std::vector<char> blob1, blob2;   // host tables of the last uploads
-        DevBuf tables1, tables2, blk_count, blk_off, nan, nout, chunk_val, seq_val, seq_tiles, stats;
+        DevBuf tables1, tables2, blk_count, blk_off, chunk_val, seq_val, seq_tiles, stats;
         // Sort hints: the kept-row map written by the last enm_prep_write
         // with ENM_P_HINTS (pm_total words), and what that call was given.
         int64_t pm_total = 0;
@@ -1449,20 +1452,19 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
     };
     if ((rc = mark(0))) return rc;
     unsigned long long* stats = W.stats.as<unsigned long long>();
-    if ((rc = chk(enm_launch_fill_u64(stats, ENM_ST_SLOTS, 0ull, st), "fill"))) return rc;
-    if ((rc = chk(enm_launch_fill_u64(W.maxabs.as<unsigned long long>(), P.n_inst, 0ull, st), "fill"))) return rc;
-    if ((rc = chk(enm_launch_fill_i32(W.counters.as<int>(),
-                                      (int64_t)P.groups.size() * (ENM_NQ + ENM_NDEF) * ENM_CSTRIDE, 0, st),
-                  "fill")))
-        return rc;
-    if ((rc = chk(enm_launch_psi_table(W.res64.as<double>() + P.psi_tab, P.psi_n, st), "fill"))) return rc;
-    nl += 4;
     const bool hints = P.hinted && P.sample_sort && hint != nullptr;
-    if (hints) {
-        if ((rc = chk(enm_launch_fill_i32(W.hint_bad.as<int>(), (int64_t)P.segs.size() + 1, 0, st), "fill")))
-            return rc;
-        ++nl;
-    }
+    InitArgs ia;
+    ia.stats = stats;
+    ia.maxabs = W.maxabs.as<unsigned long long>();
+    ia.n_maxabs = P.n_inst;
+    ia.counters = W.counters.as<int>();
+    ia.n_counters = (int64_t)P.groups.size() * (ENM_NQ + ENM_NDEF) * ENM_CSTRIDE;
+    ia.hint_bad = W.hint_bad.as<int>();
+    ia.n_hint_bad = hints ? (int64_t)P.segs.size() + 1 : 0;
+    ia.tab = W.res64.as<double>() + P.psi_tab;
+    ia.n = P.psi_n;
+    if ((rc = chk(enm_launch_init(ia, st), "fill"))) return rc;
+    ++nl;
     if ((rc = mark(1))) return rc;
     int fb = 0;
     if (P.sample_sort) {
@@ -2010,23 +2012,32 @@ int enm_prep_count(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks, co
     S.pm_total = pm;
     S.blob1.clear();
     const size_t off_t = append(S.blob1, S.tasks);
+    const size_t off_nan = append(S.blob1, std::vector<unsigned>(n_tasks, 0u));
     if (S.tables1.ensure(S.blob1.size()) != hipSuccess || S.blk_count.ensure(nb * 4 + 4) != hipSuccess ||
-        S.blk_off.ensure(nb * 8 + 8) != hipSuccess || S.nan.ensure((size_t)n_tasks * 4) != hipSuccess ||
-        S.nout.ensure((size_t)n_tasks * 8) != hipSuccess) {
+        S.blk_off.ensure(nb * 8 + 8) != hipSuccess) {
         (void)hipGetLastError();
         return fail(ctx, ENM_E_NOMEM, "hipMalloc failed for the preparation workspace");
+    }
+    if (S.n_counted < n_tasks) {
+        if (S.out) (void)hipHostFree(S.out);
+        S.out = nullptr;
+        S.n_counted = 0;
+        void* p = nullptr;
+        e = hipHostMalloc(&p, (size_t)n_tasks * sizeof(PrepCounted), hipHostMallocDefault);
+        if (e != hipSuccess) return hip_fail(ctx, e, "hipHostMalloc");
+        S.out = static_cast<PrepCounted*>(p);
+        S.n_counted = n_tasks;
     }
     e = hipMemcpyAsync(S.tables1.p, S.blob1.data(), S.blob1.size(), hipMemcpyHostToDevice, st);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipMemcpyAsync(prep tables)");
     const PrepTaskDev* dt = reinterpret_cast<const PrepTaskDev*>(S.tables1.as<char>() + off_t);
     e = enm_launch_prep_count(dt, stride, n_tasks, d_raw, d_mask, (flags & ENM_P_DROP_NAN) ? 1 : 0,
-                              S.blk_count.as<int>(), S.blk_off.as<int64_t>(), S.nan.as<unsigned>(),
-                              S.nout.as<int64_t>(), st);
+                              S.blk_count.as<int>(), S.blk_off.as<int64_t>(),
+                              reinterpret_cast<unsigned*>(S.tables1.as<char>() + off_nan), S.out, st);
     if (e != hipSuccess) return hip_fail(ctx, e, "prep count");
-    e = hipMemcpyAsync(h_n, S.nout.p, (size_t)n_tasks * 8, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(h_nan, S.nan.p, (size_t)n_tasks * 4, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(ctx, e, "prep count read-back");
+    for (int t = 0; t < n_tasks; ++t) { h_n[t] = S.out[t].n; h_nan[t] = S.out[t].nan; }
     S.n.assign(h_n, h_n + n_tasks);
     S.raw = d_raw;
     S.mask = d_mask;

@@ -350,6 +350,13 @@ struct PrepSumDev {
     int32_t n_chunks;   // blocks of ENM_PREP_SEQ_BLOCK rows (row by row; none: short)
 };
 
+// What the counting of a task's rows found.
+struct PrepCounted {
+    int64_t n;       // kept rows
+    uint32_t nan;    // a NaN is among them
+    uint32_t pad;
+};
+
 // A column summed row by row: 64 rows of it (see enm_prep.hip).
 #define ENM_PREP_SEQ_BLOCK 4096
 struct PrepSeqTile {

@@ -97,7 +97,15 @@ hipError_t enm_launch_count(const Item* items, const int* qoff, int n_items, uns
                             unsigned long long* stats, int dclass, bool f32, bool brute,
                             int grid, unsigned* deferred, unsigned* n_deferred, unsigned seg_cap,
                             int ticket, hipStream_t st);
-hipError_t enm_launch_psi_table(double* tab, int64_t n, hipStream_t st);
+// What a batch needs before its first stage: cleared counters, and the digamma
+// table tab[0 .. n].
+struct InitArgs {
+    unsigned long long *stats, *maxabs;
+    int *counters, *hint_bad;
+    double* tab;
+    int64_t n_maxabs, n_counters, n_hint_bad, n;
+};
+hipError_t enm_launch_init(const InitArgs& a, hipStream_t st);
 // items: the items of a 1-D count group.
 hipError_t enm_launch_psi_tiles(const Item* items, int n_items, const CountDev* descs, const double* psi_tab,
                                 const int* counts, double* res64, int* res32, hipStream_t st);
@@ -112,7 +120,7 @@ hipError_t enm_launch_export_cnt(const int* src, const int* perm, int64_t n, int
 hipError_t enm_launch_prep_columns(const double* rows, int64_t n, int m, double* cols, hipStream_t st);
 hipError_t enm_launch_prep_count(const PrepTaskDev* tasks, int64_t stride, int n_tasks,
                                  const double* raw, const unsigned char* mask, int drop_nan, int* blk_count,
-                                 int64_t* blk_off, unsigned* nan_flag, int64_t* n_out, hipStream_t st);
+                                 int64_t* blk_off, unsigned* nan_flag, PrepCounted* out, hipStream_t st);
 hipError_t enm_launch_prep_write(PrepTaskDev* tasks, int64_t stride, int n_tasks,
                                  const double* raw, const unsigned char* mask, int drop_nan, int rescale,
                                  const int64_t* blk_off, const PrepSumDev* sums, int n_sums,

@@ -136,10 +136,12 @@ void prep_count_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, co
 }
 
 // Per task: block offsets (exclusive scan of the block counts, in place in
-// blk_off) and the kept rows n.  One wave per task.
+// blk_off), and to host memory the kept rows n and whether a NaN is among them
+// (two copies less per call).  One wave per task.
 __global__ __launch_bounds__(ENM_WAVE)
 void prep_scan_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, int n_tasks,
-                      const int* __restrict__ blk_count, int64_t* __restrict__ blk_off, int64_t* __restrict__ n_out) {
+                      const int* __restrict__ blk_count, int64_t* __restrict__ blk_off,
+                      const unsigned* __restrict__ nan_flag, PrepCounted* __restrict__ out) {
     const int ti = blockIdx.x;
     if (ti >= n_tasks) return;
     const int64_t b0 = ti * stride, nb = tasks[ti].nblk;
@@ -155,7 +157,7 @@ void prep_scan_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, int
         if (base + lane < nb) blk_off[b0 + base + lane] = carry + inc - v;
         carry += __shfl(inc, ENM_WAVE - 1, ENM_WAVE);
     }
-    if (lane == 0) n_out[ti] = carry;
+    if (lane == 0) out[ti] = PrepCounted{carry, nan_flag[ti], 0};
 }
 
 // Phase 2a: the kept rows of every block, in row order, to the task's
@@ -827,16 +829,14 @@ hipError_t enm_launch_prep_columns(const double* rows, int64_t n, int m, double*
 
 hipError_t enm_launch_prep_count(const PrepTaskDev* tasks, int64_t stride, int n_tasks,
                                  const double* raw, const unsigned char* mask, int drop_nan, int* blk_count,
-                                 int64_t* blk_off, unsigned* nan_flag, int64_t* n_out, hipStream_t st) {
+                                 int64_t* blk_off, unsigned* nan_flag, PrepCounted* out, hipStream_t st) {
     const int64_t n_blocks = stride * n_tasks;
     if (n_tasks <= 0) return hipSuccess;
-    hipError_t e = enm_launch_fill_i32(reinterpret_cast<int*>(nan_flag), n_tasks, 0, st);
-    if (e != hipSuccess) return e;
     if (n_blocks > 0)
         hipLaunchKernelGGL(prep_count_kernel, dim3((unsigned)n_blocks), dim3(PB_THREADS), 0, st, tasks, stride,
                            raw, mask, drop_nan, blk_count, nan_flag);
     hipLaunchKernelGGL(prep_scan_kernel, dim3((unsigned)n_tasks), dim3(ENM_WAVE), 0, st, tasks, stride, n_tasks,
-                       blk_count, blk_off, n_out);
+                       blk_count, blk_off, nan_flag, out);
     return hipGetLastError();
 }
 
