@@ -340,6 +340,31 @@ int hip_fail(enm_ctx* ctx, hipError_t e, const char* what) {
 // Planning
 // ---------------------------------------------------------------------------
 
+// Cells of a scope up to which they are runs of the order by one column; beyond,
+// that order is cut into slabs that are sorted by a second column, 60 to 100 us of
+// launches and merges.  A cell's 64 leaves make up for its shape while the runs
+// are wider than the leaves would be: in two columns up to 64 of them (100,000
+// points, build and kNN 191 -> 112 us; 10 times 100,000 633 -> 533), in three 16
+// (50,000 points, three counts with it, 361 -> 278; at 25 cells the queries lose a
+// tenth), in four or five 8 (20,000 points 349 -> 280; at 13 cells they lose that).
+int tree_base_cells(int columns) { return columns <= 2 ? 64 : columns == 3 ? 16 : 8; }
+
+// Points of all two-column instances of a call up to which their neighbours are
+// found on box trees, not on strips.  A strip is one workgroup's, so few points
+// leave the chip idle, and longer lists cost strips more (their lists shift by
+// every insertion); trees cost more per point.  Strips against trees, us of sort,
+// build, kNN and counts: 1,000 points k = 3 177 / 87, k = 20 554 / 90; 100 x 1,000
+// k = 3 226 / 136, 1,000 x 1,000 418 / 547, k = 7 611 / 604, k = 12 1174 / 691;
+// 100,000 points k = 3 329 / 305, k = 20 565 / 344; 10 x 100,000 k = 7 598 / 860,
+// k = 20 934 / 1100; 1,000 x 5,000 k = 12 3388 / 3338, k = 20 5758 / 3938.
+int64_t tree_points(int k1, int64_t n) {
+    const bool one_cell = n <= ENM_CELL;
+    if (k1 <= 4) return one_cell ? 250000 : 150000;
+    if (k1 <= 8) return one_cell ? 600000 : 400000;
+    if (n <= 2 * ENM_CELL) return INT64_MAX;
+    return k1 <= 16 ? 500000 : 700000;
+}
+
 struct Planner {
     Plan& P;
     const enm_instance* inst;
@@ -504,7 +529,7 @@ struct Planner {
     // phase `ph`; returns the first one.  Scopes of one cell are cut from the
     // point order; longer ones from slabs (runs of the order by column 0, each
     // sorted by column 1: about as many slabs as cells in a slab), or, up to
-    // ENM_TREE_BASE_CELLS cells, from the order by column 0 itself.
+    // tree_base_cells cells, from the order by column 0 itself.
     int add_trees(int ii, const std::vector<int64_t>& cols, bool segmented, int ph) {
         const enm_instance& I = inst[ii];
         const int D = (int)cols.size();
@@ -518,7 +543,7 @@ struct Planner {
         }
         int64_t slab = -1;
         const int most = (int)((longest + ENM_CELL - 1) / ENM_CELL);   // cells of the longest scope
-        const bool two = most > ENM_TREE_BASE_CELLS;
+        const bool two = most > tree_base_cells(D);
         int per_slab = 1;   // cells per slab
         int sorted = -1;   // the column that the slab order has sorted within a cell
         if (most == 1) {
@@ -683,23 +708,27 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
     std::vector<enm_tuning> tunes(n_inst);
     std::set<int> cols_read;   // orders whose column-major columns a kernel reads
     // How the kNN of an instance of `cols` joint columns runs: strips staged
-    // in LDS (two columns, register lists, strips that three LDS slots hold:
-    // 20 x 100,000 points, k = 3 in 0.29 ms where trees take 0.91, k = 31 in
-    // 1.24 against 1.90), box trees (other spaces of two or more columns),
-    // or the plain key order (brute force, strips tuned off); one column by
-    // windows of its sorted keys.
-    auto route = [&](int cols, int k, const enm_tuning& T) {
+    // in LDS (two columns, register lists, strips that three LDS slots hold,
+    // many points), box trees (other spaces of two or more columns), or the
+    // plain key order (brute force, strips tuned off); one column by windows
+    // of its sorted keys.
+    int64_t points2 = 0;   // of the two-column instances that run together
+    for (int ii = 0; ii < n_inst; ++ii)
+        if (inst[ii].dx + inst[ii].dy + inst[ii].dz == 2) points2 += inst[ii].n;
+    auto route = [&](int cols, int k, int64_t n, const enm_tuning& T) {
         if (P.brute) return ENM_WALK_NONE;
         if (cols < 2) return ENM_WALK_LINE;
         if (T.strip_points <= 0 || (P.plain && (cols > 2 || k + 1 > 32))) return ENM_WALK_NONE;
-        if (cols == 2 && k + 1 <= 32 && T.strip_points <= ENM_STRIP_LDS_MAX) return ENM_WALK_STRIP;
+        if (cols == 2 && k + 1 <= 32 && T.strip_points <= ENM_STRIP_LDS_MAX &&
+            (P.plain || (P.per_instance ? n : points2) > tree_points(k + 1, n)))
+            return ENM_WALK_STRIP;
         return ENM_WALK_TREE;
     };
     int max_strip = 0;
     for (int ii = 0; ii < n_inst; ++ii) {
         const int cols = std::max(0, inst[ii].dx) + std::max(0, inst[ii].dy) + std::max(0, inst[ii].dz);
         tunes[ii] = tuning_for(ctx, cols, inst[ii].k, inst[ii].n);
-        if (route(cols, inst[ii].k, tunes[ii]) == ENM_WALK_STRIP)
+        if (route(cols, inst[ii].k, inst[ii].n, tunes[ii]) == ENM_WALK_STRIP)
             max_strip = std::max(max_strip, (int)tunes[ii].strip_points);
     }
     P.second.strip_tile = max_strip <= 512 ? 512 : max_strip <= 1024 ? 1024 : ENM_SORT_TILE;
@@ -772,7 +801,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
         }
         const enm_tuning& T = tunes[ii];
         const int S = T.strip_points;
-        const int walk = route(ncols, I.k, T);
+        const int walk = route(ncols, I.k, I.n, T);
         // Multi-column count spaces use trees unless strips are tuned off.
         const bool trees = !P.brute && !P.plain && S > 0;
         pl.inst_orders.clear();
@@ -829,7 +858,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
                     sp.ocols = {0};
                 }
         };
-        if (I.n <= ENM_CELL * ENM_TREE_BASE_CELLS) one_column();
+        if (I.n <= ENM_CELL * tree_base_cells(ncols)) one_column();
         if (walk == ENM_WALK_TREE) ktree_first = pl.add_trees(ii, acols, segA, 0);
         int ph = 0;
         for (SpaceSpec& sp : spaces) {
@@ -1506,7 +1535,8 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
             return rc;
     } else if (!P.segs.empty() &&
                (rc = chk(enm_launch_sort(tab<SortSeg>(P, P.off_segs), (int)P.segs.size(), P.ntiles, P.maxlen,
-                                         ENM_SORT_TILE, arena, nullptr,
+                                         P.maxlen <= 512 ? 512 : P.maxlen <= 1024 ? 1024 : ENM_SORT_TILE, arena,
+                                         nullptr,
                                          W.sk0.as<double>(), W.si0.as<int>(), W.sk1.as<double>(), W.si1.as<int>(),
                                          W.split.as<int>(), &fb, &nl, st), "sort"))) {
         return rc;

@@ -60,7 +60,6 @@
 #define ENM_WALK_LINE 3        // one column: windows of the sorted keys
 #define ENM_LINE_THREADS 256
 #define ENM_LINE_ITEM 2048     // positions per one-column item
-#define ENM_TREE_BASE_CELLS 4  // scopes of more cells are cut by two columns, not one
 
 // One contiguous key range to sort: keys at arena[src + t], t in [0, len),
 // carried with their instance point index p0 + t.

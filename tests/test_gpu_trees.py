@@ -160,3 +160,29 @@ def test_groups_of_cells():
         r = eps[0][i] - 1e-12
         for s, cols in enumerate(([0, 2, 3], [1, 2, 3], [2, 3])):
             assert cnts[0][s][i] == np.count_nonzero(d[:, cols].max(axis=1) <= r)
+
+
+@pytest.mark.parametrize("d, n", [(2, 64 * 4096), (2, 64 * 4096 + 1), (3, 16 * 4096), (3, 16 * 4096 + 1), (4, 8 * 4096),
+                                  (4, 8 * 4096 + 1), (5, 8 * 4096 + 1)])
+def test_cells_by_one_column_or_two(d, n):
+    nat = _nat()
+    a = _data(n, d, seed=n, form="ties" if n % 2 else "plain")
+    if d == 2:
+        _both(lambda b: b.add(nat.KIND_KSG, 20, _cols(a[:, :1]), _cols(a[:, 1:])))
+    else:
+        _both(lambda b: b.add(nat.KIND_CMI, 3, _cols(a[:, :1]), _cols(a[:, 1:2]), _cols(a[:, 2:])))
+
+
+@pytest.mark.parametrize("k", [3, 4, 7, 8, 15, 16, 31, 32])
+@pytest.mark.parametrize("n, m", [(4096, 1), (4097, 1), (8192, 2), (8193, 1), (1000, 40), (1000, 700)])
+def test_two_columns_on_trees_or_strips(k, n, m):
+    # Both sides of every limit of the two routes, on their own and together.
+    nat = _nat()
+    a = [_data(n, 2, seed=100 * k + i, form=f) for i, f in enumerate(("plain", "ties", "tails", "equal"))]
+
+    def build(b):
+        for i in range(m):
+            x = a[i % 4]
+            b.add(nat.KIND_KSG, k, _cols(x[:, :1]), _cols(x[:, 1:]))
+        b.add(nat.KIND_KL, k, _cols(a[0]))
+    _both(build)
