@@ -580,7 +580,7 @@ class DevicePrep:
             if self.arena is None or self.arena.numel() != total:
                 self.arena = torch.empty(total, dtype=torch.float64, device=self.dev)
                 self.hint = torch.empty(total, dtype=torch.int32, device=self.dev) if self.hints else None
-                self.d_const = torch.zeros(self.n_tasks, dtype=torch.int32, device=self.dev)
+                self.d_const = torch.empty(self.n_tasks, dtype=torch.int32, device=self.dev)
             if self.preprocess and noise_len > self.noise_len:
                 self.d_noise = _device_noise(noise_len, self.dev)
                 self.noise_len = noise_len

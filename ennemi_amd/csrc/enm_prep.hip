@@ -102,7 +102,8 @@ void prep_columns_kernel(const double* __restrict__ rows, int64_t n, int m, doub
 __global__ __launch_bounds__(PB_THREADS)
 void prep_count_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, const double* __restrict__ raw,
                        const unsigned char* __restrict__ mask, int drop_nan, int* __restrict__ blk_count,
-                       unsigned* __restrict__ nan_flag) {
+                       unsigned* __restrict__ nan_flag, int64_t* __restrict__ blk_off,
+                       PrepCounted* __restrict__ out) {
     __shared__ int s_cnt[PB_THREADS / ENM_WAVE];
     __shared__ int s_nan;
     const int64_t b = xcd_block(blockIdx.x, gridDim.x);   // a task's blocks on one XCD
@@ -130,8 +131,14 @@ void prep_count_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, co
     if (threadIdx.x == 0) {
         int tot = 0;
         for (int w = 0; w < PB_THREADS / ENM_WAVE; ++w) tot += s_cnt[w];
-        blk_count[b] = tot;
-        if (s_nan && !drop_nan) atomicOr(nan_flag + ti, 1u);
+        const unsigned nan = s_nan && !drop_nan ? 1u : 0u;
+        if (stride == 1) {   // the task's only block: nothing to scan
+            blk_off[b] = 0;
+            out[ti] = PrepCounted{tot, nan, 0};
+        } else {
+            blk_count[b] = tot;
+            if (nan) atomicOr(nan_flag + ti, 1u);
+        }
     }
 }
 
@@ -166,17 +173,11 @@ void prep_scan_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, int
 // them, for the sort hints.  Every
 // row's state and x, y values are read first; one barrier then gives each
 // wave the kept rows of the waves before it, round by round.
-__global__ __launch_bounds__(PB_THREADS)
-void prep_compact_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride,
-                         const double* __restrict__ raw, const unsigned char* __restrict__ mask, int drop_nan,
-                         const int64_t* __restrict__ blk_off, double* __restrict__ arena,
-                         KeptWord* __restrict__ kept) {
+__device__ __forceinline__ void compact_rows(const PrepTaskDev& t, int64_t r0, int64_t pos, const double* __restrict__ raw,
+                                             const unsigned char* __restrict__ mask, int drop_nan,
+                                             double* __restrict__ arena, KeptWord* __restrict__ kept) {
     constexpr int NW = PB_THREADS / ENM_WAVE;
     __shared__ int s_wcnt[PB_ROUNDS][NW];
-    const int64_t b = xcd_block(blockIdx.x, gridDim.x);   // a task's blocks on one XCD
-    const int ti = (int)(b / stride);
-    const PrepTaskDev& t = tasks[ti];   // read in place: a copy indexed by c would sit in scratch
-    const int64_t r0 = (b - ti * stride) * PB_ROWS;
     const int lane = threadIdx.x & (ENM_WAVE - 1), wv = threadIdx.x / ENM_WAVE;
     bool keep[PB_ROUNDS];
     double xv[PB_ROUNDS], yv[PB_ROUNDS];
@@ -197,7 +198,6 @@ void prep_compact_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride,
         if (lane == 0) s_wcnt[j][wv] = __popcll(m);
     }
     __syncthreads();
-    int64_t pos = blk_off[b];
     double* out = arena + t.arena_off;
 #pragma unroll
     for (int j = 0; j < PB_ROUNDS; ++j) {
@@ -226,6 +226,17 @@ void prep_compact_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride,
         }
         pos += total;
     }
+}
+
+__global__ __launch_bounds__(PB_THREADS)
+void prep_compact_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride,
+                         const double* __restrict__ raw, const unsigned char* __restrict__ mask, int drop_nan,
+                         const int64_t* __restrict__ blk_off, double* __restrict__ arena,
+                         KeptWord* __restrict__ kept) {
+    const int64_t b = xcd_block(blockIdx.x, gridDim.x);   // a task's blocks on one XCD
+    const int ti = (int)(b / stride);
+    // (The task is read in place: a copy indexed by c would sit in scratch.)
+    compact_rows(tasks[ti], (b - ti * stride) * PB_ROWS, blk_off[b], raw, mask, drop_nan, arena, kept);
 }
 
 // One term of a sum: the value, or its squared deviation from `mean`.
@@ -281,62 +292,57 @@ __device__ __forceinline__ double pw_full_chunk(const Term& f) {
     return ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
 }
 
-// Phase 2b: one wave per (array, chunk): the pairwise sum of a chunk of
-// values (pass 0) or of squared deviations from the array's mean (pass 1).
-// A full chunk takes pw_full_chunk; otherwise the wave builds the
-// recursion's tree in LDS level by level (slot lengths; -1 for no node),
-// sums its leaves, eight lanes to a leaf, and adds every node's two halves
+// LDS of one wave's sum.
+struct PwTree {
+    int lo[PW_HEAP], len[PW_HEAP];
+    double val[PW_HEAP];
+    short leaf[PW_HEAP];
+    int nl;
+};
+
+// Orders a wave's own LDS accesses.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The pairwise sum of m <= PW_CHUNK values (pass 0) or squared deviations (pass
+// 1) by one wave, in every lane.  A full chunk takes pw_full_chunk; otherwise the
+// wave builds the recursion's tree in LDS level by level (slot lengths; -1 for no
+// node), sums its leaves, eight lanes to a leaf, and adds every node's two halves
 // bottom-up, left + right, as NumPy does.
-__global__ __launch_bounds__(ENM_WAVE)
-void prep_chunk_kernel(const PrepSumDev* __restrict__ sums, const int* __restrict__ chunk_sum_of,
-                       const int* __restrict__ chunk_index, const int* __restrict__ list, int n_list,
-                       const double* __restrict__ arena, const double* __restrict__ stats, int pass,
-                       double* __restrict__ chunk_val) {
-    __shared__ int s_lo[PW_HEAP], s_len[PW_HEAP];
-    __shared__ double s_val[PW_HEAP];
-    __shared__ short s_leaf[PW_HEAP];
-    __shared__ int s_nl;
-    if ((int)blockIdx.x >= n_list) return;
-    const int c = list[blockIdx.x];
-    const PrepSumDev& sd = sums[chunk_sum_of[c]];
-    const int64_t first = (int64_t)chunk_index[c] * PW_CHUNK;
-    const int m = (int)min((int64_t)PW_CHUNK, sd.n - first);
-    const Term f{arena + sd.src + first, pass ? stats[sd.stat] : 0.0, pass != 0};
-    if (m == PW_CHUNK) {
-        const double sum = pw_full_chunk(f);
-        if (threadIdx.x == 0) chunk_val[c] = sum;
-        return;
-    }
-    const int lane = (int)threadIdx.x;
+__device__ double pw_chunk(const Term& f, int m, PwTree& L) {
+    if (m == PW_CHUNK) return pw_full_chunk(f);
+    const int lane = (int)threadIdx.x & (ENM_WAVE - 1);
     // The tree, top-down: slot 1 is the whole chunk; a slot's halves exist
     // when it has more than PW_LEAF values.
-    for (int i = lane; i < PW_HEAP; i += ENM_WAVE) s_len[i] = -1;
+    for (int i = lane; i < PW_HEAP; i += ENM_WAVE) L.len[i] = -1;
     if (lane == 0) {
-        s_lo[1] = 0;
-        s_len[1] = m;
-        s_nl = 0;
+        L.lo[1] = 0;
+        L.len[1] = m;
+        L.nl = 0;
     }
-    __syncthreads();
+    wave_sync();
     for (int d = 0; d < PW_DEPTH; ++d) {
         for (int i = (1 << d) + lane; i < (2 << d); i += ENM_WAVE) {
-            const int len = s_len[i];
+            const int len = L.len[i];
             if (len > PW_LEAF) {
                 int n2 = len / 2;
                 n2 -= n2 % 8;
-                s_lo[2 * i] = s_lo[i];
-                s_len[2 * i] = n2;
-                s_lo[2 * i + 1] = s_lo[i] + n2;
-                s_len[2 * i + 1] = len - n2;
+                L.lo[2 * i] = L.lo[i];
+                L.len[2 * i] = n2;
+                L.lo[2 * i + 1] = L.lo[i] + n2;
+                L.len[2 * i + 1] = len - n2;
             }
         }
-        __syncthreads();
+        wave_sync();
     }
     // The leaves, listed in any order (each is summed on its own).
     for (int i = 1 + lane; i < PW_HEAP; i += ENM_WAVE) {
-        const int len = s_len[i];
-        if (len >= 0 && len <= PW_LEAF) s_leaf[atomicAdd(&s_nl, 1)] = (short)i;
+        const int len = L.len[i];
+        if (len >= 0 && len <= PW_LEAF) L.leaf[atomicAdd(&L.nl, 1)] = (short)i;
     }
-    __syncthreads();
+    wave_sync();
     // A leaf is NumPy's pairwise_sum leaf: fewer than 8 values summed from
     // 0.0; up to 128 by 8 interleaved accumulators combined as
     // ((r0+r1)+(r2+r3))+((r4+r5)+(r6+r7)), the remainder added after.
@@ -345,11 +351,11 @@ void prep_chunk_kernel(const PrepSumDev* __restrict__ sums, const int* __restric
     // order), butterfly shuffles within the group combine the accumulators,
     // and the group's first lane adds the remainder.
     const int j = lane & 7;
-    const int nl = s_nl;
+    const int nl = L.nl;
     for (int l0 = 0; l0 < nl; l0 += ENM_WAVE / 8) {
         const int l = l0 + (lane >> 3);
-        const int slot = l < nl ? s_leaf[l] : 0;
-        const int lo = l < nl ? s_lo[slot] : 0, len = l < nl ? s_len[slot] : 0;
+        const int slot = l < nl ? L.leaf[l] : 0;
+        const int lo = l < nl ? L.lo[slot] : 0, len = l < nl ? L.len[slot] : 0;
         const int full = len >= 8 ? len - len % 8 : 0;
         double v[PW_LEAF / 8];
 #pragma unroll
@@ -370,17 +376,34 @@ void prep_chunk_kernel(const PrepSumDev* __restrict__ sums, const int* __restric
                 res = acc;
                 for (int t = full; t < len; ++t) res += f(lo + t);
             }
-            s_val[slot] = res;
+            L.val[slot] = res;
         }
     }
-    __syncthreads();
+    wave_sync();
     // Bottom-up: every split node is its left half plus its right half.
     for (int d = PW_DEPTH - 1; d >= 0; --d) {
         for (int i = (1 << d) + lane; i < (2 << d); i += ENM_WAVE)
-            if (s_len[i] > PW_LEAF) s_val[i] = s_val[2 * i] + s_val[2 * i + 1];
-        __syncthreads();
+            if (L.len[i] > PW_LEAF) L.val[i] = L.val[2 * i] + L.val[2 * i + 1];
+        wave_sync();
     }
-    if (lane == 0) chunk_val[c] = s_val[1];
+    return L.val[1];
+}
+
+// Phase 2b: the last chunk of every array, one wave each.
+__global__ __launch_bounds__(ENM_WAVE)
+void prep_chunk_kernel(const PrepSumDev* __restrict__ sums, const int* __restrict__ chunk_sum_of,
+                       const int* __restrict__ chunk_index, const int* __restrict__ list, int n_list,
+                       const double* __restrict__ arena, const double* __restrict__ stats, int pass,
+                       double* __restrict__ chunk_val) {
+    __shared__ PwTree s_tree;
+    if ((int)blockIdx.x >= n_list) return;
+    const int c = list[blockIdx.x];
+    const PrepSumDev& sd = sums[chunk_sum_of[c]];
+    const int64_t first = (int64_t)chunk_index[c] * PW_CHUNK;
+    const int m = (int)min((int64_t)PW_CHUNK, sd.n - first);
+    const Term f{arena + sd.src + first, pass ? stats[sd.stat] : 0.0, pass != 0};
+    const double sum = pw_chunk(f, m, s_tree);
+    if (threadIdx.x == 0) chunk_val[c] = sum;
 }
 
 // Full chunks only, one per wave, four waves per block (no barriers: each
@@ -718,6 +741,29 @@ __device__ double seq_sum(const PrepSumDev& sd, const double* v, double mean, in
     return s;
 }
 
+// The row-by-row sum of one array as one chain; one wave.  64 rows at a time,
+// the next 256 on their way.
+__device__ double seq_chain(const double* v, int64_t n, double mean, int pass) {
+    constexpr int AHEAD = 4;
+    const int lane = threadIdx.x & (ENM_WAVE - 1);
+    double acc = -0.0, rows[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+        const int64_t i = j * ENM_WAVE + lane;
+        rows[j] = i < n ? v[i] : 0.0;
+    }
+    for (int64_t base = 0; base < n; base += AHEAD * ENM_WAVE) {
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) {
+            const int64_t i = base + j * ENM_WAVE + lane, k = i + AHEAD * ENM_WAVE;
+            const double term = i < n ? seq_term(rows[j], mean, pass) : -0.0;
+            rows[j] = k < n ? v[k] : 0.0;
+            if (base + j * ENM_WAVE < n) acc = seq_add_rows(acc, term);
+        }
+    }
+    return acc;
+}
+
 // Phase 2c: per array, the chunk sums added in order to -0.0 (pairwise
 // arrays), or the whole column accumulated row by row (columns of a
 // multi-column condition; from its tiles if it has any); then mean = sum / n
@@ -740,23 +786,7 @@ void prep_finish_kernel(const PrepSumDev* __restrict__ sums, int n_sums, const d
         if (sd.n_chunks > 0) {
             acc = seq_sum(sd, v, mean, pass, tiles, s_ahead);
         } else {
-            // 64 rows at a time, the next 256 on their way.
-            constexpr int AHEAD = 4;
-            double rows[AHEAD];
-#pragma unroll
-            for (int j = 0; j < AHEAD; ++j) {
-                const int64_t i = j * ENM_WAVE + lane;
-                rows[j] = i < sd.n ? v[i] : 0.0;
-            }
-            for (int64_t base = 0; base < sd.n; base += AHEAD * ENM_WAVE) {
-#pragma unroll
-                for (int j = 0; j < AHEAD; ++j) {
-                    const int64_t i = base + j * ENM_WAVE + lane, k = i + AHEAD * ENM_WAVE;
-                    const double term = i < sd.n ? seq_term(rows[j], mean, pass) : -0.0;
-                    rows[j] = k < sd.n ? v[k] : 0.0;
-                    if (base + j * ENM_WAVE < sd.n) acc = seq_add_rows(acc, term);
-                }
-            }
+            acc = seq_chain(v, sd.n, mean, pass);
         }
     } else {
         for (int c = 0; c < sd.n_chunks; ++c) acc += chunk_val[sd.chunk0 + c];
@@ -767,21 +797,17 @@ void prep_finish_kernel(const PrepSumDev* __restrict__ sums, int n_sums, const d
     else stats[sd.stat + 1] = sqrt(q);
 }
 
-// Phase 2d: which variables are rescaled, where their noise starts, and
-// their flag bits (bit 0 x, bit 1 y, bit 2 z constant).  Variables of
-// raw_vars (bit 0 x, bit 1 y) are class labels: never rescaled, no noise drawn,
-// not called constant.  One thread per task.
-__global__ void prep_noise_kernel(PrepTaskDev* __restrict__ tasks, int n_tasks, const double* __restrict__ stats,
-                                  unsigned raw_vars, unsigned* __restrict__ const_flag) {
-    const int ti = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ti >= n_tasks) return;
-    PrepTaskDev& t = tasks[ti];
+// Which variables of a task are rescaled, where their noise starts, and its
+// flag bits (bit 0 x, bit 1 y, bit 2 z constant), which are returned.
+// Variables of raw_vars (bit 0 x, bit 1 y) are class labels: never rescaled, no
+// noise drawn, not called constant.
+__device__ __forceinline__ unsigned place_noise(PrepTaskDev& t, const double* stats, unsigned raw_vars) {
     unsigned fl = 0;
     if (!(raw_vars & 1u) && fabs(stats[t.stat + 1]) < 1e-20) fl |= 1u;
     if (!(raw_vars & 2u) && fabs(stats[t.stat + 3]) < 1e-20) fl |= 2u;
     for (int c = 0; c < t.dz; ++c)
         if (fabs(stats[t.stat + 4 + 2 * c + 1]) < 1e-20) fl |= 4u;
-    const_flag[ti] = fl;
+    const unsigned constant = fl;
     fl |= raw_vars;
     int64_t drawn = 0;
     t.noise_x = drawn;
@@ -790,17 +816,12 @@ __global__ void prep_noise_kernel(PrepTaskDev* __restrict__ tasks, int n_tasks, 
     if (!(fl & 2u)) drawn += t.n;
     t.noise_z = drawn;
     t.flags = fl;
+    return constant;
 }
 
-// Phase 2e: (v - mean) / std + noise for every rescaled value, in place.
-__global__ __launch_bounds__(PB_THREADS)
-void prep_scale_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, const double* __restrict__ stats,
-                       const double* __restrict__ noise, double* __restrict__ arena) {
-    const int64_t b = xcd_block(blockIdx.x, gridDim.x);   // a task's blocks on one XCD
-    const int ti = (int)(b / stride);
-    const PrepTaskDev& t = tasks[ti];   // read in place: a copy indexed by c would sit in scratch
-    const int64_t i = (b - ti * stride) * PB_THREADS + threadIdx.x;
-    if (i >= t.n) return;
+// (v - mean) / std + noise for row i of every rescaled variable, in place.
+__device__ __forceinline__ void scale_row(const PrepTaskDev& t, int64_t i, const double* stats,
+                                          const double* __restrict__ noise, double* arena) {
     double* col = arena + t.arena_off;
     if (!(t.flags & 1u)) {
         const double v = (col[i] - stats[t.stat]) / stats[t.stat + 1];
@@ -819,6 +840,62 @@ void prep_scale_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, co
     }
 }
 
+// Phase 2d.  One thread per task.
+__global__ void prep_noise_kernel(PrepTaskDev* __restrict__ tasks, int n_tasks, const double* __restrict__ stats,
+                                  unsigned raw_vars, unsigned* __restrict__ const_flag) {
+    const int ti = blockIdx.x * blockDim.x + threadIdx.x;
+    if (ti >= n_tasks) return;
+    const_flag[ti] = place_noise(tasks[ti], stats, raw_vars);
+}
+
+// Phase 2e.
+__global__ __launch_bounds__(PB_THREADS)
+void prep_scale_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, const double* __restrict__ stats,
+                       const double* __restrict__ noise, double* __restrict__ arena) {
+    const int64_t b = xcd_block(blockIdx.x, gridDim.x);   // a task's blocks on one XCD
+    const int ti = (int)(b / stride);
+    const PrepTaskDev& t = tasks[ti];   // read in place: a copy indexed by c would sit in scratch
+    const int64_t i = (b - ti * stride) * PB_THREADS + threadIdx.x;
+    if (i < t.n) scale_row(t, i, stats, noise, arena);
+}
+
+// Phase 2 of short tasks (at most PREP_SHORT kept rows each), one workgroup per
+// task: every array's mean and deviation by a wave of its own, then the
+// rescaling.  Bound by latency and launches: for a few short tasks the phases
+// take some 5 us each, mostly to be launched.  With `whole` (windows of one block
+// of rows) it does the compaction too.
+__global__ __launch_bounds__(PB_THREADS)
+void prep_short_kernel(PrepTaskDev* tasks, const double* __restrict__ raw, const unsigned char* __restrict__ mask,
+                       int drop_nan, int whole, double* stats, const double* __restrict__ noise, unsigned raw_vars,
+                       unsigned* __restrict__ const_flag, double* arena, KeptWord* __restrict__ kept) {
+    constexpr int NW = PB_THREADS / ENM_WAVE;
+    __shared__ PwTree s_tree[NW];
+    PrepTaskDev& t = tasks[blockIdx.x];
+    const int lane = threadIdx.x & (ENM_WAVE - 1), wave = threadIdx.x / ENM_WAVE;
+    if (whole) {
+        compact_rows(t, 0, 0, raw, mask, drop_nan, arena, kept);
+        __syncthreads();
+    }
+    for (int a = wave; a < 2 + t.dz; a += NW) {
+        if (a < 2 && ((raw_vars >> a) & 1u)) continue;
+        const double* v = arena + t.arena_off + a * t.n;
+        double mean = 0.0;
+        for (int pass = 0; pass < 2; ++pass) {
+            const double sum = a >= 2 && t.dz >= 2 ? seq_chain(v, t.n, mean, pass)
+                                                   : -0.0 + pw_chunk(Term{v, mean, pass != 0}, (int)t.n, s_tree[wave]);
+            const double q = sum / (double)t.n;
+            if (pass == 0) mean = q;
+            if (lane == 0) stats[t.stat + 2 * a + pass] = pass ? sqrt(q) : q;
+            wave_sync();
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) const_flag[blockIdx.x] = place_noise(t, stats, raw_vars);
+    __syncthreads();
+#pragma unroll 4
+    for (int64_t i = threadIdx.x; i < t.n; i += PB_THREADS) scale_row(t, i, stats, noise, arena);
+}
+
 }  // namespace
 
 hipError_t enm_launch_prep_columns(const double* rows, int64_t n, int m, double* cols, hipStream_t st) {
@@ -834,8 +911,9 @@ hipError_t enm_launch_prep_count(const PrepTaskDev* tasks, int64_t stride, int n
     if (n_tasks <= 0) return hipSuccess;
     if (n_blocks > 0)
         hipLaunchKernelGGL(prep_count_kernel, dim3((unsigned)n_blocks), dim3(PB_THREADS), 0, st, tasks, stride,
-                           raw, mask, drop_nan, blk_count, nan_flag);
-    hipLaunchKernelGGL(prep_scan_kernel, dim3((unsigned)n_tasks), dim3(ENM_WAVE), 0, st, tasks, stride, n_tasks,
+                           raw, mask, drop_nan, blk_count, nan_flag, blk_off, out);
+    if (stride != 1)
+        hipLaunchKernelGGL(prep_scan_kernel, dim3((unsigned)n_tasks), dim3(ENM_WAVE), 0, st, tasks, stride, n_tasks,
                        blk_count, blk_off, nan_flag, out);
     return hipGetLastError();
 }
@@ -850,10 +928,15 @@ hipError_t enm_launch_prep_write(PrepTaskDev* tasks, int64_t stride, int n_tasks
                                  KeptWord* kept, hipStream_t st) {
     if (n_tasks <= 0) return hipSuccess;
     const int64_t n_blocks = stride * n_tasks, n_sblocks = sstride * n_tasks;
-    if (n_blocks > 0)
+    const bool short_tasks = rescale && sstride * PB_THREADS <= ENM_PREP_SHORT;
+    const bool whole = short_tasks && stride == 1;
+    if (n_blocks > 0 && !whole)
         hipLaunchKernelGGL(prep_compact_kernel, dim3((unsigned)n_blocks), dim3(PB_THREADS), 0, st, tasks, stride,
                            raw, mask, drop_nan, blk_off, arena, kept);
-    if (!rescale) return hipGetLastError();
+    if (short_tasks)
+        hipLaunchKernelGGL(prep_short_kernel, dim3((unsigned)n_tasks), dim3(PB_THREADS), 0, st, tasks, raw, mask,
+                           drop_nan, whole ? 1 : 0, stats, noise, raw_vars, const_flag, arena, kept);
+    if (!rescale || short_tasks) return hipGetLastError();
     for (int pass = 0; pass < 2; ++pass) {
         if (n_chunks > 0) {
             // Full chunks four to a block; the other (last) chunks one each.
