@@ -1223,9 +1223,13 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
     };
     build(kpend, P.kitems, 0);
     build(cpend, P.citems, 1);
-    // First stage: sample sort when segments need more than one block-sort
-    // tile and none is longer than ENM_SS_MAXLEN.
-    P.sample_sort = P.maxlen > ENM_SORT_TILE && P.maxlen <= ENM_SS_MAXLEN;
+    // First stage: sample sort when segments need more than one block-sort tile,
+    // none is longer than ENM_SS_MAXLEN, and there are many keys.  Few keys are
+    // bound by the launches, many by the work: 20,000 keys in two segments 118 us
+    // by samples, 98 by merges (16,000 in two, one block each, 84); 1.6 million in
+    // sixteen 183 and 195; 5.1 million in 1,024 450 and 660.
+    constexpr int64_t kMergeKeys = 750000;
+    P.sample_sort = P.maxlen > ENM_SORT_TILE && P.maxlen <= ENM_SS_MAXLEN && (P.hinted || P.sort_elems > kMergeKeys);
     if (P.sample_sort) {
         // The orders each segment is laid out into, and its run queue, by
         // instance.
@@ -1535,8 +1539,7 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
             return rc;
     } else if (!P.segs.empty() &&
                (rc = chk(enm_launch_sort(tab<SortSeg>(P, P.off_segs), (int)P.segs.size(), P.ntiles, P.maxlen,
-                                         P.maxlen <= 512 ? 512 : P.maxlen <= 1024 ? 1024 : ENM_SORT_TILE, arena,
-                                         nullptr,
+                                         arena, nullptr,
                                          W.sk0.as<double>(), W.si0.as<int>(), W.sk1.as<double>(), W.si1.as<int>(),
                                          W.split.as<int>(), &fb, &nl, st), "sort"))) {
         return rc;
@@ -1561,7 +1564,7 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
     if (!P.second.segs.empty()) {
         const SortSeg* gsegs = tab<SortSeg>(P, P.second.off_segs);
         if ((rc = chk(enm_launch_sort(gsegs, (int)P.second.segs.size(), P.second.ntiles, P.second.maxlen,
-                                      ENM_SORT_TILE, W.col64.as<double>(), nullptr, W.sk0.as<double>(),
+                                      W.col64.as<double>(), nullptr, W.sk0.as<double>(),
                                       W.si0.as<int>(), W.sk1.as<double>(), W.si1.as<int>(), W.split.as<int>(), &fb,
                                       &nl, st), "sort")))
             return rc;
@@ -2325,7 +2328,7 @@ int enm_prep_hints(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks, co
     e = enm_launch_hint_keys(dser, (int)series.size(), maxlen, d_raw, S.hkeys.as<double>(), st);
     if (e != hipSuccess) return hip_fail(ctx, e, "hint keys");
     int fb = 0, nl = 0;
-    e = enm_launch_sort(dseg, (int)segs.size(), ntiles, maxlen, ENM_SORT_TILE, S.hkeys.as<double>(), nullptr,
+    e = enm_launch_sort(dseg, (int)segs.size(), ntiles, maxlen, S.hkeys.as<double>(), nullptr,
                         S.hk0.as<double>(), S.hi0.as<int>(), S.hk1.as<double>(), S.hi1.as<int>(),
                         S.hsplit.as<int>(), &fb, &nl, st);
     if (e != hipSuccess) return hip_fail(ctx, e, "hint series sort");
@@ -2460,7 +2463,7 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
     if (e != hipSuccess) return hip_fail(ctx, e, "hipMemcpyAsync(tables)");
     int fb = 0, nl = 0;
     e = enm_launch_sort(reinterpret_cast<const SortSeg*>(U.tables.as<char>() + o_s1), ncols, tiles1, maxlen1,
-                        ENM_SORT_TILE, d_values, nullptr, U.k0.as<double>(), U.i0.as<int>(), U.k1.as<double>(),
+                        d_values, nullptr, U.k0.as<double>(), U.i0.as<int>(), U.k1.as<double>(),
                         U.i1.as<int>(), U.split.as<int>(), &fb, &nl, st);
     if (e == hipSuccess)
         e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(U.tables.as<char>() + o_u1), ncols, tiles1,
@@ -2532,7 +2535,7 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
         fb = 0;
         if (e == hipSuccess)
             e = enm_launch_sort(reinterpret_cast<const SortSeg*>(tb + o_s2), (int)segs2.size(), tiles2, maxlen2,
-                                ENM_SORT_TILE, U.rkeys.as<double>(), nullptr, U.k0.as<double>(), U.i0.as<int>(),
+                                U.rkeys.as<double>(), nullptr, U.k0.as<double>(), U.i0.as<int>(),
                                 U.k1.as<double>(), U.i1.as<int>(), U.split.as<int>(), &fb, &nl, st);
         if (e == hipSuccess)
             e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(tb + o_u2), (int)useg2.size(), tiles2,

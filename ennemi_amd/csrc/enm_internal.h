@@ -34,6 +34,7 @@
 #define ENM_PSI_TILE 512       // positions per psi partial sum of a 1-D space
 #define ENM_SORT_TILE 2048     // elements per block-sort tile and merge chunk
 #define ENM_SORT_THREADS 256
+#define ENM_SORT_MAXTILE 8192  // largest block-sort tile
 #define ENM_MAX_SPACES 3
 // kNN list classes beyond the register lists of 4..32 slots: a per-lane
 // max-heap of k+1 values in LDS (k+1 <= ENM_LIST_LDS_MAX) or in a global

@@ -9,7 +9,9 @@
 hipError_t enm_launch_fill_u64(unsigned long long* p, int64_t n, unsigned long long v, hipStream_t st);
 hipError_t enm_launch_fill_i32(int* p, int64_t n, int v, hipStream_t st);
 
-hipError_t enm_launch_sort(const SortSeg* d_segs, int nsegs, int ntiles, int64_t maxlen, int tile,
+// Sorts segments of up to maxlen keys; the sorted runs are in k0, i0 or, with
+// *final_buf 1, in k1, i1.
+hipError_t enm_launch_sort(const SortSeg* d_segs, int nsegs, int ntiles, int64_t maxlen,
                            const double* arena, const int* iarena, double* k0, int* i0, double* k1, int* i1,
                            int* split, int* final_buf, int* n_launch, hipStream_t st,
                            const int* skip = nullptr);
