@@ -353,16 +353,17 @@ int tree_base_cells(int columns) { return columns <= 2 ? 64 : columns == 3 ? 16 
 // found on box trees, not on strips.  A strip is one workgroup's, so few points
 // leave the chip idle, and longer lists cost strips more (their lists shift by
 // every insertion); trees cost more per point.  Strips against trees, us of sort,
-// build, kNN and counts: 1,000 points k = 3 177 / 87, k = 20 554 / 90; 100 x 1,000
-// k = 3 226 / 136, 1,000 x 1,000 418 / 547, k = 7 611 / 604, k = 12 1174 / 691;
-// 100,000 points k = 3 329 / 305, k = 20 565 / 344; 10 x 100,000 k = 7 598 / 860,
-// k = 20 934 / 1100; 1,000 x 5,000 k = 12 3388 / 3338, k = 20 5758 / 3938.
+// build, kNN and counts: k = 3, 64 x 1,000 points 187 / 115, 256 x 1,000 201 / 202,
+// 100,000 points 300 / 286, 4 times 433 / 453, 16 times 568 / 1070; k = 7, 256 x
+// 2,048 347 / 349, 4 x 50,000 397 / 349, 16 times 486 / 674; k = 15, 1,024 x 2,048
+// 1506 / 1333, 64 x 10,000 636 / 646; k = 31, 1,024 x 2,048 3617 / 1753, 256 x
+// 6,000 1949 / 1552, 16 x 50,000 957 / 1005.
 int64_t tree_points(int k1, int64_t n) {
     const bool one_cell = n <= ENM_CELL;
-    if (k1 <= 4) return one_cell ? 250000 : 150000;
-    if (k1 <= 8) return one_cell ? 600000 : 400000;
-    if (n <= 2 * ENM_CELL) return INT64_MAX;
-    return k1 <= 16 ? 500000 : 700000;
+    if (k1 <= 4) return one_cell ? 250000 : 200000;
+    if (k1 <= 8) return one_cell ? 400000 : 320000;
+    if (one_cell || (k1 > 16 && n <= 2 * ENM_CELL)) return INT64_MAX;
+    return k1 <= 16 ? 550000 : 1000000;
 }
 
 struct Planner {
@@ -1622,7 +1623,7 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
                 // the LDS (three slots of the largest strip) allow.
                 const int nt = std::min(512, ((g.smax + 63) / 64) * 64);
                 const int by_waves = std::max(1, g.waves * 64 / nt);
-                const int by_lds = std::max(1, (160 * 1024) / (3 * g.smax * 16));
+                const int by_lds = std::max(1, (160 * 1024) / (3 * (g.smax + 2) * 16));
                 grid = std::max(1, std::min(g.n_items, ctx->num_cus * std::min(by_waves, by_lds)));
             }
             e = enm_launch_knn(tab<Item>(P, P.off_kitems) + g.first, qoffs + g.qoff, g.n_items,

@@ -72,7 +72,7 @@ struct KnnFar {
     int32_t i;
     int32_t open;
     int32_t pad;
-    double L[P];
+    double L[P - 1];   // the query itself is not in it
 };
 
 // Launch of the kNN kernels of one joint dimension D (one translation unit
@@ -466,7 +466,7 @@ __device__ void knn_item(const KnnArgs& A, const Item& it, const double* __restr
 // on the x axis, entering each at its y (binary search) and walking the
 // same way -- in LDS for s-1 and s+1, in global memory further out.  Every
 // candidate that could enter the list is visited, so the radii are those
-// of the per-lane walk and of brute force.  Candidate reads are LDS reads
+// of brute force.  Candidate reads are LDS reads
 // instead of one cache line per lane per load.
 
 constexpr int SK_THREADS_MAX = 512;
@@ -552,74 +552,53 @@ __device__ __forceinline__ void run_walk(L& list, double& T, const double2* __re
     }
 }
 
-// One query's walk state in run_walk2.
+// One query's walk state in run_walk2: the next candidate up and down (byte
+// offsets from the run's first).
 struct WalkQ {
     double2 q;
     double T;
     int u, dn;
-    bool up, down;
 };
 
-// Two queries walking the same run in lockstep: the four next candidates
-// (up and down of each) are read together, so their LDS latencies overlap;
-// each query still takes its candidates in its own order, up then down.
+// Two queries walking the same staged run in lockstep: the four next
+// candidates (up and down of each) are read together, so their LDS latencies
+// overlap.  A direction stops at the first candidate whose y distance is at
+// least the current radius T; the runs lie between two entries at infinite
+// distance (at -1 and at the run's length), so positions are not checked, and a
+// stopped direction stays where it is (T only falls).  The kernel is bound by
+// these instructions: 11 vector ones per candidate (20 with checks, a flag per
+// direction, a count of candidates and the query itself in its list).
 template <class L>
-__device__ __forceinline__ void run_walk2(L& l0, WalkQ& a, L& l1, WalkQ& b, const double2* __restrict__ w, int len,
+__device__ __forceinline__ void run_walk2(L& l0, WalkQ& a, L& l1, WalkQ& b, const double2* __restrict__ w,
                                           unsigned& visited) {
-    a.up = a.up && a.u < len;
-    a.down = a.down && a.dn >= 0;
-    b.up = b.up && b.u < len;
-    b.down = b.down && b.dn >= 0;
-    while (a.up || a.down || b.up || b.down) {
-        double2 ca = w[a.up ? a.u : 0], da = w[a.down ? a.dn : 0];
-        double2 cb = w[b.up ? b.u : 0], db = w[b.down ? b.dn : 0];
+    constexpr int STEP = sizeof(double2);
+    auto at = [&](int off) { return *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(w) + off); };
+    const int before = a.u - a.dn + b.u - b.dn;
+    bool au, ad, bu, bd;
+    do {
+        double2 ca = at(a.u), da = at(a.dn);
+        double2 cb = at(b.u), db = at(b.dn);
         pin(ca.x); pin(ca.y); pin(da.x); pin(da.y);
         pin(cb.x); pin(cb.y); pin(db.x); pin(db.y);
-        if (a.up) {
-            const double dy = ca.y - a.q.y;
-            if (dy < a.T) {
-                l0.insert(vmax_abs(dy, ca.x - a.q.x));
-                a.T = l0.top();
-                ++visited;
-                a.up = ++a.u < len;
-            } else {
-                a.up = false;
-            }
-        }
-        if (a.down) {
-            const double dy = a.q.y - da.y;
-            if (dy < a.T) {
-                l0.insert(vmax_abs(dy, da.x - a.q.x));
-                a.T = l0.top();
-                ++visited;
-                a.down = --a.dn >= 0;
-            } else {
-                a.down = false;
-            }
-        }
-        if (b.up) {
-            const double dy = cb.y - b.q.y;
-            if (dy < b.T) {
-                l1.insert(vmax_abs(dy, cb.x - b.q.x));
-                b.T = l1.top();
-                ++visited;
-                b.up = ++b.u < len;
-            } else {
-                b.up = false;
-            }
-        }
-        if (b.down) {
-            const double dy = b.q.y - db.y;
-            if (dy < b.T) {
-                l1.insert(vmax_abs(dy, db.x - b.q.x));
-                b.T = l1.top();
-                ++visited;
-                b.down = --b.dn >= 0;
-            } else {
-                b.down = false;
-            }
-        }
-    }
+        const double dau = ca.y - a.q.y, dad = a.q.y - da.y, dbu = cb.y - b.q.y, dbd = b.q.y - db.y;
+        au = dau < a.T;
+        if (au) l0.insert(vmax_abs(dau, ca.x - a.q.x));
+        a.u += au ? STEP : 0;
+        a.T = l0.top();
+        ad = dad < a.T;
+        if (ad) l0.insert(vmax_abs(dad, da.x - a.q.x));
+        a.dn -= ad ? STEP : 0;
+        a.T = l0.top();
+        bu = dbu < b.T;
+        if (bu) l1.insert(vmax_abs(dbu, cb.x - b.q.x));
+        b.u += bu ? STEP : 0;
+        b.T = l1.top();
+        bd = dbd < b.T;
+        if (bd) l1.insert(vmax_abs(dbd, db.x - b.q.x));
+        b.dn -= bd ? STEP : 0;
+        b.T = l1.top();
+    } while (au || ad || bu || bd);
+    visited += (unsigned)(a.u - a.dn + b.u - b.dn - before) / STEP;
 }
 
 // Strips further out than the staged neighbours, for one query: in global
@@ -653,13 +632,15 @@ __device__ __forceinline__ void far_strips(L& list, double& T, const double2* __
     }
 }
 
-// Four-slot lists are held to 80 VGPRs, six waves per SIMD (a few bytes
-// spill: the far-list bookkeeping would otherwise cost a wave per SIMD).
+// Four-slot lists (three neighbours) are held to 80 VGPRs, six waves per SIMD.
+// Bound by its instructions (run_walk2): 776 lag windows of 70,000 points, k = 3,
+// 2.33 -> 1.77 ms; 2,016 pairs of 50,000 4.94 -> 3.76.
 template <int P>
 __global__ __launch_bounds__(SK_THREADS_MAX, P == 4 ? 6 : 1)
 void knn_strip_kernel(KnnArgs A, const double* __restrict__ col64, double* __restrict__ res64,
                       unsigned long long* __restrict__ stats) {
-    extern __shared__ double2 sxy[];   // three slots of A.smax pairs: strips s-1, s, s+1
+    // Three slots of A.smax pairs and one more at each end: strips s-1, s, s+1.
+    extern __shared__ double2 sxy[];
     __shared__ unsigned s_ticket;
     const int NT = (int)blockDim.x;
     unsigned pairs = 0;   // this thread's candidates (a few thousand): one register
@@ -689,7 +670,12 @@ void knn_strip_kernel(KnnArgs A, const double* __restrict__ col64, double* __res
             for (int k = 0; k < 3; ++k) v[k] = t < slen[k] ? xy[slo[k] + t] : make_double2(0.0, 0.0);
 #pragma unroll
             for (int k = 0; k < 3; ++k)
-                if (t < slen[k]) sxy[k * A.smax + t] = v[k];
+                if (t < slen[k]) sxy[k * (A.smax + 2) + 1 + t] = v[k];
+        }
+        if (threadIdx.x < 3) {
+            double2* w = sxy + (int)threadIdx.x * (A.smax + 2) + 1;
+            w[-1] = make_double2(0.0, -INFINITY);
+            w[threadIdx.x == 0 ? slen[0] : threadIdx.x == 1 ? slen[1] : slen[2]] = make_double2(0.0, INFINITY);
         }
         // The x bounds of the neighbours: largest x left, smallest x right;
         // and of the strips beyond them.
@@ -698,43 +684,46 @@ void knn_strip_kernel(KnnArgs A, const double* __restrict__ col64, double* __res
         const double xl2 = uni_f64(s >= 2 ? xk[slo[0] - 1] : 0.0);
         const double xr2 = uni_f64(s + 2 < nstrip ? xk[lo + (s + 2) * S] : 0.0);
         __syncthreads();
-        const double2* own = sxy + A.smax;
+        const double2 *left = sxy + 1, *own = left + A.smax + 2, *right = own + A.smax + 2;
         // Two queries per thread, NT apart, walked in lockstep.
         for (int i0 = it.t0 + (int)threadIdx.x; i0 < it.t1; i0 += 2 * NT) {
             const int i1 = i0 + NT;
             const bool act1 = i1 < it.t1;
-            RegList<P> l0, l1;
-            l0.init(kd.k + 1, nullptr);
-            l1.init(kd.k + 1, nullptr);
+            RegList<P - 1> l0, l1;   // without the queries themselves
+            l0.init(kd.k, nullptr);
+            l1.init(kd.k, nullptr);
             WalkQ a, b;
             const int p0 = i0 - slo[1], p1 = act1 ? i1 - slo[1] : p0;
             a.q = own[p0];
             b.q = own[p1];
-            l0.insert(0.0);   // the queries themselves
-            if (act1) l1.insert(0.0);
             a.T = l0.top();
             b.T = l1.top();
             unsigned visited = 1 + (act1 ? 1u : 0u);
-            a.u = p0 + 1; a.dn = p0 - 1; a.up = a.down = true;
-            b.u = p1 + 1; b.dn = p1 - 1; b.up = b.down = act1;
-            run_walk2(l0, a, l1, b, own, slen[1], visited);
+            auto start = [](WalkQ& w, bool in, int u, int len) {
+                w.u = (in ? u : len) * (int)sizeof(double2);
+                w.dn = (in ? u - 1 : -1) * (int)sizeof(double2);
+            };
+            start(a, true, p0 + 1, slen[1]);
+            start(b, act1, p1 + 1, slen[1]);
+            a.dn -= (int)sizeof(double2);
+            b.dn -= act1 ? (int)sizeof(double2) : 0;
+            run_walk2(l0, a, l1, b, own, visited);
             // The staged neighbours, where the radius reaches them on x.
             const bool la = slen[0] > 0 && a.q.x - xl < a.T, lb = act1 && slen[0] > 0 && b.q.x - xl < b.T;
             if (la || lb) {
                 int e0, e1;
-                slot_lower_bound2(sxy, slen[0], a.q.y, b.q.y, e0, e1);
-                a.u = e0; a.dn = e0 - 1; a.up = a.down = la;
-                b.u = e1; b.dn = e1 - 1; b.up = b.down = lb;
-                run_walk2(l0, a, l1, b, sxy, slen[0], visited);
+                slot_lower_bound2(left, slen[0], a.q.y, b.q.y, e0, e1);
+                start(a, la, e0, slen[0]);
+                start(b, lb, e1, slen[0]);
+                run_walk2(l0, a, l1, b, left, visited);
             }
             const bool ra = slen[2] > 0 && xr - a.q.x < a.T, rb = act1 && slen[2] > 0 && xr - b.q.x < b.T;
             if (ra || rb) {
-                const double2* w = sxy + 2 * A.smax;
                 int e0, e1;
-                slot_lower_bound2(w, slen[2], a.q.y, b.q.y, e0, e1);
-                a.u = e0; a.dn = e0 - 1; a.up = a.down = ra;
-                b.u = e1; b.dn = e1 - 1; b.up = b.down = rb;
-                run_walk2(l0, a, l1, b, w, slen[2], visited);
+                slot_lower_bound2(right, slen[2], a.q.y, b.q.y, e0, e1);
+                start(a, ra, e0, slen[2]);
+                start(b, rb, e1, slen[2]);
+                run_walk2(l0, a, l1, b, right, visited);
             }
             // Further strips in global memory (a side is done once its
             // nearer strip was out of reach).  A query that needs them goes
@@ -770,7 +759,7 @@ void knn_strip_kernel(KnnArgs A, const double* __restrict__ col64, double* __res
                         f.i = i0;
                         f.open = (la ? 1 : 0) | (ra ? 2 : 0);
 #pragma unroll
-                        for (int t = 0; t < P; ++t) f.L[t] = l0.L[t];
+                        for (int t = 0; t < P - 1; ++t) f.L[t] = l0.L[t];
                     }
                     if (db) {
                         KnnFar<P>& f = far[sb];
@@ -778,7 +767,7 @@ void knn_strip_kernel(KnnArgs A, const double* __restrict__ col64, double* __res
                         f.i = i1;
                         f.open = (lb ? 1 : 0) | (rb ? 2 : 0);
 #pragma unroll
-                        for (int t = 0; t < P; ++t) f.L[t] = l1.L[t];
+                        for (int t = 0; t < P - 1; ++t) f.L[t] = l1.L[t];
                     }
                 }
             }
@@ -827,9 +816,9 @@ void knn_far_kernel(KnnArgs A, const double* __restrict__ col64, double* __restr
         const int lo = it.lo, hi = it.hi;
         const int s = (it.t0 - lo) / S;
         const int nstrip = (hi - lo + S - 1) / S;
-        RegList<P> L;
+        RegList<P - 1> L;
 #pragma unroll
-        for (int t = 0; t < P; ++t) L.L[t] = f.L[t];
+        for (int t = 0; t < P - 1; ++t) L.L[t] = f.L[t];
         double T = L.top();
         const int i = f.i;
         unsigned visited = 0;
@@ -882,7 +871,7 @@ hipError_t launch_dp(const KnnArgs& a, bool f32, int walk, int grid, const doubl
     if (walk == ENM_WALK_STRIP) {
         if constexpr (D == 2 && P > 0) {
             const int nt = a.smax >= SK_THREADS_MAX ? SK_THREADS_MAX : ((a.smax + 63) / 64) * 64;
-            const unsigned lds = (unsigned)(3 * a.smax * sizeof(double2));
+            const unsigned lds = (unsigned)(3 * (a.smax + 2) * sizeof(double2));
             hipLaunchKernelGGL((knn_strip_kernel<P>), dim3(grid), dim3(nt), lds, st, a, col64, res64, stats);
             // The far list: eight 4-wave blocks per CU of the strip grid's
             // three (latency-bound walks need every wave slot).
