@@ -34,7 +34,7 @@ class Batch:
         key = id(a)
         idx = self._col_index.get(key)
         if idx is None:
-            c = np.ascontiguousarray(a, dtype=np.float64)
+            c = np.asarray(a, dtype=np.float64)
             if c.ndim != 1:
                 raise ValueError("columns must be one-dimensional")
             idx = len(self._cols)
@@ -64,16 +64,15 @@ class Batch:
         return len(self._inst) - 1
 
     def pack(self):
-        """Host arena (float64) and the ctypes instance / class-size tables."""
-        offsets = np.zeros(len(self._cols) + 1, dtype=np.int64)
-        for i, c in enumerate(self._cols):
-            offsets[i + 1] = offsets[i] + len(c)
-        arena = np.empty(int(offsets[-1]), dtype=np.float64)
-        for i, c in enumerate(self._cols):
-            arena[offsets[i]:offsets[i + 1]] = c
+        """The ctypes instance / class-size tables; columns lie one after the other."""
+        offsets = np.cumsum([0] + [len(c) for c in self._cols])
         inst_arr = _instance_table(self._inst, offsets)
         seg_arr = (ctypes.c_int64 * max(1, len(self._seg)))(*self._seg)
-        return arena, inst_arr, seg_arr
+        return inst_arr, seg_arr
+
+    def arena(self, device, stream):
+        """The columns in HBM, sent up on `stream`; returns (arena, pinned host copy)."""
+        return upload_columns(self._cols, device, stream)
 
     def point_offsets(self) -> np.ndarray:
         n = np.array([t[2] for t in self._inst], dtype=np.int64)
@@ -123,13 +122,12 @@ class DeviceBatch:
         self.hint = getattr(batch, "device_hint", None) if hints else None
         self.ctx = nat.context()
         self.flags = flags
-        arena, self.inst_arr, self.seg_arr = batch.pack()
+        self.inst_arr, self.seg_arr = batch.pack()
         self.n_inst = len(batch)
         dev = torch.device("cuda", self.ctx.device)
         self.stream = _stream()
         with torch.cuda.stream(self.stream):
-            # A batch prepared on the device brings its arena along.
-            self.arena = batch.device_arena if arena is None else torch.from_numpy(arena).to(dev)
+            self.arena, self._pinned = batch.arena(dev, self.stream)
             self.out = torch.empty(self.n_inst, dtype=torch.float64, device=dev)
             self.offs = batch.point_offsets()
             total = int(self.offs[-1])
@@ -227,7 +225,10 @@ class ArenaBatch:
         if self._classes is not None:
             tab["n_segs"], tab["seg_index"] = self._classes[:2]
             seg_arr = (ctypes.c_int64 * len(self._classes[2]))(*self._classes[2].tolist())
-        return None, inst_arr, seg_arr
+        return inst_arr, seg_arr
+
+    def arena(self, device, stream):
+        return self.device_arena, None
 
     def point_offsets(self) -> np.ndarray:
         n = np.concatenate([np.zeros(0, dtype=np.int64)] + [r[2] for r in self._runs])
@@ -253,15 +254,14 @@ _SHORT = 1 << 14
 
 
 def upload_columns(arrays, device, stream):
-    """The values of arrays (equally long: columns, or tables of columns) as
-    float64 columns in HBM, one after the other; returns (device columns,
-    pinned host copy).  They go up from pinned host memory, asynchronously on
-    `stream`, while the host goes on; a table held row by row is turned into
-    columns on the device."""
+    """The values of arrays (columns, or tables of columns) as float64 columns
+    in HBM, one after the other; returns (device columns, pinned host copy).
+    They go up from pinned host memory, asynchronously on `stream`, while the
+    host goes on; a table held row by row is turned into columns on the device."""
     import torch
-    n = len(arrays[0])
     blocks = []   # values as they lie in memory (rows of `m`, or column by column), m
     for a in arrays:
+        n = len(a)
         m = 1 if a.ndim == 1 else a.shape[1]
         by_column = m == 1 or a.flags.f_contiguous
         blocks.append((a.reshape(n) if m == 1 else a.T if by_column else a, 1 if by_column else m, n * m))
@@ -296,7 +296,7 @@ def upload_columns(arrays, device, stream):
             if m > 1:
                 rows = up.to(torch.float64)
                 with ctx.lock:
-                    ctx.prep_columns(rows.data_ptr(), n, m, dst.data_ptr(), stream.cuda_stream)
+                    ctx.prep_columns(rows.data_ptr(), size // m, m, dst.data_ptr(), stream.cuda_stream)
             elif whole:
                 dst.copy_(up)
             at += size
