@@ -1099,10 +1099,10 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
 
     // Tree queries: an item is a leaf, shared by as many waves (of as few
     // queries each) as make four for every wave slot of the GPU.
-    auto tree_items = [&](const std::vector<TreeQueries>& all, std::vector<PendingRun>& pend) {
+    auto tree_items = [&](const std::vector<TreeQueries>& all, std::vector<PendingRun>& pend, bool counts) {
         int64_t total = 0;
         for (const TreeQueries& q : all) total = P.per_instance ? std::max(total, q.n) : total + q.n;
-        int share = 1;
+        int share = 4;   // two million points in four columns: kNN 4.9 ms with one wave per leaf, 4.5 with four
         while (share < ENM_LEAF && total * share / ENM_LEAF < (int64_t)4 * 32 * ctx->num_cus) share *= 2;
         for (const TreeQueries& q : all)
             for (int t = q.first; t < q.first + q.count; ++t) {
@@ -1111,12 +1111,12 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
                 pi.it.t0 = 0;
                 pi.it.t1 = P.trees[t].n;
                 pi.step = ENM_LEAF;
-                pi.ticket = share;
+                pi.ticket = counts ? std::min(share, ENM_LEAF / enm_tree_queries(pi.dclass)) : share;
                 pend.push_back(pi);
             }
     };
-    tree_items(ktree, kpend);
-    tree_items(ctree, cpend);
+    tree_items(ktree, kpend, false);
+    tree_items(ctree, cpend, true);
 
     for (size_t o = 0; o < P.orders.size(); ++o)
         if (P.orders[o].xy >= 0 && !cols_read.count((int)o)) P.orders[o].xy_only = 1;

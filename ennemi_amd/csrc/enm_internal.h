@@ -51,6 +51,9 @@
 #define ENM_STRIP_WIDE 4096
 // Box trees (enm_tree.hip).
 #define ENM_LEAF 64            // points per leaf (one per lane)
+// Queries that a wave counts at once on a tree of dimension class D (registers:
+// two leaves and the queries).
+constexpr int enm_tree_queries(int D) { return D <= 6 ? 4 : D <= 8 ? 2 : 1; }
 #define ENM_CELL 4096          // points per cell: ENM_LEAF leaves of ENM_LEAF points
 #define ENM_TREE_STEPS 6       // most sorted columns of a cell (one halving of its leaves each at least)
 #define ENM_TREE_LISTS 8       // most registers of a neighbour list held across a wave's lanes (64 each)

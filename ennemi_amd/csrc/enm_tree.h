@@ -3,20 +3,23 @@
 // reference (ennemi/_entropy_estimators.py:39,108,142,152-154,194,196,240,
 // 243-245) where no strip of two columns fits in LDS.
 //
-// A wave takes one query at a time.  Its 64 lanes test the boxes of 64
-// children of a node at once (groups, then cells, then leaves), and the
+// A wave takes one query at a time, or counts four.  Its 64 lanes test the boxes
+// of 64 children of a node at once (groups, then cells, then leaves), and the
 // points of a leaf are evaluated one per lane, so each (query, leaf) pair
 // whose ball and box meet costs one coalesced load and one difference and
 // maximum per column, and nothing is evaluated for the sake of other queries:
 // the boxes are tight in every column, where a window shared by 64 queries is
 // their union and is cut by two columns only.  Measured against such windows
 // (one conditional MI of 2,000,000 points with two conditions, k = 5): kNN in
-// four columns 51.6 -> 5.3 ms, the three counts 51.4 -> 15.3 ms; 100,000 points
+// four columns 51.6 -> 4.5 ms, the three counts 51.4 -> 8.0 ms; 100,000 points
 // with three conditions, kNN in five columns 2.77 -> 0.24 ms, counts 3.97 ->
-// 0.78 ms; joint entropy of four columns, 100,000 points, 1.48 -> 0.13 ms; 60
+// 0.45 ms; joint entropy of four columns, 100,000 points, 1.48 -> 0.13 ms; 60
 // conditional MIs of 1,800 points, kNN 0.110 -> 0.062 ms, counts 0.305 ->
-// 0.081 ms.  The kNN is bound by its instructions (800 vector ones a query in
-// four columns), the counts by their loads (about 85 of 512 bytes a query).
+// 0.05 ms.  The kNN is bound by its instructions (800 vector ones a query in
+// four columns).  The counts were bound by their loads from L2, about 85 of 512
+// bytes a query; four neighbouring queries at once share them (one at a time:
+// 15.3 of the 8.0 ms above; two: 10.5; eight: 9.9, their coordinates no longer
+// fit the scalar registers).
 //
 // Everything is decided by the reference's own FP64 expressions.  For a box
 // side lo <= a <= hi, fl(a - q) >= fl(lo - q) and fl(q - a) >= fl(q - hi)
@@ -212,9 +215,10 @@ __device__ __forceinline__ void load_leaf(double (&a)[D], const double* __restri
     for (int d = 0; d < D; ++d) a[d] = leaf[col_of<D>(d, ncol) * ENM_LEAF + lane];
 }
 
-// The query's distance to this lane's box, from below (FAR: and from above).
-template <int D, bool FAR>
-__device__ __forceinline__ double box_gap(const double* __restrict__ b, int ncol, const double (&q)[D], double& far) {
+// The queries' distances to this lane's box, from below (FAR: and from above).
+template <int D, int Q, bool FAR>
+__device__ __forceinline__ void box_gap(const double* __restrict__ b, int ncol, const double (&q)[Q][D], double (&gap)[Q],
+                                        double (&far)[Q]) {
     const int lane = (int)(threadIdx.x & (ENM_WAVE - 1));
     double lo[D], hi[D];
 #pragma unroll
@@ -225,42 +229,65 @@ __device__ __forceinline__ double box_gap(const double* __restrict__ b, int ncol
     }
     // Equal infinities differ by NaN, which the maxima pass over here as they
     // do in point_dist (all NaN: not inside).
-    double g = 0.0;
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-        g = vmax(g, vmax(lo[d] - q[d], q[d] - hi[d]));
-        if (FAR) {
-            const double s = vmax(hi[d] - q[d], q[d] - lo[d]);
-            far = d == 0 ? s : vmax(far, s);
+    for (int k = 0; k < Q; ++k) {
+        double g = 0.0;
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            g = vmax(g, vmax(lo[d] - q[k][d], q[k][d] - hi[d]));
+            if (FAR) {
+                const double s = vmax(hi[d] - q[k][d], q[k][d] - lo[d]);
+                far[k] = d == 0 ? s : vmax(far[k], s);
+            }
         }
+        gap[k] = g;
     }
-    return g;
+}
+
+// One query's distance to this lane's box, from below.
+template <int D>
+__device__ __forceinline__ double box_gap(const double* __restrict__ b, int ncol, const double (&q)[D]) {
+    double gap[1], far[1];
+    box_gap<D, 1, false>(b, ncol, reinterpret_cast<const double(&)[1][D]>(q), gap, far);
+    return gap[0];
 }
 
 __device__ __forceinline__ unsigned long long low_mask(int n) {
     return n >= 64 ? ~0ull : ((1ull << n) - 1ull);
 }
 
-// Points within r of q, max_d fl64(|a_d - q_d|) <= r: a node whose box lies
-// within the radius in every column adds its points unopened, one out of reach
-// adds none; the others are opened, leaves by their points.
-template <int D>
-__device__ __forceinline__ int count_cell(const TreeDev& T, const double* __restrict__ col64, int cell,
-                                          const double (&q)[D], double r, unsigned& opened) {
+// c[k] += points within r[k] of q[k], max_d fl64(|a_d - q_d|) <= r, of Q queries
+// at once: a node whose box lies within the radius in every column adds its
+// points unopened, one out of reach adds none; the others are opened, leaves by
+// their points.  A node is opened for all the queries if one of them needs it:
+// neighbours in a leaf mostly need the same ones, and the loads (48 KB a query
+// by itself, from L2) are what bounds the counts.
+template <int D, int Q>
+__device__ __forceinline__ void count_cell(const TreeDev& T, const double* __restrict__ col64, int cell,
+                                           const double (&q)[Q][D], const double (&r)[Q], int (&c)[Q], unsigned& opened) {
     const int ncol = T.ncol;
     const int cnt = min(T.cell, T.n - cell * T.cell);
     const int nleaf = (cnt + ENM_LEAF - 1) / ENM_LEAF;
     unsigned long long part = 1;
-    int c = 0;
     if (T.n > ENM_LEAF) {
-        double far;
-        const double g = box_gap<D, true>(col64 + T.box + (int64_t)cell * 2 * ncol * 64, ncol, q, far);
-        const unsigned long long inside = __builtin_amdgcn_ballot_w64(far <= r) & low_mask(nleaf);
-        part = __builtin_amdgcn_ballot_w64(g <= r) & low_mask(nleaf) & ~inside;
-        c = (int)__popcll(inside) * ENM_LEAF;
-        if ((inside >> (nleaf - 1)) & 1) c -= nleaf * ENM_LEAF - cnt;
+        double gap[Q], far[Q];
+        box_gap<D, Q, true>(col64 + T.box + (int64_t)cell * 2 * ncol * 64, ncol, q, gap, far);
+        const unsigned long long valid = low_mask(nleaf);
+        unsigned long long inside[Q];
+        part = 0;
+#pragma unroll
+        for (int k = 0; k < Q; ++k) {
+            inside[k] = __builtin_amdgcn_ballot_w64(far[k] <= r[k]) & valid;
+            part |= __builtin_amdgcn_ballot_w64(gap[k] <= r[k]) & valid & ~inside[k];
+        }
+#pragma unroll
+        for (int k = 0; k < Q; ++k) {
+            const unsigned long long whole = inside[k] & ~part;
+            c[k] += (int)__popcll(whole) * ENM_LEAF;
+            if ((whole >> (nleaf - 1)) & 1) c[k] -= nleaf * ENM_LEAF - cnt;
+        }
     }
-    opened += (unsigned)__popcll(part);
+    opened += (unsigned)__popcll(part) * Q;
     const double* leaves = col64 + T.col + (int64_t)cell * T.cell * ncol;
     // Two leaves at a time, so that their loads overlap (an odd last one is
     // loaded twice and counted once).
@@ -273,46 +300,62 @@ __device__ __forceinline__ int count_cell(const TreeDev& T, const double* __rest
         double a[D], b[D];
         load_leaf<D>(a, leaves + l0 * ENM_LEAF * ncol, ncol);
         load_leaf<D>(b, leaves + l1 * ENM_LEAF * ncol, ncol);
-        const int ca = (int)__popcll(__builtin_amdgcn_ballot_w64(point_dist<D>(a, q) <= r));
-        const int cb = (int)__popcll(__builtin_amdgcn_ballot_w64(point_dist<D>(b, q) <= r));
-        c += ca + (two ? cb : 0);
+#pragma unroll
+        for (int k = 0; k < Q; ++k) {
+            const int ca = (int)__popcll(__builtin_amdgcn_ballot_w64(point_dist<D>(a, q[k]) <= r[k]));
+            const int cb = (int)__popcll(__builtin_amdgcn_ballot_w64(point_dist<D>(b, q[k]) <= r[k]));
+            c[k] += ca + (two ? cb : 0);
+        }
     }
-    return c;
 }
 
-template <int D>
-__device__ __forceinline__ int count_query(const TreeDev& T, const double* __restrict__ col64, const double (&q)[D],
-                                           double r, unsigned& opened) {
+template <int D, int Q>
+__device__ __forceinline__ void count_queries(const TreeDev& T, const double* __restrict__ col64, const double (&q)[Q][D],
+                                              const double (&r)[Q], int (&c)[Q], unsigned& opened) {
     const int ncell = T.ncell, ncol = T.ncol;
-    if (ncell == 1) return count_cell<D>(T, col64, 0, q, r, opened);
+#pragma unroll
+    for (int k = 0; k < Q; ++k) c[k] = 0;
+    if (ncell == 1) {
+        count_cell<D, Q>(T, col64, 0, q, r, c, opened);
+        return;
+    }
     const int ngroup = (ncell + 63) / 64;
-    int c = 0;
-    double far;
-    // Groups that the ball meets, 64 at a time; then their cells.
+    double gap[Q], far[Q];
+    // Groups that the balls meet, 64 at a time; then their cells.
     for (int gb = 0; gb < ngroup; gb += 64) {
         unsigned long long gm = 1;
         if (ngroup > 1) {
-            const double g = box_gap<D, false>(col64 + T.gbox + (int64_t)(gb / 64) * 2 * ncol * 64, ncol, q, far);
-            gm = __builtin_amdgcn_ballot_w64(g <= r) & low_mask(ngroup - gb);
+            box_gap<D, Q, false>(col64 + T.gbox + (int64_t)(gb / 64) * 2 * ncol * 64, ncol, q, gap, far);
+            gm = 0;
+#pragma unroll
+            for (int k = 0; k < Q; ++k) gm |= __builtin_amdgcn_ballot_w64(gap[k] <= r[k]);
+            gm &= low_mask(ngroup - gb);
         }
         while (gm) {
             const int gr = gb + __builtin_ctzll(gm);
             gm &= gm - 1;
-            const double g = box_gap<D, true>(col64 + T.cbox + (int64_t)gr * 2 * ncol * 64, ncol, q, far);
+            box_gap<D, Q, true>(col64 + T.cbox + (int64_t)gr * 2 * ncol * 64, ncol, q, gap, far);
             const unsigned long long valid = low_mask(ncell - gr * 64);
-            const unsigned long long inside = __builtin_amdgcn_ballot_w64(far <= r) & valid;
-            unsigned long long part = __builtin_amdgcn_ballot_w64(g <= r) & valid & ~inside;
-            c += (int)__popcll(inside) * T.cell;
+            unsigned long long inside[Q], part = 0;
+#pragma unroll
+            for (int k = 0; k < Q; ++k) {
+                inside[k] = __builtin_amdgcn_ballot_w64(far[k] <= r[k]) & valid;
+                part |= __builtin_amdgcn_ballot_w64(gap[k] <= r[k]) & valid & ~inside[k];
+            }
             const int last = ncell - 1 - gr * 64;   // the scope's last cell, if it is here
-            if (last < 64 && ((inside >> last) & 1)) c -= ncell * T.cell - T.n;
+#pragma unroll
+            for (int k = 0; k < Q; ++k) {
+                const unsigned long long whole = inside[k] & ~part;
+                c[k] += (int)__popcll(whole) * T.cell;
+                if (last < 64 && ((whole >> last) & 1)) c[k] -= ncell * T.cell - T.n;
+            }
             while (part) {
                 const int k = gr * 64 + __builtin_ctzll(part);
                 part &= part - 1;
-                c += count_cell<D>(T, col64, k, q, r, opened);
+                count_cell<D, Q>(T, col64, k, q, r, c, opened);
             }
         }
     }
-    return c;
 }
 
 // Waves per SIMD that the kernels of dimension class D are held to registers

@@ -135,6 +135,7 @@ void tree_count_kernel(TreeArgs A, const CountDev* __restrict__ descs, const dou
                        unsigned long long* __restrict__ stats) {
     const TreeWork it = tree_work(A);
     if (it.nq <= 0) return;
+    constexpr int Q = enm_tree_queries(D);
     const int lane = (int)(threadIdx.x & (ENM_WAVE - 1));
     const CountDev& cd = descs[it.desc];
     const TreeDev& T = A.trees[it.tile];
@@ -150,14 +151,24 @@ void tree_count_kernel(TreeArgs A, const CountDev* __restrict__ descs, const dou
     for (int d = 0; d < D; ++d) ql[d] = leaf[col_of<D>(d, ncol) * ENM_LEAF + pos % ENM_LEAF];
     int mine = 0;
     unsigned opened = 0;
-    for (int j = 0; j < nq; ++j) {
-        const double r = lane_f64(rl, j);
-        if (r < 0.0) continue;
-        double q[D];
+    for (int j = 0; j < nq; j += Q) {
+        // (Past the last query: a radius that no point is within.)
+        double q[Q][D], r[Q];
+        int c[Q];
+        bool any = false;
 #pragma unroll
-        for (int d = 0; d < D; ++d) q[d] = lane_f64(ql[d], j);
-        const int c = count_query<D>(T, col64, q, r, opened);
-        if (lane == j) mine = c;
+        for (int k = 0; k < Q; ++k) {
+            const int t = min(j + k, nq - 1);
+            r[k] = j + k < nq ? lane_f64(rl, t) : -1.0;
+            any = any || !(r[k] < 0.0);
+#pragma unroll
+            for (int d = 0; d < D; ++d) q[k][d] = lane_f64(ql[d], t);
+        }
+        if (!any) continue;
+        count_queries<D, Q>(T, col64, q, r, c, opened);
+#pragma unroll
+        for (int k = 0; k < Q; ++k)
+            if (lane == j + k) mine = c[k];
     }
     if (lane < nq) {
         res32[cd.counts + pt] = mine;

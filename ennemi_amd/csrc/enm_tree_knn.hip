@@ -67,8 +67,7 @@ struct TreeQuery {
     // The leaves of a cell but leaf `own` (-1: all).
     __device__ __forceinline__ void visit_cell(int cell, int own) {
         const int nleaf = (min(T.cell, T.n - cell * T.cell) + ENM_LEAF - 1) / ENM_LEAF;
-        double far;
-        const double g = box_gap<D, false>(col64 + T.box + (int64_t)cell * 2 * ncol * 64, ncol, q, far);
+        const double g = box_gap<D>(col64 + T.box + (int64_t)cell * 2 * ncol * 64, ncol, q);
         unsigned long long open = low_mask(nleaf);
         if (own >= 0) open &= ~(1ull << own);
         const double* leaves = col64 + T.col + (int64_t)cell * T.cell * ncol;
@@ -83,18 +82,17 @@ struct TreeQuery {
 
     __device__ __forceinline__ void visit_others(int own_cell) {
         const int ncell = T.ncell, ngroup = (ncell + 63) / 64;
-        double far;
         for (int gb = 0; gb < ngroup; gb += 64) {
             double gg = 0.0;
             unsigned long long gopen = low_mask(ngroup - gb);
-            if (ngroup > 1) gg = box_gap<D, false>(col64 + T.gbox + (int64_t)(gb / 64) * 2 * ncol * 64, ncol, q, far);
+            if (ngroup > 1) gg = box_gap<D>(col64 + T.gbox + (int64_t)(gb / 64) * 2 * ncol * 64, ncol, q);
             for (;;) {
                 const unsigned long long gm = ngroup > 1 ? __builtin_amdgcn_ballot_w64(gg < t) & gopen : gopen;
                 if (!gm) break;
                 const int gl = ngroup > 1 ? nearest(gm, gg) : 0;
                 gopen &= ~(1ull << gl);
                 const int gr = gb + gl;
-                const double g = box_gap<D, false>(col64 + T.cbox + (int64_t)gr * 2 * ncol * 64, ncol, q, far);
+                const double g = box_gap<D>(col64 + T.cbox + (int64_t)gr * 2 * ncol * 64, ncol, q);
                 unsigned long long open = low_mask(ncell - gr * 64);
                 if (own_cell / 64 == gr) open &= ~(1ull << (own_cell % 64));
                 for (;;) {
@@ -145,7 +143,10 @@ void tree_knn_kernel(TreeArgs A, const KnnDev* __restrict__ descs, const double*
             if (T.n > ENM_LEAF) w.visit_cell(cell, leaf - cell * (T.cell / ENM_LEAF));
             if (T.ncell > 1) w.visit_others(cell);
             if (!PASSES || found + w.K1 == k1 || !(w.t < INFINITY)) break;
-            found = count_query<D>(T, col64, w.q, w.t, w.visited);
+            const double radius[1] = {w.t};
+            int within[1];
+            count_queries<D, 1>(T, col64, reinterpret_cast<const double(&)[1][D]>(w.q), radius, within, w.visited);
+            found = within[0];
             if (found >= k1) break;   // ties at the last rank
             w.above = w.t;
         }
