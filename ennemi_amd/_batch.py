@@ -11,6 +11,8 @@ one ``enm_run_batch`` call and returns one float64 value per instance.
 from __future__ import annotations
 
 import ctypes
+import functools
+import threading
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -85,9 +87,10 @@ class Batch:
     def run(self, flags: int = 0, export: bool = False):
         """Run every instance.  Returns values, or (values, eps, counts) with
         per-instance lists of radii (n,) and counts (3, n) when export=True."""
-        db = self.device(flags, export)
-        db.launch()
-        return db.results()
+        with on(_stream()):
+            db = self.device(flags, export)
+            db.launch()
+            return db.results()
 
 
 def _instance_table(inst: List[tuple], col_offsets: Optional[np.ndarray]):
@@ -126,7 +129,7 @@ class DeviceBatch:
         self.n_inst = len(batch)
         dev = torch.device("cuda", self.ctx.device)
         self.stream = _stream()
-        with torch.cuda.stream(self.stream):
+        with on(self.stream):
             self.arena, self._pinned = batch.arena(dev, self.stream)
             self.out = torch.empty(self.n_inst, dtype=torch.float64, device=dev)
             self.offs = batch.point_offsets()
@@ -158,7 +161,7 @@ class DeviceBatch:
 
     def results(self):
         import torch
-        with torch.cuda.stream(self.stream):
+        with on(self.stream):
             host = torch.empty(self.n_inst, dtype=torch.float64, pin_memory=True).copy_(self.out, non_blocking=True)
         self.stream.synchronize()
         values = host.numpy().copy()
@@ -238,9 +241,10 @@ class ArenaBatch:
         return DeviceBatch(self, flags, export, hints)
 
     def run(self, flags: int = 0, export: bool = False, hints: bool = True):
-        db = self.device(flags, export, hints)
-        db.launch()
-        return db.results()
+        with on(_stream()):
+            db = self.device(flags, export, hints)
+            db.launch()
+            return db.results()
 
 
 # Values that are copied to pinned memory and sent up at a time, so that one piece
@@ -268,7 +272,7 @@ def upload_columns(arrays, device, stream):
     total = sum(size for _, _, size in blocks)
     pinned = torch.empty(total, dtype=torch.float64, pin_memory=True)
     ctx = nat.context()
-    with torch.cuda.stream(stream):
+    with on(stream):
         if total <= _SHORT:
             host, at = pinned.numpy(), 0
             for a, m, size in blocks:
@@ -312,5 +316,39 @@ def _stream():
     global _side_stream
     import torch
     if _side_stream is None:
+        nat.context()   # says what is missing without a GPU
         _side_stream = torch.cuda.Stream()
     return _side_stream
+
+
+_entered = threading.local()   # .stream: the stream of this thread's outermost `on`
+
+
+class on:
+    """torch.cuda.stream(stream), which costs 6 us, entered once by nested uses."""
+
+    def __init__(self, stream) -> None:
+        self.stream = stream
+        self.context = None
+
+    def __enter__(self) -> None:
+        import torch
+        if getattr(_entered, "stream", None) is not self.stream:
+            self.before = getattr(_entered, "stream", None)
+            self.context = torch.cuda.stream(self.stream)
+            self.context.__enter__()
+            _entered.stream = self.stream
+
+    def __exit__(self, *exc) -> None:
+        if self.context is not None:
+            _entered.stream = self.before
+            self.context.__exit__(*exc)
+
+
+def on_stream(f):
+    """f on the dedicated stream."""
+    @functools.wraps(f)
+    def g(*args, **kwargs):
+        with on(_stream()):
+            return f(*args, **kwargs)
+    return g

@@ -69,7 +69,7 @@ def _device_unique(row_sets: Sequence[Sequence[np.ndarray]]) -> List[Tuple[np.nd
     equally long numeric columns), codes in lexicographic row order, from
     enm_unique_rows."""
     import torch
-    from ._batch import _stream
+    from ._batch import _stream, on
     ctx = nat.context()
     dev = torch.device("cuda", ctx.device)
     st = _stream()
@@ -93,7 +93,7 @@ def _device_unique(row_sets: Sequence[Sequence[np.ndarray]]) -> List[Tuple[np.nd
             sets[s].col[j] = offsets[id(c)]
         out_off.append(out_off[-1] + len(cols[0]))
     h_distinct = np.zeros(n_sets, dtype=np.int64)
-    with torch.cuda.stream(st):
+    with on(st):
         d_values = torch.from_numpy(values).to(dev)
         d_codes = torch.empty(max(out_off[-1], 1), dtype=torch.int32, device=dev)
         d_counts = torch.empty(max(out_off[-1], 1), dtype=torch.int64, device=dev)

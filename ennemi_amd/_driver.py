@@ -26,7 +26,7 @@ from warnings import warn
 import numpy as np
 
 from . import _native as nat
-from ._batch import Batch
+from ._batch import Batch, on, on_stream
 from . import _discrete
 
 DISCRETE_NORMALIZATION_WARNING = \
@@ -527,9 +527,10 @@ class DevicePrep:
         self.dz = dz
         self.n_tasks = n_tasks
         self.d_raw, self.raw_host = upload_columns(arrays, self.dev, self.st)
-        with torch.cuda.stream(self.st):
-            self.d_mask = torch.from_numpy(np.ascontiguousarray(mask, dtype=np.uint8)).to(self.dev) \
-                if mask is not None else None
+        self.d_mask = None
+        if mask is not None:
+            with on(self.st):
+                self.d_mask = torch.from_numpy(np.ascontiguousarray(mask, dtype=np.uint8)).to(self.dev)
         self.place = np.arange(n_tasks, dtype=np.int64)   # task -> its device slot
         self.tasks = (nat.EnmPrepTask * n_tasks)()
         nat.struct_array(self.tasks)["dz"] = dz
@@ -576,7 +577,7 @@ class DevicePrep:
         self.arena_off = np.concatenate([[0], np.cumsum(per)[:-1]]).astype(np.int64)
         total = int(per.sum())
         noise_len = int(per.max()) if self.preprocess else 0
-        with torch.cuda.stream(self.st):
+        with on(self.st):
             if self.arena is None or self.arena.numel() != total:
                 self.arena = torch.empty(total, dtype=torch.float64, device=self.dev)
                 self.hint = torch.empty(total, dtype=torch.int32, device=self.dev) if self.hints else None
@@ -590,7 +591,7 @@ class DevicePrep:
         with self.ctx.lock:
             self.ctx.prep_write(self.tasks, self.n_tasks, raw, mask, noise, nlen, self.flags, self.arena_off,
                                 self.arena.data_ptr(), self.d_const.data_ptr(), self.st.cuda_stream)
-            with torch.cuda.stream(self.st):
+            with on(self.st):
                 self.h_const = torch.empty(self.n_tasks, dtype=torch.int32, pin_memory=True)
                 self.h_const.copy_(self.d_const, non_blocking=True)
             if self.hints:
@@ -623,6 +624,7 @@ def _hints_pay(nlag: int, nvar: int, n_rows: int, dz: int) -> bool:
     return dz == 0 and orders >= 32 * (nvar + 1) and orders * n_rows >= 6_000_000
 
 
+@on_stream
 def _plan_mi_device(y, x, lag, k, cond, cond_lag, mask, preprocess, drop_nan, min_lag, max_lag,
                     indices, hints):
     """_plan_mi with each task prepared on the device: the raw series go up
@@ -656,6 +658,7 @@ def _classes_eligible(x, y, cond, discrete_x: bool) -> bool:
         _device_prep_arrays((cont,) if cond is None else (cont, cond), cond)
 
 
+@on_stream
 def _plan_classes_device(y, x, lag, k, cond, cond_lag, mask, discrete_x: bool, preprocess, drop_nan, min_lag, max_lag,
                          indices):
     """_plan_mi of class labels against continuous variables, prepared and
@@ -698,7 +701,7 @@ def _plan_classes_device(y, x, lag, k, cond, cond_lag, mask, discrete_x: bool, p
     g["src"][:, :1 + dz] = src
     g["dst"][:, :1 + dz] = dst
     sizes = np.zeros((prep.n_tasks, classes), dtype=np.int64)
-    with torch.cuda.stream(prep.st):
+    with on(prep.st):
         arena = torch.empty(int((n * (1 + dz)).sum()), dtype=torch.float64, device=prep.dev)
     with ctx.lock:
         ctx.group_rows(tasks, prep.n_tasks, classes, prep.arena.data_ptr(), arena.data_ptr(), sizes,
@@ -874,6 +877,7 @@ def _plan_pairwise(data, k, cond, preprocess, drop_nan, mask, discrete):
     return tasks, indices, nvar
 
 
+@on_stream
 def _plan_pairwise_device(data, k, cond, preprocess, drop_nan, mask, indices):
     """_plan_pairwise with the columns prepared on the device.  None where a
     pair fails validation (or a shared column is constant): the host path
