@@ -286,7 +286,7 @@ enum { ST_KNN_PAIRS = 0, ST_KNN_RECHECK, ST_CNT_PAIRS, ST_CNT_RECHECK, ST_CNT_1D
 
 // Device-side preparation of estimate_mi tasks (enm_prep_count / enm_prep_write).
 #define ENM_PREP_BLOCK 2048     // window rows per compaction block
-#define ENM_PREP_SHORT 8192     // kept rows of tasks rescaled by one workgroup each
+#define ENM_PREP_SHORT 4096     // kept rows of tasks rescaled by one workgroup each
 #define ENM_PREP_MAXZ 14        // condition columns of one task (ENM_MAX_COLS - 2)
 
 struct PrepTaskDev {

@@ -862,7 +862,8 @@ void prep_scale_kernel(const PrepTaskDev* __restrict__ tasks, int64_t stride, co
 // Phase 2 of short tasks (at most PREP_SHORT kept rows each), one workgroup per
 // task: every array's mean and deviation by a wave of its own, then the
 // rescaling.  Bound by latency and launches: for a few short tasks the phases
-// take some 5 us each, mostly to be launched.  With `whole` (windows of one block
+// take some 5 us each, mostly to be launched.  (36 tasks of 2,500 rows 37 us, in
+// phases 32 and five launches more; of 8,000 rows 117 and 40.)  With `whole` (windows of one block
 // of rows) it does the compaction too.
 __global__ __launch_bounds__(PB_THREADS)
 void prep_short_kernel(PrepTaskDev* tasks, const double* __restrict__ raw, const unsigned char* __restrict__ mask,
