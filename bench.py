@@ -495,7 +495,7 @@ def main() -> int:
                            "hipGraph replay of the batch: hinted orders checked and laid out, "
                            "strip-grid orders, strip kNN with LDS-staged neighbours in FP64, LDS "
                            "binary-search 1-D counts, fixed-order digamma means (FP32 filter + "
-                           "FP64 recheck only where it pays: brute force, off-grid multi-D counts)",
+                           "FP64 recheck only where it pays: brute force, counts on the plain key order)",
                    "graph_replayed": st["graph_replayed"], "n_launches_eager": stats[-1]["n_launches"],
                    "tuning": {"strip_points": tuning[0], "waves_per_cu": tuning[1],
                               "list_slots": tuning[2], "items_per_ticket": tuning[3]}},

@@ -215,7 +215,7 @@ struct Plan {
     bool plain = false;      // no trees: the key orders alone (a static batch whose trees do not fit)
     bool hinted = false;     // the call passes sort hints (first-stage segments of whole columns)
     // Kernels that read the FP32 column copies: the brute-force kNN and
-    // multi-D counts off the grid (band filter).  Only then are they made.
+    // multi-D counts on the plain key order (band filter).  Only then are they made.
     bool need32 = false;
     // device
     int64_t heap_bytes = 0;   // global heap lists of kNN groups with k+1 > ENM_LIST_LDS_MAX
@@ -263,8 +263,7 @@ struct enm_ctx {
     // by tuning_gen, which every change bumps.
     enm_tuning tuning{1024, 32, 0, 0};
     // Until a tuning is set, instances of three or more joint columns take
-    // wide strips: their grid sweeps scan the union of a wave's windows,
-    // which narrows as strips grow.
+    // wide strips: that is, box trees (see ENM_STRIP_WIDE).
     bool wide_multid = true;
     std::map<std::tuple<int, int, int>, enm_tuning> tuned;
     uint64_t tuning_gen = 0;

@@ -6,11 +6,11 @@
 // key column is all the brute-force window kernels and the 1-D binary-search
 // counts need.
 //
-// Algorithm: every segment is cut into ENM_SORT_TILE chunks; a 256-thread
-// block sorts one chunk in LDS with a bitonic network, then merge passes of
-// doubling run width merge neighbouring runs inside each segment.  Per pass,
-// one thread per chunk finds the merge-path split of the chunk's first output
-// (co_rank_kernel), then a merge block owns ENM_SORT_TILE outputs: it stages
+// Algorithm: every segment is cut into tiles of up to ENM_SORT_MAXTILE keys; a
+// block sorts one tile in LDS (networks in registers, then merge levels), then
+// merge passes of doubling run width merge neighbouring runs inside each
+// segment.  Per pass, one thread per chunk of ENM_SORT_TILE keys finds the
+// merge-path split of its first output (co_rank_kernel), then a merge block owns ENM_SORT_TILE outputs: it stages
 // its two input slices in LDS and each thread merges 8 outputs.  Keys compare as
 // (value, index) pairs, so all keys are distinct and the order is total.
 // Traffic per pass is 12 B read + 12 B written per key (HBM-bound).

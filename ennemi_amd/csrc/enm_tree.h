@@ -17,9 +17,9 @@
 // conditional MIs of 1,800 points, kNN 0.110 -> 0.062 ms, counts 0.305 ->
 // 0.05 ms.  The kNN is bound by its instructions (800 vector ones a query in
 // four columns).  The counts were bound by their loads from L2, about 85 of 512
-// bytes a query; four neighbouring queries at once share them (one at a time:
-// 15.3 of the 8.0 ms above; two: 10.5; eight: 9.9, their coordinates no longer
-// fit the scalar registers).
+// bytes a query; four neighbouring queries at once share them (the 8.0 ms above
+// are 15.3 one at a time, 10.5 two, and 9.9 eight, whose coordinates no longer fit
+// the scalar registers).
 //
 // Everything is decided by the reference's own FP64 expressions.  For a box
 // side lo <= a <= hi, fl(a - q) >= fl(lo - q) and fl(q - a) >= fl(q - hi)
