@@ -277,6 +277,8 @@ struct enm_ctx {
         if (stage_done) (void)hipEventDestroy(stage_done);
         if (stage) (void)hipHostFree(stage);
         if (prep.out) (void)hipHostFree(prep.out);
+        if (uq.out) (void)hipHostFree(uq.out);
+        if (group.sizes) (void)hipHostFree(group.sizes);
     }
     Plan* last = nullptr;
     hipStream_t last_stream = nullptr;
@@ -310,11 +312,14 @@ struct enm_ctx {
     } prep;
     // Workspace of enm_group_rows.
     struct Grouping {
-        DevBuf tables, counts, sizes;
+        DevBuf tables, counts;
+        int64_t* sizes = nullptr;   // host memory that the kernels write (n_sizes values)
+        size_t n_sizes = 0;
     } group;
     // Workspace of enm_unique_rows and enm_count_rows.
     struct Unique {
         DevBuf tables, k0, k1, i0, i1, split, heads, ccodes, cstarts, ccounts, cdist, rkeys, rstarts, rdist, hist;
+        UqShort* out = nullptr;   // host memory that a kernel writes
         std::vector<char> blob1, blob2;
     } uq;
     void* scratch = nullptr;          // this device's static workspace
@@ -2373,17 +2378,27 @@ int enm_group_rows(enm_ctx* ctx, const enm_group_task* tasks, int32_t n_tasks, i
     }
     const size_t sizes = (size_t)n_tasks * classes;
     if (G.tables.ensure(dev.size() * sizeof(GroupTaskDev)) != hipSuccess ||
-        G.counts.ensure((size_t)stride * sizes * 4) != hipSuccess || G.sizes.ensure(sizes * 8) != hipSuccess) {
+        G.counts.ensure((size_t)stride * sizes * 4) != hipSuccess) {
         (void)hipGetLastError();
         return fail(ctx, ENM_E_NOMEM, "hipMalloc failed for the class counts");
+    }
+    if (G.n_sizes < sizes) {
+        if (G.sizes) (void)hipHostFree(G.sizes);
+        G.sizes = nullptr;
+        G.n_sizes = 0;
+        void* p = nullptr;
+        e = hipHostMalloc(&p, sizes * 8, hipHostMallocDefault);
+        if (e != hipSuccess) return hip_fail(ctx, e, "hipHostMalloc");
+        G.sizes = static_cast<int64_t*>(p);
+        G.n_sizes = sizes;
     }
     e = hipMemcpyAsync(G.tables.p, dev.data(), dev.size() * sizeof(GroupTaskDev), hipMemcpyHostToDevice, st);
     if (e == hipSuccess)
         e = enm_launch_group(G.tables.as<GroupTaskDev>(), n_tasks, stride, classes, d_src, G.counts.as<int>(),
-                             G.sizes.as<int64_t>(), d_dst, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(h_sizes, G.sizes.p, sizes * 8, hipMemcpyDeviceToHost, st);
+                             G.sizes, d_dst, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(ctx, e, "group rows");
+    std::memcpy(h_sizes, G.sizes, sizes * 8);
     return ENM_OK;
 }
 
@@ -2582,32 +2597,58 @@ int enm_count_rows(enm_ctx* ctx, const enm_rowset* set, const double* d_values, 
     rows.n = set->n;
     rows.ncol = set->ncol;
     for (int c = 0; c < set->ncol; ++c) rows.col[c] = set->col[c];
+    double least[ENM_MAX_COLS], most[ENM_MAX_COLS];
+    bool odd[ENM_MAX_COLS];
+    const bool one = set->n <= ENM_UQ_SHORT;
     const int next = 3 * ENM_MAX_COLS;
+    if (one) {
+        if (!U.out) {
+            void* p = nullptr;
+            e = hipHostMalloc(&p, sizeof(UqShort), hipHostMallocDefault);
+            if (e != hipSuccess) return hip_fail(ctx, e, "hipHostMalloc");
+            U.out = static_cast<UqShort*>(p);
+        }
+        e = enm_launch_uq_short(rows, d_values, (int)cap, U.out, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        if (e != hipSuccess) return hip_fail(ctx, e, "row counts");
+        for (int c = 0; c < set->ncol; ++c) {
+            least[c] = U.out->least[c];
+            most[c] = U.out->most[c];
+            odd[c] = U.out->odd[c] != 0;
+        }
+    }
     if (U.hist.ensure((size_t)next * 8 + (size_t)cap * 4) != hipSuccess) {
         (void)hipGetLastError();
         return fail(ctx, ENM_E_NOMEM, "hipMalloc failed for the row counts");
     }
-    // ext: least, greatest and oddity of every column, then the counts.
+    // least, greatest and oddity of every column, then the counts.
     unsigned long long* ext = U.hist.as<unsigned long long>();
     unsigned* counts = reinterpret_cast<unsigned*>(ext + next);
-    unsigned long long init[3 * ENM_MAX_COLS], got[3 * ENM_MAX_COLS];
-    for (int c = 0; c < ENM_MAX_COLS; ++c) { init[3 * c] = ~0ull; init[3 * c + 1] = init[3 * c + 2] = 0; }
-    e = hipMemcpyAsync(ext, init, sizeof init, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = enm_launch_uq_range(rows, d_values, ext, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(got, ext, sizeof got, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) return hip_fail(ctx, e, "ranges of the columns");
-    auto value = [](unsigned long long m) {
-        const unsigned long long b = m >> 63 ? m & ~(1ull << 63) : ~m;
-        double v;
-        std::memcpy(&v, &b, 8);
-        return v;
-    };
+    if (!one) {
+        unsigned long long init[3 * ENM_MAX_COLS], got[3 * ENM_MAX_COLS];
+        for (int c = 0; c < ENM_MAX_COLS; ++c) { init[3 * c] = ~0ull; init[3 * c + 1] = init[3 * c + 2] = 0; }
+        e = hipMemcpyAsync(ext, init, sizeof init, hipMemcpyHostToDevice, st);
+        if (e == hipSuccess) e = enm_launch_uq_range(rows, d_values, ext, st);
+        if (e == hipSuccess) e = hipMemcpyAsync(got, ext, sizeof got, hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        if (e != hipSuccess) return hip_fail(ctx, e, "ranges of the columns");
+        auto value = [](unsigned long long m) {
+            const unsigned long long b = m >> 63 ? m & ~(1ull << 63) : ~m;
+            double v;
+            std::memcpy(&v, &b, 8);
+            return v;
+        };
+        for (int c = 0; c < set->ncol; ++c) {
+            odd[c] = got[3 * c + 2] != 0;
+            least[c] = value(got[3 * c]);
+            most[c] = value(got[3 * c + 1]);
+        }
+    }
     double keys = 1.0;
     for (int c = 0; c < set->ncol; ++c) {
-        if (got[3 * c + 2]) return fail(ctx, ENM_E_UNSUPPORTED, "a column holds values that are not whole numbers");
-        h_least[c] = value(got[3 * c]);
-        const double range = value(got[3 * c + 1]) - h_least[c] + 1.0;
+        if (odd[c]) return fail(ctx, ENM_E_UNSUPPORTED, "a column holds values that are not whole numbers");
+        h_least[c] = least[c];
+        const double range = most[c] - h_least[c] + 1.0;
         keys *= range;
         if (!(keys <= (double)cap)) return fail(ctx, ENM_E_UNSUPPORTED, "more value combinations than counters");
         h_radix[c] = (int64_t)range;
@@ -2615,6 +2656,10 @@ int enm_count_rows(enm_ctx* ctx, const enm_rowset* set, const double* d_values, 
         rows.radix[c] = (int32_t)range;
     }
     const int nk = (int)keys;
+    if (one && U.out->keys == nk) {
+        std::memcpy(h_counts, U.out->counts, (size_t)nk * 4);
+        return ENM_OK;
+    }
     e = enm_launch_fill_i32(reinterpret_cast<int*>(counts), nk, 0, st);
     if (e == hipSuccess) e = enm_launch_uq_hist(rows, d_values, nk, counts, st);
     if (e == hipSuccess) e = hipMemcpyAsync(h_counts, counts, (size_t)nk * 4, hipMemcpyDeviceToHost, st);

@@ -389,6 +389,16 @@ struct EnmRowsDev {
     int32_t ncol;
 };
 
+// What a short row set's columns and rows came to (enm_unique.hip).
+#define ENM_UQ_SHORT 16384     // rows
+#define UQ_LDS_KEYS 8192       // counters in a workgroup's LDS
+struct UqShort {
+    double least[16], most[16];
+    int32_t odd[16];            // a value is not a whole number below 2^53
+    int32_t keys, pad;
+    uint32_t counts[UQ_LDS_KEYS];
+};
+
 // The mixed-radix keys of a multi-column row set.
 struct UqRowKey {
     int64_t n;

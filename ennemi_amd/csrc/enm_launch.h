@@ -161,6 +161,7 @@ hipError_t enm_launch_group(const GroupTaskDev* tasks, int n_tasks, int64_t stri
 hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, int ntiles, const double* skeys, const int* sidx,
                                int* tile_heads, int* codes, int64_t* starts, int64_t* counts, int64_t* distinct,
                                hipStream_t st);
+hipError_t enm_launch_uq_short(const EnmRowsDev& rows, const double* values, int cap, UqShort* out, hipStream_t st);
 hipError_t enm_launch_uq_range(const EnmRowsDev& rows, const double* values, unsigned long long* ext, hipStream_t st);
 hipError_t enm_launch_uq_hist(const EnmRowsDev& rows, const double* values, int keys, unsigned* counts,
                               hipStream_t st);

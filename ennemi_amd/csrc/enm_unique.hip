@@ -23,7 +23,6 @@ namespace {
 constexpr int UQ_THREADS = 256;
 constexpr int UQ_PER = 8;                       // elements per thread of a tile
 constexpr int UQ_TILE = UQ_THREADS * UQ_PER;    // as the sort's chunks
-constexpr int UQ_LDS_KEYS = 8192;              // counters of a workgroup in LDS
 static_assert(UQ_TILE == ENM_SORT_TILE, "tiles are numbered by the segments' first_tile");
 
 __device__ __forceinline__ int uq_seg(const UqSeg* __restrict__ segs, int nsegs, int tile) {
@@ -214,6 +213,74 @@ void uq_hist_kernel(EnmRowsDev rows, const double* __restrict__ values, int keys
     }
 }
 
+// Both of a short row set by one workgroup, straight to host memory: the columns'
+// extrema, and the counts where the keys fit LDS (out->keys of them; 0: not
+// counted).  A call on a thousand labels then waits once for one kernel (9 us),
+// where clearing, two kernels and two read-backs took 69 us of it.
+constexpr int UQ_SHORT_THREADS = 1024;
+__global__ __launch_bounds__(UQ_SHORT_THREADS)
+void uq_short_kernel(EnmRowsDev rows, const double* __restrict__ values, int cap, UqShort* __restrict__ out) {
+    constexpr int NW = UQ_SHORT_THREADS / ENM_WAVE;
+    __shared__ unsigned s_counts[UQ_LDS_KEYS];
+    __shared__ double s_lo[NW], s_hi[NW], s_least[16];
+    __shared__ int s_odd[NW], s_radix[16];
+    __shared__ double s_keys;
+    const int n = (int)rows.n, tid = (int)threadIdx.x, wv = tid / ENM_WAVE;
+    if (tid == 0) s_keys = 1.0;
+    for (int c = 0; c < rows.ncol; ++c) {
+        const double* v = values + rows.col[c];
+        double lo = INFINITY, hi = -INFINITY;
+        bool odd = false;
+        for (int i = tid; i < n; i += UQ_SHORT_THREADS) {
+            const double x = v[i] + 0.0;   // (-0.0 is 0.0)
+            odd = odd || !(fabs(x) < 9007199254740992.0 && x == floor(x));
+            lo = fmin(lo, x);
+            hi = fmax(hi, x);
+        }
+        for (int off = 32; off > 0; off >>= 1) {
+            lo = fmin(lo, __shfl_xor(lo, off, ENM_WAVE));
+            hi = fmax(hi, __shfl_xor(hi, off, ENM_WAVE));
+        }
+        const bool any = wave_any(odd);
+        __syncthreads();
+        if ((tid & (ENM_WAVE - 1)) == 0) {
+            s_lo[wv] = lo;
+            s_hi[wv] = hi;
+            s_odd[wv] = any ? 1 : 0;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            for (int w = 1; w < NW; ++w) {
+                lo = fmin(lo, s_lo[w]);
+                hi = fmax(hi, s_hi[w]);
+                s_odd[0] |= s_odd[w];
+            }
+            lo = fmin(lo, s_lo[0]);
+            hi = fmax(hi, s_hi[0]);
+            out->least[c] = lo;
+            out->most[c] = hi;
+            out->odd[c] = s_odd[0];
+            const double range = s_odd[0] ? INFINITY : hi - lo + 1.0;
+            s_keys *= range;
+            s_least[c] = lo;
+            s_radix[c] = range <= UQ_LDS_KEYS ? (int)range : 0;
+        }
+    }
+    __syncthreads();
+    const int keys = s_keys <= (double)min(cap, UQ_LDS_KEYS) ? (int)s_keys : 0;
+    if (tid == 0) out->keys = keys;
+    if (keys == 0) return;
+    for (int k = tid; k < keys; k += UQ_SHORT_THREADS) s_counts[k] = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += UQ_SHORT_THREADS) {
+        int key = 0;
+        for (int c = 0; c < rows.ncol; ++c) key = key * s_radix[c] + (int)(values[rows.col[c] + i] - s_least[c]);
+        atomicAdd(s_counts + key, 1u);
+    }
+    __syncthreads();
+    for (int k = tid; k < keys; k += UQ_SHORT_THREADS) out->counts[k] = s_counts[k];
+}
+
 // Mixed-radix keys of the rows of multi-column row sets (exact doubles).
 __global__ void uq_key_kernel(const UqRowKey* __restrict__ rk, int n_rk, const int* __restrict__ ccodes,
                               double* __restrict__ keys) {
@@ -238,6 +305,11 @@ hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, int ntiles, const d
     hipLaunchKernelGGL(uq_codes_kernel, dim3(ntiles), dim3(UQ_THREADS), 0, st, segs, nsegs, skeys, sidx, tile_heads,
                        codes, starts);
     hipLaunchKernelGGL(uq_counts_kernel, dim3(ntiles), dim3(UQ_THREADS), 0, st, segs, nsegs, starts, distinct, counts);
+    return hipGetLastError();
+}
+
+hipError_t enm_launch_uq_short(const EnmRowsDev& rows, const double* values, int cap, UqShort* out, hipStream_t st) {
+    hipLaunchKernelGGL(uq_short_kernel, dim3(1), dim3(UQ_SHORT_THREADS), 0, st, rows, values, cap, out);
     return hipGetLastError();
 }
 

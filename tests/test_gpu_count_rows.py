@@ -1,6 +1,7 @@
 """Distinct rows counted directly (whole numbers in small ranges) and by
 sorting: both ways must give np.unique's rows and counts, at the edges of the
-counters (in LDS up to 8,192 keys, at most 65,536) and of the sort tiles."""
+counters (in LDS up to 8,192 keys, at most 65,536), of the row sets that one
+workgroup counts (16,384) and of the sort tiles."""
 
 import numpy as np
 import pytest
@@ -34,7 +35,7 @@ def _check(cols):
     return got is not None
 
 
-@pytest.mark.parametrize("n", [1, 2, 255, 2047, 2048, 2049, 40_001])
+@pytest.mark.parametrize("n", [1, 2, 255, 1023, 1025, 2047, 2048, 2049, 16_384, 16_385, 40_001])
 @pytest.mark.parametrize("radix,direct", [((1,), True), ((2, 3), True), ((64, 128), True), ((64, 129), True),
                                           ((256, 256), True), ((256, 257), False), ((4, 5, 6, 7), True)])
 def test_ranges(n, radix, direct):
