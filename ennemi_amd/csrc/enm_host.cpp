@@ -2156,8 +2156,8 @@ int enm_prep_write(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks, co
                       (long long)noise_len, (long long)need_noise);
         return fail(ctx, ENM_E_ARG, msg);
     }
-    // Chunks listed full ones first (8192 values: one wave each, four to a
-    // block), then the last chunk of each array.
+    // Chunks listed full ones first (8192 values), then the last chunk of each
+    // array, which takes longer to cut up: waves of a block have like work.
     std::vector<int> chunk_list;
     chunk_list.reserve(chunk_sum_of.size());
     for (int pass = 0; pass < 2; ++pass)
@@ -2165,9 +2165,6 @@ int enm_prep_write(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks, co
             const bool full = ((int64_t)chunk_index[c] + 1) * 8192 <= sums[chunk_sum_of[c]].n;
             if (full == (pass == 0)) chunk_list.push_back((int)c);
         }
-    int n_full = 0;
-    for (size_t c = 0; c < chunk_sum_of.size(); ++c)
-        n_full += ((int64_t)chunk_index[c] + 1) * 8192 <= sums[chunk_sum_of[c]].n ? 1 : 0;
     S.blob2.clear();
     const size_t o_t = append(S.blob2, S.tasks);
     const size_t o_s = append(S.blob2, sums);
@@ -2193,7 +2190,7 @@ int enm_prep_write(enm_ctx* ctx, const enm_prep_task* tasks, int32_t n_tasks, co
                               S.drop_nan ? 1 : 0, rescale ? 1 : 0, S.blk_off.as<int64_t>(),
                               reinterpret_cast<const PrepSumDev*>(base + o_s), (int)sums.size(),
                               reinterpret_cast<const int*>(base + o_cs), reinterpret_cast<const int*>(base + o_ci),
-                              reinterpret_cast<const int*>(base + o_cl), (int)chunk_sum_of.size(), n_full,
+                              reinterpret_cast<const int*>(base + o_cl), (int)chunk_sum_of.size(),
                               S.chunk_val.as<double>(), reinterpret_cast<const int*>(base + o_sq),
                               rescale ? (int)seq_sum_of.size() : 0, S.seq_val.as<double>(),
                               S.seq_tiles.as<PrepSeqTile>(), S.stats.as<double>(), sstride,

@@ -127,7 +127,7 @@ hipError_t enm_launch_prep_write(PrepTaskDev* tasks, int64_t stride, int n_tasks
                                  const double* raw, const unsigned char* mask, int drop_nan, int rescale,
                                  const int64_t* blk_off, const PrepSumDev* sums, int n_sums,
                                  const int* chunk_sum_of, const int* chunk_index, const int* chunk_list,
-                                 int n_chunks, int n_full, double* chunk_val, const int* seq_sum_of, int n_seq,
+                                 int n_chunks, double* chunk_val, const int* seq_sum_of, int n_seq,
                                  double* seq_val, PrepSeqTile* seq_tiles, double* stats, int64_t sstride,
                                  const double* noise, unsigned raw_vars, unsigned* const_flag, double* arena,
                                  KeptWord* kept, hipStream_t st);

@@ -311,8 +311,9 @@ __device__ __forceinline__ void wave_sync() {
 // wave builds the recursion's tree in LDS level by level (slot lengths; -1 for no
 // node), sums its leaves, eight lanes to a leaf, and adds every node's two halves
 // bottom-up, left + right, as NumPy does.
+template <bool FULL>   // whether m may be PW_CHUNK
 __device__ double pw_chunk(const Term& f, int m, PwTree& L) {
-    if (m == PW_CHUNK) return pw_full_chunk(f);
+    if (FULL && m == PW_CHUNK) return pw_full_chunk(f);
     const int lane = (int)threadIdx.x & (ENM_WAVE - 1);
     // The tree, top-down: slot 1 is the whole chunk; a slot's halves exist
     // when it has more than PW_LEAF values.
@@ -389,37 +390,22 @@ __device__ double pw_chunk(const Term& f, int m, PwTree& L) {
     return L.val[1];
 }
 
-// Phase 2b: the last chunk of every array, one wave each.
-__global__ __launch_bounds__(ENM_WAVE)
+// Phase 2b: one wave per chunk of every array, four waves per block (no barriers:
+// each wave sums its own chunk).
+__global__ __launch_bounds__(4 * ENM_WAVE)
 void prep_chunk_kernel(const PrepSumDev* __restrict__ sums, const int* __restrict__ chunk_sum_of,
                        const int* __restrict__ chunk_index, const int* __restrict__ list, int n_list,
                        const double* __restrict__ arena, const double* __restrict__ stats, int pass,
                        double* __restrict__ chunk_val) {
-    __shared__ PwTree s_tree;
-    if ((int)blockIdx.x >= n_list) return;
-    const int c = list[blockIdx.x];
-    const PrepSumDev& sd = sums[chunk_sum_of[c]];
-    const int64_t first = (int64_t)chunk_index[c] * PW_CHUNK;
-    const int m = (int)min((int64_t)PW_CHUNK, sd.n - first);
-    const Term f{arena + sd.src + first, pass ? stats[sd.stat] : 0.0, pass != 0};
-    const double sum = pw_chunk(f, m, s_tree);
-    if (threadIdx.x == 0) chunk_val[c] = sum;
-}
-
-// Full chunks only, one per wave, four waves per block (no barriers: each
-// wave sums its own chunk).
-__global__ __launch_bounds__(4 * ENM_WAVE)
-void prep_full_chunk_kernel(const PrepSumDev* __restrict__ sums, const int* __restrict__ chunk_sum_of,
-                            const int* __restrict__ chunk_index, const int* __restrict__ list, int n_list,
-                            const double* __restrict__ arena, const double* __restrict__ stats, int pass,
-                            double* __restrict__ chunk_val) {
-    const int idx = (int)blockIdx.x * 4 + (int)(threadIdx.x / ENM_WAVE);
+    __shared__ PwTree s_tree[4];
+    const int wave = (int)(threadIdx.x / ENM_WAVE), idx = (int)blockIdx.x * 4 + wave;
     if (idx >= n_list) return;
     const int c = list[idx];
     const PrepSumDev& sd = sums[chunk_sum_of[c]];
     const int64_t first = (int64_t)chunk_index[c] * PW_CHUNK;
+    const int m = (int)min((int64_t)PW_CHUNK, sd.n - first);
     const Term f{arena + sd.src + first, pass ? stats[sd.stat] : 0.0, pass != 0};
-    const double sum = pw_full_chunk(f);
+    const double sum = pw_chunk<true>(f, m, s_tree[wave]);
     if ((threadIdx.x & (ENM_WAVE - 1)) == 0) chunk_val[c] = sum;
 }
 
@@ -883,7 +869,7 @@ void prep_short_kernel(PrepTaskDev* tasks, const double* __restrict__ raw, const
         double mean = 0.0;
         for (int pass = 0; pass < 2; ++pass) {
             const double sum = a >= 2 && t.dz >= 2 ? seq_chain(v, t.n, mean, pass)
-                                                   : -0.0 + pw_chunk(Term{v, mean, pass != 0}, (int)t.n, s_tree[wave]);
+                                                   : -0.0 + pw_chunk<false>(Term{v, mean, pass != 0}, (int)t.n, s_tree[wave]);
             const double q = sum / (double)t.n;
             if (pass == 0) mean = q;
             if (lane == 0) stats[t.stat + 2 * a + pass] = pass ? sqrt(q) : q;
@@ -923,12 +909,13 @@ hipError_t enm_launch_prep_write(PrepTaskDev* tasks, int64_t stride, int n_tasks
                                  const double* raw, const unsigned char* mask, int drop_nan, int rescale,
                                  const int64_t* blk_off, const PrepSumDev* sums, int n_sums,
                                  const int* chunk_sum_of, const int* chunk_index, const int* chunk_list,
-                                 int n_chunks, int n_full, double* chunk_val, const int* seq_sum_of, int n_seq,
+                                 int n_chunks, double* chunk_val, const int* seq_sum_of, int n_seq,
                                  double* seq_val, PrepSeqTile* seq_tiles, double* stats, int64_t sstride,
                                  const double* noise, unsigned raw_vars, unsigned* const_flag, double* arena,
                                  KeptWord* kept, hipStream_t st) {
     if (n_tasks <= 0) return hipSuccess;
     const int64_t n_blocks = stride * n_tasks, n_sblocks = sstride * n_tasks;
+    static_assert(ENM_PREP_SHORT < PW_CHUNK, "a short task's sums are of less than a chunk");
     const bool short_tasks = rescale && sstride * PB_THREADS <= ENM_PREP_SHORT;
     const bool whole = short_tasks && stride == 1;
     if (n_blocks > 0 && !whole)
@@ -940,15 +927,9 @@ hipError_t enm_launch_prep_write(PrepTaskDev* tasks, int64_t stride, int n_tasks
     if (!rescale || short_tasks) return hipGetLastError();
     for (int pass = 0; pass < 2; ++pass) {
         if (n_chunks > 0) {
-            // Full chunks four to a block; the other (last) chunks one each.
-            if (n_full > 0)
-                hipLaunchKernelGGL(prep_full_chunk_kernel, dim3((unsigned)((n_full + 3) / 4)), dim3(4 * ENM_WAVE), 0,
-                                   st, sums, chunk_sum_of, chunk_index, chunk_list, n_full, arena, stats, pass,
-                                   chunk_val);
-            if (n_chunks > n_full)
-                hipLaunchKernelGGL(prep_chunk_kernel, dim3((unsigned)(n_chunks - n_full)), dim3(ENM_WAVE), 0, st,
-                                   sums, chunk_sum_of, chunk_index, chunk_list + n_full, n_chunks - n_full, arena,
-                                   stats, pass, chunk_val);
+            hipLaunchKernelGGL(prep_chunk_kernel, dim3((unsigned)((n_chunks + 3) / 4)), dim3(4 * ENM_WAVE), 0, st,
+                               sums, chunk_sum_of, chunk_index, chunk_list, n_chunks, arena, stats, pass,
+                               chunk_val);
         }
         if (n_seq > 0) {
             hipLaunchKernelGGL(prep_seq_block_kernel, dim3((unsigned)n_seq), dim3(SEQ_THREADS), 0, st, sums,
