@@ -2445,6 +2445,7 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
             u.count_off = tot1;
             u.slot = id;
             u.first_tile = sg.first_tile;
+            u.src = sg.src;
             segs1.push_back(sg);
             useg1.push_back(u);
             tot1 += R.n;
@@ -2477,6 +2478,10 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
     e = enm_launch_sort(reinterpret_cast<const SortSeg*>(U.tables.as<char>() + o_s1), ncols, tiles1, maxlen1,
                         d_values, nullptr, U.k0.as<double>(), U.i0.as<int>(), U.k1.as<double>(),
                         U.i1.as<int>(), U.split.as<int>(), &fb, &nl, st);
+    if (e == hipSuccess)
+        e = enm_launch_uq_nan(reinterpret_cast<const UqSeg*>(U.tables.as<char>() + o_u1), ncols, d_values,
+                              fb ? U.k1.as<double>() : U.k0.as<double>(), fb ? U.i1.as<int>() : U.i0.as<int>(),
+                              fb ? U.i0.as<int>() : U.i1.as<int>(), st);
     if (e == hipSuccess)
         e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(U.tables.as<char>() + o_u1), ncols, tiles1,
                                 fb ? U.k1.as<double>() : U.k0.as<double>(), fb ? U.i1.as<int>() : U.i0.as<int>(),

@@ -377,6 +377,7 @@ struct UqSeg {
     int64_t count_off;  // points per code
     int32_t slot;       // its distinct-count slot
     int32_t first_tile; // index of its first ENM_SORT_TILE positions
+    int64_t src;        // offset of the values that were sorted
 };
 
 // A row set of whole numbers (enm_count_rows): its columns, their least

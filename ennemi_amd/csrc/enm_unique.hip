@@ -6,9 +6,10 @@
 // A row set is one or more float64 columns of n values.  Each distinct
 // column is sorted once (the library's segmented merge sort, keys compared
 // as doubles and ties by point index, so -0.0 and 0.0 are one value, as for
-// np.unique); a run head is a position whose key differs from the previous
-// one, and a value's code is the number of run heads up to it, minus one:
-// codes number the distinct values in increasing order.  A row set of
+// np.unique, and every NaN is a value of its own after the others); a run head
+// is a position whose key differs from the previous one, and a value's code is
+// the number of run heads up to it, minus one: codes number the distinct values
+// in increasing order.  A row set of
 // several columns is keyed by the mixed-radix number of its columns' codes
 // (column 0 most significant: the order of np.unique's lexicographic row
 // sort), exact in float64 while the product of the columns' distinct counts
@@ -45,6 +46,57 @@ __device__ __forceinline__ int uq_heads(const UqSeg& sg, const double* __restric
         heads += h[j];
     }
     return heads;
+}
+
+// The sort holds NaN as +inf, in point order among the infinities.  np.unique
+// puts NaN last and keeps every one apart: the points of the last run are laid
+// out again, infinities first, and the keys of the others become NaN, which
+// differ from whatever stands before them.  One workgroup per segment; next to
+// nothing where the greatest key is finite.
+constexpr int UQ_NAN_THREADS = 1024;
+__global__ __launch_bounds__(UQ_NAN_THREADS)
+void uq_nan_kernel(const UqSeg* __restrict__ segs, const double* __restrict__ values, double* __restrict__ skeys,
+                   int* __restrict__ sidx, int* __restrict__ tmp) {
+    constexpr int NW = UQ_NAN_THREADS / ENM_WAVE;
+    __shared__ int s_inf[NW];
+    const UqSeg sg = segs[blockIdx.x];
+    skeys += sg.sbase;
+    sidx += sg.sbase;
+    tmp += sg.sbase;
+    if (skeys[sg.n - 1] < INFINITY) return;
+    int64_t lo = 0, hi = sg.n - 1;   // the first infinite key
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (skeys[mid] < INFINITY) lo = mid + 1; else hi = mid;
+    }
+    const int lane = threadIdx.x & (ENM_WAVE - 1), wv = threadIdx.x / ENM_WAVE;
+    // Real infinities, then, given their number, every point's place.
+    int64_t infinities = 0;
+    for (int place = 0; place < 2; ++place) {
+        int64_t before = 0;   // infinities among the positions done
+        for (int64_t base = lo; base < sg.n; base += UQ_NAN_THREADS) {
+            const int64_t i = base + threadIdx.x;
+            const int pt = i < sg.n ? sidx[i] : 0;
+            const bool real = i < sg.n && values[sg.src + pt] == INFINITY;
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(real);
+            __syncthreads();   // the counts of the round before are read
+            if (lane == 0) s_inf[wv] = (int)__popcll(m);
+            __syncthreads();
+            int64_t mine = before + (int)__popcll(m & ((1ull << lane) - 1ull));
+            for (int w = 0; w < NW; ++w) {
+                mine += w < wv ? s_inf[w] : 0;
+                before += s_inf[w];
+            }
+            if (place && i < sg.n) tmp[real ? lo + mine : lo + infinities + (i - lo - mine)] = pt;
+        }
+        infinities = before;
+        if (infinities == sg.n - lo) return;   // no NaN
+    }
+    __syncthreads();
+    for (int64_t i = lo + threadIdx.x; i < sg.n; i += UQ_NAN_THREADS) {
+        sidx[i] = tmp[i];
+        if (i >= lo + infinities) skeys[i] = __builtin_nan("");
+    }
 }
 
 // Three passes over tiles of 2,048 sorted positions (one workgroup per segment
@@ -295,6 +347,13 @@ __global__ void uq_key_kernel(const UqRowKey* __restrict__ rk, int n_rk, const i
 }
 
 }  // namespace
+
+hipError_t enm_launch_uq_nan(const UqSeg* segs, int nsegs, const double* values, double* skeys, int* sidx, int* tmp,
+                             hipStream_t st) {
+    if (nsegs <= 0) return hipSuccess;
+    hipLaunchKernelGGL(uq_nan_kernel, dim3(nsegs), dim3(UQ_NAN_THREADS), 0, st, segs, values, skeys, sidx, tmp);
+    return hipGetLastError();
+}
 
 hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, int ntiles, const double* skeys, const int* sidx,
                                int* tile_heads, int* codes, int64_t* starts, int64_t* counts, int64_t* distinct,

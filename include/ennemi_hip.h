@@ -330,9 +330,10 @@ int enm_group_rows(enm_ctx* ctx, const enm_group_task* tasks, int32_t n_tasks, i
  *   _estimate_conditional_discrete_mi      ennemi/_entropy_estimators.py:291-320
  *
  * A row set is ncol float64 columns of n values in d_values (numeric data;
- * -0.0 and 0.0 are one value; no NaN).  Its rows are numbered by their
- * place among the distinct rows in lexicographic order (column 0 first):
- * for row set s, placed at o_s = n_0 + ... + n_{s-1},
+ * -0.0 and 0.0 are one value; every NaN is a value of its own, above +inf, in
+ * point order).  Its rows are numbered by their place among the distinct rows
+ * in lexicographic order (column 0 first): for row set s, placed at o_s =
+ * n_0 + ... + n_{s-1},
  *   d_codes[o_s + p]   the number of point p's distinct row (int32),
  *   d_counts[o_s + r]  the points of distinct row r (int64, r < h_distinct[s]).
  * Synchronous.  ENM_E_UNSUPPORTED when the product of the distinct counts
