@@ -222,7 +222,8 @@ struct Plan {
     int64_t far_bytes = 0;    // far list of the strip kNN (queries reaching past the staged strips)
     DevBuf tables;
     Work* work = nullptr;
-    std::unique_ptr<Work> own_work;   // the static workspace's
+    std::unique_ptr<Work> own_work;   // the static workspace's, or for graphs that callers capture
+    const Work* ran = nullptr;        // of the last enqueue
     std::vector<size_t> need;         // bytes of each workspace buffer
     size_t off_segs = 0, off_gitems = 0, off_orders = 0, off_kdescs = 0, off_cdescs = 0, off_insts = 0,
            off_cls = 0, off_kitems = 0, off_citems = 0, off_trees = 0, off_rdescs = 0,
@@ -282,6 +283,7 @@ struct enm_ctx {
     }
     Plan* last = nullptr;
     hipStream_t last_stream = nullptr;
+    hipStream_t stats_stream = nullptr;   // last_stream, or the one of a caller's capture since
     // Device-side task preparation: the state enm_prep_count leaves for
     // enm_prep_write, and their workspace.
     struct Prep {
@@ -1472,6 +1474,7 @@ const T* tab(const Plan& P, size_t off) {
 int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double* out, double* d_eps, int* d_counts,
             hipStream_t st, bool timing) {
     Work& W = *P.work;
+    P.ran = P.work;
     hipError_t e;
     int nl = 0;
     auto chk = [&](hipError_t er, const char* what) -> int {
@@ -1727,6 +1730,30 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
     return ENM_OK;
 }
 
+// Whether `st` is being captured by the caller.
+bool under_capture(hipStream_t st) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    return st != nullptr && hipStreamIsCapturing(st, &c) == hipSuccess && c == hipStreamCaptureStatusActive;
+}
+
+// A run recorded into the caller's own graph.  It is replayed without this
+// library's knowledge, so its plan gets a workspace of its own, which no other
+// run moves or writes and which lives as long as the plan.
+int record(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double* out, double* d_eps, int* d_counts,
+           hipStream_t st) {
+    if (!P.own_work) P.own_work.reset(new Work());
+    // (Allocations are no part of the capture.)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return hip_fail(ctx, e, "hipThreadExchangeStreamCaptureMode");
+    P.work = P.own_work.get();
+    int rc = ensure_workspace(ctx, P);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!rc) rc = enqueue(ctx, P, arena, hint, out, d_eps, d_counts, st, false);
+    P.work = &ctx->work;
+    return rc;
+}
+
 // Plans are cached by the shape of the call: the instances (column offsets,
 // not the arena's address), class sizes, flags, which exports are asked for
 // and the tuning.  Device pointers are kernel arguments of every enqueue, so
@@ -1826,12 +1853,17 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
     hipStream_t st = (hipStream_t)stream;
-    if (ctx->last_stream != st && ctx->last_stream != nullptr) {
-        // Plans reuse their workspace; finish work queued on another stream first.
-        e = hipStreamSynchronize(ctx->last_stream);
-        if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
+    const bool captured = under_capture(st);
+    if (captured && (flags & ENM_F_GRAPH)) return fail(ctx, ENM_E_ARG, "ENM_F_GRAPH on a stream under capture");
+    ctx->stats_stream = st;
+    if (!captured) {
+        if (ctx->last_stream != st && ctx->last_stream != nullptr) {
+            // Plans reuse their workspace; finish work queued on another stream first.
+            e = hipStreamSynchronize(ctx->last_stream);
+            if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
+        }
+        ctx->last_stream = st;
     }
-    ctx->last_stream = st;
     const bool use_graph = (flags & ENM_F_GRAPH) != 0;
     const bool timing = (flags & ENM_F_TIMING) != 0;
     const std::string key = plan_key(inst, n_inst, seg_len, d_eps != nullptr, d_counts != nullptr,
@@ -1863,6 +1895,7 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
             if (it != ctx->cache.begin()) ctx->cache.splice(ctx->cache.begin(), ctx->cache, it);
             ctx->last = P;
             P->timing = false;
+            if (captured) return record(ctx, *P, d_arena, d_hint, d_out, d_eps, d_counts, st);
             const int r = ensure_workspace(ctx, *P);
             if (r) return r;
             if (use_graph) {
@@ -1870,6 +1903,7 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
                     e = hipGraphLaunch(P->graph, st);
                     if (e != hipSuccess) return hip_fail(ctx, e, "hipGraphLaunch");
                     P->n_launch = 0;
+                    P->ran = P->work;
                     return ENM_OK;
                 }
                 return capture_and_launch(*P);
@@ -1877,6 +1911,7 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
             return enqueue(ctx, *P, d_arena, d_hint, d_out, d_eps, d_counts, st, timing);
         }
     }
+    if (captured) return fail(ctx, ENM_E_ARG, "a batch is captured only after one of its shape has run");
     std::unique_ptr<Plan> up(new Plan());
     Plan& P = *up;
     P.key = key;
@@ -1946,7 +1981,7 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
         e = hipStreamSynchronize(ctx->last_stream);
         if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
     }
-    ctx->last_stream = st;
+    ctx->last_stream = ctx->stats_stream = st;
     auto rounded = [](size_t b) { return (std::max<size_t>(b, 256) + 255) & ~(size_t)255; };
     std::unique_ptr<Plan> up;
     std::vector<TablePiece> pieces;
@@ -2674,10 +2709,10 @@ int enm_get_stats(enm_ctx* ctx, enm_stats* out) {
     if (!ctx || !out) return ENM_E_ARG;
     std::memset(out, 0, sizeof(*out));
     if (!ctx->last) return fail(ctx, ENM_E_ARG, "no batch has run");
-    hipError_t e = hipStreamSynchronize(ctx->last_stream);
+    hipError_t e = hipStreamSynchronize(ctx->stats_stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
     std::vector<unsigned long long> parts(ENM_ST_SLOTS);
-    e = hipMemcpy(parts.data(), ctx->last->work->stats.p, ENM_ST_SLOTS * 8, hipMemcpyDeviceToHost);
+    e = hipMemcpy(parts.data(), ctx->last->ran->stats.p, ENM_ST_SLOTS * 8, hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipMemcpy(stats)");
     unsigned long long h[ST_N] = {};
     for (int s = 0; s < ST_N; ++s)

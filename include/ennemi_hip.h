@@ -136,7 +136,11 @@ const char* enm_last_error(const enm_ctx* ctx);
  *              instance (spaces x,y for KSG; xz,yz,z for CMI/CROSS; x for
  *              ROSS; unused slots are 0).
  * `stream` is a hipStream_t (NULL = the legacy default stream); all work is
- * enqueued on it and the call returns without synchronising.
+ * enqueued on it and the call returns without synchronising.  On a stream that
+ * the caller captures into a graph of its own, a batch of a shape that has run
+ * before is recorded, with device buffers of its own; they live until the
+ * context has run four other shapes.  (ENM_E_ARG for other shapes and with
+ * ENM_F_GRAPH; no stage times.)
  */
 int enm_run_batch(enm_ctx* ctx,
                   const enm_instance* inst, int32_t n_inst,
