@@ -282,7 +282,8 @@ struct enm_ctx {
         if (group.sizes) (void)hipHostFree(group.sizes);
     }
     Plan* last = nullptr;
-    hipStream_t last_stream = nullptr;
+    bool queued = false;                  // a run has been queued, on last_stream
+    hipStream_t last_stream = nullptr;    // (NULL: the default stream)
     hipStream_t stats_stream = nullptr;   // last_stream, or the one of a caller's capture since
     // Device-side task preparation: the state enm_prep_count leaves for
     // enm_prep_write, and their workspace.
@@ -1730,6 +1731,18 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
     return ENM_OK;
 }
 
+// Before a run on `st`: plans share their workspace, so the last run, if it was
+// queued on another stream, ends first.
+int take_stream(enm_ctx* ctx, hipStream_t st) {
+    if (ctx->queued && ctx->last_stream != st) {
+        const hipError_t e = hipStreamSynchronize(ctx->last_stream);
+        if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
+    }
+    ctx->queued = true;
+    ctx->last_stream = ctx->stats_stream = st;
+    return ENM_OK;
+}
+
 // Whether `st` is being captured by the caller.
 bool under_capture(hipStream_t st) {
     hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
@@ -1856,14 +1869,8 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     const bool captured = under_capture(st);
     if (captured && (flags & ENM_F_GRAPH)) return fail(ctx, ENM_E_ARG, "ENM_F_GRAPH on a stream under capture");
     ctx->stats_stream = st;
-    if (!captured) {
-        if (ctx->last_stream != st && ctx->last_stream != nullptr) {
-            // Plans reuse their workspace; finish work queued on another stream first.
-            e = hipStreamSynchronize(ctx->last_stream);
-            if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
-        }
-        ctx->last_stream = st;
-    }
+    int rc = captured ? ENM_OK : take_stream(ctx, st);
+    if (rc) return rc;
     const bool use_graph = (flags & ENM_F_GRAPH) != 0;
     const bool timing = (flags & ENM_F_TIMING) != 0;
     const std::string key = plan_key(inst, n_inst, seg_len, d_eps != nullptr, d_counts != nullptr,
@@ -1922,7 +1929,7 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     P.want_eps = d_eps != nullptr;
     P.hinted = d_hint != nullptr;
     P.work = &ctx->work;
-    int rc = plan_batch(ctx, P, inst, n_inst, seg_len);
+    rc = plan_batch(ctx, P, inst, n_inst, seg_len);
     if (rc) return rc;
     // Plans past the newest few leave (their runs may still be queued, and one
     // set of tables is kept for the next plan).
@@ -1977,11 +1984,8 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
     hipStream_t st = (hipStream_t)stream;
-    if (ctx->last_stream != st && ctx->last_stream != nullptr) {
-        e = hipStreamSynchronize(ctx->last_stream);
-        if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
-    }
-    ctx->last_stream = ctx->stats_stream = st;
+    int rc = take_stream(ctx, st);
+    if (rc) return rc;
     auto rounded = [](size_t b) { return (std::max<size_t>(b, 256) + 255) & ~(size_t)255; };
     std::unique_ptr<Plan> up;
     std::vector<TablePiece> pieces;
@@ -1998,7 +2002,7 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
         P.want_eps = d_eps != nullptr;
         P.compact = true;
         P.plain = plain != 0;
-        int rc = plan_batch(ctx, P, inst, n_inst, seg_len);
+        rc = plan_batch(ctx, P, inst, n_inst, seg_len);
         if (rc) return rc;
         P.own_work.reset(new Work());
         P.work = P.own_work.get();
@@ -2031,7 +2035,7 @@ int enm_run_batch_static(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     if (e != hipSuccess) return hip_fail(ctx, e, "hipMemcpyAsync(tables)");
     e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
-    const int rc = enqueue(ctx, P, d_arena, nullptr, d_out, d_eps, d_counts, st, false);
+    rc = enqueue(ctx, P, d_arena, nullptr, d_out, d_eps, d_counts, st, false);
     if (rc) return rc;
     ctx->static_plan = std::move(up);
     ctx->last = ctx->static_plan.get();
