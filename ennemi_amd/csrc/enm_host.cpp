@@ -726,11 +726,11 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
     auto route = [&](int cols, int k, int64_t n, const enm_tuning& T) {
         if (P.brute) return ENM_WALK_NONE;
         if (cols < 2) return ENM_WALK_LINE;
-        if (T.strip_points <= 0 || (P.plain && (cols > 2 || k + 1 > 32))) return ENM_WALK_NONE;
-        if (cols == 2 && k + 1 <= 32 && T.strip_points <= ENM_STRIP_LDS_MAX &&
-            (P.plain || (P.per_instance ? n : points2) > tree_points(k + 1, n)))
-            return ENM_WALK_STRIP;
-        return ENM_WALK_TREE;
+        if (T.strip_points <= 0) return ENM_WALK_NONE;
+        const bool strips = cols == 2 && k + 1 <= 32 && T.strip_points <= ENM_STRIP_LDS_MAX;
+        // (A plain plan has no trees: its count spaces count on having order A.)
+        if (P.plain) return strips ? ENM_WALK_STRIP : ENM_WALK_NONE;
+        return strips && (P.per_instance ? n : points2) > tree_points(k + 1, n) ? ENM_WALK_STRIP : ENM_WALK_TREE;
     };
     int max_strip = 0;
     for (int ii = 0; ii < n_inst; ++ii) {
@@ -892,6 +892,7 @@ int plan_batch(enm_ctx* ctx, Plan& P, const enm_instance* inst, int n_inst, cons
                 sp.order = pl.order(ii, c, seg);
                 sp.ocols = sp.cols[0] == 0 ? sp.cols : iota(0, (int)sp.cols.size());
             }
+            if (sp.order < 0) return bad("no order to count a space on");
         }
         // The radius in kNN order is kept for spaces on that order and for
         // the export; other spaces read it through the point numbering.
