@@ -252,14 +252,66 @@ class ArenaBatch:
 # caller's own program keeps all processors busy (NumPy's threads spin on after a
 # matrix product), one that waits for helpers, woken or new, waited 4 ms for them.
 _PIECE = 1 << 18
+# Pieces in use at a time: pinned memory is kept for later calls, so it is bounded
+# whatever the columns take.
+_PIECES = 4
 # Up to so many values go up in one copy, as columns: the host lays out 16,384 in
 # 20 us, what two more copies and the kernel that turns rows into columns take.
 _SHORT = 1 << 14
 
 
+class _Pieces:
+    """Pinned memory in a few pieces, each filled again once its last copy has ended."""
+
+    def __init__(self, total: int, stream) -> None:
+        import torch
+        self.size = min(_PIECE, total)
+        self.memory = torch.empty((min(_PIECES, -(-total // self.size)), self.size), dtype=torch.float64,
+                                  pin_memory=True)
+        self.sent = [None] * len(self.memory)
+        self.at = -1
+        self.stream = stream
+
+    def send(self, parts, dst) -> None:
+        """The values of parts (1-D, or rows of a table), one after the other, to dst."""
+        import torch
+        piece, host, fill, done = None, None, 0, 0
+
+        def flush():
+            nonlocal piece, done
+            dst[done:done + fill].copy_(piece[:fill], non_blocking=True)
+            if self.sent[self.at] is None:
+                self.sent[self.at] = torch.cuda.Event()
+            self.sent[self.at].record(self.stream)
+            done += fill
+            piece = None
+
+        for a in parts:
+            if a.ndim > 1 and (a.flags.c_contiguous or a.shape[1] > self.size):
+                a = np.ascontiguousarray(a).reshape(-1)
+            width = 1 if a.ndim == 1 else a.shape[1]
+            k = 0
+            while k < len(a):
+                if piece is None:
+                    self.at = (self.at + 1) % len(self.memory)
+                    if self.sent[self.at] is not None:
+                        self.sent[self.at].synchronize()
+                    piece, fill = self.memory[self.at].view(dst.dtype), 0
+                    host = piece.numpy()
+                rows = min(len(a) - k, (self.size - fill) // width)
+                if rows > 0:
+                    host[fill:fill + rows * width].reshape(a[k:k + rows].shape)[...] = a[k:k + rows]
+                    k += rows
+                    fill += rows * width
+                if fill + width > self.size:
+                    flush()
+        if piece is not None:
+            flush()
+
+
 def upload_columns(arrays, device, stream):
     """The values of arrays (columns, or tables of columns) as float64 columns
-    in HBM, one after the other; returns (device columns, pinned host copy).
+    in HBM, one after the other; returns (device columns, pinned host memory).
     They go up from pinned host memory, asynchronously on `stream`, while the
     host goes on; a table held row by row is turned into columns on the device."""
     import torch
@@ -270,41 +322,44 @@ def upload_columns(arrays, device, stream):
         by_column = m == 1 or a.flags.f_contiguous
         blocks.append((a.reshape(n) if m == 1 else a.T if by_column else a, 1 if by_column else m, n * m))
     total = sum(size for _, _, size in blocks)
-    pinned = torch.empty(total, dtype=torch.float64, pin_memory=True)
-    ctx = nat.context()
     with on(stream):
         if total <= _SHORT:
+            pinned = torch.empty(total, dtype=torch.float64, pin_memory=True)
             host, at = pinned.numpy(), 0
             for a, m, size in blocks:
                 host[at:at + size].reshape(m, -1)[...] = a.reshape(-1) if m == 1 else a.T
                 at += size
             return pinned.to(device, non_blocking=True), pinned
+        ctx = nat.context()
         d_cols = torch.empty(total, dtype=torch.float64, device=device)
-        at = 0
+        pieces = _Pieces(total, stream)
+        waiting, begin, at = [], 0, 0   # columns that go up together, from `begin` on
+
+        def send_waiting():
+            if waiting:
+                pieces.send(waiting, d_cols[begin:at])
+                waiting.clear()
+
         for a, m, size in blocks:
-            dst = d_cols[at:at + size]
             whole = a.dtype in (np.int64, np.int32)   # go up as they are, become doubles there
-            dtype = getattr(torch, a.dtype.name) if whole else torch.float64
-            up = torch.empty(size, dtype=dtype, device=device) if whole or m > 1 else dst
-            part = pinned[at:at + size].view(dtype)[:size]
-            host = part.numpy()
-            if a.flags.c_contiguous:
-                a = a.reshape(-1)
-                for i in range(0, size, _PIECE):
-                    piece = slice(i, min(i + _PIECE, size))
-                    host[piece] = a[piece]
-                    up[piece].copy_(part[piece], non_blocking=True)
+            if m > 1 or whole:
+                send_waiting()
+                dst = d_cols[at:at + size]
+                up = torch.empty(size, dtype=getattr(torch, a.dtype.name) if whole else torch.float64, device=device)
+                pieces.send([a], up)
+                if m > 1:
+                    rows = up.to(torch.float64)
+                    with ctx.lock:
+                        ctx.prep_columns(rows.data_ptr(), size // m, m, dst.data_ptr(), stream.cuda_stream)
+                else:
+                    dst.copy_(up)
+                at += size
+                begin = at
             else:
-                host.reshape(a.shape)[...] = a
-                up.copy_(part, non_blocking=True)
-            if m > 1:
-                rows = up.to(torch.float64)
-                with ctx.lock:
-                    ctx.prep_columns(rows.data_ptr(), size // m, m, dst.data_ptr(), stream.cuda_stream)
-            elif whole:
-                dst.copy_(up)
-            at += size
-    return d_cols, pinned
+                waiting.append(a)
+                at += size
+        send_waiting()
+    return d_cols, pieces.memory
 
 
 _side_stream = None

@@ -46,3 +46,36 @@ def test_estimates_with_and_without_hints(monkeypatch):
         monkeypatch.setattr(_driver, "_hints_pay", lambda *a: pays)
         got.append(estimate_mi(y, x, lag=[-1, 0, 5], drop_nan=True))
     np.testing.assert_array_equal(got[0], got[1])
+
+
+def test_pinned_memory_is_bounded():
+    import torch
+    from ennemi_amd import _batch, _native as nat
+    most = _batch._PIECES * _batch._PIECE
+    rng = np.random.default_rng(5)
+    table = rng.normal(size=(3 * most // 8 + 5, 8))
+    for arrays in ([table[:, 0].copy(), table, rng.integers(0, 9, 2 * most + 1)], [table[::2, ::2], table.T.copy().T]):
+        st = _batch._stream()
+        d, pinned = _batch.upload_columns(arrays, torch.device("cuda", nat.context().device), st)
+        assert pinned.numel() <= most
+        st.synchronize()
+        want = np.concatenate([np.asarray(a, dtype=np.float64).reshape(len(a), -1).T.reshape(-1) for a in arrays])
+        np.testing.assert_array_equal(d.cpu().numpy(), want)
+
+
+def test_many_columns_share_pieces(monkeypatch):
+    import torch
+    from ennemi_amd import _batch, _native as nat
+    monkeypatch.setattr(_batch, "_PIECE", 1000)
+    monkeypatch.setattr(_batch, "_SHORT", 0)
+    rng = np.random.default_rng(6)
+    cols = [rng.normal(size=n) for n in (1, 999, 1000, 1001, 7, 13, 3000, 1)] + [rng.normal(size=(40, 9))[:, 2]]
+    sent = []
+    send = torch.Tensor.copy_
+    monkeypatch.setattr(torch.Tensor, "copy_", lambda self, *a, **k: (sent.append(len(self)), send(self, *a, **k))[1])
+    d, _ = _batch.upload_columns(cols, torch.device("cuda", nat.context().device), _batch._stream())
+    monkeypatch.undo()
+    torch.cuda.synchronize()
+    want = np.concatenate(cols)
+    np.testing.assert_array_equal(d.cpu().numpy(), want)
+    assert sent == [1000] * (len(want) // 1000) + [len(want) % 1000]
