@@ -120,17 +120,17 @@ def _device_unique(row_sets: Sequence[Sequence[np.ndarray]]) -> List[Tuple[np.nd
 
 # Values of each column that are looked at before the columns go up to be counted
 # directly.
-_SAMPLE = 16
+_SAMPLE = 8
 
 
 def _countable(cols: Sequence[np.ndarray]) -> bool:
     """Whether a few values of every column leave it open that they are whole
     numbers in small ranges.  Two columns of 1,000 halves take 60 us to send up
-    and decline there, 3 here."""
+    and decline there, 1 here; where they are countable, this costs 2."""
     rows = 1
     for c in cols:
         v = c[::len(c) // _SAMPLE | 1].tolist()   # (an odd step: patterns of two or four values)
-        if c.dtype.kind == "f" and any(x % 1 for x in v):   # (NaN for infinities and NaN)
+        if c.dtype.kind == "f" and not all(map(float.is_integer, v)):   # (nor are infinities and NaN)
             return False
         rows *= max(v) - min(v) + 1
     return rows <= nat.COUNT_ROWS_MAX

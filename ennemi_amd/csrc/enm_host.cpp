@@ -2519,14 +2519,10 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
                         d_values, nullptr, U.k0.as<double>(), U.i0.as<int>(), U.k1.as<double>(),
                         U.i1.as<int>(), U.split.as<int>(), &fb, &nl, st);
     if (e == hipSuccess)
-        e = enm_launch_uq_nan(reinterpret_cast<const UqSeg*>(U.tables.as<char>() + o_u1), ncols, d_values,
-                              fb ? U.k1.as<double>() : U.k0.as<double>(), fb ? U.i1.as<int>() : U.i0.as<int>(),
-                              fb ? U.i0.as<int>() : U.i1.as<int>(), st);
-    if (e == hipSuccess)
-        e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(U.tables.as<char>() + o_u1), ncols, tiles1,
-                                fb ? U.k1.as<double>() : U.k0.as<double>(), fb ? U.i1.as<int>() : U.i0.as<int>(),
-                                U.heads.as<int>(), U.ccodes.as<int>(), U.cstarts.as<int64_t>(), U.ccounts.as<int64_t>(),
-                                U.cdist.as<int64_t>(), st);
+        e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(U.tables.as<char>() + o_u1), ncols, tiles1, maxlen1,
+                                d_values, (fb ? U.k1 : U.k0).as<double>(), (fb ? U.i1 : U.i0).as<int>(),
+                                (fb ? U.i0 : U.i1).as<int>(), U.heads.as<int>(), U.ccodes.as<int>(),
+                                U.cstarts.as<int64_t>(), U.ccounts.as<int64_t>(), U.cdist.as<int64_t>(), st);
     std::vector<int64_t> cdist(ncols);
     if (e == hipSuccess) e = hipMemcpyAsync(cdist.data(), U.cdist.p, (size_t)ncols * 8, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -2595,9 +2591,10 @@ int enm_unique_rows(enm_ctx* ctx, const enm_rowset* sets, int32_t n_sets, const 
                                 U.rkeys.as<double>(), nullptr, U.k0.as<double>(), U.i0.as<int>(),
                                 U.k1.as<double>(), U.i1.as<int>(), U.split.as<int>(), &fb, &nl, st);
         if (e == hipSuccess)
-            e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(tb + o_u2), (int)useg2.size(), tiles2,
-                                    fb ? U.k1.as<double>() : U.k0.as<double>(), fb ? U.i1.as<int>() : U.i0.as<int>(),
-                                    U.heads.as<int>(), d_codes, U.rstarts.as<int64_t>(), d_counts, U.rdist.as<int64_t>(), st);
+            e = enm_launch_uq_codes(reinterpret_cast<const UqSeg*>(tb + o_u2), (int)useg2.size(), tiles2, maxlen2, nullptr,
+                                    (fb ? U.k1 : U.k0).as<double>(), (fb ? U.i1 : U.i0).as<int>(), nullptr,
+                                    U.heads.as<int>(), d_codes, U.rstarts.as<int64_t>(), d_counts,
+                                    U.rdist.as<int64_t>(), st);
         if (e == hipSuccess)
             e = hipMemcpyAsync(rdist.data(), U.rdist.p, rdist.size() * 8, hipMemcpyDeviceToHost, st);
         if (e != hipSuccess) return hip_fail(ctx, e, "distinct rows");

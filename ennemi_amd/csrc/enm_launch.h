@@ -158,13 +158,12 @@ hipError_t enm_launch_hint_order(const HintCol* cols, int n_cols, int64_t max_w,
 
 hipError_t enm_launch_group(const GroupTaskDev* tasks, int n_tasks, int64_t stride, int classes, const double* src,
                             int* counts, int64_t* sizes, double* dst, hipStream_t st);
-// Sorted keys have NaN as +inf: the last run of each segment gets its real
-// infinities first and its NaN, marked as such, after them (tmp: as long as sidx).
-hipError_t enm_launch_uq_nan(const UqSeg* segs, int nsegs, const double* values, double* skeys, int* sidx, int* tmp,
-                             hipStream_t st);
-hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, int ntiles, const double* skeys, const int* sidx,
-                               int* tile_heads, int* codes, int64_t* starts, int64_t* counts, int64_t* distinct,
-                               hipStream_t st);
+// Sorted segments of up to maxlen keys: codes by point, run starts and lengths.
+// Where the keys were sorted from `values` (else NULL), which have NaN where the
+// keys are +inf, the order is np.unique's first (tmp: as long as sidx).
+hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, int ntiles, int64_t maxlen, const double* values,
+                               double* skeys, int* sidx, int* tmp, int* tile_heads, int* codes, int64_t* starts,
+                               int64_t* counts, int64_t* distinct, hipStream_t st);
 hipError_t enm_launch_uq_short(const EnmRowsDev& rows, const double* values, int cap, UqShort* out, hipStream_t st);
 hipError_t enm_launch_uq_range(const EnmRowsDev& rows, const double* values, unsigned long long* ext, hipStream_t st);
 hipError_t enm_launch_uq_hist(const EnmRowsDev& rows, const double* values, int keys, unsigned* counts,

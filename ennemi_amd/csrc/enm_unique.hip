@@ -51,15 +51,12 @@ __device__ __forceinline__ int uq_heads(const UqSeg& sg, const double* __restric
 // The sort holds NaN as +inf, in point order among the infinities.  np.unique
 // puts NaN last and keeps every one apart: the points of the last run are laid
 // out again, infinities first, and the keys of the others become NaN, which
-// differ from whatever stands before them.  One workgroup per segment; next to
-// nothing where the greatest key is finite.
-constexpr int UQ_NAN_THREADS = 1024;
-__global__ __launch_bounds__(UQ_NAN_THREADS)
-void uq_nan_kernel(const UqSeg* __restrict__ segs, const double* __restrict__ values, double* __restrict__ skeys,
-                   int* __restrict__ sidx, int* __restrict__ tmp) {
-    constexpr int NW = UQ_NAN_THREADS / ENM_WAVE;
-    __shared__ int s_inf[NW];
-    const UqSeg sg = segs[blockIdx.x];
+// differ from whatever stands before them.  Next to nothing where the greatest
+// key is finite.
+constexpr int UQ_SEG_THREADS = 1024;
+__device__ __forceinline__ void nan_last(const UqSeg& sg, const double* __restrict__ values, double* skeys, int* sidx,
+                                         int* tmp, int* s_wave) {
+    constexpr int NW = UQ_SEG_THREADS / ENM_WAVE;
     skeys += sg.sbase;
     sidx += sg.sbase;
     tmp += sg.sbase;
@@ -74,18 +71,18 @@ void uq_nan_kernel(const UqSeg* __restrict__ segs, const double* __restrict__ va
     int64_t infinities = 0;
     for (int place = 0; place < 2; ++place) {
         int64_t before = 0;   // infinities among the positions done
-        for (int64_t base = lo; base < sg.n; base += UQ_NAN_THREADS) {
+        for (int64_t base = lo; base < sg.n; base += UQ_SEG_THREADS) {
             const int64_t i = base + threadIdx.x;
             const int pt = i < sg.n ? sidx[i] : 0;
             const bool real = i < sg.n && values[sg.src + pt] == INFINITY;
             const unsigned long long m = __builtin_amdgcn_ballot_w64(real);
             __syncthreads();   // the counts of the round before are read
-            if (lane == 0) s_inf[wv] = (int)__popcll(m);
+            if (lane == 0) s_wave[wv] = (int)__popcll(m);
             __syncthreads();
             int64_t mine = before + (int)__popcll(m & ((1ull << lane) - 1ull));
             for (int w = 0; w < NW; ++w) {
-                mine += w < wv ? s_inf[w] : 0;
-                before += s_inf[w];
+                mine += w < wv ? s_wave[w] : 0;
+                before += s_wave[w];
             }
             if (place && i < sg.n) tmp[real ? lo + mine : lo + infinities + (i - lo - mine)] = pt;
         }
@@ -93,13 +90,66 @@ void uq_nan_kernel(const UqSeg* __restrict__ segs, const double* __restrict__ va
         if (infinities == sg.n - lo) return;   // no NaN
     }
     __syncthreads();
-    for (int64_t i = lo + threadIdx.x; i < sg.n; i += UQ_NAN_THREADS) {
+    for (int64_t i = lo + threadIdx.x; i < sg.n; i += UQ_SEG_THREADS) {
         sidx[i] = tmp[i];
         if (i >= lo + infinities) skeys[i] = __builtin_nan("");
     }
 }
 
-// Three passes over tiles of 2,048 sorted positions (one workgroup per segment
+__global__ __launch_bounds__(UQ_SEG_THREADS)
+void uq_nan_kernel(const UqSeg* __restrict__ segs, const double* __restrict__ values, double* skeys, int* sidx,
+                   int* tmp) {
+    __shared__ int s_wave[UQ_SEG_THREADS / ENM_WAVE];
+    nan_last(segs[blockIdx.x], values, skeys, sidx, tmp, s_wave);
+}
+
+// Codes, run starts, counts and the number of distinct values of short segments,
+// one workgroup each, 1,024 positions at a time.  Bound by launches, of which a
+// call has four fewer and, in its second stage, three; longer ones are bound by
+// the positions in sequence.  The rows of two columns, both ways: 300 positions
+// 197 us and 225 in passes, 5,000 283 and 311, 16,384 both 370, 30,000 486 and 451.
+constexpr int64_t UQ_SEG_MAX = 16384;
+__global__ __launch_bounds__(UQ_SEG_THREADS)
+void uq_seg_kernel(const UqSeg* __restrict__ segs, const double* __restrict__ values, double* skeys, int* sidx, int* tmp,
+                   int* codes, int64_t* starts, int64_t* counts, int64_t* distinct) {
+    constexpr int NW = UQ_SEG_THREADS / ENM_WAVE;
+    __shared__ int s_wave[NW];
+    const UqSeg sg = segs[blockIdx.x];
+    if (values) {
+        nan_last(sg, values, skeys, sidx, tmp, s_wave);
+        __syncthreads();
+    }
+    skeys += sg.sbase;
+    sidx += sg.sbase;
+    starts += sg.start_off;
+    const int n = (int)sg.n, lane = threadIdx.x & (ENM_WAVE - 1), wv = threadIdx.x / ENM_WAVE;
+    int heads = 0;   // before this round
+    for (int base = 0; base < n; base += UQ_SEG_THREADS) {
+        const int i = base + (int)threadIdx.x;
+        const bool head = i < n && (i == 0 || skeys[i] != skeys[i - 1]);
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(head);
+        __syncthreads();   // the counts of the round before are read
+        if (lane == 0) s_wave[wv] = (int)__popcll(m);
+        __syncthreads();
+        int rank = heads + (int)__popcll(m & ((2ull << lane) - 1ull)) - 1;
+        for (int w = 0; w < NW; ++w) {
+            rank += w < wv ? s_wave[w] : 0;
+            heads += s_wave[w];
+        }
+        if (i < n) {
+            codes[sg.code_off + sidx[i]] = rank;
+            if (head) starts[rank] = i;
+        }
+    }
+    if (threadIdx.x == 0) {
+        starts[heads] = n;
+        distinct[sg.slot] = heads;
+    }
+    __syncthreads();
+    for (int r = threadIdx.x; r < heads; r += UQ_SEG_THREADS) counts[sg.count_off + r] = starts[r + 1] - starts[r];
+}
+
+// Longer segments: three passes over tiles of 2,048 sorted positions (one workgroup per segment
 // walked its tiles in sequence: 1.9 ms for two columns of 1,000,000): the run
 // heads of every tile, their running sums per segment, then codes (by point)
 // and run starts.
@@ -348,17 +398,17 @@ __global__ void uq_key_kernel(const UqRowKey* __restrict__ rk, int n_rk, const i
 
 }  // namespace
 
-hipError_t enm_launch_uq_nan(const UqSeg* segs, int nsegs, const double* values, double* skeys, int* sidx, int* tmp,
-                             hipStream_t st) {
+hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, int ntiles, int64_t maxlen, const double* values,
+                               double* skeys, int* sidx, int* tmp, int* tile_heads, int* codes, int64_t* starts,
+                               int64_t* counts, int64_t* distinct, hipStream_t st) {
     if (nsegs <= 0) return hipSuccess;
-    hipLaunchKernelGGL(uq_nan_kernel, dim3(nsegs), dim3(UQ_NAN_THREADS), 0, st, segs, values, skeys, sidx, tmp);
-    return hipGetLastError();
-}
-
-hipError_t enm_launch_uq_codes(const UqSeg* segs, int nsegs, int ntiles, const double* skeys, const int* sidx,
-                               int* tile_heads, int* codes, int64_t* starts, int64_t* counts, int64_t* distinct,
-                               hipStream_t st) {
-    if (nsegs <= 0) return hipSuccess;
+    if (maxlen <= UQ_SEG_MAX) {
+        hipLaunchKernelGGL(uq_seg_kernel, dim3(nsegs), dim3(UQ_SEG_THREADS), 0, st, segs, values, skeys, sidx, tmp,
+                           codes, starts, counts, distinct);
+        return hipGetLastError();
+    }
+    if (values)
+        hipLaunchKernelGGL(uq_nan_kernel, dim3(nsegs), dim3(UQ_SEG_THREADS), 0, st, segs, values, skeys, sidx, tmp);
     hipLaunchKernelGGL(uq_heads_kernel, dim3(ntiles), dim3(UQ_THREADS), 0, st, segs, nsegs, skeys, tile_heads);
     hipLaunchKernelGGL(uq_scan_kernel, dim3(nsegs), dim3(ENM_WAVE), 0, st, segs, tile_heads, starts, distinct);
     hipLaunchKernelGGL(uq_codes_kernel, dim3(ntiles), dim3(UQ_THREADS), 0, st, segs, nsegs, skeys, sidx, tile_heads,

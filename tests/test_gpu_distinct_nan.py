@@ -25,7 +25,7 @@ def _column(n, form, seed):
     return a
 
 
-SIZES = [1, 2, 3, 255, 1023, 1025, 2047, 2049, 8193, 20_000]
+SIZES = [1, 2, 3, 255, 1023, 1025, 2047, 2049, 8193, 16_384, 16_385, 20_000]
 
 
 @pytest.mark.parametrize("n", SIZES)
