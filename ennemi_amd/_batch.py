@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import itertools
 import threading
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -211,8 +212,10 @@ class ArenaBatch:
 
     @property
     def _inst(self) -> List[tuple]:
-        return [(kind, k, int(n), dx, dy, dz, 1, 0, [int(o) for o in offs])
-                for kind, k, ns, dx, dy, dz, cols in self._runs for n, offs in zip(ns, cols)]
+        n_segs, seg_index = self._classes[:2] if self._classes is not None else (itertools.repeat(1), itertools.repeat(0))
+        head = ((kind, k, int(n), dx, dy, dz, [int(o) for o in offs])
+                for kind, k, ns, dx, dy, dz, cols in self._runs for n, offs in zip(ns, cols))
+        return [(*h[:6], int(m), int(first), h[6]) for h, m, first in zip(head, n_segs, seg_index)]
 
     def pack(self):
         inst_arr = (nat.EnmInstance * len(self))()
