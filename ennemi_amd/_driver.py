@@ -409,7 +409,8 @@ def _plan_mi(y, x, lag, k, cond, cond_lag, mask, discrete_x, discrete_y, preproc
     if prep != "host" and _device_prep_eligible(x, y, cond, discrete_x, discrete_y):
         return _plan_mi_device(y, x, lag, k, cond, cond_lag, mask, preprocess, drop_nan,
                                min_lag, max_lag, indices, hints), indices, nvar
-    if prep != "host" and bool(discrete_x) != bool(discrete_y) and _classes_eligible(x, y, cond, discrete_x):
+    if prep != "host" and indices and bool(discrete_x) != bool(discrete_y) and \
+            _classes_eligible(x, y, cond, discrete_x):
         tasks = _plan_classes_device(y, x, lag, k, cond, cond_lag, mask, bool(discrete_x), preprocess, drop_nan,
                                      min_lag, max_lag, indices)
         if tasks is not None:
@@ -829,7 +830,7 @@ def _plan_pairwise(data, k, cond, preprocess, drop_nan, mask, discrete):
     cond_lag = np.full(cond.shape[1], 0) if cond is not None else np.asarray(0)
 
     indices = [(i, j) for i in range(nvar) for j in range(i + 1, nvar)]
-    if len(data) and not np.any(discrete) and _device_prep_arrays((data,) if cond is None else (data, cond), cond):
+    if len(data) and indices and not np.any(discrete) and _device_prep_arrays((data,) if cond is None else (data, cond), cond):
         tasks = _plan_pairwise_device(data, k, cond, preprocess, drop_nan, mask, indices)
         if tasks is not None:
             return tasks, indices, nvar
