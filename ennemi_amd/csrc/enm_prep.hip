@@ -716,7 +716,7 @@ __device__ double seq_sum(const PrepSumDev& sd, const double* v, double mean, in
                 if (at == n_tiles) break;
             }
             const int64_t i = (int64_t)b * SEQ_BLOCK + (int64_t)at * SEQ_TILE + lane;
-            const int slot = __builtin_popcountll(which & ~from);
+            const int slot = __builtin_popcountll(which & ((1ull << at) - 1));   // (`at` has moved since `from`)
             const double x = ((which >> at) & 1) && slot < SEQ_AHEAD ? s_ahead[slot][lane] : v[i < n ? i : n - 1];
             s = seq_add_rows(s, i < n ? seq_term(x, mean, pass) : -0.0);
             ++at;
