@@ -203,6 +203,7 @@ struct Plan {
     int samp_tiles = 0;
     int64_t samp_maxlen = 0, n_samp = 0, n_counts = 0, n_buckets = 0;
     int64_t maxlen = 0;
+    int n512 = 0, n2048 = 0;         // first-stage segments of up to 512 keys, and of 513 to 2048
     int64_t sort_elems = 0;
     int64_t n_col64 = 0, n_col32 = 0, n_perm = 0, n_res64 = 0, n_res32 = 0;
     int64_t psi_tab = 0, psi_n = 0;   // res64 offset of psi(0..psi_n)
@@ -402,6 +403,7 @@ struct Planner {
         group_segs.emplace_back();
         group_pos0.emplace_back();
         int64_t p0 = 0;
+        int other = 0;
         for (int s = 0; s < nseg; ++s) {
             const int64_t len = segmented ? seg_len[I.seg_index + s] : I.n;
             if (len > 0) {
@@ -416,6 +418,7 @@ struct Planner {
                 P.ntiles += (int)((len + ENM_SORT_TILE - 1) / ENM_SORT_TILE);
                 P.sort_elems += len;
                 P.maxlen = std::max(P.maxlen, len);
+                ++(len <= 512 ? P.n512 : len <= 2048 ? P.n2048 : other);
                 group_segs[g].push_back((int)P.segs.size());
                 group_pos0[g].push_back(p0);
                 P.segs.push_back(sg);
@@ -1551,7 +1554,7 @@ int enqueue(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double*
                (rc = chk(enm_launch_sort(tab<SortSeg>(P, P.off_segs), (int)P.segs.size(), P.ntiles, P.maxlen,
                                          arena, nullptr,
                                          W.sk0.as<double>(), W.si0.as<int>(), W.sk1.as<double>(), W.si1.as<int>(),
-                                         W.split.as<int>(), &fb, &nl, st), "sort"))) {
+                                         W.split.as<int>(), &fb, &nl, st, nullptr, P.n512, P.n2048), "sort"))) {
         return rc;
     }
     if ((rc = mark(2))) return rc;

@@ -10,11 +10,12 @@ hipError_t enm_launch_fill_u64(unsigned long long* p, int64_t n, unsigned long l
 hipError_t enm_launch_fill_i32(int* p, int64_t n, int v, hipStream_t st);
 
 // Sorts segments of up to maxlen keys; the sorted runs are in k0, i0 or, with
-// *final_buf 1, in k1, i1.
+// *final_buf 1, in k1, i1.  n512, n2048: how many of them are of at most 512 keys,
+// and of more than that and at most 2048 (for the choice of tiles alone).
 hipError_t enm_launch_sort(const SortSeg* d_segs, int nsegs, int ntiles, int64_t maxlen,
                            const double* arena, const int* iarena, double* k0, int* i0, double* k1, int* i1,
                            int* split, int* final_buf, int* n_launch, hipStream_t st,
-                           const int* skip = nullptr);
+                           const int* skip = nullptr, int n512 = 0, int n2048 = 0);
 
 // Sample sort of the first-stage segments (all at most ENM_SS_MAXLEN keys),
 // laid out straight into the orders that consume them (the first-stage
