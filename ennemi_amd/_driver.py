@@ -409,7 +409,11 @@ def _plan_mi(y, x, lag, k, cond, cond_lag, mask, discrete_x, discrete_y, preproc
     if prep != "host" and _device_prep_eligible(x, y, cond, discrete_x, discrete_y):
         return _plan_mi_device(y, x, lag, k, cond, cond_lag, mask, preprocess, drop_nan,
                                min_lag, max_lag, indices, hints), indices, nvar
-    if prep != "host" and indices and bool(discrete_x) != bool(discrete_y) and \
+    # (One estimate of few rows is prepared sooner on the host: with the default
+    # options 208 and 321 us for 300 rows, 302 and 384 for 3,000, 545 and 541 for
+    # 10,000; without rescaling 177 and 334, 231 and 378, 390 and 509.)
+    few = hints is None and len(indices) == 1 and _rows_kept(y, mask) <= 4096
+    if prep != "host" and indices and not few and bool(discrete_x) != bool(discrete_y) and \
             _classes_eligible(x, y, cond, discrete_x):
         tasks = _plan_classes_device(y, x, lag, k, cond, cond_lag, mask, bool(discrete_x), preprocess, drop_nan,
                                      min_lag, max_lag, indices)
@@ -424,6 +428,10 @@ def _plan_mi(y, x, lag, k, cond, cond_lag, mask, discrete_x, discrete_y, preproc
         xs, ys, zs = _prepare_lagged(params, noise)
         _add_mi_task(tasks, xs, ys, zs, k, discrete_x, discrete_y)
     return tasks, indices, nvar
+
+
+def _rows_kept(y, mask) -> int:
+    return len(y) if mask is None else int(np.count_nonzero(mask))
 
 
 def _device_prep_eligible(x, y, cond, discrete_x: bool, discrete_y: bool) -> bool:
@@ -796,7 +804,7 @@ def pairwise_corr(data, *, k: int = 3, cond=None, mask=None, preprocess: bool = 
 
 
 def _pairwise_mi(data, k, cond, preprocess, drop_nan, mask, discrete, callback):
-    tasks, indices, nvar = _plan_pairwise(data, k, cond, preprocess, drop_nan, mask, discrete)
+    tasks, indices, nvar = _plan_pairwise(data, k, cond, preprocess, drop_nan, mask, discrete, call=True)
     values = tasks.run()
     result = np.full((nvar, nvar), np.nan)
     if indices:
@@ -825,7 +833,26 @@ def plan_pairwise_mi(data, *, k: int = 3, cond=None, mask=None, discrete=False,
     return tasks.batch, indices
 
 
-def _plan_pairwise(data, k, cond, preprocess, drop_nan, mask, discrete):
+def _pairs_sooner_on_host(data, cond, mask, preprocess, drop_nan, n_pairs: int) -> bool:
+    """Whether a call's pairs are prepared sooner on the host: few of them, of few
+    rows (one pair of 300 rows 232 us, on the device 258, of 3,000 rows 346 and
+    345, three pairs of 300 rows 287 and 260; without rescaling, where columns go up
+    as they are, one pair of 30,000 rows 346 and 468, three pairs of 300 rows 178
+    and 250, 15 pairs 274 and 256), or where a column is constant, which the
+    device would find after it has prepared them all."""
+    rows = _rows_kept(data, mask)
+    if not preprocess:
+        return n_pairs < 12 and rows <= 30_000
+    if n_pairs == 1 and rows <= 3000:
+        return True
+    if mask is not None or cond is not None or drop_nan:
+        return False   # (a constant column is prepared like any other)
+    first = data[0]
+    same = np.flatnonzero((first == data[len(data) // 2]) & (first == data[-1]))
+    return any((data[:, c] == first[c]).all() for c in same)
+
+
+def _plan_pairwise(data, k, cond, preprocess, drop_nan, mask, discrete, call: bool = False):
     _check_parameters(data, None, k, cond, mask)
     if (not (np.all(discrete) or np.all(~discrete))) and (cond is not None):
         raise ValueError("Conditioning is not supported with mixed discrete and continuous data. " +
@@ -835,7 +862,9 @@ def _plan_pairwise(data, k, cond, preprocess, drop_nan, mask, discrete):
     cond_lag = np.full(cond.shape[1], 0) if cond is not None else np.asarray(0)
 
     indices = [(i, j) for i in range(nvar) for j in range(i + 1, nvar)]
-    if len(data) and indices and not np.any(discrete) and _device_prep_arrays((data,) if cond is None else (data, cond), cond):
+    if len(data) and indices and not np.any(discrete) and \
+            _device_prep_arrays((data,) if cond is None else (data, cond), cond) and \
+            not (call and _pairs_sooner_on_host(data, cond, mask, preprocess, drop_nan, len(indices))):
         tasks = _plan_pairwise_device(data, k, cond, preprocess, drop_nan, mask, indices)
         if tasks is not None:
             return tasks, indices, nvar
