@@ -256,60 +256,73 @@ class ArenaBatch:
 # matrix product), one that waits for helpers, woken or new, waited 4 ms for them.
 _PIECE = 1 << 18
 # Pieces in use at a time: pinned memory is kept for later calls, so it is bounded
-# whatever the columns take.
-_PIECES = 4
+# (64 MB) whatever the columns take.
+_PIECES = 32
 # Up to so many values go up in one copy, as columns: the host lays out 16,384 in
 # 20 us, what two more copies and the kernel that turns rows into columns take.
 _SHORT = 1 << 14
 
 
 class _Pieces:
-    """Pinned memory in a few pieces, each filled again once its last copy has ended."""
+    """Pinned memory for `total` values, filled piece by piece from its start, or, where
+    they are more than _PIECES pieces, by turns: each quarter of it again once the
+    copies from it have ended."""
 
     def __init__(self, total: int, stream) -> None:
         import torch
-        self.size = min(_PIECE, total)
-        self.memory = torch.empty((min(_PIECES, -(-total // self.size)), self.size), dtype=torch.float64,
-                                  pin_memory=True)
-        self.sent = [None] * len(self.memory)
-        self.at = -1
+        self.size = min(total, _PIECES * _PIECE)
+        self.memory = torch.empty(self.size, dtype=torch.float64, pin_memory=True)
+        self.turns = total > self.size
+        self.sent = [None] * 4   # (with turns) the end of the last copies from each quarter
+        self.at = 0              # where the next piece starts
         self.stream = stream
+
+    def _begin(self) -> int:
+        if self.turns:
+            self.at %= self.size
+            q, rest = divmod(self.at, self.size // 4)
+            if rest == 0 and self.sent[q] is not None:
+                self.sent[q].synchronize()
+        return self.at
+
+    def _end(self, count: int) -> None:
+        import torch
+        self.at += _PIECE if self.turns else count
+        if self.turns and self.at % (self.size // 4) == 0:
+            q = self.at // (self.size // 4) - 1
+            if self.sent[q] is None:
+                self.sent[q] = torch.cuda.Event()
+            self.sent[q].record(self.stream)
 
     def send(self, parts, dst) -> None:
         """The values of parts (1-D, or rows of a table), one after the other, to dst."""
-        import torch
-        piece, host, fill, done = None, None, 0, 0
-
-        def flush():
-            nonlocal piece, done
-            dst[done:done + fill].copy_(piece[:fill], non_blocking=True)
-            if self.sent[self.at] is None:
-                self.sent[self.at] = torch.cuda.Event()
-            self.sent[self.at].record(self.stream)
-            done += fill
-            piece = None
-
+        memory = self.memory.view(dst.dtype)
+        host, scale = memory.numpy(), len(memory) // self.size
+        begin = fill = done = 0
         for a in parts:
-            if a.ndim > 1 and (a.flags.c_contiguous or a.shape[1] > self.size):
+            if a.ndim > 1 and (a.flags.c_contiguous or a.shape[1] > _PIECE):
                 a = np.ascontiguousarray(a).reshape(-1)
             width = 1 if a.ndim == 1 else a.shape[1]
-            k = 0
-            while k < len(a):
-                if piece is None:
-                    self.at = (self.at + 1) % len(self.memory)
-                    if self.sent[self.at] is not None:
-                        self.sent[self.at].synchronize()
-                    piece, fill = self.memory[self.at].view(dst.dtype), 0
-                    host = piece.numpy()
-                rows = min(len(a) - k, (self.size - fill) // width)
+            n, k = len(a), 0
+            while k < n:
+                if fill == 0:
+                    begin = self._begin() * scale
+                rows = min(n - k, (_PIECE - fill) // width)
                 if rows > 0:
-                    host[fill:fill + rows * width].reshape(a[k:k + rows].shape)[...] = a[k:k + rows]
+                    to = host[begin + fill:begin + fill + rows * width]
+                    if width > 1:
+                        to = to.reshape(rows, width)
+                    to[...] = a[k:k + rows]
                     k += rows
                     fill += rows * width
-                if fill + width > self.size:
-                    flush()
-        if piece is not None:
-            flush()
+                if fill + width > _PIECE:
+                    dst[done:done + fill].copy_(memory[begin:begin + fill], non_blocking=True)
+                    self._end(fill)
+                    done += fill
+                    fill = 0
+        if fill > 0:
+            dst[done:done + fill].copy_(memory[begin:begin + fill], non_blocking=True)
+            self._end(fill)
 
 
 def upload_columns(arrays, device, stream):

@@ -48,9 +48,10 @@ def test_estimates_with_and_without_hints(monkeypatch):
     np.testing.assert_array_equal(got[0], got[1])
 
 
-def test_pinned_memory_is_bounded():
+def test_pinned_memory_is_bounded(monkeypatch):
     import torch
     from ennemi_amd import _batch, _native as nat
+    monkeypatch.setattr(_batch, "_PIECE", 4096)
     most = _batch._PIECES * _batch._PIECE
     rng = np.random.default_rng(5)
     table = rng.normal(size=(3 * most // 8 + 5, 8))
