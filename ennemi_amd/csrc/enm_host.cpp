@@ -589,7 +589,7 @@ struct Planner {
             t.ncell = (t.n + t.cell - 1) / t.cell;
             for (int c = 0; c < D; ++c) t.src[c] = cols[c];
             t.slab = slab;
-            const int W = t.cell / ENM_LEAF, ngroup = (t.ncell + 63) / 64;
+            const int ngroup = (t.ncell + 63) / 64;
             t.col = F.n64;
             F.n64 += (int64_t)((t.n + ENM_LEAF - 1) / ENM_LEAF) * D * ENM_LEAF;
             t.box = F.n64;
@@ -600,31 +600,8 @@ struct Planner {
             if (ngroup > 1) F.n64 += (int64_t)((ngroup + 63) / 64) * 2 * D * 64;
             t.perm = F.nperm;
             F.nperm += t.n;
-            // The cell's leaves are halved log2(W) times; every halving goes
-            // to the column cut least so far, counting the cuts that made the
-            // cell.  A column the slab order has sorted comes first.
-            std::vector<double> cuts(D, 0.0);
-            if (t.ncell > 1) {
-                cuts[0] = std::log2(two ? std::max(1.0, (double)t.ncell / per_slab) : (double)t.ncell);
-                if (two) cuts[1] = std::log2((double)std::min(t.ncell, per_slab));
-            }
-            std::vector<int> bits(D, 0);
-            int log_cell = 6;
-            for (int w = 1; w < W; w *= 2) {
-                const int c = (int)(std::min_element(cuts.begin(), cuts.end()) - cuts.begin());
-                cuts[c] += 1.0;
-                ++bits[c];
-                ++log_cell;
-            }
-            int run = log_cell;
-            auto step = [&](int c) {
-                t.dim[t.nstep] = (int8_t)c;
-                t.run[t.nstep++] = (int8_t)run;
-                run -= bits[c];
-            };
-            if (sorted >= 0 && bits[sorted] > 0) { step(sorted); t.presorted = 1; }
-            for (int c = 0; c < D; ++c)
-                if (c != sorted && bits[c] > 0) step(c);
+            t.sorted = sorted;
+            while (ENM_LEAF << t.halvings < t.cell) ++t.halvings;
             const int id = (int)P.trees.size();
             for (int c = 0; c < t.ncell; ++c) F.cells.push_back(CellItem{id, c});
             if (ngroup > 1)

@@ -55,7 +55,7 @@
 // two leaves and the queries).
 constexpr int enm_tree_queries(int D) { return D <= 6 ? 4 : D <= 8 ? 2 : 1; }
 #define ENM_CELL 4096          // points per cell: ENM_LEAF leaves of ENM_LEAF points
-#define ENM_TREE_STEPS 6       // most sorted columns of a cell (one halving of its leaves each at least)
+#define ENM_TREE_STEPS 6       // most sorted columns of a cell (one halving of its points each at least)
 #define ENM_TREE_LISTS 8       // most registers of a neighbour list held across a wave's lanes (64 each)
 // How a kNN group runs (and, on trees, a count group).
 #define ENM_WALK_NONE 0        // key order: plain or brute force
@@ -179,12 +179,8 @@ struct TreeDev {
     int32_t cell;
     int32_t ncell;
     int32_t p0;       // first instance point of the scope (its first position in the slab order, too)
-    // A cell's sorts: step s sorts runs of 1 << run[s] positions by column
-    // dim[s] (the first is skipped when the slab order has it sorted already).
-    int32_t nstep;
-    int32_t presorted;
-    int8_t dim[ENM_TREE_STEPS];
-    int8_t run[ENM_TREE_STEPS];
+    int32_t sorted;   // the column that the slab order has sorted within a cell (-1: none)
+    int32_t halvings; // cuts of a cell into its leaves: log2(cell / ENM_LEAF)
 };
 
 // Tree build work: one cell.
