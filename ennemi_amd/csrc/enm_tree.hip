@@ -16,8 +16,8 @@ namespace {
 // are gathered from the arena in tree order and every leaf's box is taken.
 // (The first column 10^6 times wider than the others, joint entropies of 500,000
 // points in three, four and five columns: 18, 45 and 57 ms with the halvings dealt
-// out evenly, 3.3, 4.9 and 6.3 so; equal widths 2.0, 3.4 and 5.4 ms both ways.  The
-// build of 25 cells in four columns takes 2 us more.)
+// out evenly, 3.3, 4.9 and 6.3 so; equal widths 2.0, 3.4 and 5.4 ms both ways.  To
+// measure the widths takes a cell 3 us of 80.)
 
 constexpr int TB_THREADS = 512;
 
@@ -36,11 +36,18 @@ __device__ __forceinline__ double cell_width(const double* __restrict__ src, con
 __device__ void cell_steps(const TreeDev& T, const double* widths, int* dim, int* run, int* nstep) {
     const int lane = (int)threadIdx.x & (ENM_WAVE - 1);
     double width = lane < T.ncol ? widths[lane] : -1.0;
+    // A column that is not cut yet costs a sort (one cell of 4,096 points 18 us, which
+    // few cells wait for), and is taken up only if it is wider by a factor than the
+    // widest that is; the one sorted already costs none.  Build and kNN of 20,000 and
+    // of 400,000 points in five columns, us: factor 4, 272 and 1800; 2.5, 272 and
+    // 1700; 2, 277 and 1678; 1.5, 293 and 1681.
+    const double least = T.ncell <= 64 ? 0.25 : 0.5;
+    if (lane != T.sorted) width *= least;
     int bits = 0;
     for (int h = 0; h < T.halvings; ++h) {
         const unsigned long long widest = __builtin_amdgcn_ballot_w64(width == wave_ext_f64<true>(width));
         if (lane == __builtin_ctzll(widest)) {
-            width *= 0.5;
+            width *= bits == 0 && lane != T.sorted ? 0.5 / least : 0.5;
             ++bits;
         }
     }
