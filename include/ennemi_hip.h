@@ -375,10 +375,13 @@ int enm_get_stats(enm_ctx* ctx, enm_stats* out);
 /*
  * Tile shapes.  They change how the work is cut, never a result: every
  * radius, count and estimate is the same bits under every shape.
- *   strip_points      the kNN runs on a grid order: the key-sorted points
- *                     cut into strips of this many consecutive points, each
- *                     strip sorted by the second column (0 = plain
- *                     key-sorted order); a multiple of 64 up to 65536;
+ *   strip_points      two joint columns, k < 32 and many points: the kNN runs
+ *                     on a grid order, the key-sorted points cut into strips
+ *                     of this many consecutive points (up to 1024, three of
+ *                     which fit LDS), each strip sorted by the second column.
+ *                     Other spaces, and larger strips, run on box trees
+ *                     whatever the size; 0 = plain key-sorted order for all.
+ *                     A multiple of 64 up to 65536;
  *   waves_per_cu      sizes the persistent grids (1..64);
  *   list_slots        register-list slots of the kNN (4, 8, 16 or 32: at
  *                     least k+1 are used; 0 = the fewest that hold k+1);
@@ -389,8 +392,8 @@ int enm_get_stats(enm_ctx* ctx, enm_stats* out);
  * The planner takes each instance's shape from the context: the shape
  * enm_autotune kept for its (joint dimension class, k+1 class,
  * floor(log2 n)) if there is one, else the default; until enm_set_tuning(_ex)
- * is first called, the default gives instances of three or more joint
- * columns strips of 4096 points.  enm_autotune sweeps
+ * is first called, the default says 4096 (that is, trees) for instances of
+ * three or more joint columns.  enm_autotune sweeps
  * strips {0, 256, ..., 8192}, then waves {8, 16, 32}, then list slots
  * {0, 8, 16}, then items per ticket {0, 1, 2, 4}, each with the best of the
  * ones before (two enm_run_batch calls per shape, the second timed), and
