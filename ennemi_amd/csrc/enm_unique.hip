@@ -76,7 +76,7 @@ __device__ __forceinline__ void nan_last(const UqSeg& sg, const double* __restri
             const int pt = i < sg.n ? sidx[i] : 0;
             const bool real = i < sg.n && values[sg.src + pt] == INFINITY;
             const unsigned long long m = __builtin_amdgcn_ballot_w64(real);
-            __syncthreads();   // the counts of the round before are read
+            __syncthreads();   // the counts of the step before are read
             if (lane == 0) s_wave[wv] = (int)__popcll(m);
             __syncthreads();
             int64_t mine = before + (int)__popcll(m & ((1ull << lane) - 1ull));
@@ -123,12 +123,12 @@ void uq_seg_kernel(const UqSeg* __restrict__ segs, const double* __restrict__ va
     sidx += sg.sbase;
     starts += sg.start_off;
     const int n = (int)sg.n, lane = threadIdx.x & (ENM_WAVE - 1), wv = threadIdx.x / ENM_WAVE;
-    int heads = 0;   // before this round
+    int heads = 0;   // before this step
     for (int base = 0; base < n; base += UQ_SEG_THREADS) {
         const int i = base + (int)threadIdx.x;
         const bool head = i < n && (i == 0 || skeys[i] != skeys[i - 1]);
         const unsigned long long m = __builtin_amdgcn_ballot_w64(head);
-        __syncthreads();   // the counts of the round before are read
+        __syncthreads();   // the counts of the step before are read
         if (lane == 0) s_wave[wv] = (int)__popcll(m);
         __syncthreads();
         int rank = heads + (int)__popcll(m & ((2ull << lane) - 1ull)) - 1;
