@@ -1732,16 +1732,36 @@ bool under_capture(hipStream_t st) {
 
 // A run recorded into the caller's own graph.  It is replayed without this
 // library's knowledge, so its plan gets a workspace of its own, which no other
-// run moves or writes and which lives as long as the plan.
+// run moves or writes and which lives as long as the plan; the tables of a new
+// plan are copied at once, by a stream of their own, not by the replays.
 int record(enm_ctx* ctx, Plan& P, const double* arena, const int* hint, double* out, double* d_eps, int* d_counts,
            hipStream_t st) {
-    if (!P.own_work) P.own_work.reset(new Work());
-    // (Allocations are no part of the capture.)
+    // (Allocations and copies are no part of the capture.)
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipThreadExchangeStreamCaptureMode");
+    int rc = ENM_OK;
+    if (!P.tables.p) {
+        const std::vector<TablePiece> pieces = layout_tables(P);
+        std::vector<char> blob(P.table_bytes);
+        copy_tables(pieces, blob.data());
+        hipStream_t up = nullptr;
+        if (P.tables.ensure(std::max<size_t>(P.table_bytes, 256)) != hipSuccess) {
+            (void)hipGetLastError();
+            rc = fail(ctx, ENM_E_NOMEM, "hipMalloc failed for tables");
+        } else if ((e = hipStreamCreateWithFlags(&up, hipStreamNonBlocking)) != hipSuccess) {
+            rc = hip_fail(ctx, e, "hipStreamCreateWithFlags");
+        } else {
+            e = hipMemcpyAsync(P.tables.p, blob.data(), P.table_bytes, hipMemcpyHostToDevice, up);
+            const hipError_t done = hipStreamSynchronize(up);
+            (void)hipStreamDestroy(up);
+            if (e != hipSuccess || done != hipSuccess)
+                rc = hip_fail(ctx, e != hipSuccess ? e : done, "hipMemcpyAsync(tables)");
+        }
+    }
+    if (!P.own_work) P.own_work.reset(new Work());
     P.work = P.own_work.get();
-    int rc = ensure_workspace(ctx, P);
+    if (!rc) rc = ensure_workspace(ctx, P);
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (!rc) rc = enqueue(ctx, P, arena, hint, out, d_eps, d_counts, st, false);
     P.work = &ctx->work;
@@ -1899,7 +1919,6 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
             return enqueue(ctx, *P, d_arena, d_hint, d_out, d_eps, d_counts, st, timing);
         }
     }
-    if (captured) return fail(ctx, ENM_E_ARG, "a batch is captured only after one of its shape has run");
     std::unique_ptr<Plan> up(new Plan());
     Plan& P = *up;
     P.key = key;
@@ -1912,6 +1931,14 @@ int enm_run_batch_hinted(enm_ctx* ctx, const enm_instance* inst, int32_t n_inst,
     P.work = &ctx->work;
     rc = plan_batch(ctx, P, inst, n_inst, seg_len);
     if (rc) return rc;
+    if (captured) {
+        // (No plan leaves here: their runs may be queued on the stream that is captured.)
+        rc = record(ctx, P, d_arena, d_hint, d_out, d_eps, d_counts, st);
+        if (rc) return rc;
+        ctx->last = up.get();
+        ctx->cache.push_front(std::move(up));
+        return ENM_OK;
+    }
     // Plans past the newest few leave (their runs may still be queued, and one
     // set of tables is kept for the next plan).
     auto evict = [&](size_t keep) {

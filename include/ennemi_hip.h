@@ -137,10 +137,10 @@ const char* enm_last_error(const enm_ctx* ctx);
  *              ROSS; unused slots are 0).
  * `stream` is a hipStream_t (NULL = the legacy default stream); all work is
  * enqueued on it and the call returns without synchronising.  On a stream that
- * the caller captures into a graph of its own, a batch of a shape that has run
- * before is recorded, with device buffers of its own; they live until the
- * context has run four other shapes.  (ENM_E_ARG for other shapes and with
- * ENM_F_GRAPH; no stage times.)
+ * the caller captures into a graph of its own, the batch is recorded, with
+ * device buffers of its own; they live until the context has run or recorded
+ * four other shapes and runs a new one.  (ENM_E_ARG with ENM_F_GRAPH; no stage
+ * times.)
  */
 int enm_run_batch(enm_ctx* ctx,
                   const enm_instance* inst, int32_t n_inst,
